@@ -21,7 +21,7 @@ come from a second, open-loop run with Poisson arrivals at 80 % of that rate
 Reported beside it:
   * the resident relaunch engine (two resident batches relaunched with fresh
     noise; per-stage kernel times from HIP events; the roofline of the
-    dominant kernel, the evaluation GEMM, timed with HIP events on its stream);
+    evaluation's row kernel, timed with HIP events on its stream);
   * the plain single-instance FP64 path (same kernels in FP64, batch 1,
     host-synchronised peel loop) and the served/plain ratio;
   * NMSE against the planted spectrum, the reference decoder's own level at
@@ -47,7 +47,6 @@ sys.path.insert(0, ROOT)
 
 METRIC = "transforms/s + p99 latency @ NMSE≤1e-3: served FP32 vs plain FP64 GPU"
 K1 = dict(q=4, n=50, S=1000, b=6, C=3, R=2, snr_db=10.0)
-PEAK_F16_TFLOPS = 2500.0         # MI355X dense fp16 / bf16 MFMA, TFLOP/s
 PEAK_HBM_GBS = 8000.0            # MI355X HBM3E, GB/s
 # NMSE the reference decoder itself reaches on this workload (median over 8
 # seeds of the CPU oracle, which matches the reference's golden vectors)
@@ -81,20 +80,6 @@ def parse():
 def log(msg, quiet=False):
     if not quiet:
         print(msg, file=sys.stderr, flush=True)
-
-
-def measured_traffic(batch):
-    """HBM bytes per k_eval_mfma launch at this batch size, from the committed
-    rocprofv3 counter summary (FETCH_SIZE and WRITE_SIZE per dispatch, each
-    scaled by what the counter reads for a copy of known size); None if absent."""
-    path = os.path.join(ROOT, "profiles", "k_eval_mfma_k1_traffic.txt")
-    if not os.path.exists(path):
-        return None
-    with open(path) as f:
-        for line in f:
-            if line.startswith("bytes_per_transform"):
-                return float(line.split("=")[1]) * batch
-    return None
 
 
 def cpu_model():
@@ -218,7 +203,7 @@ def serve_open(specs, rate, batch, inflight, budget, rng, warm=256):
 
 def resident_engine(args, E, torch):
     """Two resident batches relaunched with fresh noise (inputs stay in HBM):
-    stage times, the GEMM roofline, per-batch latency."""
+    stage times, the roofline of the evaluation's row kernel, per-batch latency."""
     q, n, S, b, C, R, snr = (K1[k] for k in ("q", "n", "S", "b", "C", "R", "snr_db"))
     rng = np.random.default_rng(args.seed)
     spec_sets = [[E.random_spec(q, n, S, b, C, R, snr, rng=rng) for _ in range(args.batch)] for _ in range(2)]
@@ -257,7 +242,7 @@ def resident_engine(args, E, torch):
     for slot, packed in last.items():
         res = engines[slot].unpack(packed)
         nm += [E.nmse(k, v, sp) for (k, v, _, _), sp in zip(res, spec_sets[slot])]
-    gemm_ms = float(np.mean([m[k0].elapsed_time(m["eval"]) for m in marks]))
+    rows_ms = float(np.mean([m[k0].elapsed_time(m["eval"]) for m in marks]))
     stage_ms = {}
     for rep in range(3):
         ev = {}
@@ -270,20 +255,11 @@ def resident_engine(args, E, torch):
                 stage_ms[x] = stage_ms.get(x, 0.0) + prev.elapsed_time(ev[x][0]) / 3
                 prev = ev[x][0]
     samples = C * (R * (n + 1)) * q ** b                           # B = C * P * Q per transform
-    flops = 8.0 * samples * S * args.batch                         # B*S complex multiply-adds per launch
-    achieved = flops / (gemm_ms / 1e3) / 1e12
-    from qsft_amd.kernels import mfma_mode, mfma_ptb
-    nsp, npt = (S + 31) // 32, (R * (n + 1) + 7) // 8
-    ptb = mfma_ptb(mfma_mode(q), 1, npt)
-    npt_run = ptb * ((npt + ptb - 1) // ptb)
-    # q in {2, 4}: v_smfmac_f32_16x16x64_f16, 32 supports x 16 queries x 16 columns per
-    # instruction (one nonzero of each (Re W, Im W) k-row pair), two fp16 limbs of B
-    mfma_f16 = 2 * 2.0 * C * q ** b * (32 * nsp) * (16 * npt_run) * args.batch
-    roof = {"kernel": "k_eval_smfmac_occ2 (int8 MFMA phase + fp16x2 sparse-MFMA complex GEMM, FP32 accumulation)",
-            "bound": "mfma", "achieved": achieved, "peak": PEAK_F16_TFLOPS, "unit": "TFLOP/s",
-            "frac": achieved / PEAK_F16_TFLOPS, "traffic": measured_traffic(args.batch),
-            "algorithmic_flops_per_launch": flops, "launch_ms": gemm_ms,
-            "mfma_f16_nonzero_executed_tflops": mfma_f16 / (gemm_ms / 1e3) / 1e12}
+    nbytes = 8.0 * samples * args.batch                            # every FP32 sample written once per launch
+    achieved = nbytes / (rows_ms / 1e3) / 1e9
+    roof = {"kernel": "k_fold4_rows (folded terms, inverse [4]*6 transform in LDS and registers, samples written once)",
+            "bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
+            "frac": achieved / PEAK_HBM_GBS, "algorithmic_bytes_per_launch": nbytes, "launch_ms": rows_ms}
     out = {"value": args.batch * steps / elapsed, "ms_per_step": 1e3 * elapsed / steps,
            "latency_ms": {"p50": 1e3 * float(np.percentile(lat, 50)), "p99": 1e3 * float(np.percentile(lat, 99)),
                           "of": "a batch from launch to rows on the host, two batches in flight"},
@@ -363,11 +339,10 @@ def k2_stages(E, torch, quiet):
                 stage[x] = stage.get(x, 0.0) + prev.elapsed_time(ev[x][0]) / reps
                 prev = ev[x][0]
     samples = sum(sp.C * sp.P * sp.Q for sp in specs)
-    flops = 8.0 * sum(sp.C * sp.P * sp.Q * sp.S for sp in specs)
     nm = [E.nmse(k, v, sp) for (k, v, _, _), sp in zip(res, specs)]
     out = {"batch": len(specs), "stage_ms_per_batch": stage,
            "dft_GBps": 16.0 * samples / (stage["dft"] / 1e3) / 1e9,
-           "eval_gemm_TFLOPs": flops / (stage["eval"] / 1e3) / 1e12,
+           "eval_rows_GBps": 8.0 * samples / (stage["eval"] / 1e3) / 1e9,
            "transforms_per_s_stage_sum": len(specs) / (sum(stage.values()) / 1e3),
            "nmse_mean": float(np.mean(nm)), "dft_schedule": K.dft_schedule(20, 3, L.QSFT_F32)[0]}
     log(f"K2 stages: {stage}", quiet)
@@ -413,7 +388,7 @@ def main():
     openl = serve_open(open_specs, 0.8 * value, args.batch, args.inflight, budget, rng)
     log(f"open loop at {0.8 * value:.0f}/s: p50 {openl['p50_ms']:.2f} ms p99 {openl['p99_ms']:.2f} ms", args.quiet)
 
-    # ---- the resident relaunch engine (stages, roofline of the GEMM)
+    # ---- the resident relaunch engine (stages, roofline of the evaluation's row kernel)
     engine, roof, pspecs = resident_engine(args, E, torch)
     log(f"resident relaunch: {engine['value']:.1f} transforms/s; stages {engine['stage_ms_per_batch']}", args.quiet)
 

@@ -53,7 +53,7 @@ enum { QSFT_DEVERR_TABLE_FULL = 1, QSFT_DEVERR_TAG_COLLISION = 2, QSFT_DEVERR_OU
 const char* qsft_last_error(void);
 int qsft_abi_version(void);
 /* sizeof() of the descriptor structs, for FFI layout checks:
- * which = 0 eval, 1 eval_points, 2 dft, 3 assemble, 4 peel, 5 eval_mfma, 6 request, 7 batch sizes. */
+ * which = 0 eval, 1 eval_points, 2 dft, 3 assemble, 4 peel, 5 eval_mfma, 6 request, 7 batch sizes, 8 fold. */
 size_t qsft_sizeof(int which);
 
 /* ------------------------------------------------------------------------
@@ -118,6 +118,59 @@ int qsft_eval_mfma_blocks(const qsft_eval_mfma_desc* host_desc, int* prep_blocks
  * one word per launch. */
 int qsft_eval_mfma(const qsft_eval_mfma_desc* dev_descs, const int32_t* dev_pre_prep, const int32_t* dev_pre_main,
                    int n_inst, int prep_blocks, int main_blocks, int word, void* stream);
+
+/* The same samples through the folded spectrum (FP32 or FP64). With the bin
+ * j_s = M_c^T k_s mod q of every support, <m, k_s> = <l, j_s> + <d_p, k_s> (mod q),
+ * so a coset's samples are the unscaled inverse [q]*b transform of the terms
+ * a_s w^{<d_p, k_s>} summed into their bins. qsft_fold_prep forms the phases
+ * <d_p, k_s> and the bins by an int8 MFMA contraction (exact int32, mod q) and
+ * sorts the supports of each group by bin; qsft_fold_rows folds the terms of each
+ * row into LDS (FP64 sums in ascending s: the same bits on every run) and
+ * transforms them, n_pass launches. Replaces the same reference code as
+ * qsft_eval_cosets. */
+typedef struct qsft_fold_desc {
+    int32_t q, n, b, C, P, S;
+    int32_t n_pad;          /* multiple of 64, >= n                                         */
+    int32_t shared_d;       /* 1: every group has the same delay rows                      */
+    int32_t a_prec;         /* QSFT_F32 / QSFT_F64: type of a                               */
+    int32_t n_pass;         /* row passes (qsft_fold_rows launches), filled by qsft_fold_bind */
+    int32_t pass_d0[QSFT_DFT_MAX_PASSES], pass_d1[QSFT_DFT_MAX_PASSES], pass_ti[QSFT_DFT_MAX_PASSES];
+    int32_t pass_ta[QSFT_DFT_MAX_PASSES], pass_blocks[QSFT_DFT_MAX_PASSES], pass_lds[QSFT_DFT_MAX_PASSES];
+    int32_t tiles;          /* tiles of the first pass per row, tile_bins consecutive bins each */
+    int32_t tile_bins;
+    const int8_t* Mt;       /* [C][b][n_pad], 16-byte aligned                               */
+    const int8_t* D;        /* [C][P][n_pad] ([P][n_pad] when shared_d), 16-byte aligned    */
+    const int8_t* K;        /* [S][n_pad], 16-byte aligned                                  */
+    const void* a;          /* [S] strengths, complex FP32 or FP64, 16-byte aligned         */
+    void* x;                /* [C][P][q^b] complex samples out                              */
+    /* workspace, carved by qsft_fold_bind() */
+    uint8_t* E;             /* [groups][P][16 ceil(S / 16)] phases <d_p, k_s> mod q         */
+    double* as;             /* [C][S] complex strengths in sorted order                     */
+    uint64_t* key;          /* [C][S] bin << 32 | s, sorted                                 */
+    uint32_t* J;            /* [C][S] bins                                                  */
+    int32_t* start;         /* [C][tiles + 1] first sorted position of each tile            */
+} qsft_fold_desc;
+
+size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, int shared_d);
+/* Fills a host descriptor (schedule: k_fold4_rows for q = 4, b in {4, 6}, else the
+ * sub-DFT planner's passes). precision: of x; ws 256-byte aligned. */
+int qsft_fold_bind(qsft_fold_desc* host_desc, int q, int n, int b, int C, int P, int S, int n_pad, int shared_d,
+                   int precision, int a_precision, const int8_t* Mt, const int8_t* D, const int8_t* K, const void* a,
+                   void* x, void* ws, size_t ws_bytes);
+int qsft_fold_blocks(const qsft_fold_desc* host_desc, int* phase_blocks, int* rank_blocks);
+/* Instances of any shape share a prep launch. */
+int qsft_fold_prep(const qsft_fold_desc* dev_descs, const int32_t* dev_pre_phase, const int32_t* dev_pre_rank,
+                   int n_inst, int phase_blocks, int rank_blocks, void* stream);
+/* Row pass `pass` (dev_pre counts pass_blocks). word: low nibble QSFT_F32 / QSFT_F64, bits 8..15 = q, bits
+ * 16..23 = b: all instances of a launch share q, and b too for q = 4 with b in {4, 6} (whole rows in one
+ * launch; b = 0 for a launch of mixed b otherwise). lds_bytes: at least every instance's pass_lds[pass]. */
+int qsft_fold_rows(const qsft_fold_desc* dev_descs, const int32_t* dev_pre, int n_inst, int blocks, int pass, int word,
+                   int lds_bytes, void* stream);
+/* One instance: qsft_fold_bind and every launch, the descriptor passed to the
+ * kernels by value (nothing is uploaded). */
+int qsft_fold_one(int q, int n, int b, int C, int P, int S, int n_pad, int shared_d, int precision, int a_precision,
+                  const int8_t* Mt, const int8_t* D, const int8_t* K, const void* a, void* x, void* ws,
+                  size_t ws_bytes, void* stream);
 
 /* Stage (a) alone: the digits (M_c l + d_p) mod q of every query, written as
  * int8 [C][P][q^b][n_pad] to desc->x (a, K and S are ignored). Replaces the
@@ -420,7 +473,7 @@ int qsft_peel_pack_ordered(const qsft_peel_desc* d, int n_inst, void* dst, int64
  * result dict (qsft/qsft.py:98-281) -- for all groups, repeats and b of one
  * request as the reference's loops do one by one, and for all requests of a
  * batch in the same launches (the reference serves one request per call).
- * Samples and sub-DFTs in FP32 on the matrix cores, working transform, peeling
+ * Samples (folded spectrum) and sub-DFTs in FP32, working transform, peeling
  * and coefficients in FP64; every group shares the request's delay rows.
  *
  * Usage: qsft_batch_create (sizes) -> per request qsft_batch_pack_input into a
@@ -448,7 +501,7 @@ typedef struct qsft_request {
 
 typedef struct qsft_batch_sizes {
     size_t input_bytes;         /* inputs arena: Mt, D, K, a of every request                   */
-    size_t work_bytes;          /* work arena: samples, working transform, energies, B fragments, peel workspace */
+    size_t work_bytes;          /* work arena: samples, working transform, energies, evaluation and peel workspace */
     size_t plan_bytes;          /* descriptors and block prefixes (host plan and device plan)  */
     size_t out_bytes;           /* packed results: header + cap_rows rows of row_stride bytes   */
     int64_t cap_rows;

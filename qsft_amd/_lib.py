@@ -82,6 +82,15 @@ class EvalMfmaDesc(ctypes.Structure):
                 ("Mt", vp), ("D", vp), ("K", vp), ("a", vp), ("Bf", vp), ("x", vp)]
 
 
+class FoldDesc(ctypes.Structure):
+    _fields_ = [("q", i32), ("n", i32), ("b", i32), ("C", i32), ("P", i32), ("S", i32), ("n_pad", i32),
+                ("shared_d", i32), ("a_prec", i32), ("n_pass", i32), ("pass_d0", i32 * 4), ("pass_d1", i32 * 4),
+                ("pass_ti", i32 * 4), ("pass_ta", i32 * 4), ("pass_blocks", i32 * 4), ("pass_lds", i32 * 4),
+                ("tiles", i32), ("tile_bins", i32),
+                ("Mt", vp), ("D", vp), ("K", vp), ("a", vp), ("x", vp),
+                ("E", vp), ("as_", vp), ("key", vp), ("J", vp), ("start", vp)]
+
+
 class Request(ctypes.Structure):
     _fields_ = [("q", i32), ("n", i32), ("b", i32), ("C", i32), ("R", i32), ("S", i32), ("method", i32),
                 ("_pad0", i32), ("cutoff", ctypes.c_double), ("sigma", ctypes.c_double), ("amax", ctypes.c_double),
@@ -94,7 +103,7 @@ class BatchSizes(ctypes.Structure):
 
 
 STRUCTS = {0: EvalDesc, 1: EvalPointsDesc, 2: DftDesc, 3: AssembleDesc, 4: PeelDesc, 5: EvalMfmaDesc, 6: Request,
-           7: BatchSizes}
+           7: BatchSizes, 8: FoldDesc}
 
 # exported symbols (every function declared in include/qsft_amd.h)
 SIGNATURES = {
@@ -107,6 +116,14 @@ SIGNATURES = {
     "qsft_eval_mfma_blocks": (ctypes.c_int, [ctypes.POINTER(EvalMfmaDesc), ctypes.POINTER(ctypes.c_int),
                                              ctypes.POINTER(ctypes.c_int)]),
     "qsft_eval_mfma": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),
+    "qsft_fold_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 6),
+    "qsft_fold_bind": (ctypes.c_int, [ctypes.POINTER(FoldDesc)] + [ctypes.c_int] * 10 + [vp] * 6 + [ctypes.c_size_t]),
+    "qsft_fold_blocks": (ctypes.c_int, [ctypes.POINTER(FoldDesc), ctypes.POINTER(ctypes.c_int),
+                                        ctypes.POINTER(ctypes.c_int)]),
+    "qsft_fold_prep": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),
+    "qsft_fold_rows": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                      vp]),
+    "qsft_fold_one": (ctypes.c_int, [ctypes.c_int] * 10 + [vp] * 6 + [ctypes.c_size_t, vp]),
     "qsft_query_digits_blocks": (ctypes.c_int, [ctypes.POINTER(EvalDesc)]),
     "qsft_query_digits": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int, vp]),
     "qsft_eval_points_blocks": (ctypes.c_int, [ctypes.POINTER(EvalPointsDesc)]),

@@ -34,6 +34,7 @@ extern "C" size_t qsft_sizeof(int which) {
         case 5: return sizeof(qsft_eval_mfma_desc);
         case 6: return sizeof(qsft_request);
         case 7: return sizeof(qsft_batch_sizes);
+        case 8: return sizeof(qsft_fold_desc);
         default: return 0;
     }
 }

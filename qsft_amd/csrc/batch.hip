@@ -5,7 +5,7 @@
 // A batch is created from request shapes (sizes only), its inputs are packed
 // into a host staging arena, it is bound to caller-owned device arenas
 // (inputs, work buffers, plan) and an output buffer, and each launch enqueues
-//   upload (optional) -> eval prep + GEMM -> sub-DFTs -> assemble + noise ->
+//   upload (optional) -> samples (fold) -> sub-DFTs -> assemble + noise ->
 //   peel passes 0 .. fuse_from-1 -> fused passes fuse_from .. max_iter-1 ->
 //   (tail stream) finalize -> pack in first-detection order
 // through the library's own entry points. Nothing here allocates device
@@ -17,7 +17,7 @@
 #include <map>
 #include <new>
 #include <thread>
-#include <tuple>
+#include <utility>
 #include <vector>
 
 #include "qsft_common.h"
@@ -44,7 +44,7 @@ struct ReqLayout {
     // inside the request's input block
     size_t mt, d, kraw, a, in_size;
     // inside the request's work block
-    size_t x, u, en, bf, ws, k, work_size, ws_bytes, bf_bytes;
+    size_t x, u, en, fw, ws, k, work_size, ws_bytes, fw_bytes;
     // block offsets in the arenas
     size_t in_off, work_off;
 };
@@ -70,39 +70,19 @@ bool layout_of(const qsft_request& r, int max_iter, ReqLayout* L) {
     l.a = o;  o += al256((size_t)r.S * 16);
     l.in_size = o;
     const size_t cells = (size_t)r.C * l.P * Q;
-    l.bf_bytes = qsft_eval_mfma_workspace_bytes(1, l.P, r.S);
+    l.fw_bytes = qsft_fold_workspace_bytes(r.q, r.b, r.C, l.P, r.S, 1);
     l.ws_bytes = qsft_peel_workspace_bytes(r.q, r.n, r.b, r.C, l.P, max_iter, 0);
-    if (l.bf_bytes == 0 || l.ws_bytes == 0) return false;
+    if (l.fw_bytes == 0 || l.ws_bytes == 0) return false;
     o = 0;
     l.x = o;  o += al256(cells * 8);
     l.u = o;  o += al256(cells * 16);
     l.en = o; o += l.energy ? al256((size_t)r.C * Q * 8) : 0;
-    l.bf = o; o += al256(l.bf_bytes);
+    l.fw = o; o += al256(l.fw_bytes);
     l.ws = o; o += al256(l.ws_bytes);
     l.k = o;  o += al256((size_t)r.S * l.n_pad);                 // K [S][n_pad], staged on the device
     l.work_size = o;
     *L = l;
     return true;
-}
-
-int mfma_mode_of(int q) {
-    if (q == 2 || q == 4) return 0;
-    return (q & (q - 1)) == 0 ? 1 : 2;
-}
-
-int mfma_ptb_of(int mode, int nkb, int npt) {
-    if (mode != 0 || nkb != 1) return 8;
-    const int groups = (npt + 7) / 8;
-    const int per = (npt + groups - 1) / groups;
-    return per < 5 ? 5 : per;
-}
-
-int mfma_bexp_of(double amax) {
-    if (!(amax > 0.0)) return 0;
-    int e = 0;
-    frexp(amax, &e);
-    int v = 14 - e;
-    return v < -100 ? -100 : (v > 100 ? 100 : v);
 }
 
 // Support digits arrive as the reference holds them, locq [n][S]; the
@@ -136,7 +116,7 @@ __global__ __launch_bounds__(256) void k_stage_support(const StageDesc* __restri
     }
 }
 
-struct MfmaLaunch { size_t desc, pre_prep, pre_main; int n, prep_blocks, main_blocks, word; };
+struct FoldLaunch { size_t pre; int blocks, pass, word, lds; };
 struct Rows4Launch { size_t desc, pre; int n, blocks, word; };
 struct DftLaunch { size_t desc, pre[QSFT_DFT_MAX_PASSES]; int n, npass, blocks[QSFT_DFT_MAX_PASSES],
                    lds[QSFT_DFT_MAX_PASSES], word; };
@@ -154,7 +134,9 @@ struct Batch {
     char* plan_dev = nullptr;
     void* out = nullptr;
     bool bound = false, launched = false;
-    std::vector<MfmaLaunch> mfma;
+    size_t fold_desc = 0, fold_pre_phase = 0, fold_pre_rank = 0;
+    int fold_phase = 0, fold_rank = 0;
+    std::vector<FoldLaunch> fold;
     std::vector<Rows4Launch> rows4;
     std::vector<DftLaunch> dft;
     size_t asm_desc = 0, asm_pre = 0;
@@ -204,7 +186,7 @@ int build_plan(Batch& B, bool write) {
     const uintptr_t in_base = write ? (uintptr_t)B.in_dev : kFakeBase;
     const uintptr_t work_base = write ? (uintptr_t)B.work_dev : kFakeBase;
     PlanWriter W{B.plan_host, write};
-    B.mfma.clear();
+    B.fold.clear();
     B.rows4.clear();
     B.dft.clear();
     auto in_ptr = [&](int i, size_t off) { return (void*)(in_base + B.lay[i].in_off + off); };
@@ -232,49 +214,50 @@ int build_plan(Batch& B, bool write) {
         B.stage_pre = W.prefix(sb, &B.stage_blocks);
     }
 
-    // ---- stage (a)+(b): matrix-core evaluation, grouped by kernel variant
-    std::map<std::tuple<int, int, int, int>, std::vector<int>> eg;
-    for (int i = 0; i < nreq; ++i) {
-        const qsft_request& r = B.req[i];
-        const int nkb = B.lay[i].n_pad / 64, mode = mfma_mode_of(r.q);
-        eg[std::make_tuple(nkb, mode, mfma_ptb_of(mode, nkb, (B.lay[i].P + 7) / 8),
-                           (int)qsft::mfma_wide(r.q, r.b, B.lay[i].n_pad))].push_back(i);
-    }
-    for (auto& kv : eg) {
-        const int nkb = std::get<0>(kv.first), mode = std::get<1>(kv.first), ptb = std::get<2>(kv.first);
-        const int wide = std::get<3>(kv.first);
-        std::vector<qsft_eval_mfma_desc> descs;
-        std::vector<int> prep, mainb;
-        for (int i : kv.second) {
+    // ---- stage (a)+(b): samples through the folded spectrum; one prep for all
+    // requests, row passes per q (and per b for the whole-row kernel), each
+    // over the whole descriptor array with zero blocks for the others
+    {
+        std::map<std::pair<int, int>, std::vector<int>> groups;
+        std::vector<qsft_fold_desc> descs(nreq);
+        std::vector<int> phase(nreq), rank(nreq);
+        for (int i = 0; i < nreq; ++i) {
             const qsft_request& r = B.req[i];
             const ReqLayout& l = B.lay[i];
-            qsft_eval_mfma_desc d{};
-            d.q = r.q; d.n = r.n; d.b = r.b; d.C = r.C; d.P = l.P; d.S = r.S; d.n_pad = l.n_pad;
-            d.nsb = (r.S + 15) / 16; d.npt = (l.P + 7) / 8; d.shared_d = 1; d.bexp = mfma_bexp_of(r.amax);
-            d.ptb = ptb;
-            d.Mt = (const int8_t*)in_ptr(i, l.mt);
-            d.D = (const int8_t*)in_ptr(i, l.d);
-            d.K = (const int8_t*)work_ptr(i, l.k);
-            d.a = (const double*)in_ptr(i, l.a);
-            d.Bf = (uint16_t*)work_ptr(i, l.bf);
-            d.x = work_ptr(i, l.x);
-            int pb = 0, mb = 0;
-            if (qsft_eval_mfma_blocks(&d, &pb, &mb) != 0) {
+            const int rc = qsft_fold_bind(&descs[i], r.q, r.n, r.b, r.C, l.P, r.S, l.n_pad, 1, QSFT_F32, QSFT_F64,
+                                          (const int8_t*)in_ptr(i, l.mt), (const int8_t*)in_ptr(i, l.d),
+                                          (const int8_t*)work_ptr(i, l.k), in_ptr(i, l.a), work_ptr(i, l.x),
+                                          work_ptr(i, l.fw), l.fw_bytes);
+            if (rc != QSFT_OK) return rc;
+            if (qsft_fold_blocks(&descs[i], &phase[i], &rank[i]) != 0) {
                 qsft_set_error("qsft_batch: bad evaluation shape");
                 return QSFT_ERR_ARG;
             }
-            descs.push_back(d);
-            prep.push_back(pb);
-            mainb.push_back(mb);
+            groups[{r.q, (r.q == 4 && (r.b == 4 || r.b == 6)) ? r.b : 0}].push_back(i);
         }
-        MfmaLaunch L{};
-        L.desc = W.put(descs.data(), descs.size() * sizeof(qsft_eval_mfma_desc));
-        L.pre_prep = W.prefix(prep, &L.prep_blocks);
-        L.pre_main = W.prefix(mainb, &L.main_blocks);
-        if (L.prep_blocks < 0 || L.main_blocks < 0) { qsft_set_error("qsft_batch: launch too large"); return QSFT_ERR_ARG; }
-        L.n = (int)descs.size();
-        L.word = (nkb << 4) | (mode << 8) | (wide << 11) | (ptb << 12);
-        B.mfma.push_back(L);
+        B.fold_desc = W.put(descs.data(), descs.size() * sizeof(qsft_fold_desc));
+        B.fold_pre_phase = W.prefix(phase, &B.fold_phase);
+        B.fold_pre_rank = W.prefix(rank, &B.fold_rank);
+        if (B.fold_phase < 0 || B.fold_rank < 0) { qsft_set_error("qsft_batch: launch too large"); return QSFT_ERR_ARG; }
+        for (auto& kv : groups) {
+            int npass = 0;
+            for (int i : kv.second) npass = descs[i].n_pass > npass ? descs[i].n_pass : npass;
+            for (int p = 0; p < npass; ++p) {
+                std::vector<int> bl(nreq, 0);
+                FoldLaunch L{};
+                L.lds = 16;
+                for (int i : kv.second) {
+                    if (p >= descs[i].n_pass) continue;
+                    bl[i] = descs[i].pass_blocks[p];
+                    L.lds = descs[i].pass_lds[p] > L.lds ? descs[i].pass_lds[p] : L.lds;
+                }
+                L.pre = W.prefix(bl, &L.blocks);
+                if (L.blocks < 0) { qsft_set_error("qsft_batch: launch too large"); return QSFT_ERR_ARG; }
+                L.pass = p;
+                L.word = QSFT_F32 | (kv.first.first << 8) | (kv.first.second << 16);
+                B.fold.push_back(L);
+            }
+        }
     }
 
     // ---- stage (c): sub-DFTs in place on x (whole-row kernel for q = 4, b in {4, 6})
@@ -643,9 +626,12 @@ int enqueue(Batch* B, int upload, const void* input_host, uint64_t seed_offset, 
         e = hipGetLastError();
         if (e != hipSuccess) return qsft_hip_status(e, "qsft_batch_launch(stage)");
     }
-    for (const MfmaLaunch& L : B->mfma) {
-        rc = qsft_eval_mfma((const qsft_eval_mfma_desc*)(P + L.desc), (const int32_t*)(P + L.pre_prep),
-                            (const int32_t*)(P + L.pre_main), L.n, L.prep_blocks, L.main_blocks, L.word, st);
+    const qsft_fold_desc* fd = (const qsft_fold_desc*)(P + B->fold_desc);
+    rc = qsft_fold_prep(fd, (const int32_t*)(P + B->fold_pre_phase), (const int32_t*)(P + B->fold_pre_rank),
+                        (int)B->req.size(), B->fold_phase, B->fold_rank, st);
+    if (rc != QSFT_OK) return rc;
+    for (const FoldLaunch& L : B->fold) {
+        rc = qsft_fold_rows(fd, (const int32_t*)(P + L.pre), (int)B->req.size(), L.blocks, L.pass, L.word, L.lds, st);
         if (rc != QSFT_OK) return rc;
     }
     for (const Rows4Launch& L : B->rows4) {

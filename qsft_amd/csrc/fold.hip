@@ -1,0 +1,593 @@
+// Stage (a)+(b), coset evaluation through the folded spectrum.
+//
+// Every query of group c is m = (M_c l + d_p) mod q, and mod q is a ring
+// homomorphism, so its phase against a support vector splits exactly:
+//   <m, k_s> = <l, M_c^T k_s> + <d_p, k_s>   (mod q).
+// The first product depends on k_s only through its bin j_s = M_c^T k_s mod q,
+// so the q^b samples of a coset are
+//   x[c][p][l] = sum_j w^{<l, j>} F[c][p][j],
+//   F[c][p][j] = sum over j_s = j of a_s w^{<d_p, k_s>},
+// the unscaled inverse [q]*b transform of the S terms folded into their bins:
+// S + Q b (q - 1) operations a row where the sum over every support at every
+// query takes S Q. Every sample is still the whole sum of a_s w^{<m, k_s>};
+// terms and bin sums are formed in FP64 and rounded once.
+//
+//   * k_fold_phase: the int8 contraction K . [D; M]^T on
+//     v_mfma_i32_16x16x64_i8 (exact int32), then mod q: the phases
+//     E[p][s] = <d_p, k_s> as bytes, and the bins j_s of every group from the
+//     b products with M_c^T.
+//   * k_fold_rank: per group the supports sorted by (bin, s), each at its rank,
+//     counted against LDS tiles of the bins: the terms of a bin are adjacent
+//     and always summed in ascending s, so the sums have the same bits on
+//     every run. Also the first sorted position of every tile of the row
+//     kernel.
+//   * k_fold_pass / k_fold4_rows: a workgroup clears a tile of bins of one row
+//     in LDS, adds the tile's terms and runs the
+//     inverse transform over the tile's axes; k_fold4_rows (q = 4, b in
+//     {4, 6}) does the whole row, two digits at a time in registers. Rows
+//     larger than a tile take further k_fold_pass passes in place.
+//
+// The inverse transform is the forward one with the real and imaginary parts
+// swapped on the way in and out, so it shares the forward radix kernels: the
+// fold stores swapped terms and the last pass swaps back.
+//
+// Bound: HBM. A row is written once (8 or 16 bytes a sample) where it fits one
+// tile; nothing else of that order is read. Measured against the sums over
+// every support that these kernels replaced: one q = 4, n = 50, S = 1000,
+// b = 6, 306-row signal in FP64 463 -> 22 us a call, 64 of them in FP32 in one
+// launch 0.91 -> 0.29 ms; q = 20, S = 2000, b = 3, FP32 570 -> 32 us.
+#include <algorithm>
+
+#include "dft_tile.h"
+
+namespace qsft {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+constexpr int kPhaseThreads = 256;   // four waves, 16 supports each
+constexpr int kPhaseTiles = 4;       // 16-row tiles of [D; M] per workgroup
+constexpr int kRankThreads = 1024;
+constexpr int kRankTileKeys = 2048;
+
+__host__ __device__ __forceinline__ int fold_sp(int S) { return (S + 15) / 16 * 16; }
+// tile boundaries ranked with the supports: none where a row is one tile
+__host__ __device__ __forceinline__ int fold_bounds(int tiles) { return tiles > 1 ? tiles + 1 : 0; }
+
+// tab[r] = w^r, exact for q in {2, 4}
+__device__ __forceinline__ void fold_wtable(double2* tab, int q) {
+    for (int r = threadIdx.x; r < q; r += blockDim.x) {
+        double s, c;
+        if (q == 4) {
+            c = (double)((r == 0) - (r == 2));
+            s = (double)((r == 1) - (r == 3));
+        } else {
+            sincospi(2.0 * (double)r / (double)q, &s, &c);
+        }
+        tab[r] = make_double2(c, s);
+    }
+}
+
+// Phases and bins. A workgroup owns 64 supports (one 16-support block per
+// wave) and kPhaseTiles of the instance's 16-row tiles: first the delay-row
+// tiles (of every group that has its own), then one M^T tile per group. The
+// support digits are the A operand (lane 16 g + r: row r, digits 16 g .. +15),
+// the rows the B operand; lane 16 g + r then holds column r, supports
+// 4 g .. 4 g + 3.
+template <typename SRC>
+__global__ __launch_bounds__(kPhaseThreads) void k_fold_phase(const SRC src) {
+    int local;
+    const qsft_fold_desc& d = src.at(blockIdx.x, local);
+    const int q = d.q, b = d.b, C = d.C, P = d.P, S = d.S, n_pad = d.n_pad;
+    const int Sp = fold_sp(S);
+    const int sgroups = (S + 63) / 64;
+    const int tg = local / sgroups, sg = local - tg * sgroups;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int g = lane >> 4, r16 = lane & 15;
+    const int s0 = sg * 64 + wave * 16;
+    if (s0 >= S) return;
+    const int ptiles = (P + 15) / 16;
+    const int dtiles = (d.shared_d ? 1 : C) * ptiles;
+    const ModQ mq((uint32_t)q);
+    const int8_t* __restrict__ krow = d.K + (size_t)min(s0 + r16, S - 1) * n_pad + 16 * g;
+    v4i kf[QSFT_MAX_N / 64];
+#pragma unroll
+    for (int kb = 0; kb < QSFT_MAX_N / 64; ++kb)
+        kf[kb] = (64 * kb < n_pad) ? *reinterpret_cast<const v4i*>(krow + 64 * kb) : v4i{0, 0, 0, 0};
+    for (int tile = tg * kPhaseTiles; tile < min((tg + 1) * kPhaseTiles, dtiles + C); ++tile) {
+        const bool bins = tile >= dtiles;
+        const int c = bins ? tile - dtiles : tile / ptiles;
+        const int p = (bins ? 0 : 16 * (tile - c * ptiles)) + r16;
+        const int rows = bins ? b : P;
+        const int8_t* __restrict__ row =
+            (bins ? d.Mt : d.D) + ((size_t)c * rows + min(p, rows - 1)) * n_pad + 16 * g;
+        v4i e = {0, 0, 0, 0};
+#pragma unroll
+        for (int kb = 0; kb < QSFT_MAX_N / 64; ++kb) {
+            if (64 * kb < n_pad)
+                e = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf[kb], *reinterpret_cast<const v4i*>(row + 64 * kb), e, 0,
+                                                          0, 0);
+        }
+        if (!bins) {
+            uint32_t w = 0;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) w |= mq((uint32_t)e[v]) << (8 * v);
+            if (p < P) *reinterpret_cast<uint32_t*>(d.E + ((size_t)c * P + p) * Sp + s0 + 4 * g) = w;
+        } else {
+            int place = 0;                                         // q^(b - 1 - r16)
+            if (r16 < b) {
+                place = 1;
+                for (int t = r16 + 1; t < b; ++t) place *= q;
+            }
+            int j[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) j[v] = row_sum_i((int)mq((uint32_t)e[v]) * place);
+            const int mine = r16 == 0 ? j[0] : r16 == 1 ? j[1] : r16 == 2 ? j[2] : j[3];
+            if (r16 < 4 && s0 + 4 * g + r16 < S) d.J[(size_t)c * S + s0 + 4 * g + r16] = (uint32_t)mine;
+        }
+    }
+}
+
+// Items of one group: its S supports, then (from the next multiple of 64) the
+// tiles + 1 tile boundaries. An item's rank among the supports by (bin, s) is
+// its sorted position, where its key and strength are written; a boundary's is
+// the number of supports in lower bins. A workgroup ranks 64 items, one per
+// lane; its 16 waves each count a sixteenth of every LDS tile of bins (the
+// scan is a chain of LDS reads: one wave counting all 1000 supports of the
+// headline size took 27 us, sixteen take 5).
+template <typename SRC>
+__global__ __launch_bounds__(kRankThreads) void k_fold_rank(const SRC src) {
+    constexpr int kWaves = kRankThreads / 64;
+    __shared__ __align__(16) uint32_t keys[kRankTileKeys];
+    __shared__ uint32_t part[kWaves][64];
+    int local;
+    const qsft_fold_desc& d = src.at(blockIdx.x, local);
+    const int S = d.S, S64 = (S + 63) / 64 * 64;
+    const int per_c = (S64 + fold_bounds(d.tiles) + 63) / 64;
+    const int c = local / per_c;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int item = (local - c * per_c) * 64 + lane;
+    const bool support = item < S, bound = item >= S64 && item - S64 < fold_bounds(d.tiles);
+    const uint32_t* __restrict__ J = d.J + (size_t)c * S;
+    uint32_t j = 0;
+    if (support) j = J[item];
+    if (bound) j = (uint32_t)(item - S64) * (uint32_t)d.tile_bins;
+    const int upto = item < S64 ? item : 0;                        // equal bins count before this index
+    uint32_t rank = 0;
+    for (int t0 = 0; t0 < S; t0 += kRankTileKeys) {
+        const int tn = min(kRankTileKeys, S - t0);
+        const int share = ((tn + kWaves - 1) / kWaves + 3) & ~3;
+        __syncthreads();                                           // the previous tile is consumed
+        for (int t = threadIdx.x; t < kRankTileKeys; t += kRankThreads) keys[t] = t < tn ? J[t0 + t] : 0xFFFFFFFFu;
+        __syncthreads();
+        const int z = min(tn, (wave + 1) * share);
+#pragma unroll 4
+        for (int t = wave * share; t < z; t += 4) {                // padded keys count nowhere
+            const uint4 k = *reinterpret_cast<const uint4*>(keys + t);
+            const int at = t0 + t;
+            rank += k.x < j + (at < upto ? 1u : 0u) ? 1u : 0u;
+            rank += k.y < j + (at + 1 < upto ? 1u : 0u) ? 1u : 0u;
+            rank += k.z < j + (at + 2 < upto ? 1u : 0u) ? 1u : 0u;
+            rank += k.w < j + (at + 3 < upto ? 1u : 0u) ? 1u : 0u;
+        }
+    }
+    part[wave][lane] = rank;
+    __syncthreads();
+    if (wave != 0) return;
+    rank = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) rank += part[w][lane];
+    if (support) {
+        d.key[(size_t)c * S + rank] = ((uint64_t)j << 32) | (uint32_t)item;
+        double2 a;
+        if (d.a_prec == QSFT_F32) {
+            const float2 f = reinterpret_cast<const float2*>(d.a)[item];
+            a = make_double2(f.x, f.y);
+        } else {
+            a = reinterpret_cast<const double2*>(d.a)[item];
+        }
+        reinterpret_cast<double2*>(d.as)[(size_t)c * S + rank] = a;
+    }
+    if (bound) d.start[(size_t)c * (d.tiles + 1) + (item - S64)] = (int32_t)rank;
+}
+
+// Adds the terms of sorted positions [lo, hi) of group c, row p to their bins
+// in LDS; add(bin, re, im) adds a sum to a bin. Wave `wave` of `waves` takes an
+// equal share of the positions, moved to the ends of runs (the terms of one
+// bin), so no two waves touch a bin and none waits for another. 64 terms at a
+// time: each lane forms one, a segmented scan over the run (as many steps as
+// the longest run in the block needs) leaves a run's sum in its last lane,
+// which adds it. Equal shares keep a row's time even where one bin holds
+// most of the terms (supports of low weight), and the order of every sum
+// depends on the sorted positions only.
+template <typename F>
+__device__ __forceinline__ void fold_terms(const qsft_fold_desc& d, int c, int p, int lo, int hi, int wave, int waves,
+                                           const double2* tab, F add) {
+    const int lane = threadIdx.x & 63;
+    const int S = d.S, n = hi - lo;
+    if (n <= 0) return;
+    const QSFT_GLOBAL uint64_t* __restrict__ key = gptr(d.key) + (size_t)c * S;
+    const QSFT_GLOBAL gd2* __restrict__ as = reinterpret_cast<const QSFT_GLOBAL gd2*>(gptr(d.as)) + (size_t)c * S;
+    const QSFT_GLOBAL uint8_t* __restrict__ E = gptr(d.E) + ((size_t)(d.shared_d ? 0 : c) * d.P + p) * fold_sp(S);
+    const int first = lo + (int)((int64_t)n * wave / waves), last = lo + (int)((int64_t)n * (wave + 1) / waves);
+    if (first >= last) return;
+    bool started = first == lo;                                    // a run that began before `first` is not ours
+    for (int i0 = first; i0 < hi; i0 += 64) {
+        const int i = i0 + lane;
+        const bool in = i < hi;
+        const uint64_t k = in ? key[i] : ~0ull;
+        const uint32_t kp = (in && i > lo) ? (uint32_t)(key[i - 1] >> 32) : 0xFFFFFFFFu;
+        const gd2 a = in ? as[i] : gd2{0.0, 0.0};
+        const uint32_t j = (uint32_t)(k >> 32);
+        const bool begins = in && j != kp;                         // first term of its bin
+        const uint64_t bm = __ballot(begins);
+        const uint64_t past = __ballot(begins && i >= last);       // the runs of the next share
+        int from = 0, to = min(64, hi - i0);
+        if (!started) from = bm ? __builtin_ctzll(bm) : 64;
+        if (past) to = min(to, (int)__builtin_ctzll(past));
+        if (from < to) {
+            started = true;
+            const bool live = lane >= from && lane < to;
+            double sx = 0.0, sy = 0.0;
+            if (live) {
+                const double2 w = tab[E[(uint32_t)k]];
+                sx = a.x * w.x - a.y * w.y;
+                sy = a.x * w.y + a.y * w.x;
+            }
+            // run head of the lane inside the block (its first live lane for a run continued from the last block)
+            const uint64_t before = bm & (~0ull >> (63 - lane));
+            const int head = max(before ? 63 - (int)__builtin_clzll(before) : 0, from);
+            const int depth = live ? lane - head : 0;
+            for (int off = 1; __ballot(depth >= off); off <<= 1) {
+                const double px = __shfl_up(sx, off), py = __shfl_up(sy, off);
+                if (depth >= off) {
+                    sx += px;
+                    sy += py;
+                }
+            }
+            if (live && (lane + 1 == to || ((bm >> 1) >> lane) & 1)) add(j, sx, sy);
+        }
+        if (past) break;
+    }
+}
+
+// One pass over the axes [d0, d1) of every row (dft.hip's tile scheme). The
+// first pass (FIRST: the innermost axes, so a tile is a contiguous run of
+// bins) folds its terms into the tile; later passes read x. Between passes x
+// holds the swapped parts; the last pass swaps back.
+template <typename T, int QR, bool FIRST, typename SRC>
+__global__ __launch_bounds__(kDftThreads) void k_fold_pass(const SRC src, int pass, int lds_bytes) {
+    using C2 = cplx_t<T>;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ double2 tab[QSFT_MAX_Q];
+    C2* lds = reinterpret_cast<C2*>(smem_raw);
+    int local;
+    const qsft_fold_desc& d = src.at(blockIdx.x, local);
+    if (pass >= d.n_pass) return;
+    const int q = (QR > 0) ? QR : d.q;
+    const int b = d.b;
+    const int d0 = d.pass_d0[pass], d1 = d.pass_d1[pass], ti = d.pass_ti[pass], ta = d.pass_ta[pass];
+    const int mb = d1 - d0;
+    const int Q = ipow(q, b);
+    const int A = ipow(q, d0), M = ipow(q, mb), I = ipow(q, b - d1);
+    const bool contiguous = ti == I;
+    const int ichunks = I / ti;
+    const int tiles_per_row = (A / ta) * ichunks;
+    const int row = local / tiles_per_row;
+    const int rt = local - row * tiles_per_row;
+    const int ac = rt / ichunks;
+    const int64_t base = (int64_t)ac * ta * M * I + (rt - ac * ichunks) * ti;
+    const int E = ta * M * ti;
+    C2* tw = lds + (QR > 0 ? E : 2 * E);
+    if ((int)(((QR > 0 ? E : 2 * E) + (QR > 0 ? 0 : q)) * sizeof(C2)) > lds_bytes) return;   // launch sized too small
+    const FastDiv fti((uint32_t)ti);
+    if constexpr (QR == 0) {
+        for (int r = threadIdx.x; r < q; r += blockDim.x) {
+            double s, c;
+            sincospi(-2.0 * (double)r / (double)q, &s, &c);
+            tw[r].x = (T)c;
+            tw[r].y = (T)s;
+        }
+    }
+    auto goff = [&](int e) -> int64_t {
+        if (contiguous) return base + e;
+        const int m = (int)fti.div((uint32_t)e);
+        return base + (int64_t)m * I + (e - m * ti);
+    };
+    C2* __restrict__ x = reinterpret_cast<C2*>(d.x) + (int64_t)row * Q;
+    if constexpr (FIRST) {
+        const int c = row / d.P;
+        fold_wtable(tab, q);
+        for (int e = threadIdx.x; e < E; e += blockDim.x) lds[e] = C2{(T)0, (T)0};
+        __syncthreads();
+        int lo = 0, hi = d.S;
+        if (d.tiles > 1 && d.S > 0) {
+            const QSFT_GLOBAL int32_t* st = gptr(d.start) + (size_t)c * (d.tiles + 1) + ac;
+            lo = st[0];
+            hi = st[1];
+        }
+        fold_terms(d, c, row - c * d.P, lo, hi, threadIdx.x >> 6, kDftThreads / 64, tab,
+                   [&](uint32_t j, double sx, double sy) {
+                       C2& u = lds[j - (uint32_t)base];            // swapped parts
+                       u.x = (T)((double)u.x + sy);
+                       u.y = (T)((double)u.y + sx);
+                   });
+    } else {
+        for (int e = threadIdx.x; e < E; e += blockDim.x) lds[e] = x[goff(e)];
+    }
+    __syncthreads();
+    const C2* cur = tile_axes<T, QR>(lds, lds + E, E, q, mb, ti, tw);
+    if (pass == d.n_pass - 1) {
+        for (int e = threadIdx.x; e < E; e += blockDim.x) x[goff(e)] = C2{cur[e].y, cur[e].x};
+    } else {
+        for (int e = threadIdx.x; e < E; e += blockDim.x) x[goff(e)] = cur[e];
+    }
+}
+
+// q = 4, whole rows of 4^B samples (k_dft4_rows' register scheme, inverse):
+// 4^B / 16 threads a row, kRows rows a workgroup.
+template <int B>
+constexpr int fold4_rows() { return B == 4 ? 4 : 1; }             // b = 4: four rows of 16 threads fill a wave
+
+template <typename T, int B, typename SRC>
+__global__ __launch_bounds__(fold4_rows<B>() << (2 * B - 4)) void k_fold4_rows(const SRC src) {
+    using C2 = cplx_t<T>;
+    constexpr int Q = 1 << (2 * B), kTpr = Q / 16, kRows = fold4_rows<B>();
+    static_assert(B % 2 == 0 && B >= 4, "even digit count");
+    __shared__ C2 lds_all[kRows][Q + Q / 16];
+    __shared__ double2 tab[4];
+    int local;
+    const qsft_fold_desc& d = src.at(blockIdx.x, local);
+    if (d.q != 4 || d.b != B) return;                              // launched for other shapes
+    const int rows = d.C * d.P;
+    const int sub = threadIdx.x / kTpr, tid = threadIdx.x % kTpr;
+    const int row = local * kRows + sub;
+    const bool live = row < rows;
+    C2* lds = lds_all[sub];
+    fold_wtable(tab, 4);
+#pragma unroll
+    for (int j = 0; j < 17; ++j) lds[tid + j * kTpr] = C2{(T)0, (T)0};
+    __syncthreads();
+    // all waves of the workgroup fold one row after the other
+#pragma unroll 1
+    for (int r = 0; r < kRows; ++r) {
+        const int rr = local * kRows + r;
+        if (rr >= rows) break;
+        const int c = rr / d.P;
+        fold_terms(d, c, rr - c * d.P, 0, d.S, threadIdx.x >> 6, kRows * kTpr / 64, tab,
+                   [&](uint32_t j, double sx, double sy) {
+                       C2& u = lds_all[r][dft4_pad((int)j)];       // swapped parts
+                       u.x = (T)((double)u.x + sy);
+                       u.y = (T)((double)u.y + sx);
+                   });
+    }
+    __syncthreads();
+    C2 v[16];
+#pragma unroll
+    for (int p = 0; p < B / 2; ++p) {
+        if (p > 0) {
+            __syncthreads();                                       // the previous reads of lds are done
+#pragma unroll
+            for (int j = 0; j < 16; ++j) lds[dft4_pad(dft4_index(p - 1, tid, j))] = v[j];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = lds[dft4_pad(dft4_index(p, tid, j))];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) dft4_reg<T>(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);   // digit 2p
+#pragma unroll
+        for (int a = 0; a < 4; ++a) dft4_reg<T>(v[a], v[a + 4], v[a + 8], v[a + 12]);                 // digit 2p+1
+    }
+    if (!live) return;
+    C2* __restrict__ x = reinterpret_cast<C2*>(d.x) + (int64_t)row * Q;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) x[dft4_index(B / 2 - 1, tid, j)] = C2{v[j].y, v[j].x};
+}
+
+}  // namespace qsft
+
+using namespace qsft;
+
+extern "C" void qsft_set_error(const char* msg);
+extern "C" int qsft_hip_status(hipError_t e, const char* where);
+
+namespace {
+
+size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+bool fold_rows4(int q, int b) { return q == 4 && (b == 4 || b == 6); }
+
+bool fold_shape_ok(int q, int n, int b, int C, int P, int S, int n_pad) {
+    if (q < 2 || q > QSFT_MAX_Q || b < 1 || b > QSFT_MAX_B || n < 1 || n > n_pad || n_pad % 64 || n_pad > QSFT_MAX_N ||
+        C < 1 || P < 1 || S < 0)
+        return false;
+    long long Q = 1;
+    for (int i = 0; i < b; ++i) {
+        Q *= q;
+        if (Q > 0x7FFFFFFF) return false;                          // 32-bit bins
+    }
+    return (long long)C * P <= 0x7FFFFFFF && (long long)S + Q + 4 * kRankThreads <= 0x7FFFFFFF;
+}
+
+}  // namespace
+
+// Phases (groups x P x 16-padded S bytes), sorted strengths and keys, bins (C x S), tile
+// starts (a first-pass tile holds at least q bins).
+extern "C" size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, int shared_d) {
+    if (!fold_shape_ok(q, 1, b, C, P, S, 64)) return 0;
+    return al256((size_t)(shared_d ? 1 : C) * P * fold_sp(S)) + al256((size_t)C * S * 16) +
+           al256((size_t)C * S * 8) + al256((size_t)C * S * 4) + al256((size_t)C * (ipow(q, b) / std::min(q, 32) + 2) * 4);
+}
+
+extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int P, int S, int n_pad, int shared_d,
+                              int precision, int a_precision, const int8_t* Mt, const int8_t* D, const int8_t* K,
+                              const void* a, void* x, void* ws, size_t ws_bytes) {
+    if (!h || !fold_shape_ok(q, n, b, C, P, S, n_pad) || (shared_d != 0 && shared_d != 1) ||
+        (precision != QSFT_F32 && precision != QSFT_F64) || (a_precision != QSFT_F32 && a_precision != QSFT_F64) ||
+        (((uintptr_t)Mt | (uintptr_t)D | (uintptr_t)K | (uintptr_t)a) & 15) || ((uintptr_t)ws & 255)) {
+        qsft_set_error("qsft_fold_bind: bad shape or alignment (Mt, D, K, a 16-byte, workspace 256-byte aligned)");
+        return QSFT_ERR_ARG;
+    }
+    if (!ws || ws_bytes < qsft_fold_workspace_bytes(q, b, C, P, S, shared_d)) {
+        qsft_set_error("qsft_fold_bind: workspace too small");
+        return QSFT_ERR_ARG;
+    }
+    qsft_fold_desc d{};
+    d.q = q; d.n = n; d.b = b; d.C = C; d.P = P; d.S = S; d.n_pad = n_pad;
+    d.shared_d = shared_d; d.a_prec = a_precision;
+    d.Mt = Mt; d.D = D; d.K = K; d.a = a; d.x = x;
+    char* w = static_cast<char*>(ws);
+    d.E = reinterpret_cast<uint8_t*>(w);
+    w += al256((size_t)(shared_d ? 1 : C) * P * fold_sp(S));
+    d.as = reinterpret_cast<double*>(w);
+    w += al256((size_t)C * S * 16);
+    d.key = reinterpret_cast<uint64_t*>(w);
+    w += al256((size_t)C * S * 8);
+    d.J = reinterpret_cast<uint32_t*>(w);
+    w += al256((size_t)C * S * 4);
+    d.start = reinterpret_cast<int32_t*>(w);
+    const int Q = ipow(q, b);
+    if (fold_rows4(q, b)) {
+        const int per = b == 4 ? fold4_rows<4>() : fold4_rows<6>();
+        d.n_pass = 1;
+        d.pass_d1[0] = b;
+        d.pass_ti[0] = 1;
+        d.pass_ta[0] = 1;
+        d.pass_blocks[0] = (C * P + per - 1) / per;
+        d.pass_lds[0] = 16;
+        d.tiles = 1;
+        d.tile_bins = Q;
+    } else {
+        qsft_dft_desc s{};                                         // the sub-DFT planner's schedule, innermost first
+        s.q = q; s.b = b; s.rows = C * P; s.in_stride = 1; s.in_row_stride = Q;
+        const int rc = qsft_dft_plan(&s, precision);
+        if (rc != QSFT_OK) return rc;
+        d.n_pass = s.n_pass;
+        for (int p = 0; p < s.n_pass; ++p) {
+            d.pass_d0[p] = s.pass_d0[p];
+            d.pass_d1[p] = s.pass_d1[p];
+            d.pass_ti[p] = s.pass_ti[p];
+            d.pass_ta[p] = s.pass_ta[p];
+            d.pass_blocks[p] = s.pass_blocks[p];
+            d.pass_lds[p] = qsft_dft_lds_bytes(&s, p, precision);
+            if (d.pass_lds[p] < 0) {
+                qsft_set_error("qsft_fold_bind: tile does not fit the LDS");
+                return QSFT_ERR_ARG;
+            }
+        }
+        d.tile_bins = ipow(q, b - s.pass_d0[0]) * s.pass_ta[0];   // whole innermost axes: contiguous bins
+        d.tiles = Q / d.tile_bins;
+    }
+    *h = d;
+    return QSFT_OK;
+}
+
+extern "C" int qsft_fold_blocks(const qsft_fold_desc* h, int* phase_blocks, int* rank_blocks) {
+    if (!h || !phase_blocks || !rank_blocks || !fold_shape_ok(h->q, h->n, h->b, h->C, h->P, h->S, h->n_pad) ||
+        h->tiles < 1)
+        return -1;
+    const long long tiles = (long long)(h->shared_d ? 1 : h->C) * ((h->P + 15) / 16) + h->C;
+    const long long ph = ((h->S + 63) / 64) * ((tiles + kPhaseTiles - 1) / kPhaseTiles);
+    const long long S64 = (h->S + 63) / 64 * 64;
+    const long long rk = h->S == 0 ? 0 : h->C * ((S64 + fold_bounds(h->tiles) + 63) / 64);
+    if (ph > 0x7FFFFFFF || rk > 0x7FFFFFFF) return -1;
+    *phase_blocks = (int)ph;
+    *rank_blocks = (int)rk;
+    return 0;
+}
+
+namespace {
+
+using FoldBatch = DescBatch<qsft_fold_desc>;
+using FoldOne = DescOne<qsft_fold_desc>;
+
+template <typename SRC>
+int launch_prep(const SRC& src, int phase_blocks, int rank_blocks, hipStream_t st) {
+    if (phase_blocks > 0) {
+        hipLaunchKernelGGL(k_fold_phase<SRC>, dim3(phase_blocks), dim3(kPhaseThreads), 0, st, src);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return qsft_hip_status(e, "qsft_fold(phases)");
+    }
+    if (rank_blocks > 0) {
+        hipLaunchKernelGGL(k_fold_rank<SRC>, dim3(rank_blocks), dim3(kRankThreads), 0, st, src);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return qsft_hip_status(e, "qsft_fold(ranks)");
+    }
+    return QSFT_OK;
+}
+
+template <typename T, int QR, typename SRC>
+void launch_pass(const SRC& src, int blocks, int pass, int lds, hipStream_t st) {
+    if (pass == 0)
+        hipLaunchKernelGGL((k_fold_pass<T, QR, true, SRC>), dim3(blocks), dim3(kDftThreads), (size_t)lds, st, src, pass,
+                           lds);
+    else
+        hipLaunchKernelGGL((k_fold_pass<T, QR, false, SRC>), dim3(blocks), dim3(kDftThreads), (size_t)lds, st, src, pass,
+                           lds);
+}
+
+template <typename T, typename SRC>
+int launch_rows(int q, int b, const SRC& src, int blocks, int pass, int lds, hipStream_t st) {
+    if (blocks == 0) return QSFT_OK;
+    if (fold_rows4(q, b)) {
+        if (b == 4)
+            hipLaunchKernelGGL((k_fold4_rows<T, 4, SRC>), dim3(blocks), dim3(fold4_rows<4>() * 16), 0, st, src);
+        else
+            hipLaunchKernelGGL((k_fold4_rows<T, 6, SRC>), dim3(blocks), dim3(fold4_rows<6>() * 256), 0, st, src);
+    } else {
+        switch (q) {
+            case 2: launch_pass<T, 2>(src, blocks, pass, lds, st); break;
+            case 3: launch_pass<T, 3>(src, blocks, pass, lds, st); break;
+            case 4: launch_pass<T, 4>(src, blocks, pass, lds, st); break;
+            case 5: launch_pass<T, 5>(src, blocks, pass, lds, st); break;
+            case 20: launch_pass<T, 20>(src, blocks, pass, lds, st); break;
+            default: launch_pass<T, 0>(src, blocks, pass, lds, st); break;
+        }
+    }
+    return qsft_hip_status(hipGetLastError(), "qsft_fold(rows)");
+}
+
+}  // namespace
+
+extern "C" int qsft_fold_prep(const qsft_fold_desc* d, const int32_t* pre_phase, const int32_t* pre_rank, int n_inst,
+                              int phase_blocks, int rank_blocks, void* stream) {
+    if (!d || !pre_phase || !pre_rank || n_inst < 1 || phase_blocks < 0 || rank_blocks < 0) {
+        qsft_set_error("qsft_fold_prep: bad arguments");
+        return QSFT_ERR_ARG;
+    }
+    const int rc = launch_prep(FoldBatch{d, pre_phase, n_inst}, phase_blocks, 0, (hipStream_t)stream);
+    return rc != QSFT_OK ? rc : launch_prep(FoldBatch{d, pre_rank, n_inst}, 0, rank_blocks, (hipStream_t)stream);
+}
+
+extern "C" int qsft_fold_rows(const qsft_fold_desc* d, const int32_t* pre, int n_inst, int blocks, int pass, int word,
+                              int lds_bytes, void* stream) {
+    const int prec = word & 0xF, q = (word >> 8) & 0xFF, b = (word >> 16) & 0xFF;
+    if (!d || !pre || n_inst < 1 || blocks < 0 || pass < 0 || pass >= QSFT_DFT_MAX_PASSES || lds_bytes < 16 ||
+        lds_bytes > 65536 || (prec != QSFT_F32 && prec != QSFT_F64) || q < 2 || q > QSFT_MAX_Q ||
+        (fold_rows4(q, b) && pass != 0)) {
+        qsft_set_error("qsft_fold_rows: bad arguments");
+        return QSFT_ERR_ARG;
+    }
+    const FoldBatch src{d, pre, n_inst};
+    return prec == QSFT_F32 ? launch_rows<float>(q, b, src, blocks, pass, lds_bytes, (hipStream_t)stream)
+                            : launch_rows<double>(q, b, src, blocks, pass, lds_bytes, (hipStream_t)stream);
+}
+
+extern "C" int qsft_fold_one(int q, int n, int b, int C, int P, int S, int n_pad, int shared_d, int precision,
+                             int a_precision, const int8_t* Mt, const int8_t* D, const int8_t* K, const void* a,
+                             void* x, void* ws, size_t ws_bytes, void* stream) {
+    FoldOne src;
+    int rc = qsft_fold_bind(&src.d, q, n, b, C, P, S, n_pad, shared_d, precision, a_precision, Mt, D, K, a, x, ws,
+                            ws_bytes);
+    if (rc != QSFT_OK) return rc;
+    int pb = 0, rb = 0;
+    if (qsft_fold_blocks(&src.d, &pb, &rb) != 0) {
+        qsft_set_error("qsft_fold_one: launch too large");
+        return QSFT_ERR_ARG;
+    }
+    hipStream_t st = (hipStream_t)stream;
+    rc = launch_prep(src, pb, rb, st);
+    for (int p = 0; rc == QSFT_OK && p < src.d.n_pass; ++p)
+        rc = precision == QSFT_F32 ? launch_rows<float>(q, b, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st)
+                                   : launch_rows<double>(q, b, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st);
+    return rc;
+}

@@ -37,6 +37,30 @@ __device__ __forceinline__ int find_inst(const int32_t* __restrict__ pre, int n_
     return lo;
 }
 
+// Where a kernel's descriptor comes from. DescBatch: an uploaded array with
+// its block prefix, one launch over many instances. DescOne: the descriptor
+// itself as a kernel argument, for calls on one instance, which then need no
+// upload (a blocking copy of a few hundred bytes costs the host about 10 us).
+template <typename D>
+struct DescBatch {
+    const D* descs;
+    const int32_t* pre;
+    int n_inst;
+    __device__ __forceinline__ const D& at(int blk, int& local) const {
+        const int inst = find_inst(pre, n_inst, blk);
+        local = blk - pre[inst];
+        return descs[inst];
+    }
+};
+template <typename D>
+struct DescOne {
+    D d;
+    __device__ __forceinline__ const D& at(int blk, int& local) const {
+        local = blk;
+        return d;
+    }
+};
+
 __host__ __device__ __forceinline__ int ipow(int q, int e) {
     int r = 1;
     for (int i = 0; i < e; ++i) r *= q;

@@ -63,9 +63,9 @@ def strengths_tensor(a, precision, device):
 def evaluate_cosets(q, n, b, Mt, D, Kd, a, precision):
     """x[c][p][l] = sum_s a_s w^{<(M_c l + d_cp) mod q, k_s>} -> [C][P][q^b]."""
     C, P = Mt.shape[0], D.shape[1]
-    code, dt = PRECISIONS[precision]
+    _, dt = PRECISIONS[precision]
     x = torch.empty((C, P, q ** b), dtype=dt, device=Mt.device)
-    K.eval_cosets([dict(q=q, n=n, b=b, C=C, P=P, S=Kd.shape[0], Mt=Mt, D=D, K=Kd, a=a, x=x)], code)
+    K.eval_fold(q, n, b, Mt, D, Kd, a, x)
     return x
 
 

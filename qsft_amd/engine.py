@@ -127,9 +127,10 @@ def random_spec(q, n, S, b, C=3, R=2, snr_db=10.0, rng=None, seed=0, distinct=Tr
 
 
 class Batch:
-    """eval_mode: "mfma" (matrix-core GEMM form, FP32 only; the default for
-    FP32) or "direct" (per-query int8 MFMA phase + VALU w-table accumulation,
-    FP32 or FP64; the plain path). fused_screen: the assembler also writes each
+    """eval_mode: "fold" (the folded spectrum and its inverse transform, FP32 or
+    FP64; the default), "mfma" (matrix-core GEMM form of the direct sum, FP32
+    only) or "direct" (per-query int8 MFMA phase + VALU w-table accumulation,
+    FP32 or FP64). fused_screen: the assembler also writes each
     bin's first-pass energy (transforms with P <= 128), so the peeler's
     zeroton screen does not read U again. sparse_u (with those energies and
     FP32 samples): the assembler writes only the columns above the zeroton
@@ -144,7 +145,7 @@ class Batch:
         self.specs = list(specs)
         self.precision = precision
         if eval_mode is None:
-            eval_mode = "mfma" if precision == "fp32" else "direct"
+            eval_mode = "fold"
         if eval_mode == "mfma" and precision != "fp32":
             raise ValueError("the matrix-core evaluator produces FP32 samples")
         self.eval_mode = eval_mode
@@ -159,7 +160,7 @@ class Batch:
             Mt = dv.Mt_tensor(sp.Ms, sp.b, n_pad, dev)
             Dd = dv.D_tensor([sp.D] * C, n_pad, dev)
             Kd = dv.digits_tensor(sp.locq.T, n_pad, dev)
-            a = dv.strengths_tensor(sp.strengths, "fp64" if eval_mode == "mfma" else precision, dev)
+            a = dv.strengths_tensor(sp.strengths, "fp64" if eval_mode in ("fold", "mfma") else precision, dev)
             x = torch.empty((C, P, Q), dtype=dt, device=dev)
             U = torch.empty((C, Q, P), dtype=torch.complex128, device=dev)      # bin-major for the peeler
             # first-pass column energies come from the assembler when a bin's rows fit one tile
@@ -181,7 +182,10 @@ class Batch:
                            one_bin_waves=one_bin_waves))
             if sparse_u and energy is not None and precision == "fp32":
                 pl[-1]["sparse"] = dict(x=x, sigma=sigma)
-        self.eval = K.EvalMfma(ev) if eval_mode == "mfma" else K.EvalCosets(ev, code)
+        if eval_mode == "fold":
+            self.eval = K.EvalFold(ev, code)
+        else:
+            self.eval = K.EvalMfma(ev) if eval_mode == "mfma" else K.EvalCosets(ev, code)
         self.dft = K.Dft(df, code)
         # packed rows: at most a few per planted support entry (noise adds some), kept
         # in pinned host memory that the pack kernels write directly

@@ -208,6 +208,94 @@ class EvalMfma:
             L.check(lib.qsft_eval_mfma(_vp(dptr), _vp(pp), _vp(pm), n, 0, tm, word, st), "qsft_eval_mfma(main)")
 
 
+class EvalFold:
+    """Coset evaluation through the folded spectrum (the same samples as
+    EvalCosets, FP32 or FP64 out).
+
+    items: dicts q, n, b, C, P, S, Mt, D, K, a (complex64 or complex128 [S]),
+    x (complex [C][P][q^b]), optional shared_d (every group uses the delay
+    rows of group 0). The workspace is allocated here, one per instance.
+    """
+
+    def __init__(self, items, precision):
+        self.ws = []
+        descs, phase, rank = [], [], []
+        for it in items:
+            q, n, b, C, P, S = (it[k] for k in ("q", "n", "b", "C", "P", "S"))
+            if it["x"].dtype != (torch.complex64 if precision == L.QSFT_F32 else torch.complex128):
+                raise TypeError("EvalFold: x does not have the launch's precision")
+            shared = int(bool(it.get("shared_d")))
+            nbytes = lib.qsft_fold_workspace_bytes(q, b, C, P, S, shared)
+            ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=it["x"].device)
+            self.ws.append(ws)
+            d = L.FoldDesc()
+            # 16-byte loads: a view that starts elsewhere is copied
+            t = {k: it[k] if it[k].data_ptr() % 16 == 0 else it[k].clone() for k in ("Mt", "D", "K", "a")}
+            self.ws.append(t)
+            if lib.qsft_fold_bind(ctypes.byref(d), q, n, b, C, P, S, it["Mt"].shape[-1], shared, precision,
+                                  L.QSFT_F32 if it["a"].dtype == torch.complex64 else L.QSFT_F64, _ptr(t["Mt"]),
+                                  _ptr(t["D"]), _ptr(t["K"]), _ptr(t["a"]), _ptr(it["x"]), _ptr(ws),
+                                  nbytes) != L.QSFT_OK:
+                raise ValueError(f"bad eval shape {[it[k] for k in ('q', 'n', 'b', 'C', 'P', 'S')]}")
+            pb, rb = ctypes.c_int(), ctypes.c_int()
+            if lib.qsft_fold_blocks(ctypes.byref(d), ctypes.byref(pb), ctypes.byref(rb)) != 0:
+                raise ValueError(f"bad eval shape {[it[k] for k in ('q', 'n', 'b', 'C', 'P', 'S')]}")
+            descs.append(d)
+            phase.append(pb.value)
+            rank.append(rb.value)
+        # rows: one launch per (q, b) of the whole-row kernel, per q and pass otherwise
+        groups = defaultdict(list)
+        for i, d in enumerate(descs):
+            groups[(d.q, d.b if d.q == 4 and d.b in (4, 6) else 0)].append(i)
+        order = [i for ix in groups.values() for i in ix]
+        sd = [descs[i] for i in order]
+        lists = [[phase[i] for i in order], [rank[i] for i in order]]
+        plan, at = [], 0
+        for (q, b), ix in groups.items():
+            for p in range(max(descs[i].n_pass for i in ix)):
+                bl = [0] * len(order)
+                for k, i in enumerate(ix):
+                    bl[at + k] = descs[i].pass_blocks[p] if p < descs[i].n_pass else 0
+                plan.append((p, precision | (q << 8) | (b << 16), at,
+                             max(descs[i].pass_lds[p] for i in ix if p < descs[i].n_pass)))
+                lists.append(bl)
+            at += len(ix)
+        self.buf, self.dptr, pres, tots = pack(sd, lists, items[0]["x"].device)
+        self.n = len(sd)
+        self.prep = (pres[0], pres[1], tots[0], tots[1])
+        self.rows = [(pres[2 + k], tots[2 + k], p, word, lds) for k, (p, word, _, lds) in enumerate(plan)]
+
+    def launch(self):
+        self.launch_split(lambda: None)
+
+    def launch_split(self, between):
+        """The prep launches (phases, bins, ranks), then `between()`, then the row passes."""
+        st = stream_handle()
+        pp, pr, tp, tr = self.prep
+        L.check(lib.qsft_fold_prep(_vp(self.dptr), _vp(pp), _vp(pr), self.n, tp, tr, st), "qsft_fold_prep")
+        between()
+        for pre, tot, p, word, lds in self.rows:
+            L.check(lib.qsft_fold_rows(_vp(self.dptr), _vp(pre), self.n, tot, p, word, lds, st), "qsft_fold_rows")
+
+
+def eval_fold(q, n, b, Mt, D, K, a, x, shared_d=False):
+    """EvalFold of one instance in one native call, nothing uploaded. The
+    workspace is released on return: torch's allocator reuses it in the order
+    of the current stream, on which the launches are."""
+    C, P, S = Mt.shape[0], D.shape[1], K.shape[0]
+    Mt, D, K, a = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (Mt, D, K, a))
+    nbytes = lib.qsft_fold_workspace_bytes(q, b, C, P, S, int(shared_d))
+    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=x.device)
+    rc = lib.qsft_fold_one(q, n, b, C, P, S, Mt.shape[-1], int(shared_d),
+                           L.QSFT_F32 if x.dtype == torch.complex64 else L.QSFT_F64,
+                           L.QSFT_F32 if a.dtype == torch.complex64 else L.QSFT_F64, Mt.data_ptr(), D.data_ptr(),
+                           K.data_ptr(), a.data_ptr(), x.data_ptr(), ws.data_ptr(), nbytes,
+                           torch.cuda.current_stream().cuda_stream)
+    if rc == L.QSFT_ERR_ARG:
+        raise ValueError(f"bad eval shape {[q, n, b, C, P, S]}")
+    L.check(rc, "qsft_fold_one")
+
+
 class QueryDigits:
     """items: dicts q, n, b, C, P, Mt, D, m (int8 [C][P][q^b][n_pad] out)."""
 

@@ -7,7 +7,7 @@ The reference serves one request per `QSFT.transform` call
 (q, n, b, S, C, R, noise), and a `Server`:
 
   * admits it by its HBM footprint (`qsft_request_footprint`: inputs,
-    samples, FP64 working transform, B fragments, peel workspace) against a
+    samples, FP64 working transform, evaluation and peel workspace) against a
     byte budget; a request that could never fit is rejected at submit
     (`AdmissionError`), one that does not fit now waits in arrival order;
   * keeps up to `max_inflight` batches on the GPU at once, each on its own

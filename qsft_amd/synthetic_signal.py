@@ -3,10 +3,10 @@
 `get_random_subsampled_signal` and `SyntheticSubsampledSignal` keep the
 reference's names, arguments and global-RNG consumption order (support, then
 strengths, then M/D inside the constructor, then per transform the group and
-repeat permutation and the noise draws). Sampling runs on the device: the
-coset queries are generated and evaluated in one kernel (int8 MFMA phase
-contraction + w-table accumulation) instead of the reference's per-query
-complex exponentials on a process pool.
+repeat permutation and the noise draws). Sampling runs on the device: a
+coset's samples come from the support folded into its bins (phases and bins
+by an int8 MFMA contraction) and one inverse transform, instead of the
+reference's per-query complex exponentials on a process pool.
 
 Noise (`noise_mode`): "host" (default) draws the transform-domain noise with
 numpy's legacy RNG in the reference's order, so a seed gives the reference's
