@@ -138,6 +138,9 @@ typedef struct qsft_fold_desc {
     int32_t pass_ta[QSFT_DFT_MAX_PASSES], pass_blocks[QSFT_DFT_MAX_PASSES], pass_lds[QSFT_DFT_MAX_PASSES];
     int32_t tiles;          /* tiles of the first pass per row, tile_bins consecutive bins each */
     int32_t tile_bins;
+    int32_t rpw;            /* q = 4, b in {4, 6}: row sets of one group per workgroup      */
+    int32_t fwd;            /* 1: x receives the rows' sub-transforms (qsft_dft_pass of the *
+                             * samples), formed in the same launch: rows of one tile only  */
     const int8_t* Mt;       /* [C][b][n_pad], 16-byte aligned                               */
     const int8_t* D;        /* [C][P][n_pad] ([P][n_pad] when shared_d), 16-byte aligned    */
     const int8_t* K;        /* [S][n_pad], 16-byte aligned                                  */
@@ -153,17 +156,20 @@ typedef struct qsft_fold_desc {
 
 size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, int shared_d);
 /* Fills a host descriptor (schedule: k_fold4_rows for q = 4, b in {4, 6}, else the
- * sub-DFT planner's passes). precision: of x; ws 256-byte aligned. */
+ * sub-DFT planner's passes). precision: of x; transform: write sub-transforms
+ * instead of samples where a row is one tile (`fwd` of the descriptor says so);
+ * launch_rows: rows (C * P) of all instances of the launch; ws 256-byte aligned. */
 int qsft_fold_bind(qsft_fold_desc* host_desc, int q, int n, int b, int C, int P, int S, int n_pad, int shared_d,
-                   int precision, int a_precision, const int8_t* Mt, const int8_t* D, const int8_t* K, const void* a,
-                   void* x, void* ws, size_t ws_bytes);
+                   int precision, int a_precision, int transform, int launch_rows, const int8_t* Mt, const int8_t* D,
+                   const int8_t* K, const void* a, void* x, void* ws, size_t ws_bytes);
 int qsft_fold_blocks(const qsft_fold_desc* host_desc, int* phase_blocks, int* rank_blocks);
 /* Instances of any shape share a prep launch. */
 int qsft_fold_prep(const qsft_fold_desc* dev_descs, const int32_t* dev_pre_phase, const int32_t* dev_pre_rank,
                    int n_inst, int phase_blocks, int rank_blocks, void* stream);
 /* Row pass `pass` (dev_pre counts pass_blocks). word: low nibble QSFT_F32 / QSFT_F64, bits 8..15 = q, bits
  * 16..23 = b: all instances of a launch share q, and b too for q = 4 with b in {4, 6} (whole rows in one
- * launch; b = 0 for a launch of mixed b otherwise). lds_bytes: at least every instance's pass_lds[pass]. */
+ * launch; b = 0 for a launch of mixed b otherwise); bit 24: the descriptors' fwd (those whole-row launches).
+ * lds_bytes: at least every instance's pass_lds[pass]. */
 int qsft_fold_rows(const qsft_fold_desc* dev_descs, const int32_t* dev_pre, int n_inst, int blocks, int pass, int word,
                    int lds_bytes, void* stream);
 /* One instance: qsft_fold_bind and every launch, the descriptor passed to the

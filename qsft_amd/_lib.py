@@ -86,7 +86,7 @@ class FoldDesc(ctypes.Structure):
     _fields_ = [("q", i32), ("n", i32), ("b", i32), ("C", i32), ("P", i32), ("S", i32), ("n_pad", i32),
                 ("shared_d", i32), ("a_prec", i32), ("n_pass", i32), ("pass_d0", i32 * 4), ("pass_d1", i32 * 4),
                 ("pass_ti", i32 * 4), ("pass_ta", i32 * 4), ("pass_blocks", i32 * 4), ("pass_lds", i32 * 4),
-                ("tiles", i32), ("tile_bins", i32),
+                ("tiles", i32), ("tile_bins", i32), ("rpw", i32), ("fwd", i32),
                 ("Mt", vp), ("D", vp), ("K", vp), ("a", vp), ("x", vp),
                 ("E", vp), ("as_", vp), ("key", vp), ("J", vp), ("start", vp)]
 
@@ -117,7 +117,7 @@ SIGNATURES = {
                                              ctypes.POINTER(ctypes.c_int)]),
     "qsft_eval_mfma": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),
     "qsft_fold_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 6),
-    "qsft_fold_bind": (ctypes.c_int, [ctypes.POINTER(FoldDesc)] + [ctypes.c_int] * 10 + [vp] * 6 + [ctypes.c_size_t]),
+    "qsft_fold_bind": (ctypes.c_int, [ctypes.POINTER(FoldDesc)] + [ctypes.c_int] * 12 + [vp] * 6 + [ctypes.c_size_t]),
     "qsft_fold_blocks": (ctypes.c_int, [ctypes.POINTER(FoldDesc), ctypes.POINTER(ctypes.c_int),
                                         ctypes.POINTER(ctypes.c_int)]),
     "qsft_fold_prep": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),

@@ -124,6 +124,7 @@ struct DftLaunch { size_t desc, pre[QSFT_DFT_MAX_PASSES]; int n, npass, blocks[Q
 struct Batch {
     std::vector<qsft_request> req;
     std::vector<ReqLayout> lay;
+    std::vector<int> transformed;          // per request: its fold launch also does the sub-DFTs
     std::vector<int> sign;                 // detected delay structure per request (+1, -1, 0)
     int max_iter = 15, fuse_from = 3, max_p = 1, max_n_pad = 64;
     qsft_batch_sizes sz{};
@@ -221,14 +222,19 @@ int build_plan(Batch& B, bool write) {
         std::map<std::pair<int, int>, std::vector<int>> groups;
         std::vector<qsft_fold_desc> descs(nreq);
         std::vector<int> phase(nreq), rank(nreq);
+        long long all_rows = 0;
+        for (int i = 0; i < nreq; ++i) all_rows += (long long)B.req[i].C * B.lay[i].P;
+        const int launch_rows = (int)(all_rows < 0x7FFFFFFF ? all_rows : 0x7FFFFFFF);
+        B.transformed.assign(nreq, 0);
         for (int i = 0; i < nreq; ++i) {
             const qsft_request& r = B.req[i];
             const ReqLayout& l = B.lay[i];
             const int rc = qsft_fold_bind(&descs[i], r.q, r.n, r.b, r.C, l.P, r.S, l.n_pad, 1, QSFT_F32, QSFT_F64,
-                                          (const int8_t*)in_ptr(i, l.mt), (const int8_t*)in_ptr(i, l.d),
+                                          1, launch_rows, (const int8_t*)in_ptr(i, l.mt), (const int8_t*)in_ptr(i, l.d),
                                           (const int8_t*)work_ptr(i, l.k), in_ptr(i, l.a), work_ptr(i, l.x),
                                           work_ptr(i, l.fw), l.fw_bytes);
             if (rc != QSFT_OK) return rc;
+            B.transformed[i] = descs[i].fwd;
             if (qsft_fold_blocks(&descs[i], &phase[i], &rank[i]) != 0) {
                 qsft_set_error("qsft_batch: bad evaluation shape");
                 return QSFT_ERR_ARG;
@@ -254,16 +260,19 @@ int build_plan(Batch& B, bool write) {
                 L.pre = W.prefix(bl, &L.blocks);
                 if (L.blocks < 0) { qsft_set_error("qsft_batch: launch too large"); return QSFT_ERR_ARG; }
                 L.pass = p;
-                L.word = QSFT_F32 | (kv.first.first << 8) | (kv.first.second << 16);
+                L.word = QSFT_F32 | (kv.first.first << 8) | (kv.first.second << 16) |
+                         (kv.first.second ? 1 << 24 : 0);          // whole rows: always transformed
                 B.fold.push_back(L);
             }
         }
     }
 
-    // ---- stage (c): sub-DFTs in place on x (whole-row kernel for q = 4, b in {4, 6})
+    // ---- stage (c): sub-DFTs in place on x of the rows that are more than one tile
+    // (whole-row kernel for q = 4, b in {4, 6})
     std::map<int, std::vector<int>> fast, slow;
     for (int i = 0; i < nreq; ++i) {
         const qsft_request& r = B.req[i];
+        if (B.transformed[i]) continue;                            // done with the samples
         if (r.q == 4 && (r.b == 4 || r.b == 6)) fast[r.b].push_back(i);
         else slow[r.q].push_back(i);
     }

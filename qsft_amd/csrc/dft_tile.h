@@ -174,12 +174,25 @@ __device__ __forceinline__ cplx_t<T>* tile_axes(cplx_t<T>* cur, cplx_t<T>* alt, 
     return cur;
 }
 
+// Q = q^b: the forward scale of the last pass (a division in FP64, like numpy's
+// / q**n; a multiply by the rounded reciprocal in FP32)
+template <typename T>
+__device__ __forceinline__ cplx_t<T> dft_scaled(cplx_t<T> v, int Q) {
+    if constexpr (sizeof(T) == 8) return cplx_t<T>{v.x / (double)Q, v.y / (double)Q};
+    const T sc = (T)(1.0 / (double)Q);
+    return cplx_t<T>{v.x * sc, v.y * sc};
+}
+
 // element index of register j of thread tid when the thread holds digits 2p, 2p+1
 __device__ __forceinline__ int dft4_index(int p, int tid, int j) {
     const int lo = 4 * p;
     return ((tid >> lo) << (lo + 4)) | (j << lo) | (tid & ((1 << lo) - 1));
 }
 __device__ __forceinline__ int dft4_pad(int i) { return i + (i >> 4); }
+// dft4_pad(dft4_index(p, tid, j)) = dft4_lds_base(p, tid) + j dft4_lds_step(p):
+// one address per register pass, the 16 elements at immediate offsets
+__device__ __forceinline__ int dft4_lds_base(int p, int tid) { return dft4_pad(dft4_index(p, tid, 0)); }
+__device__ __forceinline__ constexpr int dft4_lds_step(int p) { return p == 0 ? 1 : 17 << (4 * p - 4); }
 
 
 }  // namespace qsft

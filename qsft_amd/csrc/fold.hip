@@ -34,7 +34,7 @@
 // Bound: HBM. A row is written once (8 or 16 bytes a sample) where it fits one
 // tile; nothing else of that order is read. Measured against the sums over
 // every support that these kernels replaced: one q = 4, n = 50, S = 1000,
-// b = 6, 306-row signal in FP64 463 -> 22 us a call, 64 of them in FP32 in one
+// b = 6, 306-row signal in FP64 463 -> 23 us a call, 64 of them in FP32 in one
 // launch 0.91 -> 0.29 ms; q = 20, S = 2000, b = 3, FP32 570 -> 32 us.
 #include <algorithm>
 
@@ -190,35 +190,52 @@ __global__ __launch_bounds__(kRankThreads) void k_fold_rank(const SRC src) {
     if (bound) d.start[(size_t)c * (d.tiles + 1) + (item - S64)] = (int32_t)rank;
 }
 
-// Adds the terms of sorted positions [lo, hi) of group c, row p to their bins
-// in LDS; add(bin, re, im) adds a sum to a bin. Wave `wave` of `waves` takes an
-// equal share of the positions, moved to the ends of runs (the terms of one
+// The terms of one row are added to their bins in LDS by the waves of a
+// workgroup. Wave `wave` of `waves` takes an equal share of the sorted
+// positions [lo, hi) of the group, moved to the ends of runs (the terms of one
 // bin), so no two waves touch a bin and none waits for another. 64 terms at a
 // time: each lane forms one, a segmented scan over the run (as many steps as
 // the longest run in the block needs) leaves a run's sum in its last lane,
 // which adds it. Equal shares keep a row's time even where one bin holds
 // most of the terms (supports of low weight), and the order of every sum
 // depends on the sorted positions only.
-template <typename F>
-__device__ __forceinline__ void fold_terms(const qsft_fold_desc& d, int c, int p, int lo, int hi, int wave, int waves,
-                                           const double2* tab, F add) {
-    const int lane = threadIdx.x & 63;
-    const int S = d.S, n = hi - lo;
-    if (n <= 0) return;
-    const QSFT_GLOBAL uint64_t* __restrict__ key = gptr(d.key) + (size_t)c * S;
-    const QSFT_GLOBAL gd2* __restrict__ as = reinterpret_cast<const QSFT_GLOBAL gd2*>(gptr(d.as)) + (size_t)c * S;
-    const QSFT_GLOBAL uint8_t* __restrict__ E = gptr(d.E) + ((size_t)(d.shared_d ? 0 : c) * d.P + p) * fold_sp(S);
-    const int first = lo + (int)((int64_t)n * wave / waves), last = lo + (int)((int64_t)n * (wave + 1) / waves);
-    if (first >= last) return;
-    bool started = first == lo;                                    // a run that began before `first` is not ours
-    for (int i0 = first; i0 < hi; i0 += 64) {
+//
+// What a lane needs of its position, the same for every row of the group:
+struct Term {
+    uint32_t j, s;       // bin and support
+    gd2 a;               // strength
+    int flags;           // kTermLive | kTermEmit | kTermWhole | lanes back to the run's first live lane
+};
+constexpr int kTermDepth = 63;       // mask of the distance
+constexpr int kTermLive = 64;        // a term of this wave
+constexpr int kTermEmit = 128;       // last lane of the run in the block
+constexpr int kTermWhole = 256;      // ... and the run lies inside the block: its sum is the bin's
+
+struct TermShare {
+    int lo, hi, first, last;
+    bool started;        // a run that began before `first` is another wave's
+    __device__ __forceinline__ TermShare(int lo_, int hi_, int wave, int waves)
+        : lo(lo_), hi(hi_), first(lo_ + (int)((int64_t)(hi_ - lo_) * wave / waves)),
+          last(lo_ + (int)((int64_t)(hi_ - lo_) * (wave + 1) / waves)), started(first == lo_) {}
+    // Loads the block of 64 positions from i0; false once the share has ended.
+    __device__ __forceinline__ bool load(const qsft_fold_desc& d, int c, int i0, Term& t) {
+        const int lane = threadIdx.x & 63;
+        t.flags = 0;
+        t.j = t.s = 0;
+        t.a = gd2{0.0, 0.0};
+        if (i0 >= hi || first >= last) return false;
+        const QSFT_GLOBAL uint64_t* __restrict__ key = gptr(d.key) + (size_t)c * d.S;
+        const QSFT_GLOBAL gd2* __restrict__ as =
+            reinterpret_cast<const QSFT_GLOBAL gd2*>(gptr(d.as)) + (size_t)c * d.S;
         const int i = i0 + lane;
         const bool in = i < hi;
         const uint64_t k = in ? key[i] : ~0ull;
         const uint32_t kp = (in && i > lo) ? (uint32_t)(key[i - 1] >> 32) : 0xFFFFFFFFu;
-        const gd2 a = in ? as[i] : gd2{0.0, 0.0};
-        const uint32_t j = (uint32_t)(k >> 32);
-        const bool begins = in && j != kp;                         // first term of its bin
+        const uint32_t kn = (i + 1 < hi) ? (uint32_t)(key[i + 1] >> 32) : 0xFFFFFFFFu;
+        if (in) t.a = as[i];
+        t.j = (uint32_t)(k >> 32);
+        t.s = (uint32_t)k;
+        const bool begins = in && t.j != kp;                       // first term of its bin
         const uint64_t bm = __ballot(begins);
         const uint64_t past = __ballot(begins && i >= last);       // the runs of the next share
         int from = 0, to = min(64, hi - i0);
@@ -226,28 +243,72 @@ __device__ __forceinline__ void fold_terms(const qsft_fold_desc& d, int c, int p
         if (past) to = min(to, (int)__builtin_ctzll(past));
         if (from < to) {
             started = true;
-            const bool live = lane >= from && lane < to;
-            double sx = 0.0, sy = 0.0;
-            if (live) {
-                const double2 w = tab[E[(uint32_t)k]];
-                sx = a.x * w.x - a.y * w.y;
-                sy = a.x * w.y + a.y * w.x;
+            if (lane >= from && lane < to) {
+                const uint64_t before = bm & (~0ull >> (63 - lane));
+                t.flags = kTermLive | (lane - max(before ? 63 - (int)__builtin_clzll(before) : 0, from));
+                if (lane + 1 == to || t.j != kn) t.flags |= kTermEmit | (before && t.j != kn ? kTermWhole : 0);
             }
-            // run head of the lane inside the block (its first live lane for a run continued from the last block)
-            const uint64_t before = bm & (~0ull >> (63 - lane));
-            const int head = max(before ? 63 - (int)__builtin_clzll(before) : 0, from);
-            const int depth = live ? lane - head : 0;
-            for (int off = 1; __ballot(depth >= off); off <<= 1) {
-                const double px = __shfl_up(sx, off), py = __shfl_up(sy, off);
-                if (depth >= off) {
-                    sx += px;
-                    sy += py;
-                }
-            }
-            if (live && (lane + 1 == to || ((bm >> 1) >> lane) & 1)) add(j, sx, sy);
         }
-        if (past) break;
+        return past == 0;
     }
+};
+
+// The value one lane below (lane 0: unspecified), on the VALU.
+__device__ __forceinline__ double lane_below(double v) {
+    return dpp_f64<0x138>(v);                                      // wave_shr:1
+}
+
+// Sums of one block's runs: term(t, sx, sy) forms a live lane's term,
+// put(t, sx, sy) takes the sum of a run in its last lane.
+template <typename TM, typename F>
+__device__ __forceinline__ void term_add(const Term& t, TM term, F put) {
+    if (!__ballot(t.flags & kTermLive)) return;
+    double sx = 0.0, sy = 0.0;
+    if (t.flags & kTermLive) term(t, sx, sy);
+    const int depth = t.flags & kTermDepth;
+    if (__ballot(depth >= 1)) {
+        const double px = lane_below(sx), py = lane_below(sy);
+        if (depth >= 1) {
+            sx += px;
+            sy += py;
+        }
+        for (int off = 2; __ballot(depth >= off); off <<= 1) {
+            const double qx = __shfl_up(sx, off), qy = __shfl_up(sy, off);
+            if (depth >= off) {
+                sx += qx;
+                sy += qy;
+            }
+        }
+    }
+    if (t.flags & kTermEmit) put(t, sx, sy);
+}
+
+template <typename TM, typename F>
+__device__ __forceinline__ void fold_terms(const qsft_fold_desc& d, int c, int lo, int hi, int wave, int waves,
+                                           TM term, F put) {
+    TermShare sh(lo, hi, wave, waves);
+    Term t;
+    bool more = true;
+    for (int i0 = sh.first; more; i0 += 64) {
+        more = sh.load(d, c, i0, t);
+        term_add(t, term, put);
+    }
+}
+
+// A run's sum into its bin (swapped parts): stored where the run is the whole
+// bin, else added to the bin's earlier blocks.
+template <typename T>
+__device__ __forceinline__ void bin_put(cplx_t<T>& u, const Term& t, double sx, double sy) {
+    if (!(t.flags & kTermWhole)) {
+        sx += (double)u.y;
+        sy += (double)u.x;
+    }
+    u = cplx_t<T>{(T)sy, (T)sx};
+}
+
+// Phases of row p of group c.
+__device__ __forceinline__ const QSFT_GLOBAL uint8_t* phase_row(const qsft_fold_desc& d, int c, int p) {
+    return gptr(d.E) + ((size_t)(d.shared_d ? 0 : c) * d.P + p) * fold_sp(d.S);
 }
 
 // One pass over the axes [d0, d1) of every row (dft.hip's tile scheme). The
@@ -305,82 +366,178 @@ __global__ __launch_bounds__(kDftThreads) void k_fold_pass(const SRC src, int pa
             lo = st[0];
             hi = st[1];
         }
-        fold_terms(d, c, row - c * d.P, lo, hi, threadIdx.x >> 6, kDftThreads / 64, tab,
-                   [&](uint32_t j, double sx, double sy) {
-                       C2& u = lds[j - (uint32_t)base];            // swapped parts
-                       u.x = (T)((double)u.x + sy);
-                       u.y = (T)((double)u.y + sx);
-                   });
+        const QSFT_GLOBAL uint8_t* ph = phase_row(d, c, row - c * d.P);
+        fold_terms(d, c, lo, hi, threadIdx.x >> 6, kDftThreads / 64,
+                   [&](const Term& t, double& sx, double& sy) {
+                       const double2 w = tab[ph[t.s]];
+                       sx = t.a.x * w.x - t.a.y * w.y;
+                       sy = t.a.x * w.y + t.a.y * w.x;
+                   },
+                   [&](const Term& t, double sx, double sy) { bin_put<T>(lds[t.j - (uint32_t)base], t, sx, sy); });
     } else {
         for (int e = threadIdx.x; e < E; e += blockDim.x) lds[e] = x[goff(e)];
     }
     __syncthreads();
-    const C2* cur = tile_axes<T, QR>(lds, lds + E, E, q, mb, ti, tw);
-    if (pass == d.n_pass - 1) {
+    C2* cur = tile_axes<T, QR>(lds, lds + E, E, q, mb, ti, tw);
+    if (FIRST && d.fwd) {
+        // the tile holds whole rows of samples: their sub-transform, scaled by
+        // q^-b as k_dft_pass scales it
+        for (int e = threadIdx.x; e < E; e += blockDim.x) cur[e] = C2{cur[e].y, cur[e].x};
+        __syncthreads();
+        cur = tile_axes<T, QR>(cur, cur == lds ? lds + E : lds, E, q, mb, ti, tw);
+        for (int e = threadIdx.x; e < E; e += blockDim.x) x[base + e] = dft_scaled<T>(cur[e], Q);
+    } else if (pass == d.n_pass - 1) {
         for (int e = threadIdx.x; e < E; e += blockDim.x) x[goff(e)] = C2{cur[e].y, cur[e].x};
     } else {
         for (int e = threadIdx.x; e < E; e += blockDim.x) x[goff(e)] = cur[e];
     }
 }
 
-// q = 4, whole rows of 4^B samples (k_dft4_rows' register scheme, inverse):
-// 4^B / 16 threads a row, kRows rows a workgroup.
+// q = 4, whole rows of 4^B samples (k_dft4_rows' register scheme): 4^B / 16
+// threads a row, kRows rows at a time, d.rpw times over for the rows of one
+// group, so that what the rows share (positions, strengths, run structure) is
+// loaded into registers once and the next row's phases arrive while this one
+// is transformed: a row alone spent most of its time in three dependent loads
+// before its first LDS write. Terms that do not fit the registers, or phases
+// their LDS buffer, are read per row.
+//
+// With d.fwd the row's samples are transformed back to its sub-transform
+// before they leave the registers (digit pairs 2, 0, 1 for B = 6: the first
+// needs no exchange, the last stores 128-byte segments), and x receives that.
+typedef float gf2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void store_c2(QSFT_GLOBAL float2* p, float2 v) {
+    *reinterpret_cast<QSFT_GLOBAL gf2*>(p) = gf2{v.x, v.y};
+}
+__device__ __forceinline__ void store_c2(QSFT_GLOBAL double2* p, double2 v) {
+    *reinterpret_cast<QSFT_GLOBAL gd2*>(p) = gd2{v.x, v.y};
+}
+
 template <int B>
 constexpr int fold4_rows() { return B == 4 ? 4 : 1; }             // b = 4: four rows of 16 threads fill a wave
+constexpr int kTermBlocks = 4;       // blocks of 64 terms a wave keeps in registers
+constexpr int kPhaseBytes = 4096;    // phases of one row in LDS (b = 6)
 
-template <typename T, int B, typename SRC>
-__global__ __launch_bounds__(fold4_rows<B>() << (2 * B - 4)) void k_fold4_rows(const SRC src) {
+template <typename T, int B, bool FWD, typename SRC>
+__global__ __launch_bounds__(fold4_rows<B>() << (2 * B - 4)) __attribute__((
+    amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2))) void k_fold4_rows(const SRC src) {
     using C2 = cplx_t<T>;
-    constexpr int Q = 1 << (2 * B), kTpr = Q / 16, kRows = fold4_rows<B>();
-    static_assert(B % 2 == 0 && B >= 4, "even digit count");
-    __shared__ C2 lds_all[kRows][Q + Q / 16];
-    __shared__ double2 tab[4];
+    constexpr int Q = 1 << (2 * B), kTpr = Q / 16, kRows = fold4_rows<B>(), kThreads = kRows * kTpr;
+    constexpr bool kPhLds = B == 6;
+    static_assert(B == 4 || B == 6, "two digits per register pass");
+    __shared__ __align__(16) C2 lds_all[kRows][Q + Q / 16];
+    __shared__ __align__(16) uint8_t phl[kPhLds ? kPhaseBytes : 16];
     int local;
     const qsft_fold_desc& d = src.at(blockIdx.x, local);
-    if (d.q != 4 || d.b != B) return;                              // launched for other shapes
-    const int rows = d.C * d.P;
-    const int sub = threadIdx.x / kTpr, tid = threadIdx.x % kTpr;
-    const int row = local * kRows + sub;
-    const bool live = row < rows;
+    if (d.q != 4 || d.b != B || (d.fwd != 0) != FWD) return;       // launched for other shapes
+    const int P = d.P, Sp = fold_sp(d.S), per = d.rpw * kRows, wpg = (P + per - 1) / per;
+    const int c = local / wpg, p0 = (local - c * wpg) * per, p1 = min(P, p0 + per);
+    const int sub = threadIdx.x / kTpr, tid = threadIdx.x % kTpr, wave = threadIdx.x >> 6;
     C2* lds = lds_all[sub];
-    fold_wtable(tab, 4);
+    const bool phases_staged = kPhLds && Sp <= kPhaseBytes;
+    gu4 ph_next = {0, 0, 0, 0};                                    // the next row's phases, 16 per thread
+    auto fetch = [&](int p) {
+        if (phases_staged && 16 * (int)threadIdx.x < Sp)
+            ph_next = *reinterpret_cast<const QSFT_GLOBAL gu4*>(phase_row(d, c, p) + 16 * threadIdx.x);
+    };
+    fetch(p0);
+    Term kept[kTermBlocks];
+    TermShare share(0, d.S, wave, kThreads / 64);
+    bool more = true;
 #pragma unroll
-    for (int j = 0; j < 17; ++j) lds[tid + j * kTpr] = C2{(T)0, (T)0};
-    __syncthreads();
-    // all waves of the workgroup fold one row after the other
+    for (int i = 0; i < kTermBlocks; ++i) {
+        kept[i].flags = 0;
+        if (more) more = share.load(d, c, share.first + 64 * i, kept[i]);
+    }
+    more = more && share.first < share.last && share.first + 64 * kTermBlocks < d.S;   // terms beyond the registers
+    for (int p = p0; p < p1; p += kRows) {
+        __syncthreads();                                           // the last row's reads are done
+        if (phases_staged && 16 * (int)threadIdx.x < Sp) reinterpret_cast<gu4*>(phl)[threadIdx.x] = ph_next;
+        for (int e = threadIdx.x; e < (int)(sizeof(lds_all) / 16); e += kThreads)
+            reinterpret_cast<gu4*>(lds_all)[e] = gu4{0, 0, 0, 0};
+        __syncthreads();
+        if (p + kRows < p1) fetch(p + kRows);
 #pragma unroll 1
-    for (int r = 0; r < kRows; ++r) {
-        const int rr = local * kRows + r;
-        if (rr >= rows) break;
-        const int c = rr / d.P;
-        fold_terms(d, c, rr - c * d.P, 0, d.S, threadIdx.x >> 6, kRows * kTpr / 64, tab,
-                   [&](uint32_t j, double sx, double sy) {
-                       C2& u = lds_all[r][dft4_pad((int)j)];       // swapped parts
-                       u.x = (T)((double)u.x + sy);
-                       u.y = (T)((double)u.y + sx);
-                   });
-    }
-    __syncthreads();
-    C2 v[16];
+        for (int r = 0; r < kRows; ++r) {                          // the workgroup folds one row after the other
+            if (p + r >= p1) break;
+            const QSFT_GLOBAL uint8_t* ph = phase_row(d, c, p + r);
+            auto term = [&](const Term& t, double& sx, double& sy) {
+                // a w^e, w^e in {1, i, -1, -i}: parts exchanged for odd e, signs from e
+                const uint32_t e = phases_staged ? phl[t.s] : ph[t.s];
+                const bool odd = e & 1;
+                sx = odd ? -t.a.y : t.a.x;
+                sy = odd ? t.a.x : t.a.y;
+                if (e & 2) {
+                    sx = -sx;
+                    sy = -sy;
+                }
+            };
+            auto put = [&](const Term& t, double sx, double sy) { bin_put<T>(lds_all[r][dft4_pad((int)t.j)], t, sx, sy); };
 #pragma unroll
-    for (int p = 0; p < B / 2; ++p) {
-        if (p > 0) {
-            __syncthreads();                                       // the previous reads of lds are done
-#pragma unroll
-            for (int j = 0; j < 16; ++j) lds[dft4_pad(dft4_index(p - 1, tid, j))] = v[j];
-            __syncthreads();
+            for (int i = 0; i < kTermBlocks; ++i) {
+                Term t = kept[i];
+                __asm__ volatile("" : "+v"(t.flags));              // or every step's run masks are kept across rows
+                term_add(t, term, put);
+            }
+            if (more) {
+                TermShare rest = share;
+                Term t;
+                bool go = true;
+                for (int i0 = share.first + 64 * kTermBlocks; go; i0 += 64) {
+                    go = rest.load(d, c, i0, t);
+                    term_add(t, term, put);
+                }
+            }
         }
+        __syncthreads();
+        C2 v[16];
+        auto exchange = [&](int from, int to) {                     // registers hold digit pair `from`, then `to`
+            if (from >= 0) {
+                __syncthreads();                                   // the previous reads of lds are done
+                C2* w = lds + dft4_lds_base(from, tid);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) v[j] = lds[dft4_pad(dft4_index(p, tid, j))];
+                for (int j = 0; j < 16; ++j) w[j * dft4_lds_step(from)] = v[j];
+                __syncthreads();
+            }
+            const C2* r = lds + dft4_lds_base(to, tid);
 #pragma unroll
-        for (int a = 0; a < 4; ++a) dft4_reg<T>(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);   // digit 2p
+            for (int j = 0; j < 16; ++j) v[j] = r[j * dft4_lds_step(to)];
+        };
+        auto digits = [&]() {                                      // the transforms along the pair in registers
 #pragma unroll
-        for (int a = 0; a < 4; ++a) dft4_reg<T>(v[a], v[a + 4], v[a + 8], v[a + 12]);                 // digit 2p+1
+            for (int a = 0; a < 4; ++a) dft4_reg<T>(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);
+#pragma unroll
+            for (int a = 0; a < 4; ++a) dft4_reg<T>(v[a], v[a + 4], v[a + 8], v[a + 12]);
+        };
+#pragma unroll
+        for (int k = 0; k < B / 2; ++k) {
+            exchange(k - 1, k);
+            digits();
+        }
+        int row = c * P + p;
+        __asm__ volatile("" : "+s"(row));                          // not an induction variable per store address
+        QSFT_GLOBAL C2* x = gptr(reinterpret_cast<C2*>(d.x)) + (int64_t)row * Q;
+        const bool live = p + sub < p1;
+        const uint32_t xo = (uint32_t)sub * Q;
+        if constexpr (FWD) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) v[j] = C2{v[j].y, v[j].x};   // the samples
+            digits();                                              // pair B / 2 - 1, still in registers
+            exchange(B / 2 - 1, 0);
+            digits();
+            if constexpr (B == 6) {
+                exchange(0, 1);
+                digits();
+            }
+            if (live) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    store_c2(x + (xo + dft4_index(B / 2 - 2, tid, 0) + (j << (4 * (B / 2 - 2)))), dft_scaled<T>(v[j], Q));
+            }
+        } else if (live) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) store_c2(x + (xo + tid + j * kTpr), C2{v[j].y, v[j].x});
+        }
     }
-    if (!live) return;
-    C2* __restrict__ x = reinterpret_cast<C2*>(d.x) + (int64_t)row * Q;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) x[dft4_index(B / 2 - 1, tid, j)] = C2{v[j].y, v[j].x};
 }
 
 }  // namespace qsft
@@ -419,8 +576,8 @@ extern "C" size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, i
 }
 
 extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int P, int S, int n_pad, int shared_d,
-                              int precision, int a_precision, const int8_t* Mt, const int8_t* D, const int8_t* K,
-                              const void* a, void* x, void* ws, size_t ws_bytes) {
+                              int precision, int a_precision, int transform, int launch_rows, const int8_t* Mt,
+                              const int8_t* D, const int8_t* K, const void* a, void* x, void* ws, size_t ws_bytes) {
     if (!h || !fold_shape_ok(q, n, b, C, P, S, n_pad) || (shared_d != 0 && shared_d != 1) ||
         (precision != QSFT_F32 && precision != QSFT_F64) || (a_precision != QSFT_F32 && a_precision != QSFT_F64) ||
         (((uintptr_t)Mt | (uintptr_t)D | (uintptr_t)K | (uintptr_t)a) & 15) || ((uintptr_t)ws & 255)) {
@@ -447,12 +604,15 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
     d.start = reinterpret_cast<int32_t*>(w);
     const int Q = ipow(q, b);
     if (fold_rows4(q, b)) {
-        const int per = b == 4 ? fold4_rows<4>() : fold4_rows<6>();
+        // rows of a group per workgroup: one where the launch has fewer rows than
+        // the chip holds (256 CUs x 4 workgroups), up to four where it has many
+        d.rpw = launch_rows >= 8192 ? 4 : launch_rows >= 4096 ? 2 : 1;
+        const int per = d.rpw * (b == 4 ? fold4_rows<4>() : fold4_rows<6>());
         d.n_pass = 1;
         d.pass_d1[0] = b;
         d.pass_ti[0] = 1;
         d.pass_ta[0] = 1;
-        d.pass_blocks[0] = (C * P + per - 1) / per;
+        d.pass_blocks[0] = C * ((P + per - 1) / per);
         d.pass_lds[0] = 16;
         d.tiles = 1;
         d.tile_bins = Q;
@@ -477,6 +637,7 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
         d.tile_bins = ipow(q, b - s.pass_d0[0]) * s.pass_ta[0];   // whole innermost axes: contiguous bins
         d.tiles = Q / d.tile_bins;
     }
+    d.fwd = transform && d.n_pass == 1;                            // whole rows in one tile
     *h = d;
     return QSFT_OK;
 }
@@ -526,13 +687,14 @@ void launch_pass(const SRC& src, int blocks, int pass, int lds, hipStream_t st) 
 }
 
 template <typename T, typename SRC>
-int launch_rows(int q, int b, const SRC& src, int blocks, int pass, int lds, hipStream_t st) {
+int launch_rows(int q, int b, bool fwd, const SRC& src, int blocks, int pass, int lds, hipStream_t st) {
     if (blocks == 0) return QSFT_OK;
     if (fold_rows4(q, b)) {
-        if (b == 4)
-            hipLaunchKernelGGL((k_fold4_rows<T, 4, SRC>), dim3(blocks), dim3(fold4_rows<4>() * 16), 0, st, src);
-        else
-            hipLaunchKernelGGL((k_fold4_rows<T, 6, SRC>), dim3(blocks), dim3(fold4_rows<6>() * 256), 0, st, src);
+        const dim3 g(blocks), t4(fold4_rows<4>() * 16), t6(fold4_rows<6>() * 256);
+        if (b == 4 && fwd) hipLaunchKernelGGL((k_fold4_rows<T, 4, true, SRC>), g, t4, 0, st, src);
+        else if (b == 4) hipLaunchKernelGGL((k_fold4_rows<T, 4, false, SRC>), g, t4, 0, st, src);
+        else if (fwd) hipLaunchKernelGGL((k_fold4_rows<T, 6, true, SRC>), g, t6, 0, st, src);
+        else hipLaunchKernelGGL((k_fold4_rows<T, 6, false, SRC>), g, t6, 0, st, src);
     } else {
         switch (q) {
             case 2: launch_pass<T, 2>(src, blocks, pass, lds, st); break;
@@ -561,6 +723,7 @@ extern "C" int qsft_fold_prep(const qsft_fold_desc* d, const int32_t* pre_phase,
 extern "C" int qsft_fold_rows(const qsft_fold_desc* d, const int32_t* pre, int n_inst, int blocks, int pass, int word,
                               int lds_bytes, void* stream) {
     const int prec = word & 0xF, q = (word >> 8) & 0xFF, b = (word >> 16) & 0xFF;
+    const bool fwd = (word >> 24) & 1;
     if (!d || !pre || n_inst < 1 || blocks < 0 || pass < 0 || pass >= QSFT_DFT_MAX_PASSES || lds_bytes < 16 ||
         lds_bytes > 65536 || (prec != QSFT_F32 && prec != QSFT_F64) || q < 2 || q > QSFT_MAX_Q ||
         (fold_rows4(q, b) && pass != 0)) {
@@ -568,16 +731,16 @@ extern "C" int qsft_fold_rows(const qsft_fold_desc* d, const int32_t* pre, int n
         return QSFT_ERR_ARG;
     }
     const FoldBatch src{d, pre, n_inst};
-    return prec == QSFT_F32 ? launch_rows<float>(q, b, src, blocks, pass, lds_bytes, (hipStream_t)stream)
-                            : launch_rows<double>(q, b, src, blocks, pass, lds_bytes, (hipStream_t)stream);
+    return prec == QSFT_F32 ? launch_rows<float>(q, b, fwd, src, blocks, pass, lds_bytes, (hipStream_t)stream)
+                            : launch_rows<double>(q, b, fwd, src, blocks, pass, lds_bytes, (hipStream_t)stream);
 }
 
 extern "C" int qsft_fold_one(int q, int n, int b, int C, int P, int S, int n_pad, int shared_d, int precision,
                              int a_precision, const int8_t* Mt, const int8_t* D, const int8_t* K, const void* a,
                              void* x, void* ws, size_t ws_bytes, void* stream) {
     FoldOne src;
-    int rc = qsft_fold_bind(&src.d, q, n, b, C, P, S, n_pad, shared_d, precision, a_precision, Mt, D, K, a, x, ws,
-                            ws_bytes);
+    int rc = qsft_fold_bind(&src.d, q, n, b, C, P, S, n_pad, shared_d, precision, a_precision, 0, C * P, Mt, D, K, a,
+                            x, ws, ws_bytes);
     if (rc != QSFT_OK) return rc;
     int pb = 0, rb = 0;
     if (qsft_fold_blocks(&src.d, &pb, &rb) != 0) {
@@ -587,7 +750,7 @@ extern "C" int qsft_fold_one(int q, int n, int b, int C, int P, int S, int n_pad
     hipStream_t st = (hipStream_t)stream;
     rc = launch_prep(src, pb, rb, st);
     for (int p = 0; rc == QSFT_OK && p < src.d.n_pass; ++p)
-        rc = precision == QSFT_F32 ? launch_rows<float>(q, b, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st)
-                                   : launch_rows<double>(q, b, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st);
+        rc = precision == QSFT_F32 ? launch_rows<float>(q, b, src.d.fwd, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st)
+                                   : launch_rows<double>(q, b, src.d.fwd, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st);
     return rc;
 }

@@ -215,10 +215,13 @@ class EvalFold:
     items: dicts q, n, b, C, P, S, Mt, D, K, a (complex64 or complex128 [S]),
     x (complex [C][P][q^b]), optional shared_d (every group uses the delay
     rows of group 0). The workspace is allocated here, one per instance.
+    transform: x receives the sub-transforms of the samples wherever a row is
+    one tile (`transformed[i]`), in the same launch; the samples elsewhere.
     """
 
-    def __init__(self, items, precision):
+    def __init__(self, items, precision, transform=False):
         self.ws = []
+        launch_rows = sum(it["C"] * it["P"] for it in items)
         descs, phase, rank = [], [], []
         for it in items:
             q, n, b, C, P, S = (it[k] for k in ("q", "n", "b", "C", "P", "S"))
@@ -233,8 +236,8 @@ class EvalFold:
             t = {k: it[k] if it[k].data_ptr() % 16 == 0 else it[k].clone() for k in ("Mt", "D", "K", "a")}
             self.ws.append(t)
             if lib.qsft_fold_bind(ctypes.byref(d), q, n, b, C, P, S, it["Mt"].shape[-1], shared, precision,
-                                  L.QSFT_F32 if it["a"].dtype == torch.complex64 else L.QSFT_F64, _ptr(t["Mt"]),
-                                  _ptr(t["D"]), _ptr(t["K"]), _ptr(t["a"]), _ptr(it["x"]), _ptr(ws),
+                                  L.QSFT_F32 if it["a"].dtype == torch.complex64 else L.QSFT_F64, int(transform),
+                                  launch_rows, _ptr(t["Mt"]), _ptr(t["D"]), _ptr(t["K"]), _ptr(t["a"]), _ptr(it["x"]), _ptr(ws),
                                   nbytes) != L.QSFT_OK:
                 raise ValueError(f"bad eval shape {[it[k] for k in ('q', 'n', 'b', 'C', 'P', 'S')]}")
             pb, rb = ctypes.c_int(), ctypes.c_int()
@@ -243,6 +246,7 @@ class EvalFold:
             descs.append(d)
             phase.append(pb.value)
             rank.append(rb.value)
+        self.transformed = [bool(d.fwd) for d in descs]
         # rows: one launch per (q, b) of the whole-row kernel, per q and pass otherwise
         groups = defaultdict(list)
         for i, d in enumerate(descs):
@@ -256,7 +260,7 @@ class EvalFold:
                 bl = [0] * len(order)
                 for k, i in enumerate(ix):
                     bl[at + k] = descs[i].pass_blocks[p] if p < descs[i].n_pass else 0
-                plan.append((p, precision | (q << 8) | (b << 16), at,
+                plan.append((p, precision | (q << 8) | (b << 16) | ((int(transform) << 24) if b else 0), at,
                              max(descs[i].pass_lds[p] for i in ix if p < descs[i].n_pass)))
                 lists.append(bl)
             at += len(ix)

@@ -13,7 +13,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
+    from qsft_amd import _lib as L
     from qsft_amd import device as dv
+    from qsft_amd import kernels as K
 
 # whole-row kernels (q = 4, b in {4, 6}) with rows that do not fill the last
 # workgroup; one tile, several tiles and several passes of the others (b = 7,
@@ -80,3 +82,50 @@ def test_fold_of_crowded_bins(q, b, S):
         x = _run(q, n, b, Ms, Ds, crowd, a, "fp64")
         ref = _direct(q, b, Ms, Ds, crowd, a)
         assert np.max(np.abs(x - ref)) <= 1e-12 * np.max(np.abs(ref))
+
+
+def _item(q, n, b, Ms, Ds, loc, a, precision):
+    dev, n_pad = dv.current_device(), dv.n_pad_of(n)
+    dt = torch.complex64 if precision == "fp32" else torch.complex128
+    return dict(q=q, n=n, b=b, C=len(Ms), P=Ds[0].shape[0], S=loc.shape[1], Mt=dv.Mt_tensor(Ms, b, n_pad, dev),
+                D=dv.D_tensor(Ds, n_pad, dev), K=dv.digits_tensor(loc.T, n_pad, dev),
+                a=dv.strengths_tensor(a, "fp64", dev),
+                x=torch.empty((len(Ms), Ds[0].shape[0], q ** b), dtype=dt, device=dev))
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 2e-6)])
+@pytest.mark.parametrize("q,n,b,S,C,P", [c for c in CASES if c[3] > 0])
+def test_fold_with_the_sub_transform_in_the_same_launch(q, n, b, S, C, P, precision, tol):
+    """transform=True: rows of one tile come out as their sub-transforms, other
+    rows as samples. A sample's error is at most tol of the largest sample and
+    independent of its neighbours', so the error of a mean of q^b of them is
+    that over sqrt(q^b), times 6 for the largest of all values, and as much
+    again for the forward transform's own rounding."""
+    print(f"fold + sub-DFT q={q} n={n} b={b} S={S} C={C} P={P} {precision}", flush=True)
+    Ms, Ds, loc, a = _inputs(q, n, b, S, C, P, seed=q * 97 + n + S)
+    it = _item(q, n, b, Ms, Ds, loc, a, precision)
+    ev = K.EvalFold([it], L.QSFT_F32 if precision == "fp32" else L.QSFT_F64, transform=True)
+    ev.launch()
+    got, ref = it["x"].cpu().numpy(), _direct(q, b, Ms, Ds, loc, a)
+    bound = tol * np.max(np.abs(ref))
+    if ev.transformed[0]:
+        ref = np.fft.fftn(ref.reshape(C, P, *[q] * b), axes=range(2, 2 + b)).reshape(C, P, -1) / q ** b
+        bound *= 12 / q ** (b / 2)
+    else:
+        assert b > 6 or q > 4                                      # q = 4, b <= 6 always fits one tile
+    assert np.max(np.abs(got - ref)) <= bound
+
+
+@pytest.mark.parametrize("b,count", [(4, 15), (4, 29), (6, 15), (6, 29)])
+def test_fold_of_many_rows_gives_the_bits_of_one_instance(b, count):
+    """Launches of 4096 and 8192 rows and more give a workgroup two or four sets
+    of rows of a group (P = 101 leaves the last one short): the same bits."""
+    print(f"fold many rows b={b} count={count}", flush=True)
+    g = [_inputs(4, 50, b, 300 + 40 * i, 3, 101, seed=i) for i in range(count)]
+    items = [_item(4, 50, b, *x, "fp32") for x in g]
+    assert sum(it["C"] * it["P"] for it in items) >= (4096 if count == 15 else 8192)
+    K.EvalFold(items, L.QSFT_F32).launch()
+    for i in (0, count // 2, count - 1):
+        alone = _item(4, 50, b, *g[i], "fp32")
+        K.EvalFold([alone], L.QSFT_F32).launch()
+        assert torch.equal(torch.view_as_real(alone["x"]), torch.view_as_real(items[i]["x"]))
