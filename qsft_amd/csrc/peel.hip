@@ -51,8 +51,30 @@ constexpr int kBinThreads = 64 * kWaves;
 constexpr int kBinsPerWave = 64;      // consecutive bins owned by one wave (one per lane) in the per-bin kernels
 constexpr int kRowsPerLane = kColRowsPerLane;   // P <= 256
 constexpr int kSlotThreads = 256;
+// Most parts (log2) of a wave's bins, first and later passes. The first pass
+// classifies four bins at once and nearly every block ends with atomics on the
+// shared counters: 16 bins a wave (one request at the K1 size: 64 bins 43 us,
+// 32 33, 16 25, 4 39). Later passes take one bin after the other: 4 bins (two
+// passes 87 us at 64 bins, 37 at 8, 31 at 4).
+constexpr int kSplitFirst = 2;
+constexpr int kSplitLater = 4;
 constexpr uint32_t kNil = 0xFFFFFFFFu;
 constexpr int kHeldMulti = 1 << 30;   // mark bit: multiton when last scanned, no ball queued on it since
+
+// The per-bin kernels' partition. A batch's block prefix counts blocks of
+// kWaves x 64 bins. A wave walks its due bins one step after another, so a
+// launch of few blocks is as long as its longest wave while most of the chip
+// idles: it runs 2^split times the blocks, each wave with 64 >> split of the
+// bins (see bin_split).
+struct BinShare {
+    int inst, base, nbins;
+    __device__ __forceinline__ BinShare(const int32_t* pre, int n_inst, int split) {
+        const int blk = blockIdx.x >> split, part = blockIdx.x & ((1 << split) - 1);
+        inst = find_inst(pre, n_inst, blk);
+        nbins = kBinsPerWave >> split;
+        base = ((blk - pre[inst]) * kWaves + (int)(threadIdx.x >> 6)) * kBinsPerWave + part * nbins;
+    }
+};
 
 // numpy's remainder(x, 2 pi) for finite x: fmod, then shift negatives up.
 __device__ __forceinline__ double rem_2pi(double x) {
@@ -186,24 +208,24 @@ __device__ __forceinline__ void load_col(double2 (&u)[kRowsPerLane], const doubl
     }
 }
 
-// First-pass screen. Wave w owns bins [64 w, 64 w + 64); lane L stamps bin
-// 64 w + L for pass 0 iff it is not a zeroton, and -1 (never) otherwise. With
+// First-pass screen. Wave w owns bins [64 w, 64 w + 64) (or a part of them, see
+// BinShare); lane L stamps its bin L for pass 0 iff it is not a zeroton, and -1 (never) otherwise. With
 // energies from the assembler it compares one number per bin; otherwise four
 // columns are loaded before their energies are reduced, so several loads per
 // lane are in flight and U streams once at HBM speed. Kernel A then visits
 // only the stamped bins.
 __global__ __launch_bounds__(kBinThreads) void k_peel_screen(const qsft_peel_desc* __restrict__ descs,
-                                                             const int32_t* __restrict__ pre, int n_inst) {
-    const int inst = find_inst(pre, n_inst, blockIdx.x);
-    const qsft_peel_desc& d = descs[inst];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+                                                             const int32_t* __restrict__ pre, int n_inst, int split) {
+    const BinShare share(pre, n_inst, split);
+    const qsft_peel_desc& d = descs[share.inst];
+    const int lane = threadIdx.x & 63;
     const int CQ = d.C * d.Q, P = d.P;
-    const int base = ((blockIdx.x - pre[inst]) * kWaves + wave) * kBinsPerWave;
+    const int base = share.base;
     if (base >= CQ) return;
-    const int nb = min(kBinsPerWave, CQ - base);
+    const int nb = min(share.nbins, CQ - base);
     const double thr = d.cutoff * (double)P;
     if (d.energy) {
-        if (base + lane < CQ) d.mark[base + lane] = (d.energy[base + lane] > thr) ? 0 : -1;
+        if (lane < nb) d.mark[base + lane] = (d.energy[base + lane] > thr) ? 0 : -1;
         return;
     }
     const double2* __restrict__ Ub = reinterpret_cast<const double2*>(d.U) + (size_t)base * P;
@@ -225,7 +247,7 @@ __global__ __launch_bounds__(kBinThreads) void k_peel_screen(const qsft_peel_des
             if (lane == g + k) nz = e > thr;
         }
     }
-    if (base + lane < CQ) d.mark[base + lane] = nz ? 0 : -1;
+    if (lane < nb) d.mark[base + lane] = nz ? 0 : -1;
 }
 
 // w^{<D_c row p, k>} for this lane's rows p = lane + 64 r (zero past P); k is
@@ -784,26 +806,32 @@ __device__ __noinline__ void rs_decode_wave(const qsft_peel_desc& d, const int8_
 // anyway, buffers all 64.
 constexpr int kSbCap = 16;
 
+template <int CAP>
+struct SingletonBuf {
+    double2 rho[CAP];
+    uint64_t h[CAP];
+    int32_t t[CAP];
+};
+
 template <int NR, int CAP = kSbCap>
 struct DetectWaveLds {
+    SingletonBuf<CAP> sb;                                          // (first, as in QuadWaveLds)
     __align__(16) uint32_t kws[QSFT_MAX_N / 4];
     int8_t syn[kRsMaxSyn];                                         // coded source: syndrome digits
     int32_t rs[kRsScratch];                                        // coded source: decoder state
     __align__(16) PendingSlot pslot[2];                            // first queued ball, per column slot
     __align__(16) double2 colw[2][64 * NR];                        // current / next column
-    uint64_t sb_h[CAP];
-    double2 sb_rho[CAP];
-    int32_t sb_t[CAP];
 };
 
-// The wave's bins due this pass among the 64 from `base` (bit i: bin base + i).
+// The wave's bins due this pass among the nbins from `base` (bit i: bin base + i).
 // A held multiton (a multiton last pass that no ball has been queued on since)
 // keeps its column, so it is a multiton again: it is counted (nheld) and
 // re-stamped without being read.
-__device__ __forceinline__ uint64_t scan_marks(const qsft_peel_desc& d, int it, int base, uint32_t& nheld) {
+__device__ __forceinline__ uint64_t scan_marks(const qsft_peel_desc& d, int it, int base, uint32_t& nheld,
+                                               int nbins = kBinsPerWave) {
     const int lane = threadIdx.x & 63;
     QSFT_GLOBAL int32_t* __restrict__ mark = gptr(d.mark);
-    const int mk = (base + lane < d.C * d.Q) ? mark[base + lane] : -1;
+    const int mk = (lane < nbins && base + lane < d.C * d.Q) ? mark[base + lane] : -1;
     const bool due = (mk & ~kHeldMulti) == it;
     const bool held = due && (mk & kHeldMulti) != 0;
     nheld = (uint32_t)__popcll(__ballot(held));
@@ -811,17 +839,12 @@ __device__ __forceinline__ uint64_t scan_marks(const qsft_peel_desc& d, int it, 
     return __ballot(due && !held);
 }
 
-// One wave classifies the due bins `todo` among the 64 from `base` and
-// registers its singletons (kernel A's body; the fused tail kernel runs it
-// with PERSIST). tab, offbuf and mtbuf are the block's staged tables.
-// End of a wave's detection: the pass counters (bins scanned, singletons,
-// multitons: one atomic each per wave), then the hash registration of the
-// wave's buffered singletons, one lane each, so the atomics of up to 64
-// registrations are in flight together.
-// Hash registration of the wave's ns buffered singletons (sb_*), one lane
-// each. Every lane of the wave takes part (ballots).
-__device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int it, int ns, const int32_t* sb_t,
-                                                    const uint64_t* sb_h, const double2* sb_rho, int lane) {
+// Hash registration of a wave's ns buffered singletons, one lane each, so the
+// atomics of up to 64 registrations are in flight together. Every lane of the
+// wave takes part (ballots).
+template <int CAP>
+__device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int it, int ns,
+                                                    const SingletonBuf<CAP>& sb, int lane) {
     uint32_t* __restrict__ ctr = d.ctr;
     const int CQ = d.C * d.Q;
     int slot = -1;
@@ -831,9 +854,9 @@ __device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int
     uint64_t tm = 0;
     double2 rho = make_double2(0.0, 0.0);
     if (lane < ns) {
-        t = sb_t[lane];
-        rho = sb_rho[lane];
-        const uint64_t hv = sb_h[lane];
+        t = sb.t[lane];
+        rho = sb.rho[lane];
+        const uint64_t hv = sb.h[lane];
         const uint64_t tg = hv | 1ull;
         const uint32_t mask = (1u << d.hcap_log2) - 1u;
         uint32_t pos = (uint32_t)(hv >> 32) & mask;
@@ -883,31 +906,164 @@ __device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int
     }
 }
 
-// End of a wave's detection: the pass counters over the whole wave (scanned
-// bins, ns singletons, nz - ns multitons) and the registration of the nbuf
-// singletons still buffered.
-__device__ __forceinline__ void finish_wave(const qsft_peel_desc& d, int it, uint32_t scanned, int nz, int ns,
-                                            const int32_t* sb_t, const uint64_t* sb_h, const double2* sb_rho,
-                                            int lane, int nbuf) {
-    if (lane == 0) {
-        uint32_t* pc = d.ctr + it * QSFT_CTR_ITER_STRIDE;
-        atomicAdd(pc + 4, scanned);
-        if (ns) atomicAdd(pc + 0, (uint32_t)ns);
-        if (nz > ns) atomicAdd(pc + 1, (uint32_t)(nz - ns));
+// The same in two parts, for waves that end together (finish_block): first the
+// slots; then, with the first record and list position of the wave, the records.
+struct Claim {
+    int slot, t;
+    bool claimed;                                              // this lane's k took a new slot
+    double2 rho;
+    uint64_t nb_mask, ok_mask, cl_mask;                        // new balls, registered, claimed
+};
+
+template <int CAP>
+__device__ __forceinline__ Claim claim_slots(const qsft_peel_desc& d, int it, int ns, const SingletonBuf<CAP>& sb, int lane) {
+    uint32_t* __restrict__ ctr = d.ctr;
+    Claim c{-1, 0, false, make_double2(0.0, 0.0), 0, 0, 0};
+    bool newball = false;
+    if (lane < ns) {
+        c.t = sb.t[lane];
+        c.rho = sb.rho[lane];
+        const uint64_t hv = sb.h[lane];
+        const uint64_t tg = hv | 1ull;
+        const uint32_t mask = (1u << d.hcap_log2) - 1u;
+        uint32_t pos = (uint32_t)(hv >> 32) & mask;
+        for (uint32_t probe = 0; probe <= mask; ++probe) {
+            const unsigned long long old = atomicCAS((unsigned long long*)&d.tag[pos], 0ull, (unsigned long long)tg);
+            if (old == 0ull || old == tg) {
+                c.slot = (int)pos;
+                c.claimed = old == 0ull;
+                break;
+            }
+            pos = (pos + 1) & mask;
+        }
+        if (c.slot < 0) {
+            atomicOr(&ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_TABLE_FULL);
+        } else {
+            d.slot_bin[c.t] = c.slot;
+            d.sstamp[c.t] = it + 1;                               // kernel B peels only registered bins
+            const uint64_t tm = ((uint64_t)(it + 1) << 32) | (uint32_t)c.t;
+            atomicMin((unsigned long long*)&d.owner[c.slot], (unsigned long long)tm);
+            const unsigned long long prev = atomicMax((unsigned long long*)&d.last[c.slot], (unsigned long long)tm);
+            newball = (prev >> 32) != (unsigned long long)(it + 1);
+        }
     }
-    if (nbuf > 0) register_singletons(d, it, nbuf, sb_t, sb_h, sb_rho, lane);
+    c.nb_mask = __ballot(newball);
+    c.ok_mask = __ballot(c.slot >= 0);
+    c.cl_mask = __ballot(c.claimed);
+    return c;
 }
 
+// rbase / lbase: the wave's first record and first live-list position
+__device__ __forceinline__ void write_records(const qsft_peel_desc& d, int it, const Claim& c, uint32_t rbase,
+                                              uint32_t lbase, int lane) {
+    const uint64_t below = (1ull << lane) - 1ull;
+    if (c.claimed) d.live[lbase + (uint32_t)__popcll(c.cl_mask & below)] = (uint32_t)c.slot;
+    if (c.slot >= 0) {
+        const uint32_t rix = rbase + (uint32_t)__popcll(c.ok_mask & below);
+        if ((uint64_t)rix >= (uint64_t)d.max_iter * (uint64_t)(d.C * d.Q)) {   // cannot happen: one record per bin per pass
+            atomicOr(&d.ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_BAD_SHAPE);
+        } else {
+            d.rec_time[rix] = ((uint64_t)(it + 1) << 32) | (uint32_t)c.t;
+            d.rec_rho[2 * (size_t)rix] = c.rho.x;
+            d.rec_rho[2 * (size_t)rix + 1] = c.rho.y;
+            d.rec_next[rix] = atomicExch(&d.head[c.slot], rix);
+            atomicAdd(&d.count[c.slot], 1u);
+        }
+    }
+}
+
+// records << 0 | claimed slots << 32 added to the adjacent LOG and LIVE words
+// in one atomic (neither word overflows into the other: both count at most the
+// records); the counts before.
+__device__ __forceinline__ uint64_t take_records(uint32_t* ctr, uint32_t records, uint32_t slots) {
+    static_assert(QSFT_CTR_LOG % 2 == 0 && QSFT_CTR_LIVE == QSFT_CTR_LOG + 1, "one 64-bit word");
+    if (records == 0 && slots == 0) return 0;
+    return atomicAdd((unsigned long long*)&ctr[QSFT_CTR_LOG], (unsigned long long)records | ((unsigned long long)slots << 32));
+}
+
+// The pass counters of a block: singletons and multitons (adjacent words, one
+// atomic), new balls, bins scanned.
+__device__ __forceinline__ void add_counters(uint32_t* ctr, int it, uint32_t scanned, uint32_t ns, uint32_t nm,
+                                             uint32_t nb) {
+    static_assert(QSFT_CTR_ITER_STRIDE % 2 == 0, "64-bit aligned counter pairs");
+    uint32_t* pc = ctr + it * QSFT_CTR_ITER_STRIDE;
+    if (ns | nm) atomicAdd((unsigned long long*)pc, (unsigned long long)ns | ((unsigned long long)nm << 32));
+    if (nb) atomicAdd(pc + 2, nb);
+    if (scanned) atomicAdd(pc + 4, scanned);
+}
+
+// What a wave's detection leaves to its end: its pass counts (nz non-zerotons,
+// ns of them singletons) and the nbuf singletons still buffered.
+struct WaveEnd {
+    uint32_t scanned;
+    int nz, ns, nbuf;
+};
+
+template <int CAP>
+__device__ __forceinline__ void finish_wave(const qsft_peel_desc& d, int it, const WaveEnd& e,
+                                            const SingletonBuf<CAP>& sb, int lane) {
+    if (lane == 0) {
+        uint32_t* pc = d.ctr + it * QSFT_CTR_ITER_STRIDE;
+        if (e.scanned) atomicAdd(pc + 4, e.scanned);
+        if (e.ns) atomicAdd(pc + 0, (uint32_t)e.ns);
+        if (e.nz > e.ns) atomicAdd(pc + 1, (uint32_t)(e.nz - e.ns));
+    }
+    if (e.nbuf > 0) register_singletons(d, it, e.nbuf, sb, lane);
+}
+
+// The same for a block whose waves all take part: the shared counters get one
+// set of atomics per block. They serialise on their cache line, and a launch
+// split into many small waves has thousands of ends (one request at the K1
+// size in 768 blocks: 18 432 atomics, 80 us; per block 3 072, 39 us).
+struct BlockEnd {
+    uint32_t cnt[kWaves][6];
+    uint64_t base;
+};
+
+template <int CAP>
+__device__ __forceinline__ void finish_block(const qsft_peel_desc& d, int it, const WaveEnd& e,
+                                             const SingletonBuf<CAP>& sb, BlockEnd& B) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const Claim c = claim_slots(d, it, e.nbuf, sb, lane);
+    if (lane == 0) {
+        uint32_t* w = B.cnt[wave];
+        w[0] = e.scanned;
+        w[1] = (uint32_t)e.ns;
+        w[2] = (uint32_t)(e.nz - e.ns);
+        w[3] = (uint32_t)__popcll(c.nb_mask);
+        w[4] = (uint32_t)__popcll(c.ok_mask);
+        w[5] = (uint32_t)__popcll(c.cl_mask);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t[6];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            t[i] = 0;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) t[i] += B.cnt[w][i];
+        }
+        B.base = take_records(d.ctr, t[4], t[5]);
+        add_counters(d.ctr, it, t[0], t[1], t[2], t[3]);
+    }
+    __syncthreads();
+    uint32_t rbase = (uint32_t)B.base, lbase = (uint32_t)(B.base >> 32);
+    for (int w = 0; w < wave; ++w) {
+        rbase += B.cnt[w][4];
+        lbase += B.cnt[w][5];
+    }
+    write_records(d, it, c, rbase, lbase, lane);
+}
+
+// One wave classifies the due bins `todo` among the 64 from `base` and
+// buffers its singletons (kernel A's body; the fused tail kernel runs it
+// with PERSIST). tab, offbuf and mtbuf are the block's staged tables.
 template <int NR, bool PERSIST, int CAP>
-__device__ __forceinline__ void detect_bins(const qsft_peel_desc& d, int it, int base, uint64_t todo, uint32_t nheld,
+__device__ __forceinline__ WaveEnd detect_bins(const qsft_peel_desc& d, int it, int base, uint64_t todo, uint32_t nheld,
                                             DetectWaveLds<NR, CAP>& W, const double2* tab, const int8_t* offbuf,
                                             bool offs_staged, const int8_t* mtbuf, bool mt_staged) {
-    uint32_t* __restrict__ ctr = d.ctr;
     const int lane = threadIdx.x & 63;
-    if (todo == 0) {
-        if (lane == 0 && nheld) atomicAdd(ctr + it * QSFT_CTR_ITER_STRIDE + 1, nheld);
-        return;
-    }
+    if (todo == 0) return WaveEnd{0, (int)nheld, 0, 0};
     const int q = d.q, n = d.n, b = d.b, C = d.C, P = d.P, Q = d.Q, n_pad = d.n_pad;
     const int nw = n_pad >> 2;
     const int CQ = C * Q;
@@ -1067,9 +1223,9 @@ __device__ __forceinline__ void detect_bins(const qsft_peel_desc& d, int it, int
             if (single) {
                 const uint64_t hk = hash_k(kk, nw, lane);
                 if (lane == 0) {
-                    W.sb_t[nb] = t;
-                    W.sb_h[nb] = hk;
-                    W.sb_rho[nb] = make_double2(rho_x, rho_y);
+                    W.sb.t[nb] = t;
+                    W.sb.h[nb] = hk;
+                    W.sb.rho[nb] = make_double2(rho_x, rho_y);
                 }
                 ++ns;
                 ++nb;
@@ -1094,14 +1250,14 @@ __device__ __forceinline__ void detect_bins(const qsft_peel_desc& d, int it, int
         wave_lds_sync();                                           // kk / this slot are rewritten next
         if constexpr (CAP < kBinsPerWave) {
             if (nb == CAP) {                                       // the buffer is full: register it
-                register_singletons(d, it, nb, W.sb_t, W.sb_h, W.sb_rho, lane);
+                register_singletons(d, it, nb, W.sb, lane);
                 nb = 0;
                 wave_lds_sync();
             }
         }
     }
 
-    finish_wave(d, it, scanned, nz, ns, W.sb_t, W.sb_h, W.sb_rho, lane, nb);
+    return WaveEnd{scanned, nz, ns, nb};
 }
 
 // ---- The first pass, four bins per wave ------------------------------------
@@ -1121,12 +1277,10 @@ constexpr int kQuad = 4;                 // bins a wave classifies at once
 constexpr int kQRows = 8;                // rows per lane (P <= 128)
 
 struct QuadWaveLds {
+    SingletonBuf<kSbCap> sb;
     __align__(16) double2 col[kQuad][128];         // the current quad's columns
     __align__(16) uint32_t kws[kQuad][16];         // each bin's k (n_pad = 64)
     __align__(16) int32_t off[kQuad][4];           // each bin's <offset_r, k> mod q (unit delays)
-    uint64_t sb_h[kSbCap];
-    double2 sb_rho[kSbCap];
-    int32_t sb_t[kSbCap];
 };
 
 // In-row (16 lanes) part of wave_sum: the same DPP butterfly.
@@ -1155,7 +1309,7 @@ __device__ __forceinline__ uint64_t hash_k16(uint32_t word, int l16) {
 // The wave's due bins (first pass), four at a time. Preconditions (checked by
 // the caller): no coded source, n_pad = 64, P <= 128, unit delays with R <= 4
 // staged offset rows (or general delays), every due bin written.
-__device__ __forceinline__ void detect_quads(const qsft_peel_desc& d, int base, uint64_t todo, uint32_t nheld, QuadWaveLds& W,
+__device__ __forceinline__ WaveEnd detect_quads(const qsft_peel_desc& d, int base, uint64_t todo, uint32_t nheld, QuadWaveLds& W,
                              const double2* tab, const int8_t* offbuf, const int8_t* mtbuf, bool mt_staged) {
     constexpr int it = 0;
     const int lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
@@ -1165,7 +1319,6 @@ __device__ __forceinline__ void detect_quads(const qsft_peel_desc& d, int base, 
     const double thr = d.cutoff * (double)P;
     const double inv_p = 1.0 / (double)P;
     const double2* __restrict__ Ub = reinterpret_cast<const double2*>(d.U);
-    const int CQ = d.C * Q;
     QSFT_GLOBAL int32_t* __restrict__ mark = gptr(d.mark);
     QSFT_GLOBAL int8_t* __restrict__ kcur = gptr(d.kbin);         // pass 0: slot (it & 1) = 0
     QSFT_GLOBAL double* __restrict__ rcur = gptr(d.rho_bin);
@@ -1278,15 +1431,17 @@ __device__ __forceinline__ void detect_quads(const qsft_peel_desc& d, int base, 
             const int p = l16 + 16 * r;
             double2 w = make_double2(0.0, 0.0);
             if (nonzero && p < P) {
-                if (unit) {
-                    const int blk = (int)__umulhi((uint32_t)p, m1);
-                    const int i = p - blk * p1;
+                int pp = p;
+                __asm__ volatile("" : "+v"(pp));                   // or eight rows' indexes and addresses are kept
+                if (unit) {                                        // (and spilled) across the quads
+                    const int blk = (int)__umulhi((uint32_t)pp, m1);
+                    const int i = pp - blk * p1;
                     int e = blk == 0 ? o[0] : blk == 1 ? o[1] : blk == 2 ? o[2] : o[3];
                     if (i > 0) e += neg ? q - (int)kb8[i - 1] : (int)kb8[i - 1];
                     if (e >= q) e -= q;
                     w = tab[e];
                 } else {
-                    w = tab[mq(dot_row(Dc + (size_t)p * n_pad, kk, nw))];
+                    w = tab[mq(dot_row(Dc + (size_t)pp * n_pad, kk, nw))];
                 }
             }
             return w;
@@ -1327,15 +1482,15 @@ __device__ __forceinline__ void detect_quads(const qsft_peel_desc& d, int base, 
         const uint64_t smask = __ballot(l16 == 0 && single);
         const int nnew = (int)__popcll(smask);
         if (nbuf + nnew > kSbCap) {                                // no room: register the buffer first
-            register_singletons(d, it, nbuf, W.sb_t, W.sb_h, W.sb_rho, lane);
+            register_singletons(d, it, nbuf, W.sb, lane);
             nbuf = 0;
             wave_lds_sync();
         }
         if (l16 == 0 && single) {
             const int at = nbuf + (int)__popcll(smask & ((1ull << lane) - 1ull));
-            W.sb_t[at] = t;
-            W.sb_h[at] = hk;
-            W.sb_rho[at] = make_double2(rho_x, rho_y);
+            W.sb.t[at] = t;
+            W.sb.h[at] = hk;
+            W.sb.rho[at] = make_double2(rho_x, rho_y);
         }
         ns += nnew;
         nbuf += nnew;
@@ -1352,8 +1507,7 @@ __device__ __forceinline__ void detect_quads(const qsft_peel_desc& d, int base, 
         for (int k = 0; k < kQuad; ++k) cb[k] = nb[k];
         wave_lds_sync();                                           // kws / the column buffer are rewritten next
     }
-    (void)CQ;
-    finish_wave(d, it, scanned, nz, ns, W.sb_t, W.sb_h, W.sb_rho, lane, nbuf);
+    return WaveEnd{scanned, nz, ns, nbuf};
 }
 
 // Kernel A of the first pass: detect_quads where its preconditions hold (and
@@ -1367,8 +1521,11 @@ __device__ __forceinline__ void detect_quads(const qsft_peel_desc& d, int base, 
 constexpr int kQuadOffBytes = 1024;
 constexpr int kQuadMtBytes = 2048;
 
+// SPLIT: a launch of split waves ends its blocks together (finish_block); the
+// full waves of a large launch each register their own.
+template <bool SPLIT>
 __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_peel_detect0(
-    const qsft_peel_desc* __restrict__ descs, const int32_t* __restrict__ pre, int n_inst) {
+    const qsft_peel_desc* __restrict__ descs, const int32_t* __restrict__ pre, int n_inst, int split) {
     __shared__ double2 tab[QSFT_MAX_Q];
     __shared__ union WaveLds {
         QuadWaveLds quad;
@@ -1376,16 +1533,16 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_waves_per_eu(4))
     } wl[kWaves];
     __shared__ __align__(16) int8_t offbuf[kQuadOffBytes];
     __shared__ __align__(16) int8_t mtbuf[kQuadMtBytes];
-    const int inst = find_inst(pre, n_inst, blockIdx.x);
-    const qsft_peel_desc& d = descs[inst];
+    __shared__ BlockEnd end;
+    const BinShare share(pre, n_inst, split);
+    const qsft_peel_desc& d = descs[share.inst];
     uint32_t* __restrict__ ctr = d.ctr;
     constexpr int it = 0;
     if (it >= d.max_iter) return;
     if (cptr(ctr)[it * QSFT_CTR_ITER_STRIDE + 3] == 0) return;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int base = ((blockIdx.x - pre[inst]) * kWaves + wave) * kBinsPerWave;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, base = share.base;
     uint32_t nheld;
-    const uint64_t todo = scan_marks(d, it, base, nheld);
+    const uint64_t todo = scan_marks(d, it, base, nheld, share.nbins);
     if (!__syncthreads_or(todo != 0)) {
         if (lane == 0 && nheld) atomicAdd(ctr + it * QSFT_CTR_ITER_STRIDE + 1, nheld);
         return;
@@ -1399,8 +1556,23 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_waves_per_eu(4))
     const bool written = !sparse_u(d) || __ballot(((todo >> lane) & 1) && !gptr(d.written)[base + lane]) == 0;
     const bool quads = !(d.flags & QSFT_PEEL_ONE_BIN_WAVES) && !(d.method & QSFT_DETECT_CODED) && d.n_pad == 64 &&
                        d.P <= 128 && (!unit || (offs_staged && d.P / d.p1 <= 4)) && written;
-    if (quads) detect_quads(d, base, todo, nheld, wl[wave].quad, tab, offbuf, mtbuf, mt_staged);
-    else detect_bins<2, false>(d, it, base, todo, nheld, wl[wave].one, tab, offbuf, offs_staged, mtbuf, mt_staged);
+    if constexpr (SPLIT) {
+        // (quads is the same for a wave, not for a block)
+        const WaveEnd e = quads ? detect_quads(d, base, todo, nheld, wl[wave].quad, tab, offbuf, mtbuf, mt_staged)
+                                : detect_bins<2, false>(d, it, base, todo, nheld, wl[wave].one, tab, offbuf,
+                                                        offs_staged, mtbuf, mt_staged);
+        wave_lds_sync();
+        finish_block(d, it, e, wl[wave].quad.sb, end);             // (the same place in both layouts)
+    } else if (quads) {
+        const WaveEnd e = detect_quads(d, base, todo, nheld, wl[wave].quad, tab, offbuf, mtbuf, mt_staged);
+        wave_lds_sync();
+        finish_wave(d, it, e, wl[wave].quad.sb, lane);
+    } else {
+        const WaveEnd e =
+            detect_bins<2, false>(d, it, base, todo, nheld, wl[wave].one, tab, offbuf, offs_staged, mtbuf, mt_staged);
+        wave_lds_sync();
+        finish_wave(d, it, e, wl[wave].one.sb, lane);
+    }
 }
 
 // Kernel A. Wave w of an instance owns bins [64 w, 64 w + 64): it classifies
@@ -1414,21 +1586,22 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_waves_per_eu(4))
 // reserved across the whole loop, are out of line.
 template <int NR>
 __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_waves_per_eu(NR == 2 ? 4 : 3))) void k_peel_detect(const qsft_peel_desc* __restrict__ descs,
-                                                             const int32_t* __restrict__ pre, int n_inst, int it) {
+                                                             const int32_t* __restrict__ pre, int n_inst, int it,
+                                                             int split) {
     __shared__ double2 tab[QSFT_MAX_Q];
     __shared__ DetectWaveLds<NR> wl[kWaves];
     __shared__ __align__(16) int8_t offbuf[kStageOffBytes];
     __shared__ __align__(16) int8_t mtbuf[kStageMtBytes];
-    const int inst = find_inst(pre, n_inst, blockIdx.x);
-    const qsft_peel_desc& d = descs[inst];
+    __shared__ BlockEnd end;
+    const BinShare share(pre, n_inst, split);
+    const qsft_peel_desc& d = descs[share.inst];
     uint32_t* __restrict__ ctr = d.ctr;
     if (it >= d.max_iter) return;                                  // beyond the bound workspace
     if (cptr(ctr)[it * QSFT_CTR_ITER_STRIDE + 3] == 0) return;    // loop already stopped (set by the
                                                                    // previous pass; scalar load)
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int base = ((blockIdx.x - pre[inst]) * kWaves + wave) * kBinsPerWave;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, base = share.base;
     uint32_t nheld;
-    const uint64_t todo = scan_marks(d, it, base, nheld);
+    const uint64_t todo = scan_marks(d, it, base, nheld, share.nbins);
     if (!__syncthreads_or(todo != 0)) {                            // nothing to read in this block
         if (lane == 0 && nheld) atomicAdd(ctr + it * QSFT_CTR_ITER_STRIDE + 1, nheld);
         return;
@@ -1437,7 +1610,10 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_waves_per_eu(NR 
     const bool offs_staged = stage_offsets(d, offbuf);
     const bool mt_staged = stage_mt(d, mtbuf);
     __syncthreads();
-    detect_bins<NR, false>(d, it, base, todo, nheld, wl[wave], tab, offbuf, offs_staged, mtbuf, mt_staged);
+    const WaveEnd e =
+        detect_bins<NR, false>(d, it, base, todo, nheld, wl[wave], tab, offbuf, offs_staged, mtbuf, mt_staged);
+    wave_lds_sync();
+    finish_block(d, it, e, wl[wave].sb, end);
 }
 
 constexpr int kKeyChunks = QSFT_MAX_N / 16;                        // 16-byte chunks of a k row
@@ -1634,9 +1810,13 @@ __global__ __launch_bounds__(64 * tail_waves<NR>()) void k_peel_tail(const qsft_
             for (int i = 0; i < kTailBatch; ++i) {
                 const uint64_t todo = tdue[wave][i];
                 const uint32_t nheld = theld[wave][i];
-                if (todo != 0 || nheld != 0)
-                    detect_bins<NR, true>(d, it, g0 + i * kGroupStride, todo, nheld, wl[wave], tab, offbuf,
-                                          offs_staged, mtbuf, mt_staged);
+                if (todo != 0 || nheld != 0) {
+                    const WaveEnd e = detect_bins<NR, true>(d, it, g0 + i * kGroupStride, todo, nheld, wl[wave], tab,
+                                                            offbuf, offs_staged, mtbuf, mt_staged);
+                    wave_lds_sync();
+                    finish_wave(d, it, e, wl[wave].sb, lane);
+                    wave_lds_sync();                               // the buffer is rewritten next
+                }
             }
             wave_lds_sync();                                       // tdue is rewritten next
         }
@@ -2015,6 +2195,15 @@ extern "C" int qsft_peel_slot_blocks(const qsft_peel_desc* h) {
     return (int)(((H > CQ ? H : CQ) + kSlotThreads - 1) / kSlotThreads);
 }
 
+// log2 of the parts a launch's 64-bin waves are divided into: as many as keep
+// the blocks within the 1024 that are resident at once (256 CUs x 4), at most
+// `most`.
+static int bin_split(int blocks, int most) {
+    int split = 0;
+    while (split < most && ((long long)blocks << (split + 1)) <= 1024) ++split;
+    return split;
+}
+
 extern "C" int qsft_peel_init(const qsft_peel_desc* d, const int32_t* pre_bins, const int32_t* pre_slots,
                               int n_inst, int blocks_bins, int blocks_slots, void* stream) {
     if (!d || !pre_bins || !pre_slots || n_inst < 1 || blocks_bins < 1 || blocks_slots < 1) {
@@ -2025,7 +2214,8 @@ extern "C" int qsft_peel_init(const qsft_peel_desc* d, const int32_t* pre_bins, 
     hipLaunchKernelGGL(k_peel_init, dim3(blocks_slots), dim3(kSlotThreads), 0, st, d, pre_slots, n_inst);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return qsft_hip_status(e, "qsft_peel_init");
-    hipLaunchKernelGGL(k_peel_screen, dim3(blocks_bins), dim3(kBinThreads), 0, st, d, pre_bins, n_inst);
+    const int split = bin_split(blocks_bins, 4);
+    hipLaunchKernelGGL(k_peel_screen, dim3(blocks_bins << split), dim3(kBinThreads), 0, st, d, pre_bins, n_inst, split);
     return qsft_hip_status(hipGetLastError(), "qsft_peel_init(screen)");
 }
 
@@ -2039,12 +2229,16 @@ extern "C" int qsft_peel_iteration(const qsft_peel_desc* d, const int32_t* pre_b
     hipStream_t st = (hipStream_t)stream;
     // rows per lane: 2 when every instance has P <= 128, else 4; the first
     // pass of the former four bins per wave where it can
-    if (max_p <= 128 && it == 0)
-        hipLaunchKernelGGL(k_peel_detect0, dim3(blocks_bins), dim3(kBinThreads), 0, st, d, pre_bins, n_inst);
+    const int split = bin_split(blocks_bins, it == 0 ? kSplitFirst : kSplitLater);
+    const dim3 grid(blocks_bins << split), threads(kBinThreads);
+    if (max_p <= 128 && it == 0 && split > 0)
+        hipLaunchKernelGGL(k_peel_detect0<true>, grid, threads, 0, st, d, pre_bins, n_inst, split);
+    else if (max_p <= 128 && it == 0)
+        hipLaunchKernelGGL(k_peel_detect0<false>, grid, threads, 0, st, d, pre_bins, n_inst, split);
     else if (max_p <= 128)
-        hipLaunchKernelGGL(k_peel_detect<2>, dim3(blocks_bins), dim3(kBinThreads), 0, st, d, pre_bins, n_inst, it);
+        hipLaunchKernelGGL(k_peel_detect<2>, grid, threads, 0, st, d, pre_bins, n_inst, it, split);
     else
-        hipLaunchKernelGGL(k_peel_detect<4>, dim3(blocks_bins), dim3(kBinThreads), 0, st, d, pre_bins, n_inst, it);
+        hipLaunchKernelGGL(k_peel_detect<4>, grid, threads, 0, st, d, pre_bins, n_inst, it, split);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return qsft_hip_status(e, "qsft_peel_iteration(detect)");
     hipLaunchKernelGGL(k_peel_apply, dim3(blocks_bins), dim3(kBinThreads), 0, st, d, pre_bins, n_inst, it);

@@ -381,3 +381,28 @@ def test_k3_uneven_mix_batch_equals_alone():
         planted += sp.S
     print(f"noiseless K3 copies: {found} of {planted} keys", flush=True)
     assert found >= 0.95 * planted
+
+
+@pytest.mark.parametrize("q,n,S,b,R,method,snr", [(4, 50, 1000, 6, 2, "nso", 10.0), (4, 10, 100, 4, 1, "identity", None),
+                                                  (3, 90, 200, 5, 2, "nso", 15.0), (2, 100, 60, 7, 1, "nso", 20.0)])
+def test_split_waves_match_full_waves(q, n, S, b, R, method, snr):
+    """Launches of few blocks give each wave a part of its 64 bins and end their
+    blocks together; launches of many do not. One instance alone (split) and the
+    same instance among enough copies to fill the chip (1024 blocks and more):
+    the same rows, bits and order."""
+    rng = np.random.default_rng(q * 100 + n)
+    specs = [E.random_spec(q, n, S, b, 3, R, snr, rng=rng, method=method) for _ in range(2)]
+    per = -(-3 * q ** b // 256)
+    copies = -(-520 // per)
+    print(f"split waves q={q} n={n} b={b}: {per} blocks alone, {2 * copies * per} together", flush=True)
+    many = E.Batch(specs * copies, precision="fp32")
+    many.launch(seed_offset=3)
+    got = many.results(with_info=False)
+    for i in (0, 1):
+        alone = E.Batch([specs[i]], precision="fp32")
+        alone.launch(seed_offset=3)
+        (k, v, order, info), = alone.results(with_info=True)
+        for j in (i, 2 * (copies - 1) + i):
+            assert np.array_equal(got[j][0], k) and np.array_equal(got[j][2], order)
+            assert np.array_equal(got[j][1].view(np.float64), v.view(np.float64))
+        assert info["trace"] == many.peel.info(i)["trace"] and info["records"] == many.peel.info(i)["records"]
