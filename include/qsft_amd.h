@@ -462,9 +462,9 @@ size_t qsft_peel_pack_header_bytes(int n_inst);
 int qsft_peel_pack(const qsft_peel_desc* dev_descs, int n_inst, void* dst, int64_t cap_rows, int row_stride,
                    void* stream);
 
-/* The same rows, each instance's in first-detection order (the reference's
- * dict insertion order, qsft/qsft.py:247-255): a row's position is its
- * instance offset plus its rank by the order word, so readers need no sort. */
+/* qsft_peel_finalize leaves every instance's rows in first-detection order (the
+ * reference's dict insertion order, qsft/qsft.py:247-255), so both packs write
+ * them in that order and readers need no sort. */
 int qsft_peel_pack_ordered(const qsft_peel_desc* d, int n_inst, void* dst, int64_t cap_rows, int row_stride,
                            void* stream);
 

@@ -42,6 +42,8 @@
 // bit instead of merging two keys), writes the key of new slots, and lets the
 // last detection of each key queue the ball on its bin in every group. No
 // kernel waits on another thread's progress.
+#include <algorithm>
+
 #include "qsft_common.h"
 
 namespace qsft {
@@ -1274,7 +1276,6 @@ __device__ __forceinline__ WaveEnd detect_bins(const qsft_peel_desc& d, int it, 
 // swaps of wave_sum do: energies, rho, residuals, digits, phases and hashes
 // come out bit for bit as in the one-bin layout.
 constexpr int kQuad = 4;                 // bins a wave classifies at once
-constexpr int kQRows = 8;                // rows per lane (P <= 128)
 
 struct QuadWaveLds {
     SingletonBuf<kSbCap> sb;
@@ -1839,27 +1840,25 @@ __global__ __launch_bounds__(64 * tail_waves<NR>()) void k_peel_tail(const qsft_
     }
 }
 
-// Output of one key: the running mean of its records in time order, gathered
-// kFinRecs at a time by walks of the key's list.
+// The output table. Each key's value is the running mean of its records in
+// time order, and its row is its rank by first detection (the reference's dict
+// insertion order; the order words are distinct: one first detection per pass
+// and bin), so packing is a plain copy. A workgroup takes 64 keys: wave 0 walks
+// their record lists (a chain of dependent loads) while the other three count the
+// keys' ranks against LDS tiles of all order words. kFinRecs records are
+// gathered at a time by walks of the key's list.
+// 64 K1 instances (1000 keys each): the table and the ranked copy took 97 us
+// and 194 us as a thread per key writing its own rows, now 33 and 98 us; one
+// instance 12 and 57 us, now 12 and 5. (512 and 1024 threads: 52 and 45 us for
+// 64 instances, 10 us for one.)
 constexpr int kFinRecs = 8;
+constexpr int kFinThreads = 256;
+constexpr int kFinTile = 2048;
 
-__global__ __launch_bounds__(kSlotThreads) void k_peel_finalize(const qsft_peel_desc* __restrict__ descs,
-                                                                const int32_t* __restrict__ pre, int n_inst) {
-    // one thread per claimed slot (the claim order of the registration), so
-    // the output row of a key is its position in that list
-    const int inst = find_inst(pre, n_inst, blockIdx.x);
-    const qsft_peel_desc& d = descs[inst];
-    const uint32_t nlive = d.ctr[QSFT_CTR_LIVE];
-    const uint32_t o = (uint32_t)(blockIdx.x - pre[inst]) * kSlotThreads + threadIdx.x;
-    if (o == 0) {
-        d.ctr[QSFT_CTR_OUT] = nlive;
-        if (nlive > (uint32_t)d.out_cap) atomicOr(&d.ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_OUT_FULL);
-    }
-    if (o >= nlive || o >= (uint32_t)d.out_cap) return;
-    const uint32_t h = d.live[o];
+// Running mean over the m records of hash slot h.
+__device__ __forceinline__ double2 mean_of_records(const qsft_peel_desc& d, uint32_t h, uint32_t L) {
     const uint32_t m = d.count[h];
-    const uint32_t L = d.ctr[QSFT_CTR_LOG];
-    // running mean over the records in time order: g <- (g * c + v) / (c + 1)
+    // g <- (g * c + v) / (c + 1)
     double gx = 0.0, gy = 0.0;
     auto accumulate = [&](uint32_t cnt, double vx, double vy) {
         if (cnt == 0) {
@@ -1885,10 +1884,13 @@ __global__ __launch_bounds__(kSlotThreads) void k_peel_finalize(const qsft_peel_
             rx[a] = ry[a] = 0.0;
         }
         uint32_t steps = 0;
-        for (uint32_t r = d.head[h]; r != kNil && steps <= L; r = d.rec_next[r], ++steps) {
+        for (uint32_t r = d.head[h]; r != kNil && steps <= L; ++steps) {
+            const uint32_t next = d.rec_next[r];
             uint64_t t = d.rec_time[r];
+            const double2 v = reinterpret_cast<const double2*>(d.rec_rho)[r];
+            r = next;
             if (t <= prev || t >= tr[kFinRecs - 1]) continue;
-            double vx = d.rec_rho[2 * (size_t)r], vy = d.rec_rho[2 * (size_t)r + 1];
+            double vx = v.x, vy = v.y;
 #pragma unroll
             for (int a = 0; a < kFinRecs; ++a) {                   // insertion: the later entries shift up
                 if (t < tr[a]) {
@@ -1915,22 +1917,73 @@ __global__ __launch_bounds__(kSlotThreads) void k_peel_finalize(const qsft_peel_
         }
         if (got == 0) break;                                       // (a list shorter than its count)
     }
-    const int nw = d.n_pad >> 2;
-    const uint32_t* ksrc = reinterpret_cast<const uint32_t*>(d.key + (size_t)h * d.n_pad);
-    uint32_t* kdst = reinterpret_cast<uint32_t*>(d.out_k + (size_t)o * d.n_pad);
-    for (int w = 0; w < nw; ++w) kdst[w] = ksrc[w];
-    d.out_val[2 * (size_t)o] = gx;
-    d.out_val[2 * (size_t)o + 1] = gy;
-    d.out_order[o] = d.owner[h];
+    return make_double2(gx, gy);
 }
 
-// Exclusive scan of the per-instance output counts into the pack header:
-// hdr[i] = count_i, hdr[n + i] = offset_i, hdr[2n] = total, hdr[2n + 1] = OR of
-// error bits, hdr[2n + 2] = most passes run, hdr[2n + 3] = instances whose loop
-// asked for a pass beyond those launched.
-__global__ __launch_bounds__(64) void k_pack_scan(const qsft_peel_desc* __restrict__ descs, int n_inst,
-                                                  int64_t* __restrict__ hdr, int64_t cap_rows) {
-    const int lane = threadIdx.x;
+__global__ __launch_bounds__(kFinThreads) void k_peel_finalize(const qsft_peel_desc* __restrict__ descs,
+                                                               int per_inst) {
+    constexpr int kFinWaves = kFinThreads / 64;
+    __shared__ __align__(16) uint64_t tile[kFinTile];
+    __shared__ uint32_t part[kFinWaves][64];
+    const int inst = blockIdx.x / per_inst, local = blockIdx.x - inst * per_inst;
+    const qsft_peel_desc& d = descs[inst];
+    const uint32_t nlive = d.ctr[QSFT_CTR_LIVE];
+    if (local == 0 && threadIdx.x == 0) {
+        d.ctr[QSFT_CTR_OUT] = nlive;
+        if (nlive > (uint32_t)d.out_cap) atomicOr(&d.ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_OUT_FULL);
+    }
+    const int m = (int)min(nlive, (uint32_t)d.out_cap);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t L = d.ctr[QSFT_CTR_LOG];
+    for (int o0 = local * 64; o0 < m; o0 += per_inst * 64) {       // (block-uniform)
+        const int o = o0 + lane;
+        const bool mine = o < m;
+        const uint32_t h = mine ? d.live[o] : 0u;
+        const uint64_t order = mine ? d.owner[h] : 0ull;
+        double2 g = make_double2(0.0, 0.0);
+        uint32_t rank = 0;
+        for (int t0 = 0; t0 < m; t0 += kFinTile) {
+            const int tn = min(kFinTile, m - t0), te = (tn + 1) & ~1;
+            __syncthreads();                                       // the previous tile is consumed
+            for (int t = threadIdx.x; t < te; t += kFinThreads) tile[t] = t < tn ? d.owner[d.live[t0 + t]] : ~0ull;
+            __syncthreads();
+            if (wave == 0) {
+                if (t0 == 0 && mine) g = mean_of_records(d, h, L);
+                continue;
+            }
+            const int share = ((te + kFinWaves - 2) / (kFinWaves - 1) + 1) & ~1;
+            const int z = min(te, wave * share);
+#pragma unroll 4
+            for (int t = (wave - 1) * share; t < z; t += 2) {      // (the pad word is above every order)
+                const ulonglong2 k = *reinterpret_cast<const ulonglong2*>(tile + t);
+                rank += (k.x < order ? 1u : 0u) + (k.y < order ? 1u : 0u);
+            }
+        }
+        part[wave][lane] = rank;
+        __syncthreads();
+        if (wave == 0 && mine) {
+            rank = 0;
+#pragma unroll
+            for (int w = 1; w < kFinWaves; ++w) rank += part[w][lane];
+            const uint4* ks = reinterpret_cast<const uint4*>(d.key + (size_t)h * d.n_pad);
+            uint4* kd = reinterpret_cast<uint4*>(d.out_k + (size_t)rank * d.n_pad);
+            for (int w = 0; w < (d.n_pad >> 4); ++w) kd[w] = ks[w];
+            reinterpret_cast<double2*>(d.out_val)[rank] = g;
+            d.out_order[rank] = order;
+        }
+    }
+}
+
+// Exclusive scan of the per-instance output counts into the pack header (one
+// wave): hdr[i] = count_i, hdr[n + i] = offset_i, hdr[2n] = total, hdr[2n + 1] =
+// OR of error bits, hdr[2n + 2] = most passes run, hdr[2n + 3] = instances whose
+// loop asked for a pass beyond those launched.
+__device__ __forceinline__ int64_t rows_of(const qsft_peel_desc& d) {
+    return (int64_t)min(d.ctr[QSFT_CTR_OUT], (uint32_t)d.out_cap);
+}
+
+__device__ __forceinline__ void pack_header(const qsft_peel_desc* __restrict__ descs, int n_inst,
+                                            int64_t* __restrict__ hdr, int64_t cap_rows, int lane) {
     long long carry = 0;
     uint32_t err = 0;
     int iters = 0, unfinished = 0;
@@ -1939,10 +1992,8 @@ __global__ __launch_bounds__(64) void k_pack_scan(const qsft_peel_desc* __restri
         long long m = 0;
         if (i < n_inst) {
             const qsft_peel_desc& d = descs[i];
-            uint32_t c = d.ctr[QSFT_CTR_OUT];
-            if ((int)c > d.out_cap) c = (uint32_t)d.out_cap;
+            m = rows_of(d);
             err |= d.ctr[QSFT_CTR_ERROR];
-            m = c;
             // passes that ran, and whether the loop asked for one more than were launched
             const int it = (int)d.ctr[QSFT_CTR_ITERS];
             iters = max(iters, it);
@@ -1975,68 +2026,38 @@ __global__ __launch_bounds__(64) void k_pack_scan(const qsft_peel_desc* __restri
     }
 }
 
-// One block per instance copies its rows: k digits (n_pad bytes), value (2 doubles), order (u64).
-__global__ __launch_bounds__(256) void k_pack_rows(const qsft_peel_desc* __restrict__ descs, int n_inst,
-                                                   const int64_t* __restrict__ hdr, unsigned char* __restrict__ rows,
-                                                   int64_t cap_rows, int row_stride) {
-    const int i = blockIdx.x;
+// Rows: k digits (n_pad bytes), value (2 doubles), order (u64), row_stride
+// apart. per_inst blocks share an instance; each sums the counts before it, and
+// the first block also writes the header. Consecutive lanes write consecutive
+// 8-byte words, so what crosses PCIe into pinned host memory is whole lines
+// (bound: the link; rows written word by word by one thread each took twice as
+// long for 64 instances and ten times for one).
+__global__ __launch_bounds__(256) void k_pack(const qsft_peel_desc* __restrict__ descs, int n_inst, int per_inst,
+                                              int64_t* __restrict__ hdr, unsigned char* __restrict__ rows,
+                                              int64_t cap_rows, int row_stride) {
+    __shared__ int64_t sums[4];
+    const int i = blockIdx.x / per_inst, g = blockIdx.x - i * per_inst;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (blockIdx.x == 0 && wave == 3) pack_header(descs, n_inst, hdr, cap_rows, lane);
+    long long before = 0;
+    for (int t = threadIdx.x; t < i; t += 256) before += rows_of(descs[t]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) before += __shfl_xor(before, off);
+    if (lane == 0) sums[wave] = before;
+    __syncthreads();
+    const int64_t off = sums[0] + sums[1] + sums[2] + sums[3];
     const qsft_peel_desc& d = descs[i];
-    const int64_t m = hdr[i], off = hdr[n_inst + i];
-    const int nw = d.n_pad >> 2;
-    for (int64_t r = threadIdx.x; r < m; r += blockDim.x) {
-        if (off + r >= cap_rows) break;
-        unsigned char* dst = rows + (off + r) * row_stride;
-        const uint32_t* ks = reinterpret_cast<const uint32_t*>(d.out_k + r * d.n_pad);
-        uint32_t* kd = reinterpret_cast<uint32_t*>(dst);
-        for (int w = 0; w < nw; ++w) kd[w] = ks[w];
-        double* vd = reinterpret_cast<double*>(dst + d.n_pad);
-        vd[0] = d.out_val[2 * r];
-        vd[1] = d.out_val[2 * r + 1];
-        *reinterpret_cast<uint64_t*>(dst + d.n_pad + 16) = d.out_order[r];
-    }
-}
-
-// The same rows, each written at its instance offset plus its rank in first
-// detection order (the reference's dict insertion order), so a caller reads
-// every instance's rows already ordered. The rank of a row is the number of
-// the instance's rows with a smaller order word (order words are distinct:
-// one first detection per pass and bin), counted against LDS tiles of the
-// order words. kRankGroups blocks share an instance (block g ranks rows
-// g*256 + tid, stepping by kRankGroups*256), so an instance with thousands
-// of rows spreads its m^2 comparisons over many CUs.
-constexpr int kRankTile = 2048;
-constexpr int kRankGroups = 32;
-
-__global__ __launch_bounds__(256) void k_pack_rows_ordered(const qsft_peel_desc* __restrict__ descs, int n_inst,
-                                                           const int64_t* __restrict__ hdr,
-                                                           unsigned char* __restrict__ rows, int64_t cap_rows,
-                                                           int row_stride) {
-    __shared__ uint64_t tile[kRankTile];
-    const int i = blockIdx.x / kRankGroups, g = blockIdx.x % kRankGroups;
-    const qsft_peel_desc& d = descs[i];
-    const int64_t m = hdr[i], off = hdr[n_inst + i];
-    const int nw = d.n_pad >> 2;
-    for (int64_t r0 = (int64_t)g * blockDim.x; r0 < m; r0 += (int64_t)kRankGroups * blockDim.x) {   // block-uniform
-        const int64_t r = r0 + threadIdx.x;
-        const uint64_t mine = r < m ? d.out_order[r] : ~0ull;
-        int64_t rank = 0;
-        for (int64_t t0 = 0; t0 < m; t0 += kRankTile) {
-            const int tn = (int)min((int64_t)kRankTile, m - t0);
-            __syncthreads();                                       // the previous tile is consumed
-            for (int j = threadIdx.x; j < tn; j += blockDim.x) tile[j] = d.out_order[t0 + j];
-            __syncthreads();
-            for (int j = 0; j < tn; ++j) rank += tile[j] < mine ? 1 : 0;
-        }
-        if (r < m && off + rank < cap_rows) {
-            unsigned char* dst = rows + (off + rank) * row_stride;
-            const uint32_t* ks = reinterpret_cast<const uint32_t*>(d.out_k + r * d.n_pad);
-            uint32_t* kd = reinterpret_cast<uint32_t*>(dst);
-            for (int w = 0; w < nw; ++w) kd[w] = ks[w];
-            double* vd = reinterpret_cast<double*>(dst + d.n_pad);
-            vd[0] = d.out_val[2 * r];
-            vd[1] = d.out_val[2 * r + 1];
-            *reinterpret_cast<uint64_t*>(dst + d.n_pad + 16) = mine;
-        }
+    const int64_t m = min(rows_of(d), max(cap_rows - off, (int64_t)0));
+    const int kw = d.n_pad >> 3;                                   // 8-byte words of the digits
+    const uint32_t used = (uint32_t)kw + 3;
+    const uint64_t* __restrict__ ok = reinterpret_cast<const uint64_t*>(d.out_k);
+    const uint64_t* __restrict__ ov = reinterpret_cast<const uint64_t*>(d.out_val);
+    const int64_t total = m * used;
+    for (int64_t e = (int64_t)g * 256 + threadIdx.x; e < total; e += (int64_t)per_inst * 256) {
+        const int64_t r = e / used;
+        const int c = (int)(e - r * used);
+        const uint64_t v = c < kw ? ok[r * kw + c] : c < kw + 2 ? ov[2 * r + (c - kw)] : d.out_order[r];
+        *reinterpret_cast<uint64_t*>(rows + (off + r) * row_stride + 8 * c) = v;
     }
 }
 
@@ -2257,7 +2278,11 @@ extern "C" int qsft_peel_finalize(const qsft_peel_desc* d, const int32_t* pre_sl
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return qsft_hip_status(e, "qsft_peel_finalize(flush)");
     }
-    hipLaunchKernelGGL(k_peel_finalize, dim3(blocks_slots), dim3(kSlotThreads), 0, (hipStream_t)stream, d, pre_slots, n_inst);
+    // blocks per instance: 64 take 4096 keys in one step (the large job of the
+    // serving mix, 5000 keys, needs two); an empty block costs a large batch
+    // about 4 ns (K1 x 64: 48 blocks 30 us, 96 41 us; mix 82 and 56 us)
+    const int per = std::min(128, std::max(64, 1024 / n_inst));
+    hipLaunchKernelGGL(k_peel_finalize, dim3(n_inst * per), dim3(kFinThreads), 0, (hipStream_t)stream, d, per);
     return qsft_hip_status(hipGetLastError(), "qsft_peel_finalize");
 }
 
@@ -2294,29 +2319,17 @@ extern "C" int qsft_peel_pack(const qsft_peel_desc* d, int n_inst, void* dst, in
         qsft_set_error("qsft_peel_pack: bad arguments");
         return QSFT_ERR_ARG;
     }
-    hipStream_t st = (hipStream_t)stream;
     int64_t* hdr = static_cast<int64_t*>(dst);
     unsigned char* rows = static_cast<unsigned char*>(dst) + qsft_peel_pack_header_bytes(n_inst);
-    hipLaunchKernelGGL(k_pack_scan, dim3(1), dim3(64), 0, st, d, n_inst, hdr, cap_rows);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return qsft_hip_status(e, "qsft_peel_pack(scan)");
-    hipLaunchKernelGGL(k_pack_rows, dim3(n_inst), dim3(256), 0, st, d, n_inst, hdr, rows, cap_rows, row_stride);
-    return qsft_hip_status(hipGetLastError(), "qsft_peel_pack(rows)");
+    const int per = std::min(32, std::max(4, 512 / n_inst));
+    hipLaunchKernelGGL(k_pack, dim3(n_inst * per), dim3(256), 0, (hipStream_t)stream, d, n_inst, per, hdr, rows,
+                       cap_rows, row_stride);
+    return qsft_hip_status(hipGetLastError(), "qsft_peel_pack");
 }
 
+// qsft_peel_finalize leaves the table in first-detection order, so the two
+// packs are one.
 extern "C" int qsft_peel_pack_ordered(const qsft_peel_desc* d, int n_inst, void* dst, int64_t cap_rows,
                                       int row_stride, void* stream) {
-    if (!d || !dst || n_inst < 1 || cap_rows < 0 || row_stride < 24 + 64 || row_stride % 8) {
-        qsft_set_error("qsft_peel_pack_ordered: bad arguments");
-        return QSFT_ERR_ARG;
-    }
-    hipStream_t st = (hipStream_t)stream;
-    int64_t* hdr = static_cast<int64_t*>(dst);
-    unsigned char* rows = static_cast<unsigned char*>(dst) + qsft_peel_pack_header_bytes(n_inst);
-    hipLaunchKernelGGL(k_pack_scan, dim3(1), dim3(64), 0, st, d, n_inst, hdr, cap_rows);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return qsft_hip_status(e, "qsft_peel_pack_ordered(scan)");
-    hipLaunchKernelGGL(k_pack_rows_ordered, dim3(n_inst * kRankGroups), dim3(256), 0, st, d, n_inst, hdr, rows,
-                       cap_rows, row_stride);
-    return qsft_hip_status(hipGetLastError(), "qsft_peel_pack_ordered(rows)");
+    return qsft_peel_pack(d, n_inst, dst, cap_rows, row_stride, stream);
 }

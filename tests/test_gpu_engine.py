@@ -406,3 +406,25 @@ def test_split_waves_match_full_waves(q, n, S, b, R, method, snr):
             assert np.array_equal(got[j][0], k) and np.array_equal(got[j][2], order)
             assert np.array_equal(got[j][1].view(np.float64), v.view(np.float64))
         assert info["trace"] == many.peel.info(i)["trace"] and info["records"] == many.peel.info(i)["records"]
+
+
+@pytest.mark.parametrize("S,count", [(40, 3), (63, 1), (64, 1), (65, 2), (2500, 1), (5000, 2)])
+def test_output_table_is_ranked_by_first_detection(S, count):
+    """Rows come packed in ascending first-detection order with the instances'
+    offsets in the header, for key counts around a wave, over one rank tile
+    (2048) and over one step of the blocks (4096): noiseless, so every planted
+    key is a row."""
+    b = 4 if S < 100 else 7
+    rng = np.random.default_rng(S)
+    specs = [E.random_spec(4, 20, S, b, 3, 2, None, rng=rng) for _ in range(count)]
+    print(f"output table S={S} x {count}", flush=True)
+    bt = E.Batch(specs, precision="fp32")
+    bt.launch()
+    counts, offs, rows = bt.fetch()
+    assert list(offs) == list(np.cumsum(counts) - counts) and rows.shape[0] == counts.sum()
+    for i, (sp, (k, v, order, _)) in enumerate(zip(specs, bt.unpack((counts, offs, rows)))):
+        packed = rows[offs[i]:offs[i] + counts[i], 80:88].copy().view(np.uint64).reshape(-1)
+        assert np.all(packed[1:] > packed[:-1]) and np.array_equal(packed, order)
+        truth = {tuple(c): a for c, a in zip(sp.locq.T, sp.strengths)}
+        assert {tuple(r) for r in k} == set(truth)
+        assert max(abs(x - truth[tuple(r)]) for r, x in zip(k, v)) < 1e-4
