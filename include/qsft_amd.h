@@ -138,9 +138,11 @@ typedef struct qsft_fold_desc {
     int32_t pass_ta[QSFT_DFT_MAX_PASSES], pass_blocks[QSFT_DFT_MAX_PASSES], pass_lds[QSFT_DFT_MAX_PASSES];
     int32_t tiles;          /* tiles of the first pass per row, tile_bins consecutive bins each */
     int32_t tile_bins;
-    int32_t rpw;            /* q = 4, b in {4, 6}: row sets of one group per workgroup      */
-    int32_t fwd;            /* 1: x receives the rows' sub-transforms (qsft_dft_pass of the *
-                             * samples), formed in the same launch: rows of one tile only  */
+    int32_t rpw;            /* whole-row kernel (q = 4, b = 4..6, FP32 also 7): row sets of *
+                             * one group per workgroup; 0: the tile kernel                  */
+    int32_t fwd;            /* 1: the last pass transforms its samples back along its axes  *
+                             * (all of them where n_pass = 1: x receives sub-transforms);   *
+                             * qsft_fold_rest gives the passes that remain                  */
     const int8_t* Mt;       /* [C][b][n_pad], 16-byte aligned                               */
     const int8_t* D;        /* [C][P][n_pad] ([P][n_pad] when shared_d), 16-byte aligned    */
     const int8_t* K;        /* [S][n_pad], 16-byte aligned                                  */
@@ -155,10 +157,9 @@ typedef struct qsft_fold_desc {
 } qsft_fold_desc;
 
 size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, int shared_d);
-/* Fills a host descriptor (schedule: k_fold4_rows for q = 4, b in {4, 6}, else the
- * sub-DFT planner's passes). precision: of x; transform: write sub-transforms
- * instead of samples where a row is one tile (`fwd` of the descriptor says so);
- * launch_rows: rows (C * P) of all instances of the launch; ws 256-byte aligned. */
+/* Fills a host descriptor (schedule: whole rows where they fit the LDS, else the
+ * sub-DFT planner's passes). precision: of x; transform: sub-transforms instead of
+ * samples, the passes of qsft_fold_rest included; launch_rows: rows (C * P) of all instances of the launch; ws 256-byte aligned. */
 int qsft_fold_bind(qsft_fold_desc* host_desc, int q, int n, int b, int C, int P, int S, int n_pad, int shared_d,
                    int precision, int a_precision, int transform, int launch_rows, const int8_t* Mt, const int8_t* D,
                    const int8_t* K, const void* a, void* x, void* ws, size_t ws_bytes);
@@ -167,8 +168,8 @@ int qsft_fold_blocks(const qsft_fold_desc* host_desc, int* phase_blocks, int* ra
 int qsft_fold_prep(const qsft_fold_desc* dev_descs, const int32_t* dev_pre_phase, const int32_t* dev_pre_rank,
                    int n_inst, int phase_blocks, int rank_blocks, void* stream);
 /* Row pass `pass` (dev_pre counts pass_blocks). word: low nibble QSFT_F32 / QSFT_F64, bits 8..15 = q, bits
- * 16..23 = b: all instances of a launch share q, and b too for q = 4 with b in {4, 6} (whole rows in one
- * launch; b = 0 for a launch of mixed b otherwise); bit 24: the descriptors' fwd (those whole-row launches).
+ * 16..23 = b of a whole-row launch (descriptors with rpw > 0, all of one b; 0: the tile kernel, any b);
+ * bit 24: the descriptors' fwd (whole-row launches). All instances of a launch share q.
  * lds_bytes: at least every instance's pass_lds[pass]. */
 int qsft_fold_rows(const qsft_fold_desc* dev_descs, const int32_t* dev_pre, int n_inst, int blocks, int pass, int word,
                    int lds_bytes, void* stream);
@@ -231,6 +232,8 @@ typedef struct qsft_dft_desc {
  * and inner-run lengths). Every schedule applies the same axis transforms in
  * the same order (innermost axis first), so results do not depend on it. */
 int qsft_dft_plan(qsft_dft_desc* host_desc, int precision);
+/* The same, but one pass over whole rows where a row of several passes fits 144 KiB of LDS. */
+int qsft_dft_plan_rows(qsft_dft_desc* host_desc, int precision);
 /* The planner's candidate `index` (0 = the model's best, in the order the
  * autotuner tries them); QSFT_ERR_ARG past the last. */
 int qsft_dft_plan_candidate(qsft_dft_desc* host_desc, int precision, int index);
@@ -244,12 +247,14 @@ int qsft_dft_autotune(int q, int b, int precision, int rows, void* buf, size_t b
 /* The schedule qsft_dft_plan returns for (q, b, precision): pass count, axis
  * groups [d0, d1), TI and TA per pass (arrays of 4); *tuned = 1 if measured. */
 int qsft_dft_schedule(int q, int b, int precision, int* n_pass, int* d0, int* d1, int* ti, int* ta, int* tuned);
-/* Dynamic LDS bytes one instance's pass needs (tile + twiddles, <= 64 KiB). */
+/* Dynamic LDS bytes one instance's pass needs (tile + twiddles; <= 64 KiB for a qsft_dft_plan schedule). */
 int qsft_dft_lds_bytes(const qsft_dft_desc* host_desc, int pass, int precision);
 /* lds_bytes: dynamic LDS of the launch, at least qsft_dft_lds_bytes() of every
  * instance's pass; smaller tiles leave more workgroups resident per CU. */
 int qsft_dft_pass(const qsft_dft_desc* dev_descs, const int32_t* dev_pre, int n_inst,
                   int total_blocks, int pass, int precision, int lds_bytes, void* stream);
+/* After the row passes of a descriptor bound with transform: the qsft_dft_pass passes that are left. */
+int qsft_fold_rest(const qsft_fold_desc* host_desc, qsft_dft_desc* out);
 /* q = 4 and b in {4, 6} with in_stride 1 (the served sub-transforms): one
  * workgroup per row (dev_pre counts rows), the axis transforms two digits at a
  * time in registers, one launch instead of qsft_dft_pass's passes. word: low

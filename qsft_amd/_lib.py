@@ -118,6 +118,7 @@ SIGNATURES = {
     "qsft_eval_mfma": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),
     "qsft_fold_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 6),
     "qsft_fold_bind": (ctypes.c_int, [ctypes.POINTER(FoldDesc)] + [ctypes.c_int] * 12 + [vp] * 6 + [ctypes.c_size_t]),
+    "qsft_fold_rest": (ctypes.c_int, [ctypes.POINTER(FoldDesc), ctypes.POINTER(DftDesc)]),
     "qsft_fold_blocks": (ctypes.c_int, [ctypes.POINTER(FoldDesc), ctypes.POINTER(ctypes.c_int),
                                         ctypes.POINTER(ctypes.c_int)]),
     "qsft_fold_prep": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),
@@ -129,6 +130,7 @@ SIGNATURES = {
     "qsft_eval_points_blocks": (ctypes.c_int, [ctypes.POINTER(EvalPointsDesc)]),
     "qsft_eval_points": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),
     "qsft_dft_plan": (ctypes.c_int, [ctypes.POINTER(DftDesc), ctypes.c_int]),
+    "qsft_dft_plan_rows": (ctypes.c_int, [ctypes.POINTER(DftDesc), ctypes.c_int]),
     "qsft_dft_lds_bytes": (ctypes.c_int, [ctypes.POINTER(DftDesc), ctypes.c_int, ctypes.c_int]),
     "qsft_dft_plan_candidate": (ctypes.c_int, [ctypes.POINTER(DftDesc), ctypes.c_int, ctypes.c_int]),
     "qsft_dft_autotune": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, ctypes.c_size_t,

@@ -117,14 +117,13 @@ __global__ __launch_bounds__(256) void k_stage_support(const StageDesc* __restri
 }
 
 struct FoldLaunch { size_t pre; int blocks, pass, word, lds; };
-struct Rows4Launch { size_t desc, pre; int n, blocks, word; };
 struct DftLaunch { size_t desc, pre[QSFT_DFT_MAX_PASSES]; int n, npass, blocks[QSFT_DFT_MAX_PASSES],
                    lds[QSFT_DFT_MAX_PASSES], word; };
 
 struct Batch {
     std::vector<qsft_request> req;
     std::vector<ReqLayout> lay;
-    std::vector<int> transformed;          // per request: its fold launch also does the sub-DFTs
+    std::vector<qsft_dft_desc> rest;       // per request: the sub-DFT passes its fold launches leave
     std::vector<int> sign;                 // detected delay structure per request (+1, -1, 0)
     int max_iter = 15, fuse_from = 3, max_p = 1, max_n_pad = 64;
     qsft_batch_sizes sz{};
@@ -138,7 +137,6 @@ struct Batch {
     size_t fold_desc = 0, fold_pre_phase = 0, fold_pre_rank = 0;
     int fold_phase = 0, fold_rank = 0;
     std::vector<FoldLaunch> fold;
-    std::vector<Rows4Launch> rows4;
     std::vector<DftLaunch> dft;
     size_t asm_desc = 0, asm_pre = 0;
     int asm_blocks = 0, asm_word = 0;
@@ -188,7 +186,6 @@ int build_plan(Batch& B, bool write) {
     const uintptr_t work_base = write ? (uintptr_t)B.work_dev : kFakeBase;
     PlanWriter W{B.plan_host, write};
     B.fold.clear();
-    B.rows4.clear();
     B.dft.clear();
     auto in_ptr = [&](int i, size_t off) { return (void*)(in_base + B.lay[i].in_off + off); };
     auto work_ptr = [&](int i, size_t off) { return (void*)(work_base + B.lay[i].work_off + off); };
@@ -225,7 +222,7 @@ int build_plan(Batch& B, bool write) {
         long long all_rows = 0;
         for (int i = 0; i < nreq; ++i) all_rows += (long long)B.req[i].C * B.lay[i].P;
         const int launch_rows = (int)(all_rows < 0x7FFFFFFF ? all_rows : 0x7FFFFFFF);
-        B.transformed.assign(nreq, 0);
+        B.rest.assign(nreq, qsft_dft_desc{});
         for (int i = 0; i < nreq; ++i) {
             const qsft_request& r = B.req[i];
             const ReqLayout& l = B.lay[i];
@@ -234,12 +231,13 @@ int build_plan(Batch& B, bool write) {
                                           (const int8_t*)work_ptr(i, l.k), in_ptr(i, l.a), work_ptr(i, l.x),
                                           work_ptr(i, l.fw), l.fw_bytes);
             if (rc != QSFT_OK) return rc;
-            B.transformed[i] = descs[i].fwd;
+            const int rr = qsft_fold_rest(&descs[i], &B.rest[i]);
+            if (rr != QSFT_OK) return rr;
             if (qsft_fold_blocks(&descs[i], &phase[i], &rank[i]) != 0) {
                 qsft_set_error("qsft_batch: bad evaluation shape");
                 return QSFT_ERR_ARG;
             }
-            groups[{r.q, (r.q == 4 && (r.b == 4 || r.b == 6)) ? r.b : 0}].push_back(i);
+            groups[{r.q, descs[i].rpw ? r.b : 0}].push_back(i);       // rpw: the whole-row kernel of q = 4
         }
         B.fold_desc = W.put(descs.data(), descs.size() * sizeof(qsft_fold_desc));
         B.fold_pre_phase = W.prefix(phase, &B.fold_phase);
@@ -267,46 +265,13 @@ int build_plan(Batch& B, bool write) {
         }
     }
 
-    // ---- stage (c): sub-DFTs in place on x of the rows that are more than one tile
-    // (whole-row kernel for q = 4, b in {4, 6})
-    std::map<int, std::vector<int>> fast, slow;
-    for (int i = 0; i < nreq; ++i) {
-        const qsft_request& r = B.req[i];
-        if (B.transformed[i]) continue;                            // done with the samples
-        if (r.q == 4 && (r.b == 4 || r.b == 6)) fast[r.b].push_back(i);
-        else slow[r.q].push_back(i);
-    }
-    auto dft_desc = [&](int i) {
-        const qsft_request& r = B.req[i];
-        const ReqLayout& l = B.lay[i];
-        qsft_dft_desc d{};
-        d.q = r.q; d.b = r.b; d.rows = r.C * l.P; d.in_stride = 1; d.in_row_stride = l.Q;
-        d.in = work_ptr(i, l.x);
-        d.out = work_ptr(i, l.x);
-        return d;
-    };
-    for (auto& kv : fast) {
-        std::vector<qsft_dft_desc> descs;
-        std::vector<int> rows;
-        for (int i : kv.second) {
-            descs.push_back(dft_desc(i));
-            rows.push_back(descs.back().rows);
-        }
-        Rows4Launch L{};
-        L.desc = W.put(descs.data(), descs.size() * sizeof(qsft_dft_desc));
-        L.pre = W.prefix(rows, &L.blocks);
-        L.n = (int)descs.size();
-        L.word = QSFT_F32 | (kv.first << 8);
-        B.rows4.push_back(L);
-    }
+    // ---- stage (c): the sub-DFT passes that are left, in place on x (rows of more than one tile)
+    std::map<int, std::vector<int>> slow;
+    for (int i = 0; i < nreq; ++i)
+        if (B.rest[i].n_pass > 0) slow[B.req[i].q].push_back(i);
     for (auto& kv : slow) {
         std::vector<qsft_dft_desc> descs;
-        for (int i : kv.second) {
-            qsft_dft_desc d = dft_desc(i);
-            const int rc = qsft_dft_plan(&d, QSFT_F32);
-            if (rc != QSFT_OK) return rc;
-            descs.push_back(d);
-        }
+        for (int i : kv.second) descs.push_back(B.rest[i]);
         DftLaunch L{};
         L.npass = 0;
         for (auto& d : descs) L.npass = d.n_pass > L.npass ? d.n_pass : L.npass;
@@ -641,10 +606,6 @@ int enqueue(Batch* B, int upload, const void* input_host, uint64_t seed_offset, 
     if (rc != QSFT_OK) return rc;
     for (const FoldLaunch& L : B->fold) {
         rc = qsft_fold_rows(fd, (const int32_t*)(P + L.pre), (int)B->req.size(), L.blocks, L.pass, L.word, L.lds, st);
-        if (rc != QSFT_OK) return rc;
-    }
-    for (const Rows4Launch& L : B->rows4) {
-        rc = qsft_dft4_rows((const qsft_dft_desc*)(P + L.desc), (const int32_t*)(P + L.pre), L.n, L.blocks, L.word, st);
         if (rc != QSFT_OK) return rc;
     }
     for (const DftLaunch& L : B->dft)

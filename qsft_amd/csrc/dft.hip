@@ -39,11 +39,10 @@
 
 namespace qsft {
 
-constexpr int kDftLdsBytes = 65536;                 // dynamic LDS per workgroup (at most)
 constexpr int kDftTwBytes = QSFT_MAX_Q * 16;        // twiddle table of the generic radix, after the tiles
 
-template <typename T, int QR>
-__global__ __launch_bounds__(kDftThreads) void k_dft_pass(const qsft_dft_desc* __restrict__ descs,
+template <typename T, int QR, int TH>
+__global__ __launch_bounds__(TH) void k_dft_pass(const qsft_dft_desc* __restrict__ descs,
                                                           const int32_t* __restrict__ pre, int n_inst,
                                                           int pass, int lds_bytes) {
     using C2 = cplx_t<T>;
@@ -92,7 +91,7 @@ __global__ __launch_bounds__(kDftThreads) void k_dft_pass(const qsft_dft_desc* _
             ? reinterpret_cast<const C2*>(d.in) + (int64_t)row * d.in_row_stride
             : reinterpret_cast<const C2*>(d.out) + (int64_t)row * Q;
         const int64_t stride = pass == 0 ? d.in_stride : 1;
-        for (int e = threadIdx.x; e < E; e += blockDim.x) lds[e] = in[goff(e) * stride];
+        tile_load(lds, E, [&](int e) { return in[goff(e) * stride]; });
     }
     __syncthreads();
 
@@ -100,27 +99,10 @@ __global__ __launch_bounds__(kDftThreads) void k_dft_pass(const qsft_dft_desc* _
 
     const bool last = (pass == d.n_pass - 1);
     C2* __restrict__ out = reinterpret_cast<C2*>(d.out) + (int64_t)row * Q;
-    if (last) {
-        if constexpr (sizeof(T) == 8) {
-            const double qd = (double)Q;
-            for (int e = threadIdx.x; e < E; e += blockDim.x) {
-                C2 v = cur[e];
-                v.x = v.x / qd;
-                v.y = v.y / qd;
-                out[goff(e)] = v;
-            }
-        } else {
-            const T sc = (T)(1.0 / (double)Q);
-            for (int e = threadIdx.x; e < E; e += blockDim.x) {
-                C2 v = cur[e];
-                v.x *= sc;
-                v.y *= sc;
-                out[goff(e)] = v;
-            }
-        }
-    } else {
-        for (int e = threadIdx.x; e < E; e += blockDim.x) out[goff(e)] = cur[e];
-    }
+    if (last)
+        tile_store(cur, E, [&](int e, C2 v) { out[goff(e)] = dft_scaled<T>(v, Q); });
+    else
+        tile_store(cur, E, [&](int e, C2 v) { out[goff(e)] = v; });
 }
 
 // q = 4, whole rows of Q = 4^B samples (B even), one workgroup per row,
@@ -154,10 +136,10 @@ __global__ __launch_bounds__(1 << (2 * B - 4)) void k_dft4_rows(const qsft_dft_d
         if (p > 0) {
             __syncthreads();                                       // the previous reads of lds are done
 #pragma unroll
-            for (int j = 0; j < 16; ++j) lds[dft4_pad(dft4_index(p - 1, tid, j))] = v[j];
+            for (int j = 0; j < 16; ++j) lds[dft4_pad(dft4_index(2 * (p - 1), tid, j))] = v[j];
             __syncthreads();
 #pragma unroll
-            for (int j = 0; j < 16; ++j) v[j] = lds[dft4_pad(dft4_index(p, tid, j))];
+            for (int j = 0; j < 16; ++j) v[j] = lds[dft4_pad(dft4_index(2 * p, tid, j))];
         }
 #pragma unroll
         for (int a = 0; a < 4; ++a) dft4_reg<T>(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);   // digit 2p
@@ -175,7 +157,7 @@ __global__ __launch_bounds__(1 << (2 * B - 4)) void k_dft4_rows(const qsft_dft_d
             x.x *= sc;
             x.y *= sc;
         }
-        out[dft4_index(B / 2 - 1, tid, j)] = x;
+        out[dft4_index(B - 2, tid, j)] = x;
     }
 }
 
@@ -352,6 +334,21 @@ extern "C" int qsft_dft_plan(qsft_dft_desc* h, int precision) {
     return apply_schedule(h, sc);
 }
 
+// One pass over whole rows where the planned schedule takes several and a row
+// fits the LDS of a CU. The planner's own schedules stay within 64 KiB.
+extern "C" int qsft_dft_plan_rows(qsft_dft_desc* h, int precision) {
+    const int rc = qsft_dft_plan(h, precision);
+    if (rc != QSFT_OK || h->n_pass == 1) return rc;
+    const long long elem = precision == QSFT_F32 ? 8 : 16, Q = ipow_ll(h->q, h->b);
+    const long long bytes = radix_compiled(h->q) ? Q * elem : (2 * Q + h->q) * elem;
+    if (bytes > kRowLdsBytes) return rc;
+    Sched sc;
+    sc.np = 1;
+    sc.d1[0] = h->b;
+    sc.ti[0] = sc.ta[0] = 1;
+    return apply_schedule(h, sc);
+}
+
 // The planner's candidate number `index` (0 = the model's best; the order
 // qsft_dft_autotune tries them in); QSFT_ERR_ARG past the last one.
 extern "C" int qsft_dft_plan_candidate(qsft_dft_desc* h, int precision, int index) {
@@ -373,20 +370,33 @@ extern "C" int qsft_dft_lds_bytes(const qsft_dft_desc* h, int pass, int precisio
     const long long elem = (precision == QSFT_F32) ? 8 : 16;
     const long long E = ipow_ll(h->q, h->pass_d1[pass] - h->pass_d0[pass]) * h->pass_ti[pass] * h->pass_ta[pass];
     const long long bytes = radix_compiled(h->q) ? E * elem : 2 * E * elem + (long long)h->q * elem;
-    return bytes > kDftLdsBytes ? -1 : (int)(bytes < 16 ? 16 : bytes);
+    return bytes > kRowLdsBytes ? -1 : (int)(bytes < 16 ? 16 : bytes);
+}
+
+template <typename T, int QR>
+static void launch_dft_pass(const qsft_dft_desc* d, const int32_t* pre, int n_inst, int blocks, int pass, int lds,
+                            hipStream_t st) {
+    if (lds > kDftLdsBytes)
+        hipLaunchKernelGGL((k_dft_pass<T, QR, row_threads<T>()>), dim3(blocks), dim3(row_threads<T>()), (size_t)lds, st,
+                           d, pre, n_inst, pass, lds);
+    else if (lds > kDftMidBytes && pass == 0)
+        hipLaunchKernelGGL((k_dft_pass<T, QR, kDftMidThreads>), dim3(blocks), dim3(kDftMidThreads), (size_t)lds, st, d,
+                           pre, n_inst, pass, lds);
+    else
+        hipLaunchKernelGGL((k_dft_pass<T, QR, kDftThreads>), dim3(blocks), dim3(kDftThreads), (size_t)lds, st, d, pre,
+                           n_inst, pass, lds);
 }
 
 template <typename T>
 static hipError_t launch_dft(int radix, const qsft_dft_desc* d, const int32_t* pre, int n_inst, int blocks,
                              int pass, int lds, hipStream_t st) {
-    const size_t sh = (size_t)lds;
     switch (radix) {
-        case 2: hipLaunchKernelGGL((k_dft_pass<T, 2>), dim3(blocks), dim3(kDftThreads), sh, st, d, pre, n_inst, pass, lds); break;
-        case 3: hipLaunchKernelGGL((k_dft_pass<T, 3>), dim3(blocks), dim3(kDftThreads), sh, st, d, pre, n_inst, pass, lds); break;
-        case 4: hipLaunchKernelGGL((k_dft_pass<T, 4>), dim3(blocks), dim3(kDftThreads), sh, st, d, pre, n_inst, pass, lds); break;
-        case 5: hipLaunchKernelGGL((k_dft_pass<T, 5>), dim3(blocks), dim3(kDftThreads), sh, st, d, pre, n_inst, pass, lds); break;
-        case 20: hipLaunchKernelGGL((k_dft_pass<T, 20>), dim3(blocks), dim3(kDftThreads), sh, st, d, pre, n_inst, pass, lds); break;
-        default: hipLaunchKernelGGL((k_dft_pass<T, 0>), dim3(blocks), dim3(kDftThreads), sh, st, d, pre, n_inst, pass, lds); break;
+        case 2: launch_dft_pass<T, 2>(d, pre, n_inst, blocks, pass, lds, st); break;
+        case 3: launch_dft_pass<T, 3>(d, pre, n_inst, blocks, pass, lds, st); break;
+        case 4: launch_dft_pass<T, 4>(d, pre, n_inst, blocks, pass, lds, st); break;
+        case 5: launch_dft_pass<T, 5>(d, pre, n_inst, blocks, pass, lds, st); break;
+        case 20: launch_dft_pass<T, 20>(d, pre, n_inst, blocks, pass, lds, st); break;
+        default: launch_dft_pass<T, 0>(d, pre, n_inst, blocks, pass, lds, st); break;
     }
     return hipGetLastError();
 }
@@ -398,7 +408,7 @@ static hipError_t launch_dft(int radix, const qsft_dft_desc* d, const int32_t* p
 extern "C" int qsft_dft_pass(const qsft_dft_desc* d, const int32_t* pre, int n_inst, int blocks, int pass,
                              int precision, int lds_bytes, void* stream) {
     if (!d || !pre || n_inst < 1 || blocks < 0 || pass < 0 || pass >= QSFT_DFT_MAX_PASSES || lds_bytes < 16 ||
-        lds_bytes > kDftLdsBytes) {
+        lds_bytes > kRowLdsBytes) {
         qsft_set_error("qsft_dft_pass: bad arguments");
         return QSFT_ERR_ARG;
     }

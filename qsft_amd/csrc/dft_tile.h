@@ -6,7 +6,19 @@
 
 namespace qsft {
 
+// Workgroups of the tile kernels by their LDS: 256 threads up to 32 KiB (four
+// and more per CU), 512 up to 64 KiB (two per CU; a strided pass, bound by its
+// loads, stays at 256: 134 against 149 us on a serving mix's q = 20, b = 4
+// rows), and for whole rows beyond that, at most 144 of the 160 KiB of a CU, as
+// many as the registers allow. q = 20, b = 3: the samples of 102 rows in FP32
+// (64 KiB) 19.6 us with 256 threads, 13.4 with 512; their FP64 sub-DFT 29 us in
+// two passes, 17 as whole rows of 128 KiB.
 constexpr int kDftThreads = 256;
+constexpr int kDftMidBytes = 32768;
+constexpr int kDftMidThreads = 512;
+constexpr int kDftLdsBytes = 65536;
+constexpr int kRowLdsBytes = 147456;
+template <typename T> constexpr int row_threads() { return sizeof(T) == 8 ? 512 : 1024; }
 
 template <typename T>
 __device__ __forceinline__ cplx_t<T> cmul(cplx_t<T> a, cplx_t<T> b) {
@@ -142,6 +154,46 @@ __host__ __device__ __forceinline__ bool radix_compiled(int q) {
     return q == 2 || q == 3 || q == 4 || q == 5 || q == 20;
 }
 
+// A tile of E elements into LDS, get(e) being the global load of element e:
+// kTileLoads loads of a thread are in flight together (one at a time, each
+// waited for before the next was issued, a 64 KiB tile of 256 threads spent 31
+// memory latencies on its way in).
+constexpr int kTileLoads = 8;
+template <typename C2, typename G>
+__device__ __forceinline__ void tile_load(C2* lds, int E, G get) {
+    for (int e0 = threadIdx.x; e0 < E; e0 += kTileLoads * blockDim.x) {
+        C2 v[kTileLoads];
+#pragma unroll
+        for (int k = 0; k < kTileLoads; ++k) {
+            const int e = e0 + k * blockDim.x;
+            if (e < E) v[k] = get(e);
+        }
+#pragma unroll
+        for (int k = 0; k < kTileLoads; ++k) {
+            const int e = e0 + k * blockDim.x;
+            if (e < E) lds[e] = v[k];
+        }
+    }
+}
+
+// And out again: put(e, value).
+template <typename C2, typename F>
+__device__ __forceinline__ void tile_store(const C2* lds, int E, F put) {
+    for (int e0 = threadIdx.x; e0 < E; e0 += kTileLoads * blockDim.x) {
+        C2 v[kTileLoads];
+#pragma unroll
+        for (int k = 0; k < kTileLoads; ++k) {
+            const int e = e0 + k * blockDim.x;
+            if (e < E) v[k] = lds[e];
+        }
+#pragma unroll
+        for (int k = 0; k < kTileLoads; ++k) {
+            const int e = e0 + k * blockDim.x;
+            if (e < E) put(e, v[k]);
+        }
+    }
+}
+
 // The axis transforms of a tile of E elements, [.., q^mb, ti] with its mb axes
 // innermost first (axis t has stride q^(mb-1-t) ti in the tile), by the whole
 // workgroup, which has synchronised after filling `cur`. The generic radix is
@@ -183,16 +235,16 @@ __device__ __forceinline__ cplx_t<T> dft_scaled(cplx_t<T> v, int Q) {
     return cplx_t<T>{v.x * sc, v.y * sc};
 }
 
-// element index of register j of thread tid when the thread holds digits 2p, 2p+1
-__device__ __forceinline__ int dft4_index(int p, int tid, int j) {
-    const int lo = 4 * p;
+// q = 4, whole rows held 16 samples a thread: element index of register j when
+// the thread holds digits w, w + 1 (base-4 digit t at bits 2t, 2t + 1)
+__device__ __forceinline__ int dft4_index(int w, int tid, int j) {
+    const int lo = 2 * w;
     return ((tid >> lo) << (lo + 4)) | (j << lo) | (tid & ((1 << lo) - 1));
 }
 __device__ __forceinline__ int dft4_pad(int i) { return i + (i >> 4); }
-// dft4_pad(dft4_index(p, tid, j)) = dft4_lds_base(p, tid) + j dft4_lds_step(p):
-// one address per register pass, the 16 elements at immediate offsets
-__device__ __forceinline__ int dft4_lds_base(int p, int tid) { return dft4_pad(dft4_index(p, tid, 0)); }
-__device__ __forceinline__ constexpr int dft4_lds_step(int p) { return p == 0 ? 1 : 17 << (4 * p - 4); }
-
+// dft4_pad(dft4_index(w, tid, j)) = dft4_lds_base(w, tid) + j dft4_lds_step(w) for
+// w = 0 or w >= 2: one address per window, the 16 elements at immediate offsets
+__device__ __forceinline__ int dft4_lds_base(int w, int tid) { return dft4_pad(dft4_index(w, tid, 0)); }
+__device__ __forceinline__ constexpr int dft4_lds_step(int w) { return w == 0 ? 1 : 17 << (2 * w - 4); }
 
 }  // namespace qsft

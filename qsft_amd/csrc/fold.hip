@@ -23,8 +23,8 @@
 //     kernel.
 //   * k_fold_pass / k_fold4_rows: a workgroup clears a tile of bins of one row
 //     in LDS, adds the tile's terms and runs the
-//     inverse transform over the tile's axes; k_fold4_rows (q = 4, b in
-//     {4, 6}) does the whole row, two digits at a time in registers. Rows
+//     inverse transform over the tile's axes; k_fold4_rows (q = 4, b = 4
+//     .. 7) does the whole row, two digits at a time in registers. Rows
 //     larger than a tile take further k_fold_pass passes in place.
 //
 // The inverse transform is the forward one with the real and imaginary parts
@@ -191,13 +191,14 @@ __global__ __launch_bounds__(kRankThreads) void k_fold_rank(const SRC src) {
 }
 
 // The terms of one row are added to their bins in LDS by the waves of a
-// workgroup. Wave `wave` of `waves` takes an equal share of the sorted
-// positions [lo, hi) of the group, moved to the ends of runs (the terms of one
-// bin), so no two waves touch a bin and none waits for another. 64 terms at a
-// time: each lane forms one, a segmented scan over the run (as many steps as
-// the longest run in the block needs) leaves a run's sum in its last lane,
-// which adds it. Equal shares keep a row's time even where one bin holds
-// most of the terms (supports of low weight), and the order of every sum
+// workgroup. Wave `wave` of `waves` takes an equal share of the blocks of 64
+// sorted positions that hold [lo, hi) of the group, moved to the ends of runs
+// (the terms of one bin), so no two waves touch a bin and none waits for
+// another. A block at a time: each lane forms one term, a segmented scan over
+// the run (as many steps as the longest run in the block needs) leaves a run's
+// sum in its last lane, which adds it. Equal shares keep a row's time even
+// where one bin holds most of the terms (supports of low weight). The blocks
+// are the same for every tile and workgroup size, so the order of a sum
 // depends on the sorted positions only.
 //
 // What a lane needs of its position, the same for every row of the group:
@@ -214,9 +215,12 @@ constexpr int kTermWhole = 256;      // ... and the run lies inside the block: i
 struct TermShare {
     int lo, hi, first, last;
     bool started;        // a run that began before `first` is another wave's
-    __device__ __forceinline__ TermShare(int lo_, int hi_, int wave, int waves)
-        : lo(lo_), hi(hi_), first(lo_ + (int)((int64_t)(hi_ - lo_) * wave / waves)),
-          last(lo_ + (int)((int64_t)(hi_ - lo_) * (wave + 1) / waves)), started(first == lo_) {}
+    __device__ __forceinline__ TermShare(int lo_, int hi_, int wave, int waves) : lo(lo_), hi(hi_) {
+        const int b0 = lo >> 6, nb = hi > lo ? ((hi + 63) >> 6) - b0 : 0;
+        first = (b0 + (int)((int64_t)nb * wave / waves)) << 6;
+        last = (b0 + (int)((int64_t)nb * (wave + 1) / waves)) << 6;
+        started = first <= lo;
+    }
     // Loads the block of 64 positions from i0; false once the share has ended.
     __device__ __forceinline__ bool load(const qsft_fold_desc& d, int c, int i0, Term& t) {
         const int lane = threadIdx.x & 63;
@@ -228,17 +232,17 @@ struct TermShare {
         const QSFT_GLOBAL gd2* __restrict__ as =
             reinterpret_cast<const QSFT_GLOBAL gd2*>(gptr(d.as)) + (size_t)c * d.S;
         const int i = i0 + lane;
-        const bool in = i < hi;
+        const bool in = i >= lo && i < hi;
         const uint64_t k = in ? key[i] : ~0ull;
         const uint32_t kp = (in && i > lo) ? (uint32_t)(key[i - 1] >> 32) : 0xFFFFFFFFu;
-        const uint32_t kn = (i + 1 < hi) ? (uint32_t)(key[i + 1] >> 32) : 0xFFFFFFFFu;
+        const uint32_t kn = (in && i + 1 < hi) ? (uint32_t)(key[i + 1] >> 32) : 0xFFFFFFFFu;
         if (in) t.a = as[i];
         t.j = (uint32_t)(k >> 32);
         t.s = (uint32_t)k;
         const bool begins = in && t.j != kp;                       // first term of its bin
         const uint64_t bm = __ballot(begins);
         const uint64_t past = __ballot(begins && i >= last);       // the runs of the next share
-        int from = 0, to = min(64, hi - i0);
+        int from = max(0, lo - i0), to = min(64, hi - i0);
         if (!started) from = bm ? __builtin_ctzll(bm) : 64;
         if (past) to = min(to, (int)__builtin_ctzll(past));
         if (from < to) {
@@ -315,8 +319,8 @@ __device__ __forceinline__ const QSFT_GLOBAL uint8_t* phase_row(const qsft_fold_
 // first pass (FIRST: the innermost axes, so a tile is a contiguous run of
 // bins) folds its terms into the tile; later passes read x. Between passes x
 // holds the swapped parts; the last pass swaps back.
-template <typename T, int QR, bool FIRST, typename SRC>
-__global__ __launch_bounds__(kDftThreads) void k_fold_pass(const SRC src, int pass, int lds_bytes) {
+template <typename T, int QR, bool FIRST, int TH, typename SRC>
+__global__ __launch_bounds__(TH) void k_fold_pass(const SRC src, int pass, int lds_bytes) {
     using C2 = cplx_t<T>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ double2 tab[QSFT_MAX_Q];
@@ -367,7 +371,7 @@ __global__ __launch_bounds__(kDftThreads) void k_fold_pass(const SRC src, int pa
             hi = st[1];
         }
         const QSFT_GLOBAL uint8_t* ph = phase_row(d, c, row - c * d.P);
-        fold_terms(d, c, lo, hi, threadIdx.x >> 6, kDftThreads / 64,
+        fold_terms(d, c, lo, hi, threadIdx.x >> 6, TH / 64,
                    [&](const Term& t, double& sx, double& sy) {
                        const double2 w = tab[ph[t.s]];
                        sx = t.a.x * w.x - t.a.y * w.y;
@@ -375,21 +379,22 @@ __global__ __launch_bounds__(kDftThreads) void k_fold_pass(const SRC src, int pa
                    },
                    [&](const Term& t, double sx, double sy) { bin_put<T>(lds[t.j - (uint32_t)base], t, sx, sy); });
     } else {
-        for (int e = threadIdx.x; e < E; e += blockDim.x) lds[e] = x[goff(e)];
+        tile_load(lds, E, [&](int e) { return x[goff(e)]; });
     }
     __syncthreads();
     C2* cur = tile_axes<T, QR>(lds, lds + E, E, q, mb, ti, tw);
-    if (FIRST && d.fwd) {
-        // the tile holds whole rows of samples: their sub-transform, scaled by
-        // q^-b as k_dft_pass scales it
+    if (d.fwd && pass == d.n_pass - 1) {
+        // the tile now holds samples: back along the same axes, scaled by q^-b as
+        // k_dft_pass scales it if these are all (else its last pass does that)
         for (int e = threadIdx.x; e < E; e += blockDim.x) cur[e] = C2{cur[e].y, cur[e].x};
         __syncthreads();
         cur = tile_axes<T, QR>(cur, cur == lds ? lds + E : lds, E, q, mb, ti, tw);
-        for (int e = threadIdx.x; e < E; e += blockDim.x) x[base + e] = dft_scaled<T>(cur[e], Q);
+        if (FIRST) tile_store(cur, E, [&](int e, C2 v) { x[goff(e)] = dft_scaled<T>(v, Q); });
+        else tile_store(cur, E, [&](int e, C2 v) { x[goff(e)] = v; });
     } else if (pass == d.n_pass - 1) {
-        for (int e = threadIdx.x; e < E; e += blockDim.x) x[goff(e)] = C2{cur[e].y, cur[e].x};
+        tile_store(cur, E, [&](int e, C2 v) { x[goff(e)] = C2{v.y, v.x}; });
     } else {
-        for (int e = threadIdx.x; e < E; e += blockDim.x) x[goff(e)] = cur[e];
+        tile_store(cur, E, [&](int e, C2 v) { x[goff(e)] = v; });
     }
 }
 
@@ -401,9 +406,17 @@ __global__ __launch_bounds__(kDftThreads) void k_fold_pass(const SRC src, int pa
 // before its first LDS write. Terms that do not fit the registers, or phases
 // their LDS buffer, are read per row.
 //
-// With d.fwd the row's samples are transformed back to its sub-transform
-// before they leave the registers (digit pairs 2, 0, 1 for B = 6: the first
-// needs no exchange, the last stores 128-byte segments), and x receives that.
+// A thread's 16 samples differ in the two digits of a window. The inverse
+// transform runs through the windows 0, 2, 4 (two digits each), an odd B ends
+// with the window of its two top digits, of which only the last is left. With
+// d.fwd the row's samples are transformed back to its sub-transform before
+// they leave the registers (the last window first, which needs no exchange,
+// then the others upwards, so that the stores are 128-byte segments), and x
+// receives that.
+// 64 instances of q = 4, S = 1000, b = 6, P = 102 in FP32: 0.227 ms for the
+// samples and 0.268 ms for k_dft4_rows as two launches, 0.214 ms in one (3.0
+// TB/s of writes: bound by the chain of exchanges at four waves per SIMD, all
+// that 34 KiB of LDS a row allow).
 typedef float gf2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void store_c2(QSFT_GLOBAL float2* p, float2 v) {
     *reinterpret_cast<QSFT_GLOBAL gf2*>(p) = gf2{v.x, v.y};
@@ -413,19 +426,25 @@ __device__ __forceinline__ void store_c2(QSFT_GLOBAL double2* p, double2 v) {
 }
 
 template <int B>
-constexpr int fold4_rows() { return B == 4 ? 4 : 1; }             // b = 4: four rows of 16 threads fill a wave
+constexpr int fold4_rows() { return B <= 5 ? 4 : 1; }             // rows of 16 (b = 4) or 64 threads at a time
+template <int B>
+constexpr int fold4_threads() { return fold4_rows<B>() << (2 * B - 4); }
+template <int B>
+constexpr int fold4_phases() { return B == 6 ? 4096 : B == 7 ? 8192 : 0; }   // phases of one row in LDS
 constexpr int kTermBlocks = 4;       // blocks of 64 terms a wave keeps in registers
-constexpr int kPhaseBytes = 4096;    // phases of one row in LDS (b = 6)
+// window k of the inverse transform: its lower digit
+template <int B>
+__device__ __forceinline__ constexpr int fold4_window(int k) { return 2 * k < B - 1 ? 2 * k : B - 2; }
 
 template <typename T, int B, bool FWD, typename SRC>
-__global__ __launch_bounds__(fold4_rows<B>() << (2 * B - 4)) __attribute__((
+__global__ __launch_bounds__(fold4_threads<B>()) __attribute__((
     amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2))) void k_fold4_rows(const SRC src) {
     using C2 = cplx_t<T>;
     constexpr int Q = 1 << (2 * B), kTpr = Q / 16, kRows = fold4_rows<B>(), kThreads = kRows * kTpr;
-    constexpr bool kPhLds = B == 6;
-    static_assert(B == 4 || B == 6, "two digits per register pass");
+    constexpr int kPhases = fold4_phases<B>(), kWindows = (B + 1) / 2;
+    static_assert(B >= 4 && B <= 7, "16 samples a thread, at most 1024 threads a row");
     __shared__ __align__(16) C2 lds_all[kRows][Q + Q / 16];
-    __shared__ __align__(16) uint8_t phl[kPhLds ? kPhaseBytes : 16];
+    __shared__ __align__(16) uint8_t phl[kPhases ? kPhases : 16];
     int local;
     const qsft_fold_desc& d = src.at(blockIdx.x, local);
     if (d.q != 4 || d.b != B || (d.fwd != 0) != FWD) return;       // launched for other shapes
@@ -433,7 +452,7 @@ __global__ __launch_bounds__(fold4_rows<B>() << (2 * B - 4)) __attribute__((
     const int c = local / wpg, p0 = (local - c * wpg) * per, p1 = min(P, p0 + per);
     const int sub = threadIdx.x / kTpr, tid = threadIdx.x % kTpr, wave = threadIdx.x >> 6;
     C2* lds = lds_all[sub];
-    const bool phases_staged = kPhLds && Sp <= kPhaseBytes;
+    const bool phases_staged = Sp <= kPhases;
     gu4 ph_next = {0, 0, 0, 0};                                    // the next row's phases, 16 per thread
     auto fetch = [&](int p) {
         if (phases_staged && 16 * (int)threadIdx.x < Sp)
@@ -490,7 +509,7 @@ __global__ __launch_bounds__(fold4_rows<B>() << (2 * B - 4)) __attribute__((
         }
         __syncthreads();
         C2 v[16];
-        auto exchange = [&](int from, int to) {                     // registers hold digit pair `from`, then `to`
+        auto exchange = [&](int from, int to) {                     // registers hold window `from`, then `to`
             if (from >= 0) {
                 __syncthreads();                                   // the previous reads of lds are done
                 C2* w = lds + dft4_lds_base(from, tid);
@@ -502,16 +521,19 @@ __global__ __launch_bounds__(fold4_rows<B>() << (2 * B - 4)) __attribute__((
 #pragma unroll
             for (int j = 0; j < 16; ++j) v[j] = r[j * dft4_lds_step(to)];
         };
-        auto digits = [&]() {                                      // the transforms along the pair in registers
+        // the transforms along the digits of the window that are its own
+        auto digits = [&](int w) {
+            if (w % 2 == 0) {
 #pragma unroll
-            for (int a = 0; a < 4; ++a) dft4_reg<T>(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);
+                for (int a = 0; a < 4; ++a) dft4_reg<T>(v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]);
+            }
 #pragma unroll
             for (int a = 0; a < 4; ++a) dft4_reg<T>(v[a], v[a + 4], v[a + 8], v[a + 12]);
         };
 #pragma unroll
-        for (int k = 0; k < B / 2; ++k) {
-            exchange(k - 1, k);
-            digits();
+        for (int k = 0; k < kWindows; ++k) {
+            exchange(k ? fold4_window<B>(k - 1) : -1, fold4_window<B>(k));
+            digits(fold4_window<B>(k));
         }
         int row = c * P + p;
         __asm__ volatile("" : "+s"(row));                          // not an induction variable per store address
@@ -521,21 +543,21 @@ __global__ __launch_bounds__(fold4_rows<B>() << (2 * B - 4)) __attribute__((
         if constexpr (FWD) {
 #pragma unroll
             for (int j = 0; j < 16; ++j) v[j] = C2{v[j].y, v[j].x};   // the samples
-            digits();                                              // pair B / 2 - 1, still in registers
-            exchange(B / 2 - 1, 0);
-            digits();
-            if constexpr (B == 6) {
-                exchange(0, 1);
-                digits();
+            digits(B - 2);                                         // the last window, still in registers
+#pragma unroll
+            for (int k = 0; k < kWindows - 1; ++k) {
+                exchange(k ? fold4_window<B>(k - 1) : B - 2, fold4_window<B>(k));
+                digits(fold4_window<B>(k));
             }
             if (live) {
+                constexpr int w = fold4_window<B>(kWindows - 2);
 #pragma unroll
                 for (int j = 0; j < 16; ++j)
-                    store_c2(x + (xo + dft4_index(B / 2 - 2, tid, 0) + (j << (4 * (B / 2 - 2)))), dft_scaled<T>(v[j], Q));
+                    store_c2(x + (xo + dft4_index(w, tid, 0) + (j << (2 * w))), dft_scaled<T>(v[j], Q));
             }
         } else if (live) {
 #pragma unroll
-            for (int j = 0; j < 16; ++j) store_c2(x + (xo + tid + j * kTpr), C2{v[j].y, v[j].x});
+            for (int j = 0; j < 16; ++j) store_c2(x + (xo + tid + j * kTpr), C2{v[j].y, v[j].x});   // (window B - 2)
         }
     }
 }
@@ -551,7 +573,8 @@ namespace {
 
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-bool fold_rows4(int q, int b) { return q == 4 && (b == 4 || b == 6); }
+// rows that k_fold4_rows takes: q = 4, b = 4..6, and in FP32 b = 7 (139 KiB of LDS)
+bool fold_rows4(int q, int b, int precision) { return q == 4 && b >= 4 && b <= (precision == QSFT_F32 ? 7 : 6); }
 
 bool fold_shape_ok(int q, int n, int b, int C, int P, int S, int n_pad) {
     if (q < 2 || q > QSFT_MAX_Q || b < 1 || b > QSFT_MAX_B || n < 1 || n > n_pad || n_pad % 64 || n_pad > QSFT_MAX_N ||
@@ -603,11 +626,11 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
     w += al256((size_t)C * S * 4);
     d.start = reinterpret_cast<int32_t*>(w);
     const int Q = ipow(q, b);
-    if (fold_rows4(q, b)) {
+    if (fold_rows4(q, b, precision)) {
         // rows of a group per workgroup: one where the launch has fewer rows than
         // the chip holds (256 CUs x 4 workgroups), up to four where it has many
         d.rpw = launch_rows >= 8192 ? 4 : launch_rows >= 4096 ? 2 : 1;
-        const int per = d.rpw * (b == 4 ? fold4_rows<4>() : fold4_rows<6>());
+        const int per = d.rpw * (b <= 5 ? fold4_rows<4>() : fold4_rows<6>());
         d.n_pass = 1;
         d.pass_d1[0] = b;
         d.pass_ti[0] = 1;
@@ -617,9 +640,10 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
         d.tiles = 1;
         d.tile_bins = Q;
     } else {
-        qsft_dft_desc s{};                                         // the sub-DFT planner's schedule, innermost first
+        // whole rows where they fit the LDS, else the sub-DFT planner's schedule, innermost first
+        qsft_dft_desc s{};
         s.q = q; s.b = b; s.rows = C * P; s.in_stride = 1; s.in_row_stride = Q;
-        const int rc = qsft_dft_plan(&s, precision);
+        const int rc = qsft_dft_plan_rows(&s, precision);
         if (rc != QSFT_OK) return rc;
         d.n_pass = s.n_pass;
         for (int p = 0; p < s.n_pass; ++p) {
@@ -637,8 +661,35 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
         d.tile_bins = ipow(q, b - s.pass_d0[0]) * s.pass_ta[0];   // whole innermost axes: contiguous bins
         d.tiles = Q / d.tile_bins;
     }
-    d.fwd = transform && d.n_pass == 1;                            // whole rows in one tile
+    d.fwd = transform != 0;
     *h = d;
+    return QSFT_OK;
+}
+
+// The forward passes a fwd descriptor's launches leave: those over the axes of
+// every pass but the last, in place on x (n_pass 0: none).
+extern "C" int qsft_fold_rest(const qsft_fold_desc* h, qsft_dft_desc* out) {
+    if (!h || !out || !h->fwd || h->n_pass < 1) {
+        qsft_set_error("qsft_fold_rest: a descriptor bound with transform is needed");
+        return QSFT_ERR_ARG;
+    }
+    qsft_dft_desc r{};
+    r.q = h->q;
+    r.b = h->b;
+    r.rows = h->C * h->P;
+    r.in_stride = 1;
+    r.in_row_stride = ipow(h->q, h->b);
+    r.in = h->x;
+    r.out = h->x;
+    r.n_pass = h->n_pass - 1;
+    for (int p = 0; p < r.n_pass; ++p) {
+        r.pass_d0[p] = h->pass_d0[p];
+        r.pass_d1[p] = h->pass_d1[p];
+        r.pass_ti[p] = h->pass_ti[p];
+        r.pass_ta[p] = h->pass_ta[p];
+        r.pass_blocks[p] = h->pass_blocks[p];
+    }
+    *out = r;
     return QSFT_OK;
 }
 
@@ -678,23 +729,35 @@ int launch_prep(const SRC& src, int phase_blocks, int rank_blocks, hipStream_t s
 
 template <typename T, int QR, typename SRC>
 void launch_pass(const SRC& src, int blocks, int pass, int lds, hipStream_t st) {
-    if (pass == 0)
-        hipLaunchKernelGGL((k_fold_pass<T, QR, true, SRC>), dim3(blocks), dim3(kDftThreads), (size_t)lds, st, src, pass,
-                           lds);
+    const dim3 g(blocks), th(kDftThreads), mid(kDftMidThreads), big(row_threads<T>());
+    const size_t sh = (size_t)lds;
+    if (lds > kDftLdsBytes)                                        // whole rows: the first pass is the only one
+        hipLaunchKernelGGL((k_fold_pass<T, QR, true, row_threads<T>(), SRC>), g, big, sh, st, src, pass, lds);
+    else if (pass == 0 && lds > kDftMidBytes)
+        hipLaunchKernelGGL((k_fold_pass<T, QR, true, kDftMidThreads, SRC>), g, mid, sh, st, src, pass, lds);
+    else if (pass == 0)
+        hipLaunchKernelGGL((k_fold_pass<T, QR, true, kDftThreads, SRC>), g, th, sh, st, src, pass, lds);
     else
-        hipLaunchKernelGGL((k_fold_pass<T, QR, false, SRC>), dim3(blocks), dim3(kDftThreads), (size_t)lds, st, src, pass,
-                           lds);
+        hipLaunchKernelGGL((k_fold_pass<T, QR, false, kDftThreads, SRC>), g, th, sh, st, src, pass, lds);
+}
+
+template <typename T, int B, typename SRC>
+void launch_rows4(bool fwd, const SRC& src, int blocks, hipStream_t st) {
+    if (fwd) hipLaunchKernelGGL((k_fold4_rows<T, B, true, SRC>), dim3(blocks), dim3(fold4_threads<B>()), 0, st, src);
+    else hipLaunchKernelGGL((k_fold4_rows<T, B, false, SRC>), dim3(blocks), dim3(fold4_threads<B>()), 0, st, src);
 }
 
 template <typename T, typename SRC>
 int launch_rows(int q, int b, bool fwd, const SRC& src, int blocks, int pass, int lds, hipStream_t st) {
     if (blocks == 0) return QSFT_OK;
-    if (fold_rows4(q, b)) {
-        const dim3 g(blocks), t4(fold4_rows<4>() * 16), t6(fold4_rows<6>() * 256);
-        if (b == 4 && fwd) hipLaunchKernelGGL((k_fold4_rows<T, 4, true, SRC>), g, t4, 0, st, src);
-        else if (b == 4) hipLaunchKernelGGL((k_fold4_rows<T, 4, false, SRC>), g, t4, 0, st, src);
-        else if (fwd) hipLaunchKernelGGL((k_fold4_rows<T, 6, true, SRC>), g, t6, 0, st, src);
-        else hipLaunchKernelGGL((k_fold4_rows<T, 6, false, SRC>), g, t6, 0, st, src);
+    if (fold_rows4(q, b, sizeof(T) == 4 ? QSFT_F32 : QSFT_F64)) {
+        switch (b) {
+            case 4: launch_rows4<T, 4>(fwd, src, blocks, st); break;
+            case 5: launch_rows4<T, 5>(fwd, src, blocks, st); break;
+            case 6: launch_rows4<T, 6>(fwd, src, blocks, st); break;
+            default:
+                if constexpr (sizeof(T) == 4) launch_rows4<T, 7>(fwd, src, blocks, st);
+        }
     } else {
         switch (q) {
             case 2: launch_pass<T, 2>(src, blocks, pass, lds, st); break;
@@ -725,8 +788,8 @@ extern "C" int qsft_fold_rows(const qsft_fold_desc* d, const int32_t* pre, int n
     const int prec = word & 0xF, q = (word >> 8) & 0xFF, b = (word >> 16) & 0xFF;
     const bool fwd = (word >> 24) & 1;
     if (!d || !pre || n_inst < 1 || blocks < 0 || pass < 0 || pass >= QSFT_DFT_MAX_PASSES || lds_bytes < 16 ||
-        lds_bytes > 65536 || (prec != QSFT_F32 && prec != QSFT_F64) || q < 2 || q > QSFT_MAX_Q ||
-        (fold_rows4(q, b) && pass != 0)) {
+        lds_bytes > kRowLdsBytes || (lds_bytes > kDftLdsBytes && pass != 0) || (prec != QSFT_F32 && prec != QSFT_F64) || q < 2 || q > QSFT_MAX_Q ||
+        (fold_rows4(q, b, prec) && pass != 0)) {
         qsft_set_error("qsft_fold_rows: bad arguments");
         return QSFT_ERR_ARG;
     }

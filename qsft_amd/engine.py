@@ -7,7 +7,7 @@ workspace per instance, builds every stage's descriptors once, and then
 
     stage (a)+(b)  eval      x[c][p][l] = sum_s a_s w^{<M_c l + d_p, k_s>}   (FP32 or FP64)
     stage (c)      DFT       in place, x -> q^-b fftn over [q]*b (in the evaluation's
-                             launch where a row is one tile)
+                             launches as far as a tile of samples allows)
     get_MDU step   assemble  FP64 working copy + transform-domain noise (Philox)
     stage (d)      peel      device loop (no host sync), finalize, pack
 
@@ -185,7 +185,7 @@ class Batch:
                 pl[-1]["sparse"] = dict(x=x, sigma=sigma)
         if eval_mode == "fold":
             self.eval = K.EvalFold(ev, code, transform=True)
-            df = [it for it, done in zip(df, self.eval.transformed) if not done]   # the others' sub-transforms
+            df = self.eval.rest                                    # what is left of the sub-transforms
         else:
             self.eval = K.EvalMfma(ev) if eval_mode == "mfma" else K.EvalCosets(ev, code)
         self.dft = K.Dft(df, code)

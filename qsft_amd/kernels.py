@@ -215,8 +215,9 @@ class EvalFold:
     items: dicts q, n, b, C, P, S, Mt, D, K, a (complex64 or complex128 [S]),
     x (complex [C][P][q^b]), optional shared_d (every group uses the delay
     rows of group 0). The workspace is allocated here, one per instance.
-    transform: x receives the sub-transforms of the samples wherever a row is
-    one tile (`transformed[i]`), in the same launch; the samples elsewhere.
+    transform: x receives the sub-transforms of the samples, transformed in the
+    same launch where a row is one tile; elsewhere `rest` (Dft items) are the
+    passes that Dft still has to run.
     """
 
     def __init__(self, items, precision, transform=False):
@@ -246,11 +247,16 @@ class EvalFold:
             descs.append(d)
             phase.append(pb.value)
             rank.append(rb.value)
-        self.transformed = [bool(d.fwd) for d in descs]
+        self.rest = []
+        for it, d in zip(items, descs):
+            if transform and d.n_pass > 1:
+                r = L.DftDesc()
+                L.check(lib.qsft_fold_rest(ctypes.byref(d), ctypes.byref(r)), "qsft_fold_rest")
+                self.rest.append(dict(q=d.q, b=d.b, rows=r.rows, inp=it["x"], out=it["x"], desc=r))
         # rows: one launch per (q, b) of the whole-row kernel, per q and pass otherwise
         groups = defaultdict(list)
         for i, d in enumerate(descs):
-            groups[(d.q, d.b if d.q == 4 and d.b in (4, 6) else 0)].append(i)
+            groups[(d.q, d.b if d.rpw else 0)].append(i)          # rpw: the whole-row kernel of q = 4
         order = [i for ix in groups.values() for i in ix]
         sd = [descs[i] for i in order]
         lists = [[phase[i] for i in order], [rank[i] for i in order]]
@@ -365,7 +371,8 @@ def eval_points(items, precision):
 
 
 class Dft:
-    """items: dicts q, b, rows, inp (tensor), in_stride, in_row_stride, out (tensor [rows][q^b]).
+    """items: dicts q, b, rows, inp (tensor), in_stride, in_row_stride, out (tensor [rows][q^b]),
+    optional desc (a planned descriptor to run as it is, see EvalFold).
     rows4: q = 4, b in {4, 6} contiguous rows go to the whole-row kernel."""
 
     def __init__(self, items, precision, rows4=True, candidate=None):
@@ -374,7 +381,7 @@ class Dft:
         groups = defaultdict(list)
         fast = defaultdict(list)
         for it in items:
-            if rows4 and it["q"] == 4 and it["b"] in (4, 6) and it.get("in_stride", 1) == 1:
+            if rows4 and it["q"] == 4 and it["b"] in (4, 6) and it.get("in_stride", 1) == 1 and "desc" not in it:
                 fast[it["b"]].append(it)                           # whole rows in one launch
             else:
                 groups[it["q"]].append(it)
@@ -389,11 +396,15 @@ class Dft:
         for q, its in groups.items():
             descs = []
             for it in its:
+                if "desc" in it:
+                    descs.append(it["desc"])
+                    continue
                 d = L.DftDesc(q=q, b=it["b"], rows=it["rows"], in_stride=it.get("in_stride", 1),
                               in_row_stride=it.get("in_row_stride", q ** it["b"]), in_=_ptr(it["inp"]),
                               out=_ptr(it["out"]))
                 if candidate is None:
-                    L.check(lib.qsft_dft_plan(ctypes.byref(d), precision), "qsft_dft_plan")
+                    plan = lib.qsft_dft_plan_rows if rows4 else lib.qsft_dft_plan
+                    L.check(plan(ctypes.byref(d), precision), "qsft_dft_plan")
                 else:
                     L.check(lib.qsft_dft_plan_candidate(ctypes.byref(d), precision, int(candidate)),
                             "qsft_dft_plan_candidate")

@@ -17,14 +17,16 @@ if torch.cuda.is_available():
     from qsft_amd import device as dv
     from qsft_amd import kernels as K
 
-# whole-row kernels (q = 4, b in {4, 6}) with rows that do not fill the last
-# workgroup; one tile, several tiles and several passes of the others (b = 7,
+# whole-row kernels (q = 4, b = 4..7, the last in FP32 only) with rows that do
+# not fill the last workgroup and phases beyond their LDS buffer (S = 5000, 9000); one tile, several tiles and several passes of the others (b = 7,
 # q = 2 b = 13, q = 20 b = 4), the generic radix (q = 7, 50, 64), one to four
 # digit blocks; supports around the 16-, 64- and 2048-wide blocks of the prep
 CASES = [(4, 10, 4, 100, 3, 11), (4, 50, 6, 1000, 2, 21), (4, 64, 6, 65, 1, 17), (4, 100, 7, 2049, 2, 33),
          (4, 9, 5, 64, 3, 10), (4, 20, 2, 16, 2, 5), (2, 8, 1, 1, 1, 9), (2, 30, 13, 63, 2, 16), (3, 67, 7, 777, 2, 19),
          (20, 16, 3, 2000, 2, 7), (20, 12, 4, 300, 1, 2), (5, 130, 4, 129, 2, 15), (7, 200, 3, 500, 2, 4),
-         (50, 11, 2, 33, 1, 3), (64, 256, 2, 17, 2, 3), (4, 12, 3, 5000, 1, 12), (2, 40, 6, 0, 2, 3)]
+         (50, 11, 2, 33, 1, 3), (64, 256, 2, 17, 2, 3), (4, 12, 3, 5000, 1, 12), (2, 40, 6, 0, 2, 3),
+         (4, 30, 5, 700, 2, 13), (4, 33, 6, 5000, 1, 3), (4, 70, 7, 9000, 1, 2), (4, 8, 7, 0, 1, 2), (2, 60, 14, 500, 1, 3),
+         (5, 20, 6, 900, 2, 3)]
 
 
 def _inputs(q, n, b, S, C, P, seed, loc=None):
@@ -96,8 +98,8 @@ def _item(q, n, b, Ms, Ds, loc, a, precision):
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 2e-6)])
 @pytest.mark.parametrize("q,n,b,S,C,P", [c for c in CASES if c[3] > 0])
 def test_fold_with_the_sub_transform_in_the_same_launch(q, n, b, S, C, P, precision, tol):
-    """transform=True: rows of one tile come out as their sub-transforms, other
-    rows as samples. A sample's error is at most tol of the largest sample and
+    """transform=True: rows come out as their sub-transforms, after the passes
+    left to Dft where they are more than one tile. A sample's error is at most tol of the largest sample and
     independent of its neighbours', so the error of a mean of q^b of them is
     that over sqrt(q^b), times 6 for the largest of all values, and as much
     again for the forward transform's own rounding."""
@@ -106,17 +108,15 @@ def test_fold_with_the_sub_transform_in_the_same_launch(q, n, b, S, C, P, precis
     it = _item(q, n, b, Ms, Ds, loc, a, precision)
     ev = K.EvalFold([it], L.QSFT_F32 if precision == "fp32" else L.QSFT_F64, transform=True)
     ev.launch()
+    assert bool(ev.rest) == (q ** b * (8 if precision == "fp32" else 16) * (1 if q in (2, 3, 4, 5, 20) else 2) > 147456)
+    K.Dft(ev.rest, L.QSFT_F32 if precision == "fp32" else L.QSFT_F64).launch()
     got, ref = it["x"].cpu().numpy(), _direct(q, b, Ms, Ds, loc, a)
-    bound = tol * np.max(np.abs(ref))
-    if ev.transformed[0]:
-        ref = np.fft.fftn(ref.reshape(C, P, *[q] * b), axes=range(2, 2 + b)).reshape(C, P, -1) / q ** b
-        bound *= 12 / q ** (b / 2)
-    else:
-        assert b > 6 or q > 4                                      # q = 4, b <= 6 always fits one tile
+    bound = tol * np.max(np.abs(ref)) * 12 / q ** (b / 2)
+    ref = np.fft.fftn(ref.reshape(C, P, *[q] * b), axes=range(2, 2 + b)).reshape(C, P, -1) / q ** b
     assert np.max(np.abs(got - ref)) <= bound
 
 
-@pytest.mark.parametrize("b,count", [(4, 15), (4, 29), (6, 15), (6, 29)])
+@pytest.mark.parametrize("b,count", [(4, 15), (4, 29), (5, 29), (6, 15), (6, 29)])
 def test_fold_of_many_rows_gives_the_bits_of_one_instance(b, count):
     """Launches of 4096 and 8192 rows and more give a workgroup two or four sets
     of rows of a group (P = 101 leaves the last one short): the same bits."""
@@ -129,3 +129,17 @@ def test_fold_of_many_rows_gives_the_bits_of_one_instance(b, count):
         alone = _item(4, 50, b, *g[i], "fp32")
         K.EvalFold([alone], L.QSFT_F32).launch()
         assert torch.equal(torch.view_as_real(alone["x"]), torch.view_as_real(items[i]["x"]))
+
+
+def test_fold_gives_the_same_bits_alone_and_beside_larger_rows():
+    """A launch's workgroup size follows its largest tile: q = 2 and q = 3
+    instances with crowded bins alone and beside rows of up to 128 KiB."""
+    print("fold alone and beside larger rows", flush=True)
+    shapes = [(2, 6, 1500), (2, 10, 700), (2, 14, 300), (3, 4, 1000), (3, 8, 200), (20, 2, 3000), (20, 3, 500)]
+    g = [(q, b, _inputs(q, 20, b, S, 2, 5, seed=S)) for q, b, S in shapes]
+    items = [_item(q, 20, b, *x, "fp32") for q, b, x in g]
+    K.EvalFold(items, L.QSFT_F32, transform=True).launch()
+    for (q, b, x), it in zip(g, items):
+        alone = _item(q, 20, b, *x, "fp32")
+        K.EvalFold([alone], L.QSFT_F32, transform=True).launch()
+        assert torch.equal(torch.view_as_real(alone["x"]), torch.view_as_real(it["x"])), (q, b)
