@@ -199,6 +199,9 @@ typedef struct qsft_eval_points_desc {
 } qsft_eval_points_desc;
 
 int qsft_eval_points_blocks(const qsft_eval_points_desc* host_desc);
+/* 1: the instance may run in the exact integer form (q in {2, 3, 4}, S < 2^23), which a
+ * launch whose instances all may asks for with bit 9 of its precision word. */
+int qsft_eval_points_int(const qsft_eval_points_desc* host_desc);
 int qsft_eval_points(const qsft_eval_points_desc* dev_descs, const int32_t* dev_pre, int n_inst,
                      int total_blocks, int precision, void* stream);
 

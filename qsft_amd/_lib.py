@@ -128,6 +128,7 @@ SIGNATURES = {
     "qsft_query_digits_blocks": (ctypes.c_int, [ctypes.POINTER(EvalDesc)]),
     "qsft_query_digits": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int, vp]),
     "qsft_eval_points_blocks": (ctypes.c_int, [ctypes.POINTER(EvalPointsDesc)]),
+    "qsft_eval_points_int": (ctypes.c_int, [ctypes.POINTER(EvalPointsDesc)]),
     "qsft_eval_points": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),
     "qsft_dft_plan": (ctypes.c_int, [ctypes.POINTER(DftDesc), ctypes.c_int]),
     "qsft_dft_plan_rows": (ctypes.c_int, [ctypes.POINTER(DftDesc), ctypes.c_int]),

@@ -335,26 +335,26 @@ def query_digits(items):
 
 
 class EvalPoints:
-    """items: dicts q, n, S, m (int8 [N][n_pad]), K, a, x."""
+    """items: dicts q, n, S, m (int8 [N][n_pad]), K, a, x.
+    table: every item by the w-table, also where the exact integer form applies (q in {2, 3, 4})."""
 
-    def __init__(self, items, precision):
+    def __init__(self, items, precision, table=False):
         groups = defaultdict(list)
         for it in items:
-            groups[(it["m"].shape[-1] // 64, is_pow2(it["q"]))].append(it)
+            d = L.EvalPointsDesc(q=it["q"], n=it["n"], S=it["S"], n_pad=it["m"].shape[-1],
+                                 N=it["m"].shape[0], m=_ptr(it["m"]), K=_ptr(it["K"]), a=_ptr(it["a"]),
+                                 x=_ptr(it["x"]))
+            nb = lib.qsft_eval_points_blocks(ctypes.byref(d))
+            if nb < 0:
+                raise ValueError("bad eval_points shape")
+            exact = int(not table and lib.qsft_eval_points_int(ctypes.byref(d)))
+            groups[d.n_pad // 64, exact, int(is_pow2(d.q) and not exact)].append((d, nb, it["x"].device))
         self.launches = []
-        for (nkb, pow2), its in groups.items():
-            descs, blocks = [], []
-            for it in its:
-                d = L.EvalPointsDesc(q=it["q"], n=it["n"], S=it["S"], n_pad=it["m"].shape[-1],
-                                     N=it["m"].shape[0], m=_ptr(it["m"]), K=_ptr(it["K"]), a=_ptr(it["a"]),
-                                     x=_ptr(it["x"]))
-                nb = lib.qsft_eval_points_blocks(ctypes.byref(d))
-                if nb < 0:
-                    raise ValueError("bad eval_points shape")
-                descs.append(d)
-                blocks.append(nb)
-            buf, dptr, (pre,), (tot,) = pack(descs, [blocks], its[0]["x"].device)
-            self.launches.append((buf, dptr, pre, len(descs), tot, precision | (nkb << 4) | (int(pow2) << 8)))
+        for (nkb, exact, pow2), its in groups.items():
+            descs = [d for d, _, _ in its]
+            buf, dptr, (pre,), (tot,) = pack(descs, [[nb for _, nb, _ in its]], its[0][2])
+            self.launches.append((buf, dptr, pre, len(descs), tot,
+                                  precision | (nkb << 4) | (pow2 << 8) | (exact << 9)))
 
     def launch(self):
         for _, dptr, pre, n, tot, word in self.launches:
