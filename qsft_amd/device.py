@@ -27,6 +27,16 @@ def n_pad_of(n):
     return (n + 63) // 64 * 64
 
 
+def upload(arrays, device):
+    """int8 host arrays -> device tensors of the same shapes, in one buffer and one copy."""
+    starts = np.cumsum([0] + [(a.size + 255) // 256 * 256 for a in arrays])
+    host = np.zeros(starts[-1], np.int8)
+    for a, s in zip(arrays, starts):
+        host[s:s + a.size] = a.ravel()
+    buf = torch.from_numpy(host).to(device)
+    return [buf[s:s + a.size].view(a.shape) for a, s in zip(arrays, starts)]
+
+
 def digits_tensor(rows, n_pad, device):
     """int digit rows (R, n) -> int8 [R][n_pad] on the device (zero padded)."""
     rows = np.asarray(rows)
@@ -35,24 +45,32 @@ def digits_tensor(rows, n_pad, device):
     return torch.from_numpy(out).to(device)
 
 
-def Mt_tensor(Ms, b, n_pad, device):
-    """List of C (n, >=b) matrices -> Mt [C][b][n_pad]."""
+def Mt_rows(Ms, b, n_pad):
     C = len(Ms)
     n = Ms[0].shape[0]
     out = np.zeros((C, b, n_pad), np.int8)
     for c, M in enumerate(Ms):
         out[c, :, :n] = np.asarray(M)[:, :b].T
-    return torch.from_numpy(out).to(device)
+    return out
 
 
-def D_tensor(Ds, n_pad, device):
-    """List of C arrays (P, n) -> D [C][P][n_pad]."""
+def Mt_tensor(Ms, b, n_pad, device):
+    """List of C (n, >=b) matrices -> Mt [C][b][n_pad]."""
+    return torch.from_numpy(Mt_rows(Ms, b, n_pad)).to(device)
+
+
+def D_rows(Ds, n_pad):
     Ds = [np.asarray(D) for D in Ds]
     C, (P, n) = len(Ds), Ds[0].shape
     out = np.zeros((C, P, n_pad), np.int8)
     for c, D in enumerate(Ds):
         out[c, :, :n] = D
-    return torch.from_numpy(out).to(device)
+    return out
+
+
+def D_tensor(Ds, n_pad, device):
+    """List of C arrays (P, n) -> D [C][P][n_pad]."""
+    return torch.from_numpy(D_rows(Ds, n_pad)).to(device)
 
 
 def strengths_tensor(a, precision, device):

@@ -111,8 +111,8 @@ class SubsampledSignal(Signal):
         C, R, p1 = self._layout()
         self._dev = dev
         self._n_pad = n_pad
-        self._Mt = dv.Mt_tensor(self.Ms, self.b, n_pad, dev)
-        self._Dall = dv.D_tensor([np.vstack(self.Ds[i]) for i in range(C)], n_pad, dev)
+        self._Mt, self._Dall = dv.upload([dv.Mt_rows(self.Ms, self.b, n_pad),
+                                          dv.D_rows([np.vstack(self.Ds[i]) for i in range(C)], n_pad)], dev)
 
     def _subsample_qsft(self):
         """input_signal_subsampled.py:107-155: samples, then sub-DFTs per b in all_bs.

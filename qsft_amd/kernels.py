@@ -549,6 +549,20 @@ def unit_delay_sign(D, q, n, p1):
     return 0
 
 
+def delay_form(D, q, n, p1):
+    """shared_d and unit_d of a peel item (see PeelBatch) from delay rows on the host, int8 [C][P][n_pad]:
+    what the comparisons on the device give, without their launches and waits."""
+    shared = bool((D[1:] == D[0]).all())
+    G = D[:1] if shared else D
+    C, P, _ = G.shape
+    unit = 0
+    if p1 == n + 1 and P % p1 == 0 and P // p1 <= 64 and not G[:, :, n:].any():
+        Gn = G[:, :, :n].reshape(C, P // p1, p1, n).astype(np.int16)
+        E = np.eye(p1, n, -1, dtype=np.int16)
+        unit = next((s for s in (-1, 1) if ((Gn[:, :, :1] + s * E) % q == Gn).all()), 0)
+    return dict(shared_d=shared, unit_d=unit)
+
+
 def peel_flags(it):
     """QSFT_PEEL_SHARED_D / UNIT_D / UNIT_D_NEG (/ ONE_BIN_WAVES) bits of a peel item (see PeelBatch)."""
     C, q, n = it["C"], it["q"], it["n"]
@@ -581,20 +595,24 @@ def peel_noalloc(it, dst, cap_rows, row_stride, max_iter=15):
         int(cap_rows), int(row_stride), stream_handle()), "qsft_peel_transform_noalloc")
 
 
+def _unpack(r, n, n_pad):
+    """(k int64 [m][n], values complex128 [m], order uint64 [m]) of one instance's packed rows, sorted by
+    first detection (the order that the output table is written in)."""
+    k = r[:, :n].astype(np.int64)
+    v = np.ascontiguousarray(r[:, n_pad:n_pad + 16]).view(np.complex128).reshape(-1)
+    order = np.ascontiguousarray(r[:, n_pad + 16:n_pad + 24]).view(np.uint64).reshape(-1)
+    if (order[1:] < order[:-1]).any():
+        srt = np.argsort(order, kind="stable")
+        k, v, order = k[srt], v[srt], order[srt]
+    return k, v, order
+
+
 def unpack_rows(hdr, rows, n_inst, ns, n_pads):
     """Per instance (k int64 [m][n], values complex128 [m], order uint64 [m]),
     sorted by first detection, from a packed header (int64) and rows (uint8
     [total][row_stride])."""
     counts, offs = hdr[:n_inst], hdr[n_inst:2 * n_inst]
-    out = []
-    for i in range(n_inst):
-        r = rows[offs[i]:offs[i] + counts[i]]
-        k = r[:, :ns[i]].astype(np.int64)
-        v = r[:, n_pads[i]:n_pads[i] + 16].copy().view(np.float64).reshape(-1, 2)
-        order = r[:, n_pads[i] + 16:n_pads[i] + 24].copy().view(np.uint64).reshape(-1)
-        srt = np.argsort(order, kind="stable")
-        out.append((k[srt], (v[:, 0] + 1j * v[:, 1])[srt], order[srt]))
-    return out
+    return [_unpack(rows[offs[i]:offs[i] + counts[i]], ns[i], n_pads[i]) for i in range(n_inst)]
 
 
 class PeelBatch:
@@ -666,10 +684,10 @@ class PeelBatch:
         self.hdr_bytes = lib.qsft_peel_pack_header_bytes(len(self.descs))
         size = self.hdr_bytes + self.cap_rows * self.row_stride
         if host_rows:
-            self.packed = torch.empty(size, dtype=torch.uint8).pin_memory()
+            self.packed = torch.empty(size, dtype=torch.uint8, pin_memory=True)
         else:
             self.packed = torch.empty(size, dtype=torch.uint8, device=dev)
-            self.hdr_host = torch.empty(self.hdr_bytes, dtype=torch.uint8).pin_memory()
+            self.hdr_host = torch.empty(self.hdr_bytes, dtype=torch.uint8, pin_memory=True)
 
     def sparse_targets(self, i):
         """(written, noise_key) device addresses of instance i, for its assembler."""
@@ -770,7 +788,7 @@ class PeelBatch:
         total = int(hdr[2 * n])
         nbytes = total * self.row_stride
         if getattr(self, "rows_host", None) is None or self.rows_host.numel() < nbytes:
-            self.rows_host = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8).pin_memory()
+            self.rows_host = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, pin_memory=True)
         src = self.packed[self.hdr_bytes:self.hdr_bytes + nbytes]
         if copy_stream is None:
             self.rows_host[:nbytes].copy_(src)
@@ -795,13 +813,8 @@ class PeelBatch:
         counts, offs, rows = self.fetch_packed() if packed is None else packed
         out = []
         for i, d in enumerate(self.descs):
-            r = rows[offs[i]:offs[i] + counts[i]]
-            k = r[:, :d.n].astype(np.int64)
-            v = r[:, d.n_pad:d.n_pad + 16].copy().view(np.float64).reshape(-1, 2)
-            order = r[:, d.n_pad + 16:d.n_pad + 24].copy().view(np.uint64).reshape(-1)
-            srt = np.argsort(order, kind="stable")
-            info = self.info(i) if with_info else {}
-            out.append((k[srt], (v[:, 0] + 1j * v[:, 1])[srt], order[srt], info))
+            k, v, order = _unpack(rows[offs[i]:offs[i] + counts[i]], d.n, d.n_pad)
+            out.append((k, v, order, self.info(i) if with_info else {}))
         return out
 
     def info(self, i):

@@ -20,7 +20,7 @@ from . import device as dv
 from . import kernels
 from .input_signal_subsampled import SubsampledSignal
 from .reed_solomon import ReedSolomon
-from .utils import calc_hamming_weight, sort_qary_vecs
+from .utils import calc_hamming_weight, digit_tuples, lex_order
 
 MAX_ITER = 15
 
@@ -89,12 +89,12 @@ class QSFT:
         C, Q, P = U.shape
         dev = U.device
         n_pad = dv.n_pad_of(n)
-        Mt = dv.Mt_tensor(Ms, b, n_pad, dev)
-        Dd = dv.D_tensor(Ds, n_pad, dev)
+        Dh = dv.D_rows(Ds, n_pad)
+        Mt, Dd = dv.upload([dv.Mt_rows(Ms, b, n_pad), Dh], dev)
         torch.cuda.synchronize()
         t0 = time.time()
         item = dict(q=q, n=n, b=b, C=C, P=P, p1=signal.get_source_parity(), method=method, cutoff=cutoff, Mt=Mt,
-                    D=Dd, U=U)
+                    D=Dd, U=U, **kernels.delay_form(Dh, q, n, signal.get_source_parity()))
         if method & L.QSFT_DETECT_CODED:
             rs = self._code(n, q)
             item["coded"] = dict(t=rs.t, s=rs.s, tables=torch.from_numpy(rs.device_tables()).to(dev))
@@ -108,15 +108,16 @@ class QSFT:
         if verbosity >= 2:
             for it, (ns, nm, nb) in enumerate(info["trace"]):
                 print(f"iter {it + 1}: singletons {ns} multitons {nm} balls {nb}", flush=True)
-        gwht = {tuple(row): v for row, v in zip(k, vals)}
+        keys = digit_tuples(k)
+        gwht = dict(zip(keys, vals))
         self.last_info = info
         if not report:
             return gwht
-        loc = list(gwht.keys())
+        loc = keys
         if loc:
+            hw = calc_hamming_weight(k)
             if kwargs.get("sort", False):
-                loc = sort_qary_vecs(loc)
-            hw = calc_hamming_weight(loc)
+                loc = k[lex_order(k)]
             avg_hw, max_hw = np.mean(hw), np.max(hw)
         else:
             loc, avg_hw, max_hw = [], 0, 0
