@@ -14,6 +14,12 @@
 // logical element only, so both layouts draw the same values. With `energy`,
 // each wave reduces its two columns from registers exactly as the peeler does
 // (all rows of a bin are in one tile when R*p1 <= 128).
+//
+// Where it draws noise it is bound by its VALU, most of that Philox's 32 x 32
+// bit products: one three-way XOR per word and round instead of two XORs took
+// 64 x (3 x 102 x 4096) FP32 cells from 268 to 250 us. Drawing over (row, pair)
+// flattened, without the idle lanes of the last 64 rows, needs the sums in LDS
+// and half the loads in flight: 359 us. 32 bins per tile (256 B segments): 254.
 #include "qsft_common.h"
 
 namespace qsft {

@@ -96,6 +96,14 @@ template <typename T> using cplx_t = typename cplx<T>::type;
 // easy as 1, 2, 3", SC 2011): multipliers 0xD2511F53 / 0xCD9E8D57, Weyl key
 // increments 0x9E3779B9 / 0xBB67AE85, ten rounds.
 struct u4 { uint32_t x, y, z, w; };
+// a ^ b ^ c as one instruction on the device
+__host__ __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+    return a ^ b ^ c;
+#endif
+}
 __host__ __device__ __forceinline__ u4 philox4x32_10(u4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
@@ -103,7 +111,7 @@ __host__ __device__ __forceinline__ u4 philox4x32_10(u4 c, uint32_t k0, uint32_t
         const uint64_t p1 = (uint64_t)0xCD9E8D57u * c.z;
         const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0;
         const uint32_t hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
-        c = u4{hi1 ^ c.y ^ k0, lo1, hi0 ^ c.w ^ k1, lo0};
+        c = u4{xor3(hi1, c.y, k0), lo1, xor3(hi0, c.w, k1), lo0};
         k0 += 0x9E3779B9u;
         k1 += 0xBB67AE85u;
     }
