@@ -33,15 +33,15 @@ __device__ __forceinline__ double2 src_value(const qsft_assemble_desc& d, int c,
     const int r = p / d.p1, i = p - r * d.p1;
     const int64_t src_idx = ((int64_t)d.gsel[c] * d.src_rows + (int64_t)d.rsel[r] * d.p1 + i) * d.Q + j;
     if (d.src_prec == QSFT_F32) {
-        const float2 v = reinterpret_cast<const float2*>(d.src)[src_idx];
+        const float2 v = in_global(reinterpret_cast<const float2*>(d.src))[src_idx];
         return make_double2(v.x, v.y);
     }
-    return reinterpret_cast<const double2*>(d.src)[src_idx];
+    return in_global(reinterpret_cast<const double2*>(d.src))[src_idx];
 }
 
 __device__ __forceinline__ double2 add_array_noise(const qsft_assemble_desc& d, double2 v, int64_t e) {
     if (d.noise_mode == QSFT_NOISE_ARRAY) {
-        const double2 z = reinterpret_cast<const double2*>(d.noise)[e];
+        const double2 z = in_global(reinterpret_cast<const double2*>(d.noise))[e];
         v.x = v.x + z.x;
         v.y = v.y + z.y;
     }
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(const qsft_assemble_de
             const int p = (int)(rowg - (int64_t)c * rows);
             double2 v = add_array_noise(d, src_value(d, c, p, j), e);
             if (d.noise_mode == QSFT_NOISE_PHILOX) v = add_philox(v, c, p, rows, Q, j, comp_sd, seed);
-            reinterpret_cast<double2*>(d.U)[e] = v;
+            in_global(reinterpret_cast<double2*>(d.U))[e] = v;
         }
         return;
     }
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(const qsft_assemble_de
             const int e = threadIdx.x + k * kAsmThreads;
             const int pr = e >> 4, jj = e & 15;
             v[k] = make_float2(0.0f, 0.0f);
-            if (pr < Pc && jj < Jc) v[k] = reinterpret_cast<const float2*>(d.src)[srow[pr] + j0 + jj];
+            if (pr < Pc && jj < Jc) v[k] = in_global(reinterpret_cast<const float2*>(d.src))[srow[pr] + j0 + jj];
         }
 #pragma unroll
         for (int k = 0; k < kReads; ++k) {
@@ -126,10 +126,10 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(const qsft_assemble_de
             if (pr < Pc && jj < Jc) {
                 const int64_t si = srow[pr] + j0 + jj;
                 if (d.src_prec == QSFT_F32) {
-                    const float2 f = reinterpret_cast<const float2*>(d.src)[si];
+                    const float2 f = in_global(reinterpret_cast<const float2*>(d.src))[si];
                     v[k] = make_double2(f.x, f.y);
                 } else {
-                    v[k] = reinterpret_cast<const double2*>(d.src)[si];
+                    v[k] = in_global(reinterpret_cast<const double2*>(d.src))[si];
                 }
             }
         }
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(const qsft_assemble_de
     // is 1 KiB contiguous and the energies reduce straight from registers. With
     // `written` (energies, so all rows are in this chunk) a column is stored
     // only if its energy is above the peeler's zeroton cutoff.
-    double2* __restrict__ U = reinterpret_cast<double2*>(d.U);
+    double2* __restrict__ U = in_global(reinterpret_cast<double2*>(d.U));
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int npairs = (Jc + 1) >> 1;
     const bool philox = d.noise_mode == QSFT_NOISE_PHILOX;
@@ -186,11 +186,11 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(const qsft_assemble_de
                 w1 = two && e1 > thr;
             }
             if (lane == 0) {
-                d.energy[(int64_t)c * Q + j] = e0;
-                if (two) d.energy[(int64_t)c * Q + j + 1] = e1;
+                in_global(d.energy)[(int64_t)c * Q + j] = e0;
+                if (two) in_global(d.energy)[(int64_t)c * Q + j + 1] = e1;
                 if (d.written) {
-                    d.written[(int64_t)c * Q + j] = w0 ? 1 : 0;
-                    if (two) d.written[(int64_t)c * Q + j + 1] = w1 ? 1 : 0;
+                    in_global(d.written)[(int64_t)c * Q + j] = w0 ? 1 : 0;
+                    if (two) in_global(d.written)[(int64_t)c * Q + j + 1] = w1 ? 1 : 0;
                 }
             }
         }

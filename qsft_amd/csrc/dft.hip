@@ -85,7 +85,8 @@ __global__ __launch_bounds__(TH) void k_dft_pass(const qsft_dft_desc* __restrict
         const int m = (int)fti.div((uint32_t)e);
         return base + (int64_t)m * I + (e - m * ti);
     };
-    // load the tile
+    // load the tile. (Generic pointers: with global ones the q = 20, b = 4 rows
+    // of a serving mix take 322 against 305 us.)
     {
         const C2* __restrict__ in = pass == 0
             ? reinterpret_cast<const C2*>(d.in) + (int64_t)row * d.in_row_stride
@@ -125,8 +126,8 @@ __global__ __launch_bounds__(1 << (2 * B - 4)) void k_dft4_rows(const qsft_dft_d
     const int row = blockIdx.x - pre[inst];
     if (d.q != 4 || d.b != B || d.in_stride != 1 || row >= d.rows) return;   // launched for other shapes
     const int tid = threadIdx.x;
-    const C2* __restrict__ in = reinterpret_cast<const C2*>(d.in) + (int64_t)row * d.in_row_stride;
-    C2* __restrict__ out = reinterpret_cast<C2*>(d.out) + (int64_t)row * Q;
+    const C2* __restrict__ in = in_global(reinterpret_cast<const C2*>(d.in)) + (int64_t)row * d.in_row_stride;
+    C2* __restrict__ out = in_global(reinterpret_cast<C2*>(d.out)) + (int64_t)row * Q;
 
     C2 v[16];
 #pragma unroll

@@ -151,11 +151,11 @@ __global__ __launch_bounds__(256) void k_eval_cosets(const qsft_eval_desc* __res
     }
 
     C2 sum[4];
-    accumulate<T, POW2, NKB>(afrag, d.K, reinterpret_cast<const C2*>(d.a), d.S, n_pad, tab, mq,
+    accumulate<T, POW2, NKB>(afrag, in_global(d.K), in_global(reinterpret_cast<const C2*>(d.a)), d.S, n_pad, tab, mq,
                              (uint32_t)(q - 1), sum);
     if (r16 < 4) {
         const int ql = lq0 + 4 * g + r16;
-        if (ql < Q) reinterpret_cast<C2*>(d.x)[(size_t)row * Q + ql] = pick4<T>(sum, r16);
+        if (ql < Q) in_global(reinterpret_cast<C2*>(d.x))[(size_t)row * Q + ql] = pick4<T>(sum, r16);
     }
 }
 
@@ -175,15 +175,15 @@ __device__ __forceinline__ void points_by_table(const qsft_eval_points_desc& d, 
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
         v4i z = {0, 0, 0, 0};
-        if (l < d.N) z = *reinterpret_cast<const v4i*>(d.m + (size_t)l * n_pad + 64 * kb + 16 * g);
+        if (l < d.N) z = *reinterpret_cast<const v4i*>(in_global(d.m) + (size_t)l * n_pad + 64 * kb + 16 * g);
         afrag[kb] = z;
     }
     C2 sum[4];
-    accumulate<T, POW2, NKB>(afrag, d.K, reinterpret_cast<const C2*>(d.a), d.S, n_pad, tab, mq,
+    accumulate<T, POW2, NKB>(afrag, in_global(d.K), in_global(reinterpret_cast<const C2*>(d.a)), d.S, n_pad, tab, mq,
                              (uint32_t)(q - 1), sum);
     if (r16 < 4) {
         const int64_t ql = lq0 + 4 * g + r16;
-        if (ql < d.N) reinterpret_cast<C2*>(d.x)[ql] = pick4<T>(sum, r16);
+        if (ql < d.N) in_global(reinterpret_cast<C2*>(d.x))[ql] = pick4<T>(sum, r16);
     }
 }
 
@@ -251,8 +251,8 @@ __global__ __launch_bounds__(256, NKB <= 2 ? 4 : 1) void k_eval_points_int(const
     const qsft_eval_points_desc& d = descs[inst];
     const int64_t local = blockIdx.x - pre[inst];
     const int q = d.q, S = d.S, n_pad = d.n_pad;
-    const C2* __restrict__ a = reinterpret_cast<const C2*>(d.a);
-    const int8_t* __restrict__ K = d.K;
+    const C2* __restrict__ a = in_global(reinterpret_cast<const C2*>(d.a));
+    const int8_t* __restrict__ K = in_global(d.K);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = lane >> 4, r16 = lane & 15;
 
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256, NKB <= 2 ? 4 : 1) void k_eval_points_int(const
     for (int k = 0; k < NKB; ++k) {
         const int i = threadIdx.x + 256 * k, row = i / (4 * NKB), col = 16 * (i - row * (4 * NKB));
         v4i z = {0, 0, 0, 0};
-        if (local * 64 + row < d.N) z = *reinterpret_cast<const v4i*>(d.m + (size_t)(local * 64 + row) * n_pad + col);
+        if (local * 64 + row < d.N) z = *reinterpret_cast<const v4i*>(in_global(d.m) + (size_t)(local * 64 + row) * n_pad + col);
         *reinterpret_cast<v4i*>(&sh.s.query[row][col]) = z;
     }
     for (int i = threadIdx.x; i < 2 * 64 * kSumPitch; i += 256) (&sh.s.sum[0][0][0])[i] = 0;
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(256, NKB <= 2 ? 4 : 1) void k_eval_points_int(const
     } else {
         x = fma((double)(c1 + z1), 4294967296.0, (double)(c0 + z0));
     }
-    reinterpret_cast<T*>(d.x)[2 * ql + part] = (T)ldexp(x, e - 62);
+    in_global(reinterpret_cast<T*>(d.x))[2 * ql + part] = (T)ldexp(x, e - 62);
 }
 
 

@@ -88,7 +88,7 @@ __global__ __launch_bounds__(kPhaseThreads) void k_fold_phase(const SRC src) {
     const int ptiles = (P + 15) / 16;
     const int dtiles = (d.shared_d ? 1 : C) * ptiles;
     const ModQ mq((uint32_t)q);
-    const int8_t* __restrict__ krow = d.K + (size_t)min(s0 + r16, S - 1) * n_pad + 16 * g;
+    const int8_t* __restrict__ krow = in_global(d.K) + (size_t)min(s0 + r16, S - 1) * n_pad + 16 * g;
     v4i kf[QSFT_MAX_N / 64];
 #pragma unroll
     for (int kb = 0; kb < QSFT_MAX_N / 64; ++kb)
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(kPhaseThreads) void k_fold_phase(const SRC src) {
             uint32_t w = 0;
 #pragma unroll
             for (int v = 0; v < 4; ++v) w |= mq((uint32_t)e[v]) << (8 * v);
-            if (p < P) *reinterpret_cast<uint32_t*>(d.E + ((size_t)c * P + p) * Sp + s0 + 4 * g) = w;
+            if (p < P) *reinterpret_cast<uint32_t*>(in_global(d.E) + ((size_t)c * P + p) * Sp + s0 + 4 * g) = w;
         } else {
             int place = 0;                                         // q^(b - 1 - r16)
             if (r16 < b) {
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(kPhaseThreads) void k_fold_phase(const SRC src) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) j[v] = row_sum_i((int)mq((uint32_t)e[v]) * place);
             const int mine = r16 == 0 ? j[0] : r16 == 1 ? j[1] : r16 == 2 ? j[2] : j[3];
-            if (r16 < 4 && s0 + 4 * g + r16 < S) d.J[(size_t)c * S + s0 + 4 * g + r16] = (uint32_t)mine;
+            if (r16 < 4 && s0 + 4 * g + r16 < S) in_global(d.J)[(size_t)c * S + s0 + 4 * g + r16] = (uint32_t)mine;
         }
     }
 }
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(kRankThreads) void k_fold_rank(const SRC src) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int item = (local - c * per_c) * 64 + lane;
     const bool support = item < S, bound = item >= S64 && item - S64 < fold_bounds(d.tiles);
-    const uint32_t* __restrict__ J = d.J + (size_t)c * S;
+    const uint32_t* __restrict__ J = in_global(d.J) + (size_t)c * S;
     uint32_t j = 0;
     if (support) j = J[item];
     if (bound) j = (uint32_t)(item - S64) * (uint32_t)d.tile_bins;
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kRankThreads) void k_fold_rank(const SRC src) {
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) rank += part[w][lane];
     if (support) {
-        d.key[(size_t)c * S + rank] = ((uint64_t)j << 32) | (uint32_t)item;
+        in_global(d.key)[(size_t)c * S + rank] = ((uint64_t)j << 32) | (uint32_t)item;
         double2 a;
         if (d.a_prec == QSFT_F32) {
             const float2 f = reinterpret_cast<const float2*>(d.a)[item];
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kRankThreads) void k_fold_rank(const SRC src) {
         }
         reinterpret_cast<double2*>(d.as)[(size_t)c * S + rank] = a;
     }
-    if (bound) d.start[(size_t)c * (d.tiles + 1) + (item - S64)] = (int32_t)rank;
+    if (bound) in_global(d.start)[(size_t)c * (d.tiles + 1) + (item - S64)] = (int32_t)rank;
 }
 
 // The terms of one row are added to their bins in LDS by the waves of a
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(TH) void k_fold_pass(const SRC src, int pass, int l
         const int m = (int)fti.div((uint32_t)e);
         return base + (int64_t)m * I + (e - m * ti);
     };
-    C2* __restrict__ x = reinterpret_cast<C2*>(d.x) + (int64_t)row * Q;
+    C2* __restrict__ x = in_global(reinterpret_cast<C2*>(d.x)) + (int64_t)row * Q;
     if constexpr (FIRST) {
         const int c = row / d.P;
         fold_wtable(tab, q);

@@ -187,17 +187,17 @@ __global__ __launch_bounds__(kSlotThreads) void k_peel_init(const qsft_peel_desc
     const int local = blockIdx.x - pre[inst];
     const int H = 1 << d.hcap_log2;
     const int h = local * kSlotThreads + threadIdx.x;
-    if (local == 0 && threadIdx.x < QSFT_CTR_WORDS) d.ctr[threadIdx.x] = (threadIdx.x == 3) ? 1u : 0u;
+    if (local == 0 && threadIdx.x < QSFT_CTR_WORDS) in_global(d.ctr)[threadIdx.x] = (threadIdx.x == 3) ? 1u : 0u;
     if (h < H) {
-        d.tag[h] = 0;
-        d.owner[h] = ~0ull;
-        d.last[h] = 0;
-        d.head[h] = kNil;
-        d.count[h] = 0;
+        in_global(d.tag)[h] = 0;
+        in_global(d.owner)[h] = ~0ull;
+        in_global(d.last)[h] = 0;
+        in_global(d.head)[h] = kNil;
+        in_global(d.count)[h] = 0;
     }
     if (h < d.C * d.Q) {
-        d.sstamp[h] = 0;
-        d.pend_head[h] = -1;
+        in_global(d.sstamp)[h] = 0;
+        in_global(d.pend_head)[h] = -1;
     }
 }
 
@@ -210,12 +210,41 @@ __device__ __forceinline__ void load_col(double2 (&u)[kRowsPerLane], const doubl
     }
 }
 
+// Whether column `lane` of a wave's nb columns has an energy above thr, kGroup
+// columns at a time. Every load is issued (the rows past P read row P - 1, the
+// columns past nb column nb - 1, and count as zero or not at all), so that none
+// waits for the column before it.
+template <int NR>
+__device__ __forceinline__ bool screen_columns(const double2* __restrict__ Ub, int P, int nb, double thr, int lane) {
+    constexpr int kGroup = NR == 4 ? 4 : 8;
+    bool nz = false;
+    for (int g = 0; g < nb; g += kGroup) {
+        double2 u[kGroup][NR];
+#pragma unroll
+        for (int k = 0; k < kGroup; ++k) {
+            const double2* col = Ub + (size_t)min(g + k, nb - 1) * P;
+#pragma unroll
+            for (int r = 0; r < NR; ++r) u[k][r] = col[min(lane + 64 * r, P - 1)];
+        }
+#pragma unroll
+        for (int k = 0; k < kGroup; ++k) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r)
+                if (lane + 64 * r >= P) u[k][r] = make_double2(0.0, 0.0);
+            const double e = bin_energy(u[k]);
+            if (lane == g + k) nz = e > thr;
+        }
+    }
+    return nz;
+}
+
 // First-pass screen. Wave w owns bins [64 w, 64 w + 64) (or a part of them, see
 // BinShare); lane L stamps its bin L for pass 0 iff it is not a zeroton, and -1 (never) otherwise. With
-// energies from the assembler it compares one number per bin; otherwise four
-// columns are loaded before their energies are reduced, so several loads per
+// energies from the assembler it compares one number per bin; otherwise four or
+// eight columns are loaded before their energies are reduced, so 16 loads per
 // lane are in flight and U streams once at HBM speed. Kernel A then visits
-// only the stamped bins.
+// only the stamped bins. 161 MB (P = 102): 45 -> 28.5 us since no load waits for
+// an earlier column; a serving mix's P = 202 columns 228 -> 185 us.
 __global__ __launch_bounds__(kBinThreads) void k_peel_screen(const qsft_peel_desc* __restrict__ descs,
                                                              const int32_t* __restrict__ pre, int n_inst, int split) {
     const BinShare share(pre, n_inst, split);
@@ -227,29 +256,14 @@ __global__ __launch_bounds__(kBinThreads) void k_peel_screen(const qsft_peel_des
     const int nb = min(share.nbins, CQ - base);
     const double thr = d.cutoff * (double)P;
     if (d.energy) {
-        if (lane < nb) d.mark[base + lane] = (d.energy[base + lane] > thr) ? 0 : -1;
+        if (lane < nb) in_global(d.mark)[base + lane] = (in_global(d.energy)[base + lane] > thr) ? 0 : -1;
         return;
     }
-    const double2* __restrict__ Ub = reinterpret_cast<const double2*>(d.U) + (size_t)base * P;
-    bool nz = false;
-    for (int g = 0; g < nb; g += 4) {
-        double2 u[4][kRowsPerLane];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (g + k < nb) {
-                load_col(u[k], Ub + (size_t)(g + k) * P, P, lane);
-            } else {
-#pragma unroll
-                for (int r = 0; r < kRowsPerLane; ++r) u[k][r] = make_double2(0.0, 0.0);
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const double e = bin_energy(u[k]);
-            if (lane == g + k) nz = e > thr;
-        }
-    }
-    if (lane < nb) d.mark[base + lane] = nz ? 0 : -1;
+    const double2* __restrict__ Ub = in_global(reinterpret_cast<const double2*>(d.U)) + (size_t)base * P;
+    const bool nz = P > 128 ? screen_columns<4>(Ub, P, nb, thr, lane)
+                  : P > 64  ? screen_columns<2>(Ub, P, nb, thr, lane)
+                            : screen_columns<1>(Ub, P, nb, thr, lane);
+    if (lane < nb) in_global(d.mark)[base + lane] = nz ? 0 : -1;
 }
 
 // w^{<D_c row p, k>} for this lane's rows p = lane + 64 r (zero past P); k is
@@ -847,7 +861,7 @@ __device__ __forceinline__ uint64_t scan_marks(const qsft_peel_desc& d, int it, 
 template <int CAP>
 __device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int it, int ns,
                                                     const SingletonBuf<CAP>& sb, int lane) {
-    uint32_t* __restrict__ ctr = d.ctr;
+    uint32_t* __restrict__ ctr = in_global(d.ctr);
     const int CQ = d.C * d.Q;
     int slot = -1;
     bool claimed = false;                                      // this lane's k took a new slot
@@ -863,7 +877,7 @@ __device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int
         const uint32_t mask = (1u << d.hcap_log2) - 1u;
         uint32_t pos = (uint32_t)(hv >> 32) & mask;
         for (uint32_t probe = 0; probe <= mask; ++probe) {
-            const unsigned long long old = atomicCAS((unsigned long long*)&d.tag[pos], 0ull, (unsigned long long)tg);
+            const unsigned long long old = atomicCAS((unsigned long long*)&in_global(d.tag)[pos], 0ull, (unsigned long long)tg);
             if (old == 0ull || old == tg) {
                 slot = (int)pos;
                 claimed = old == 0ull;
@@ -874,11 +888,11 @@ __device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int
         if (slot < 0) {
             atomicOr(&ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_TABLE_FULL);
         } else {
-            d.slot_bin[t] = slot;
-            d.sstamp[t] = it + 1;                                 // kernel B peels only registered bins
+            in_global(d.slot_bin)[t] = slot;
+            in_global(d.sstamp)[t] = it + 1;                                 // kernel B peels only registered bins
             tm = ((uint64_t)(it + 1) << 32) | (uint32_t)t;
-            atomicMin((unsigned long long*)&d.owner[slot], (unsigned long long)tm);
-            const unsigned long long prev = atomicMax((unsigned long long*)&d.last[slot], (unsigned long long)tm);
+            atomicMin((unsigned long long*)&in_global(d.owner)[slot], (unsigned long long)tm);
+            const unsigned long long prev = atomicMax((unsigned long long*)&in_global(d.last)[slot], (unsigned long long)tm);
             newball = (prev >> 32) != (unsigned long long)(it + 1);
         }
     }
@@ -893,17 +907,17 @@ __device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int
     }
     rbase = __shfl(rbase, 0);
     lbase = __shfl(lbase, 0);
-    if (claimed) d.live[lbase + (uint32_t)__popcll(cl_mask & ((1ull << lane) - 1ull))] = (uint32_t)slot;
+    if (claimed) in_global(d.live)[lbase + (uint32_t)__popcll(cl_mask & ((1ull << lane) - 1ull))] = (uint32_t)slot;
     if (slot >= 0) {
         const uint32_t rix = rbase + (uint32_t)__popcll(ok_mask & ((1ull << lane) - 1ull));
         if ((uint64_t)rix >= (uint64_t)d.max_iter * (uint64_t)CQ) {   // cannot happen: one record per bin per pass
             atomicOr(&ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_BAD_SHAPE);
         } else {
-            d.rec_time[rix] = tm;
-            d.rec_rho[2 * (size_t)rix] = rho.x;
-            d.rec_rho[2 * (size_t)rix + 1] = rho.y;
-            d.rec_next[rix] = atomicExch(&d.head[slot], rix);
-            atomicAdd(&d.count[slot], 1u);
+            in_global(d.rec_time)[rix] = tm;
+            in_global(d.rec_rho)[2 * (size_t)rix] = rho.x;
+            in_global(d.rec_rho)[2 * (size_t)rix + 1] = rho.y;
+            in_global(d.rec_next)[rix] = atomicExch(&in_global(d.head)[slot], rix);
+            atomicAdd(&in_global(d.count)[slot], 1u);
         }
     }
 }
@@ -919,7 +933,7 @@ struct Claim {
 
 template <int CAP>
 __device__ __forceinline__ Claim claim_slots(const qsft_peel_desc& d, int it, int ns, const SingletonBuf<CAP>& sb, int lane) {
-    uint32_t* __restrict__ ctr = d.ctr;
+    uint32_t* __restrict__ ctr = in_global(d.ctr);
     Claim c{-1, 0, false, make_double2(0.0, 0.0), 0, 0, 0};
     bool newball = false;
     if (lane < ns) {
@@ -930,7 +944,7 @@ __device__ __forceinline__ Claim claim_slots(const qsft_peel_desc& d, int it, in
         const uint32_t mask = (1u << d.hcap_log2) - 1u;
         uint32_t pos = (uint32_t)(hv >> 32) & mask;
         for (uint32_t probe = 0; probe <= mask; ++probe) {
-            const unsigned long long old = atomicCAS((unsigned long long*)&d.tag[pos], 0ull, (unsigned long long)tg);
+            const unsigned long long old = atomicCAS((unsigned long long*)&in_global(d.tag)[pos], 0ull, (unsigned long long)tg);
             if (old == 0ull || old == tg) {
                 c.slot = (int)pos;
                 c.claimed = old == 0ull;
@@ -941,11 +955,11 @@ __device__ __forceinline__ Claim claim_slots(const qsft_peel_desc& d, int it, in
         if (c.slot < 0) {
             atomicOr(&ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_TABLE_FULL);
         } else {
-            d.slot_bin[c.t] = c.slot;
-            d.sstamp[c.t] = it + 1;                               // kernel B peels only registered bins
+            in_global(d.slot_bin)[c.t] = c.slot;
+            in_global(d.sstamp)[c.t] = it + 1;                               // kernel B peels only registered bins
             const uint64_t tm = ((uint64_t)(it + 1) << 32) | (uint32_t)c.t;
-            atomicMin((unsigned long long*)&d.owner[c.slot], (unsigned long long)tm);
-            const unsigned long long prev = atomicMax((unsigned long long*)&d.last[c.slot], (unsigned long long)tm);
+            atomicMin((unsigned long long*)&in_global(d.owner)[c.slot], (unsigned long long)tm);
+            const unsigned long long prev = atomicMax((unsigned long long*)&in_global(d.last)[c.slot], (unsigned long long)tm);
             newball = (prev >> 32) != (unsigned long long)(it + 1);
         }
     }
@@ -959,17 +973,17 @@ __device__ __forceinline__ Claim claim_slots(const qsft_peel_desc& d, int it, in
 __device__ __forceinline__ void write_records(const qsft_peel_desc& d, int it, const Claim& c, uint32_t rbase,
                                               uint32_t lbase, int lane) {
     const uint64_t below = (1ull << lane) - 1ull;
-    if (c.claimed) d.live[lbase + (uint32_t)__popcll(c.cl_mask & below)] = (uint32_t)c.slot;
+    if (c.claimed) in_global(d.live)[lbase + (uint32_t)__popcll(c.cl_mask & below)] = (uint32_t)c.slot;
     if (c.slot >= 0) {
         const uint32_t rix = rbase + (uint32_t)__popcll(c.ok_mask & below);
         if ((uint64_t)rix >= (uint64_t)d.max_iter * (uint64_t)(d.C * d.Q)) {   // cannot happen: one record per bin per pass
-            atomicOr(&d.ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_BAD_SHAPE);
+            atomicOr(&in_global(d.ctr)[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_BAD_SHAPE);
         } else {
-            d.rec_time[rix] = ((uint64_t)(it + 1) << 32) | (uint32_t)c.t;
-            d.rec_rho[2 * (size_t)rix] = c.rho.x;
-            d.rec_rho[2 * (size_t)rix + 1] = c.rho.y;
-            d.rec_next[rix] = atomicExch(&d.head[c.slot], rix);
-            atomicAdd(&d.count[c.slot], 1u);
+            in_global(d.rec_time)[rix] = ((uint64_t)(it + 1) << 32) | (uint32_t)c.t;
+            in_global(d.rec_rho)[2 * (size_t)rix] = c.rho.x;
+            in_global(d.rec_rho)[2 * (size_t)rix + 1] = c.rho.y;
+            in_global(d.rec_next)[rix] = atomicExch(&in_global(d.head)[c.slot], rix);
+            atomicAdd(&in_global(d.count)[c.slot], 1u);
         }
     }
 }
@@ -1005,7 +1019,7 @@ template <int CAP>
 __device__ __forceinline__ void finish_wave(const qsft_peel_desc& d, int it, const WaveEnd& e,
                                             const SingletonBuf<CAP>& sb, int lane) {
     if (lane == 0) {
-        uint32_t* pc = d.ctr + it * QSFT_CTR_ITER_STRIDE;
+        uint32_t* pc = in_global(d.ctr) + it * QSFT_CTR_ITER_STRIDE;
         if (e.scanned) atomicAdd(pc + 4, e.scanned);
         if (e.ns) atomicAdd(pc + 0, (uint32_t)e.ns);
         if (e.nz > e.ns) atomicAdd(pc + 1, (uint32_t)(e.nz - e.ns));
@@ -1045,8 +1059,8 @@ __device__ __forceinline__ void finish_block(const qsft_peel_desc& d, int it, co
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) t[i] += B.cnt[w][i];
         }
-        B.base = take_records(d.ctr, t[4], t[5]);
-        add_counters(d.ctr, it, t[0], t[1], t[2], t[3]);
+        B.base = take_records(in_global(d.ctr), t[4], t[5]);
+        add_counters(in_global(d.ctr), it, t[0], t[1], t[2], t[3]);
     }
     __syncthreads();
     uint32_t rbase = (uint32_t)B.base, lbase = (uint32_t)(B.base >> 32);
@@ -1537,7 +1551,7 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_waves_per_eu(4))
     __shared__ BlockEnd end;
     const BinShare share(pre, n_inst, split);
     const qsft_peel_desc& d = descs[share.inst];
-    uint32_t* __restrict__ ctr = d.ctr;
+    uint32_t* __restrict__ ctr = in_global(d.ctr);
     constexpr int it = 0;
     if (it >= d.max_iter) return;
     if (cptr(ctr)[it * QSFT_CTR_ITER_STRIDE + 3] == 0) return;
@@ -1596,7 +1610,7 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_waves_per_eu(NR 
     __shared__ BlockEnd end;
     const BinShare share(pre, n_inst, split);
     const qsft_peel_desc& d = descs[share.inst];
-    uint32_t* __restrict__ ctr = d.ctr;
+    uint32_t* __restrict__ ctr = in_global(d.ctr);
     if (it >= d.max_iter) return;                                  // beyond the bound workspace
     if (cptr(ctr)[it * QSFT_CTR_ITER_STRIDE + 3] == 0) return;    // loop already stopped (set by the
                                                                    // previous pass; scalar load)
@@ -1626,17 +1640,17 @@ __device__ __forceinline__ void apply_singleton(const qsft_peel_desc& d, int t, 
                                                 int n_pad, int nq, uint32_t* ctr, const int8_t* mt) {
     const int CQ = C * Q;
     const ModQ mq((uint32_t)q);
-    const int8_t* __restrict__ kcur = d.kbin + (size_t)(it & 1) * CQ * n_pad;
+    const int8_t* __restrict__ kcur = in_global(d.kbin) + (size_t)(it & 1) * CQ * n_pad;
     const uint4* __restrict__ krow = reinterpret_cast<const uint4*>(kcur + (size_t)t * n_pad);
     uint4 k[kKeyChunks];
 #pragma unroll
     for (int w = 0; w < kKeyChunks; ++w) k[w] = (w < nq) ? krow[w] : make_uint4(0u, 0u, 0u, 0u);
-    const int slot = d.slot_bin[t];
+    const int slot = in_global(d.slot_bin)[t];
     const uint64_t tm = ((uint64_t)(it + 1) << 32) | (uint32_t)t;
-    const uint64_t own = d.owner[slot];
-    const uint64_t lst = d.last[slot];
+    const uint64_t own = in_global(d.owner)[slot];
+    const uint64_t lst = in_global(d.last)[slot];
     // the detection's k must equal its slot's key
-    uint4* kslot = reinterpret_cast<uint4*>(d.key + (size_t)slot * n_pad);
+    uint4* kslot = reinterpret_cast<uint4*>(in_global(d.key) + (size_t)slot * n_pad);
     bool same = true;
     if (own == tm) {                                               // first detection of the key: it writes the key
 #pragma unroll
@@ -1678,7 +1692,7 @@ __device__ __forceinline__ void apply_singleton(const qsft_peel_desc& d, int t, 
                     }
                 }
             } else {
-                const uint4* __restrict__ mrow = reinterpret_cast<const uint4*>(d.Mt + mo);
+                const uint4* __restrict__ mrow = reinterpret_cast<const uint4*>(in_global(d.Mt) + mo);
 #pragma unroll
                 for (int w = 0; w < kKeyChunks; ++w) {
                     if (w < nq) {
@@ -1694,8 +1708,8 @@ __device__ __forceinline__ void apply_singleton(const qsft_peel_desc& d, int t, 
         }
         const int target = l * Q + jl;
         const int e = t * C + l;
-        d.pend_next[e] = atomicExch(&d.pend_head[target], e);
-        d.mark[target] = it + 1;                                   // the peeled bin is rescanned
+        in_global(d.pend_next)[e] = atomicExch(&in_global(d.pend_head)[target], e);
+        in_global(d.mark)[target] = it + 1;                                   // the peeled bin is rescanned
     }
 }
 
@@ -1712,7 +1726,7 @@ __device__ __forceinline__ void apply_singleton(const qsft_peel_desc& d, int t, 
 // pass ran and found a singleton and a multiton, below the peel cap.
 template <bool PERSIST>
 __device__ __forceinline__ void loop_control(const qsft_peel_desc& d, int it, uint32_t active) {
-    uint32_t* __restrict__ ctr = d.ctr;
+    uint32_t* __restrict__ ctr = in_global(d.ctr);
     auto rd = [&](int w) -> uint32_t {
         if constexpr (PERSIST) return __hip_atomic_load(ctr + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         else return ctr[w];
@@ -1735,7 +1749,7 @@ __global__ __launch_bounds__(kBinThreads) void k_peel_apply(const qsft_peel_desc
     __shared__ __align__(16) int8_t mtbuf[kStageMtBytes];
     const int inst = find_inst(pre, n_inst, blockIdx.x);
     const qsft_peel_desc& d = descs[inst];
-    uint32_t* __restrict__ ctr = d.ctr;
+    uint32_t* __restrict__ ctr = in_global(d.ctr);
     const int local = blockIdx.x - pre[inst];
     if (it >= d.max_iter) return;
     const uint32_t active = cptr(ctr)[it * QSFT_CTR_ITER_STRIDE + 3];   // written before this kernel
@@ -1746,7 +1760,7 @@ __global__ __launch_bounds__(kBinThreads) void k_peel_apply(const qsft_peel_desc
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int CQ = C * Q;
     const int t = (local * kWaves + wave) * kBinsPerWave + lane;
-    const bool mine = t < CQ && d.sstamp[t] == it + 1;
+    const bool mine = t < CQ && in_global(d.sstamp)[t] == it + 1;
     if (!__syncthreads_or(mine)) return;                           // (active is the same for the whole block)
     const bool mt_staged = stage_mt(d, mtbuf);                     // the targets' bin digits read M^T from LDS
     __syncthreads();
@@ -1781,7 +1795,7 @@ __global__ __launch_bounds__(64 * tail_waves<NR>()) void k_peel_tail(const qsft_
     __shared__ uint32_t theld[kW][kTailBatch];
     __shared__ uint32_t go;
     const qsft_peel_desc& d = descs[blockIdx.x];
-    uint32_t* __restrict__ ctr = d.ctr;
+    uint32_t* __restrict__ ctr = in_global(d.ctr);
     const int end = min(it_end, min(d.max_iter, 15));
     if (it0 >= end) return;                                        // (block-uniform)
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -1857,7 +1871,7 @@ constexpr int kFinTile = 2048;
 
 // Running mean over the m records of hash slot h.
 __device__ __forceinline__ double2 mean_of_records(const qsft_peel_desc& d, uint32_t h, uint32_t L) {
-    const uint32_t m = d.count[h];
+    const uint32_t m = in_global(d.count)[h];
     // g <- (g * c + v) / (c + 1)
     double gx = 0.0, gy = 0.0;
     auto accumulate = [&](uint32_t cnt, double vx, double vy) {
@@ -1884,10 +1898,10 @@ __device__ __forceinline__ double2 mean_of_records(const qsft_peel_desc& d, uint
             rx[a] = ry[a] = 0.0;
         }
         uint32_t steps = 0;
-        for (uint32_t r = d.head[h]; r != kNil && steps <= L; ++steps) {
-            const uint32_t next = d.rec_next[r];
-            uint64_t t = d.rec_time[r];
-            const double2 v = reinterpret_cast<const double2*>(d.rec_rho)[r];
+        for (uint32_t r = in_global(d.head)[h]; r != kNil && steps <= L; ++steps) {
+            const uint32_t next = in_global(d.rec_next)[r];
+            uint64_t t = in_global(d.rec_time)[r];
+            const double2 v = reinterpret_cast<const double2*>(in_global(d.rec_rho))[r];
             r = next;
             if (t <= prev || t >= tr[kFinRecs - 1]) continue;
             double vx = v.x, vy = v.y;
@@ -1927,25 +1941,25 @@ __global__ __launch_bounds__(kFinThreads) void k_peel_finalize(const qsft_peel_d
     __shared__ uint32_t part[kFinWaves][64];
     const int inst = blockIdx.x / per_inst, local = blockIdx.x - inst * per_inst;
     const qsft_peel_desc& d = descs[inst];
-    const uint32_t nlive = d.ctr[QSFT_CTR_LIVE];
+    const uint32_t nlive = in_global(d.ctr)[QSFT_CTR_LIVE];
     if (local == 0 && threadIdx.x == 0) {
-        d.ctr[QSFT_CTR_OUT] = nlive;
-        if (nlive > (uint32_t)d.out_cap) atomicOr(&d.ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_OUT_FULL);
+        in_global(d.ctr)[QSFT_CTR_OUT] = nlive;
+        if (nlive > (uint32_t)d.out_cap) atomicOr(&in_global(d.ctr)[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_OUT_FULL);
     }
     const int m = (int)min(nlive, (uint32_t)d.out_cap);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint32_t L = d.ctr[QSFT_CTR_LOG];
+    const uint32_t L = in_global(d.ctr)[QSFT_CTR_LOG];
     for (int o0 = local * 64; o0 < m; o0 += per_inst * 64) {       // (block-uniform)
         const int o = o0 + lane;
         const bool mine = o < m;
-        const uint32_t h = mine ? d.live[o] : 0u;
-        const uint64_t order = mine ? d.owner[h] : 0ull;
+        const uint32_t h = mine ? in_global(d.live)[o] : 0u;
+        const uint64_t order = mine ? in_global(d.owner)[h] : 0ull;
         double2 g = make_double2(0.0, 0.0);
         uint32_t rank = 0;
         for (int t0 = 0; t0 < m; t0 += kFinTile) {
             const int tn = min(kFinTile, m - t0), te = (tn + 1) & ~1;
             __syncthreads();                                       // the previous tile is consumed
-            for (int t = threadIdx.x; t < te; t += kFinThreads) tile[t] = t < tn ? d.owner[d.live[t0 + t]] : ~0ull;
+            for (int t = threadIdx.x; t < te; t += kFinThreads) tile[t] = t < tn ? in_global(d.owner)[in_global(d.live)[t0 + t]] : ~0ull;
             __syncthreads();
             if (wave == 0) {
                 if (t0 == 0 && mine) g = mean_of_records(d, h, L);
@@ -1965,11 +1979,11 @@ __global__ __launch_bounds__(kFinThreads) void k_peel_finalize(const qsft_peel_d
             rank = 0;
 #pragma unroll
             for (int w = 1; w < kFinWaves; ++w) rank += part[w][lane];
-            const uint4* ks = reinterpret_cast<const uint4*>(d.key + (size_t)h * d.n_pad);
-            uint4* kd = reinterpret_cast<uint4*>(d.out_k + (size_t)rank * d.n_pad);
+            const uint4* ks = reinterpret_cast<const uint4*>(in_global(d.key) + (size_t)h * d.n_pad);
+            uint4* kd = reinterpret_cast<uint4*>(in_global(d.out_k) + (size_t)rank * d.n_pad);
             for (int w = 0; w < (d.n_pad >> 4); ++w) kd[w] = ks[w];
-            reinterpret_cast<double2*>(d.out_val)[rank] = g;
-            d.out_order[rank] = order;
+            reinterpret_cast<double2*>(in_global(d.out_val))[rank] = g;
+            in_global(d.out_order)[rank] = order;
         }
     }
 }
@@ -2050,13 +2064,13 @@ __global__ __launch_bounds__(256) void k_pack(const qsft_peel_desc* __restrict__
     const int64_t m = min(rows_of(d), max(cap_rows - off, (int64_t)0));
     const int kw = d.n_pad >> 3;                                   // 8-byte words of the digits
     const uint32_t used = (uint32_t)kw + 3;
-    const uint64_t* __restrict__ ok = reinterpret_cast<const uint64_t*>(d.out_k);
-    const uint64_t* __restrict__ ov = reinterpret_cast<const uint64_t*>(d.out_val);
+    const uint64_t* __restrict__ ok = reinterpret_cast<const uint64_t*>(in_global(d.out_k));
+    const uint64_t* __restrict__ ov = reinterpret_cast<const uint64_t*>(in_global(d.out_val));
     const int64_t total = m * used;
     for (int64_t e = (int64_t)g * 256 + threadIdx.x; e < total; e += (int64_t)per_inst * 256) {
         const int64_t r = e / used;
         const int c = (int)(e - r * used);
-        const uint64_t v = c < kw ? ok[r * kw + c] : c < kw + 2 ? ov[2 * r + (c - kw)] : d.out_order[r];
+        const uint64_t v = c < kw ? ok[r * kw + c] : c < kw + 2 ? ov[2 * r + (c - kw)] : in_global(d.out_order)[r];
         *reinterpret_cast<uint64_t*>(rows + (off + r) * row_stride + 8 * c) = v;
     }
 }

@@ -13,6 +13,10 @@ namespace qsft {
 // gptr() so the accesses compile to global_* instructions.
 #define QSFT_GLOBAL __attribute__((address_space(1)))
 template <typename T> __device__ __forceinline__ QSFT_GLOBAL T* gptr(T* p) { return (QSFT_GLOBAL T*)p; }
+// in_global() does the same for code that keeps generic pointers and HIP's
+// vector classes: the way through the integer is not folded, and the compiler
+// carries the address space on to the accesses.
+template <typename T> __device__ __forceinline__ T* in_global(T* p) { return (T*)(QSFT_GLOBAL T*)(uintptr_t)p; }
 // Data that no thread writes while a kernel runs may be read through the
 // constant address space: wave-uniform reads then compile to scalar loads
 // (the LDS/scalar wait counter, not the vector-memory one).
