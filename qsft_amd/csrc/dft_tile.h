@@ -158,40 +158,52 @@ __host__ __device__ __forceinline__ bool radix_compiled(int q) {
 // kTileLoads loads of a thread are in flight together (one at a time, each
 // waited for before the next was issued, a 64 KiB tile of 256 threads spent 31
 // memory latencies on its way in).
+// A tile of at most two elements per thread moves without the other six steps'
+// conditions (q = 20, b = 2, 1347 rows in FP64: 20.2 -> 16.6 us back to back).
 constexpr int kTileLoads = 8;
-template <typename C2, typename G>
-__device__ __forceinline__ void tile_load(C2* lds, int E, G get) {
-    for (int e0 = threadIdx.x; e0 < E; e0 += kTileLoads * blockDim.x) {
-        C2 v[kTileLoads];
+template <int N, typename C2, typename G>
+__device__ __forceinline__ void tile_load_steps(C2* lds, int E, G get) {
+    for (int e0 = threadIdx.x; e0 < E; e0 += N * blockDim.x) {
+        C2 v[N];
 #pragma unroll
-        for (int k = 0; k < kTileLoads; ++k) {
+        for (int k = 0; k < N; ++k) {
             const int e = e0 + k * blockDim.x;
             if (e < E) v[k] = get(e);
         }
 #pragma unroll
-        for (int k = 0; k < kTileLoads; ++k) {
+        for (int k = 0; k < N; ++k) {
             const int e = e0 + k * blockDim.x;
             if (e < E) lds[e] = v[k];
         }
     }
 }
+template <typename C2, typename G>
+__device__ __forceinline__ void tile_load(C2* lds, int E, G get) {
+    if (E <= 2 * (int)blockDim.x) tile_load_steps<2>(lds, E, get);
+    else tile_load_steps<kTileLoads>(lds, E, get);
+}
 
 // And out again: put(e, value).
-template <typename C2, typename F>
-__device__ __forceinline__ void tile_store(const C2* lds, int E, F put) {
-    for (int e0 = threadIdx.x; e0 < E; e0 += kTileLoads * blockDim.x) {
-        C2 v[kTileLoads];
+template <int N, typename C2, typename F>
+__device__ __forceinline__ void tile_store_steps(const C2* lds, int E, F put) {
+    for (int e0 = threadIdx.x; e0 < E; e0 += N * blockDim.x) {
+        C2 v[N];
 #pragma unroll
-        for (int k = 0; k < kTileLoads; ++k) {
+        for (int k = 0; k < N; ++k) {
             const int e = e0 + k * blockDim.x;
             if (e < E) v[k] = lds[e];
         }
 #pragma unroll
-        for (int k = 0; k < kTileLoads; ++k) {
+        for (int k = 0; k < N; ++k) {
             const int e = e0 + k * blockDim.x;
             if (e < E) put(e, v[k]);
         }
     }
+}
+template <typename C2, typename F>
+__device__ __forceinline__ void tile_store(const C2* lds, int E, F put) {
+    if (E <= 2 * (int)blockDim.x) tile_store_steps<2>(lds, E, put);
+    else tile_store_steps<kTileLoads>(lds, E, put);
 }
 
 // The axis transforms of a tile of E elements, [.., q^mb, ti] with its mb axes
