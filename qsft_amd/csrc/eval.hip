@@ -207,13 +207,19 @@ __device__ __forceinline__ uint32_t quad_transpose(uint32_t x, int lane) {
 // q in {2, 3, 4}: cosine and sine of every phase are small integers (q = 3: of
 // 2 cos and sin / (sqrt(3)/2)), so the sum over the support is a contraction of
 // an int8 matrix with the coefficients, and runs on the matrix cores without a
-// rounding: each coefficient, as a fixed-point number of 63 bits below the
-// largest one, is eight signed base-256 digits; [cos | sin] (16 queries x 64
-// supports) times [re | im digits] (64 x 16) accumulates exactly in int32 (S <
-// 2^23), and the digit sums meet in int64 once per query. The error is the
-// final rounding and 2^-64 of the largest coefficient per term, less than a
-// sum in FP64 makes. A coefficient that is not finite sends the workgroup to
-// the table form, which carries it through as before.
+// rounding: each component of a coefficient is an integer of a common unit, in
+// 62-bit limbs of eight signed base-256 digits; [cos | sin] (16 queries x 64
+// supports) times [re | im digits] (64 x 16) per limb accumulates exactly in
+// int32 (S < 2^23), and the digit sums meet in a wide integer once per query.
+//
+// The unit is one that every component is a whole multiple of, so nothing is
+// lost on the way in: one limb where the largest component is below 2^62 units,
+// two up to 2^124 (FP64 components of random phases: 53 bits and a spread of
+// about log2 S more), four, two after the other, up to 2^248, the table form
+// beyond that and where a coefficient is not finite. For q = 2 the real and the imaginary parts never meet and have units
+// of their own. The result is the exact sum rounded once for q = 2 and 4; for
+// q = 3 the two sums are carried to about 2^-96 and sqrt(3)/2 to 2^-107, so
+// that the last rounding is the only one that shows.
 //
 // The phases come from the MFMA with the support along its rows: a lane then
 // holds 4 supports of one query per tile, and four tiles are the 16 bytes of
@@ -226,38 +232,297 @@ __device__ __forceinline__ uint32_t quad_transpose(uint32_t x, int lane) {
 // The table form is bound by its VALU and LDS reads (one 16 B entry and six
 // FP64 operations per term); this one by the conversion and packing (about 1.5
 // operations per term) and, as a launch of 100k queries is one and a half
-// rounds of the four waves per SIMD, by its last round. S = 1000, n = 50, q = 4,
-// FP64: 100003 queries 53 -> 20 us, 1000 queries 23 -> 7.5 us; S = 4000, n =
-// 100, 50000 queries 250 -> 65 us; q = 3, 100003 queries 58 -> 30 us; S = 10,
-// 100000 queries 22 -> 8 us. Fetching the next block's support ahead costs the
-// registers of a wave (20 us); eight waves per workgroup 24 us. Digits of the
-// queries stay in LDS for the same reason (n = 100: 110 us in registers).
-template <typename T, int NKB>
-__global__ __launch_bounds__(256, NKB <= 2 ? 4 : 1) void k_eval_points_int(const qsft_eval_points_desc* __restrict__ descs,
-                                                         const int32_t* __restrict__ pre, int n_inst) {
+// rounds of the four waves per SIMD, by its last round. Fetching the next
+// block's support ahead costs the registers of a wave; digits of the queries
+// stay in LDS for the same reason. Table and this form, FP64 strengths of 53
+// bits (two limbs): S = 1000, n = 50, q = 4, 100003 queries 53 and 32 us (one
+// limb, strengths of 24 bits: 23), 1000 queries 23 and 11; S = 4000, n = 100,
+// 50000 queries 249 and 126 (70); q = 3, 100003 queries 58 and 43 (35); S = 10,
+// 100000 queries 22 and 11.
+constexpr int kPointTiles = 4;                    // query tiles of 16 per workgroup
+constexpr int kSumPitch = 36;                     // rows 4 g + v of one column in 64 distinct banks
+
+template <int NKB>
+struct PointsLds {
+    int32_t sum[2][64][kSumPitch];                // [cos | sin][query][re, im digits of a limb | of the next]
+    int8_t dig[4][2][16][64];                     // [wave][limb][digit column][support of the block]
+    int8_t query[64][64 * NKB + 16];              // digits of the queries
+};
+
+// The magnitude of sum_i g[i] 2^(32 i), |g[i]| < 2^62, as m 2^e with m in
+// [2^63, 2^64) (or 0), the 32 bits below m, and whether any bit follows those.
+template <int N>
+struct WideInt {
+    uint64_t m;
+    uint32_t next;
+    int e;
+    bool neg, more;
+    __device__ __forceinline__ explicit WideInt(int64_t (&g)[N]) {
+        uint32_t w[N - 1];                        // the words below the top, carries passed up
+#pragma unroll
+        for (int i = 0; i < N - 1; ++i) {
+            w[i] = (uint32_t)g[i];
+            g[i + 1] += g[i] >> 32;
+        }
+        neg = g[N - 1] < 0;
+        m = (uint64_t)g[N - 1];
+        if (neg) {                                // two's complement
+            uint64_t carry = 1;
+#pragma unroll
+            for (int i = 0; i < N - 1; ++i) {
+                carry += (uint32_t)~w[i];
+                w[i] = (uint32_t)carry;
+                carry >>= 32;
+            }
+            m = ~m + carry;
+        }
+        e = 32 * (N - 1);
+        next = 0;
+        more = false;
+        bool full = false;                        // m has 33 bits or more and `next` is taken
+#pragma unroll
+        for (int i = N - 2; i >= 0; --i) {
+            if (full) {
+                more |= w[i] != 0;
+            } else if (m >> 32) {
+                next = w[i];
+                full = true;
+            } else {
+                m = m << 32 | w[i];
+                e -= 32;
+            }
+        }
+        const int lz = m ? (int)__builtin_clzll(m) : 0;            // (above 31 only without a next word)
+        m = m << lz | ((uint64_t)next << (lz & 31)) >> 32;
+        next = lz < 32 ? next << lz : 0;
+        e -= lz;
+    }
+    // rounded to nearest, in units of 2^e
+    template <typename T>
+    __device__ __forceinline__ T rounded() const {
+        const T v = (T)(m | (next != 0 || more ? 1u : 0u));
+        return neg ? -v : v;
+    }
+    // hi + lo to about 2^-96 of it, times 2^e
+    __device__ __forceinline__ double2 pair() const {
+        double hi = (double)(m & ~0x7FFull), lo = (double)(m & 0x7FFull) + (double)next * 0x1p-32;
+        if (neg) {
+            hi = -hi;
+            lo = -lo;
+        }
+        return make_double2(ldexp(hi, e), ldexp(lo, e));
+    }
+};
+
+// Limb `first` (and the next, where H = 2) of v, a whole number of units 2^unit
+// below 2^(62 LIMBS) of them: v is the sum of limb h times 2^(62 h), each rounded
+// to nearest from the top (|limb| <= 2^61 below the highest; a remainder has no
+// more bits than v, so every step is exact). Byte i of a word is the limb's
+// signed base-256 digit i: (x + b) ^ b with b = 0x80 in every byte turns the
+// bytes of a two's complement number into them.
+template <int LIMBS, int H>
+__device__ __forceinline__ void signed_digits(double v, int unit, int first, uint64_t (&w)[H]) {
+    constexpr uint64_t bias = 0x8080808080808080ull;
+    double r = ldexp(v, -unit), limb[H];
+#pragma unroll
+    for (int h = LIMBS - 1; h >= 0; --h) {
+        double t = r;
+        if (h > 0) {
+            t = rint(ldexp(r, -62 * h));
+            r = fma(-t, __builtin_bit_cast(double, (uint64_t)(1023 + 62 * h) << 52), r);
+        }
+        if (LIMBS == H || (h & ~(H - 1)) == first) limb[h & (H - 1)] = t;
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) w[h] = ((uint64_t)__double2ll_rn(limb[h]) + bias) ^ bias;
+}
+
+template <typename T, int NKB, int LIMBS>
+__device__ __forceinline__ void points_exact(const qsft_eval_points_desc& d, int64_t local, PointsLds<NKB>& sh,
+                                             const int (&unit)[2]) {
     using C2 = cplx_t<T>;
-    constexpr int kTiles = 4;                     // query tiles of 16
-    constexpr int kSumPitch = 20;                 // rows 4 g + v of one column in 64 distinct banks
-    __shared__ union {
-        struct {
-            int32_t sum[2][64][kSumPitch];        // [cos | sin][query][re, im digits]
-            int8_t dig[4][16][64];                // [wave][digit column][support of the block]
-            int8_t query[64][64 * NKB + 16];      // digits of the queries
-        } s;
-        C2 tab[QSFT_MAX_Q];
-    } sh;
-    __shared__ uint32_t top;
-    const int inst = find_inst(pre, n_inst, blockIdx.x);
-    const qsft_eval_points_desc& d = descs[inst];
-    const int64_t local = blockIdx.x - pre[inst];
+    constexpr int kHeld = LIMBS < 2 ? LIMBS : 2;  // limbs at once
+    // query tiles at once: with two limbs and two digit blocks the accumulators of all four do not fit the
+    // registers of four waves per SIMD
+    constexpr int kTiles = kHeld == 2 && NKB > 1 ? 2 : kPointTiles;
     const int q = d.q, S = d.S, n_pad = d.n_pad;
     const C2* __restrict__ a = in_global(reinterpret_cast<const C2*>(d.a));
     const int8_t* __restrict__ K = in_global(d.K);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = lane >> 4, r16 = lane & 15;
+    const uint32_t cosine = q == 4 ? 0x00FF0001u : q == 2 ? 0x0000FF01u : 0x00FFFF02u;
+    const uint32_t sine = q == 4 ? 0xFF000100u : q == 2 ? 0u : 0x00FF0100u;
+    const uint32_t mask = q == 4 ? 0x03030303u : q == 2 ? 0x01010101u : 0xFFFFFFFFu;
 
-    // exponent of the largest |re|, |im|
-    if (threadIdx.x == 0) top = 0;
+    const int qi = threadIdx.x >> 1, part = threadIdx.x & 1;      // query, re or im
+    const int64_t ql = local * 64 + qi;
+    int64_t c[2 * LIMBS], z[2 * LIMBS];           // four digits each, of the two sums
+#pragma unroll 1
+    for (int first = 0; first < LIMBS; first += kHeld) {
+#pragma unroll 1
+        for (int t0 = 0; t0 < kPointTiles; t0 += kTiles) {
+            v4i csum[kHeld][kTiles], ssum[kHeld][kTiles];
+#pragma unroll
+            for (int h = 0; h < kHeld; ++h) {
+#pragma unroll
+                for (int t = 0; t < kTiles; ++t) {
+                    csum[h][t] = v4i{0, 0, 0, 0};
+                    ssum[h][t] = v4i{0, 0, 0, 0};
+                }
+            }
+            for (int s0 = 64 * wave; s0 < S; s0 += 256) {
+                v4i kfrag[4][NKB];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int s = s0 + 16 * t + r16;
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb) {
+                        v4i z = {0, 0, 0, 0};
+                        if (s < S) z = *reinterpret_cast<const v4i*>(K + (size_t)s * n_pad + 64 * kb + 16 * g);
+                        kfrag[t][kb] = z;
+                    }
+                }
+                C2 as;
+                as.x = as.y = (T)0;
+                if (s0 + lane < S) as = a[s0 + lane];
+                // digits of this lane's support, at its place in the fragments' order:
+                // support 16 t + 4 g + v is byte 16 g + 4 t + v, so four neighbouring
+                // lanes hold the four bytes of a word of each digit's row
+                uint64_t word[2][kHeld];
+                signed_digits<LIMBS>((double)as.x, unit[0], first, word[0]);
+                signed_digits<LIMBS>((double)as.y, unit[1], first, word[1]);
+                const int pos = 16 * ((lane >> 2) & 3) + 4 * (lane >> 4);
+#pragma unroll
+                for (int h = 0; h < kHeld; ++h) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        *reinterpret_cast<uint32_t*>(&sh.dig[wave][h][4 * j + (lane & 3)][pos]) =
+                            quad_transpose((uint32_t)(word[j >> 1][h] >> (32 * (j & 1))), lane);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                v4i bfrag[kHeld];
+#pragma unroll
+                for (int h = 0; h < kHeld; ++h) bfrag[h] = *reinterpret_cast<const v4i*>(&sh.dig[wave][h][r16][16 * g]);
+#pragma unroll
+                for (int t = 0; t < kTiles; ++t) {
+                    v4i qfrag[NKB], cf, sf;
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb)
+                        qfrag[kb] = *reinterpret_cast<const v4i*>(&sh.query[16 * (t0 + t) + r16][64 * kb + 16 * g]);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        v4i p = {0, 0, 0, 0};
+#pragma unroll
+                        for (int kb = 0; kb < NKB; ++kb)
+                            p = __builtin_amdgcn_mfma_i32_16x16x64_i8(kfrag[u][kb], qfrag[kb], p, 0, 0, 0);
+                        if (q == 3) {
+                            // p - 3 floor((p + 1/2) / 3) in FP32: p < 2^22, so the quotient is off by less than 0.09
+                            // of the 1/6 that it may be
+#pragma unroll
+                            for (int w = 0; w < 4; ++w)
+                                p[w] -= 3 * (int)fmaf((float)p[w], 1.0f / 3.0f, 1.0f / 6.0f);
+                        }
+                        const uint32_t lo = __builtin_amdgcn_perm((uint32_t)p[1], (uint32_t)p[0], 0x0C0C0400u);
+                        const uint32_t up = __builtin_amdgcn_perm((uint32_t)p[3], (uint32_t)p[2], 0x04000C0Cu);
+                        const uint32_t r = (lo | up) & mask;
+                        cf[u] = (int)__builtin_amdgcn_perm(0u, cosine, r);
+                        sf[u] = (int)__builtin_amdgcn_perm(0u, sine, r);
+                    }
+#pragma unroll
+                    for (int h = 0; h < kHeld; ++h) {
+                        csum[h][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cf, bfrag[h], csum[h][t], 0, 0, 0);
+                        ssum[h][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(sf, bfrag[h], ssum[h][t], 0, 0, 0);
+                    }
+                }
+                __builtin_amdgcn_wave_barrier();      // the fragments are read before the next block's digits
+            }
+#pragma unroll
+            for (int h = 0; h < kHeld; ++h) {
+#pragma unroll
+                for (int t = 0; t < kTiles; ++t) {
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        atomicAdd(&sh.sum[0][16 * (t0 + t) + 4 * g + w][16 * h + r16], csum[h][t][w]);
+                        atomicAdd(&sh.sum[1][16 * (t0 + t) + 4 * g + w][16 * h + r16], ssum[h][t][w]);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2 * kHeld; ++i) {
+            const int at = 16 * (i >> 1) + 4 * (i & 1);
+            int64_t cv = 0, zv = 0;
+            if (qi < 64) {
+#pragma unroll
+                for (int j = 3; j >= 0; --j) {
+                    cv = cv * 256 + sh.sum[0][qi][at + 8 * part + j];
+                    zv = zv * 256 + sh.sum[1][qi][at + 8 * (1 - part) + j];
+                }
+            }
+            // limb h counts 2^(62 h) units = 2^(64 h) 4^(LIMBS - 1 - h) quarters of them, LIMBS - 1 times over
+            const int up = 2 * (LIMBS - 1 - first - (i >> 1));
+            c[2 * first + i] = cv << up;
+            z[2 * first + i] = (part ? zv : -zv) << up;            // re: cos re - sin im; im: cos im + sin re
+        }
+        if (first + kHeld < LIMBS) {
+            __syncthreads();                      // the sums are read
+            for (int i = threadIdx.x; i < 2 * 64 * kSumPitch; i += 256) (&sh.sum[0][0][0])[i] = 0;
+            __syncthreads();
+        }
+    }
+    if (qi >= 64 || ql >= d.N) return;
+    T x;
+    if (q == 3) {                                 // c / 2 + sqrt(3)/2 z
+#pragma clang fp contract(off)
+        const double h0 = 0.8660254037844386, h1 = 5.0175421109034514e-17;
+        const double2 cs = WideInt<2 * LIMBS>(c).pair(), zs = WideInt<2 * LIMBS>(z).pair();
+        const double p = h0 * zs.x, a0 = 0.5 * cs.x, s = a0 + p;
+        const double bb = s - a0, err = (a0 - (s - bb)) + (p - bb);                   // s + err = a0 + p
+        const double rest = fma(h0, zs.x, -p) + fma(h0, zs.y, fma(h1, zs.x, 0.5 * cs.y));
+        x = (T)ldexp(s + (err + rest), unit[part] - 2 * (LIMBS - 1));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2 * LIMBS; ++i) c[i] += z[i];
+        const WideInt<2 * LIMBS> w(c);
+        x = ldexp(w.template rounded<T>(), w.e + unit[part] - 2 * (LIMBS - 1));
+    }
+    in_global(reinterpret_cast<T*>(d.x))[2 * ql + part] = x;
+}
+
+// Bits of one component: the exponent that it stays below, and that of its
+// lowest set bit.
+__device__ __forceinline__ void component_range(double v, int& top, int& low) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v) & ~(1ull << 63);
+    if (b == 0) return;
+    const int f = (int)(b >> 52);
+    const uint64_t mant = (b & ((1ull << 52) - 1)) | (f ? 1ull << 52 : 0ull);
+    top = max(top, max(f, 1) - 1022);
+    low = min(low, max(f, 1) - 1075 + (int)__builtin_ctzll(mant));
+}
+
+template <typename T, int NKB>
+__global__ __launch_bounds__(256, NKB <= 2 ? 4 : 1) void k_eval_points_int(const qsft_eval_points_desc* __restrict__ descs,
+                                                         const int32_t* __restrict__ pre, int n_inst) {
+    using C2 = cplx_t<T>;
+    constexpr int kNotFinite = 0x7FF - 1022;
+    __shared__ union {
+        PointsLds<NKB> s;
+        C2 tab[QSFT_MAX_Q];
+    } sh;
+    __shared__ int range[2][2];                   // [re | im][top, low]
+    const int inst = find_inst(pre, n_inst, blockIdx.x);
+    const qsft_eval_points_desc& d = descs[inst];
+    const int64_t local = blockIdx.x - pre[inst];
+    const int q = d.q, S = d.S, n_pad = d.n_pad;
+    const C2* __restrict__ a = in_global(reinterpret_cast<const C2*>(d.a));
+    const int lane = threadIdx.x & 63;
+    constexpr int kNone = 4096;                   // beyond every exponent
+    if (threadIdx.x < 2) {
+        range[threadIdx.x][0] = -kNone;
+        range[threadIdx.x][1] = kNone;
+    }
 #pragma unroll
     for (int k = 0; k < NKB; ++k) {
         const int i = threadIdx.x + 256 * k, row = i / (4 * NKB), col = 16 * (i - row * (4 * NKB));
@@ -266,127 +531,52 @@ __global__ __launch_bounds__(256, NKB <= 2 ? 4 : 1) void k_eval_points_int(const
         *reinterpret_cast<v4i*>(&sh.s.query[row][col]) = z;
     }
     for (int i = threadIdx.x; i < 2 * 64 * kSumPitch; i += 256) (&sh.s.sum[0][0][0])[i] = 0;
-    uint32_t hi = 0;
+    int top[2] = {-kNone, -kNone}, low[2] = {kNone, kNone};
     for (int s = threadIdx.x; s < S; s += 256) {
         const C2 v = a[s];
-        hi = max(hi, max((uint32_t)__double2hiint((double)v.x) & 0x7FFFFFFFu,
-                         (uint32_t)__double2hiint((double)v.y) & 0x7FFFFFFFu));
+        component_range((double)v.x, top[0], low[0]);
+        component_range((double)v.y, top[1], low[1]);
     }
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) hi = max(hi, (uint32_t)__shfl_xor((int)hi, off));
+    for (int off = 1; off < 64; off <<= 1) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            top[p] = max(top[p], __shfl_xor(top[p], off));
+            low[p] = min(low[p], __shfl_xor(low[p], off));
+        }
+    }
     __syncthreads();
-    if (lane == 0) atomicMax(&top, hi);
+    if (lane == 0) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            atomicMax(&range[p][0], top[p]);
+            atomicMin(&range[p][1], low[p]);
+        }
+    }
     __syncthreads();
-    const int field = (int)(top >> 20);
-    if (field == 0x7FF) {                         // infinity or NaN (the same word in all threads)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {                 // (the same words in all threads)
+        top[p] = __builtin_amdgcn_readfirstlane(range[p][0]);
+        low[p] = __builtin_amdgcn_readfirstlane(range[p][1]);
+    }
+    if (q != 2) {
+        top[0] = top[1] = max(top[0], top[1]);
+        low[0] = low[1] = min(low[0], low[1]);
+    }
+    const int bits = max(top[0] - low[0], top[1] - low[1]);       // (negative where all are zero)
+    if (bits <= 62 && top[0] < kNotFinite && top[1] < kNotFinite) {
+        const int unit[2] = {low[0] < kNone ? top[0] - 62 : 0, low[1] < kNone ? top[1] - 62 : 0};
+        points_exact<T, NKB, 1>(d, local, sh.s, unit);
+    } else if (bits <= 124 && top[0] < kNotFinite && top[1] < kNotFinite) {
+        const int unit[2] = {low[0] < kNone ? top[0] - 124 : 0, low[1] < kNone ? top[1] - 124 : 0};
+        points_exact<T, NKB, 2>(d, local, sh.s, unit);
+    } else if (bits <= 248 && top[0] < kNotFinite && top[1] < kNotFinite) {
+        const int unit[2] = {low[0] < kNone ? top[0] - 248 : 0, low[1] < kNone ? top[1] - 248 : 0};
+        points_exact<T, NKB, 4>(d, local, sh.s, unit);
+    } else {
         __syncthreads();
         points_by_table<T, false, NKB>(d, local, sh.tab);
-        return;
     }
-    const int e = max(field, 1) - 1022;           // largest component < 2^e
-    const uint32_t cosine = q == 4 ? 0x00FF0001u : q == 2 ? 0x0000FF01u : 0x00FFFF02u;
-    const uint32_t sine = q == 4 ? 0xFF000100u : q == 2 ? 0u : 0x00FF0100u;
-    const uint32_t mask = q == 4 ? 0x03030303u : q == 2 ? 0x01010101u : 0xFFFFFFFFu;
-
-    v4i csum[kTiles], ssum[kTiles];
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-        csum[t] = v4i{0, 0, 0, 0};
-        ssum[t] = v4i{0, 0, 0, 0};
-    }
-    int8_t(*dig)[64] = sh.s.dig[wave];
-    for (int s0 = 64 * wave; s0 < S; s0 += 256) {
-        v4i kfrag[4][NKB];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int s = s0 + 16 * t + r16;
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-                v4i z = {0, 0, 0, 0};
-                if (s < S) z = *reinterpret_cast<const v4i*>(K + (size_t)s * n_pad + 64 * kb + 16 * g);
-                kfrag[t][kb] = z;
-            }
-        }
-        C2 as;
-        as.x = as.y = (T)0;
-        if (s0 + lane < S) as = a[s0 + lane];
-        // digits of this lane's support, at its place in the fragments' order:
-        // support 16 t + 4 g + v is byte 16 g + 4 t + v, so four neighbouring
-        // lanes hold the four bytes of a word of each digit's row
-        const uint64_t bias = 0x8080808080808080ull;
-        const uint64_t re = ((uint64_t)__double2ll_rn(ldexp((double)as.x, 62 - e)) + bias) ^ bias;
-        const uint64_t im = ((uint64_t)__double2ll_rn(ldexp((double)as.y, 62 - e)) + bias) ^ bias;
-        const uint32_t word[4] = {(uint32_t)re, (uint32_t)(re >> 32), (uint32_t)im, (uint32_t)(im >> 32)};
-        const int pos = 16 * ((lane >> 2) & 3) + 4 * (lane >> 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            *reinterpret_cast<uint32_t*>(&dig[4 * j + (lane & 3)][pos]) = quad_transpose(word[j], lane);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        const v4i bfrag = *reinterpret_cast<const v4i*>(&dig[r16][16 * g]);
-#pragma unroll
-        for (int t = 0; t < kTiles; ++t) {
-            v4i qfrag[NKB], cf, sf;
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb)
-                qfrag[kb] = *reinterpret_cast<const v4i*>(&sh.s.query[16 * t + r16][64 * kb + 16 * g]);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                v4i p = {0, 0, 0, 0};
-#pragma unroll
-                for (int kb = 0; kb < NKB; ++kb)
-                    p = __builtin_amdgcn_mfma_i32_16x16x64_i8(kfrag[u][kb], qfrag[kb], p, 0, 0, 0);
-                if (q == 3) {
-                    // p - 3 floor((p + 1/2) / 3) in FP32: p < 2^22, so the quotient is off by less than 0.09
-                    // of the 1/6 that it may be
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        p[v] -= 3 * (int)fmaf((float)p[v], 1.0f / 3.0f, 1.0f / 6.0f);
-                }
-                const uint32_t lo = __builtin_amdgcn_perm((uint32_t)p[1], (uint32_t)p[0], 0x0C0C0400u);
-                const uint32_t up = __builtin_amdgcn_perm((uint32_t)p[3], (uint32_t)p[2], 0x04000C0Cu);
-                const uint32_t r = (lo | up) & mask;
-                cf[u] = (int)__builtin_amdgcn_perm(0u, cosine, r);
-                sf[u] = (int)__builtin_amdgcn_perm(0u, sine, r);
-            }
-            csum[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cf, bfrag, csum[t], 0, 0, 0);
-            ssum[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(sf, bfrag, ssum[t], 0, 0, 0);
-        }
-        __builtin_amdgcn_wave_barrier();          // the fragment is read before the next block's digits
-    }
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            atomicAdd(&sh.s.sum[0][16 * t + 4 * g + v][r16], csum[t][v]);
-            atomicAdd(&sh.s.sum[1][16 * t + 4 * g + v][r16], ssum[t][v]);
-        }
-    }
-    __syncthreads();
-    const int qi = threadIdx.x >> 1, part = threadIdx.x & 1;      // query, re or im
-    const int64_t ql = local * 64 + qi;
-    if (qi >= 64 || ql >= d.N) return;
-    int64_t c0 = 0, c1 = 0, z0 = 0, z1 = 0;       // low and high four digits of the two sums
-#pragma unroll
-    for (int j = 3; j >= 0; --j) {
-        c0 = c0 * 256 + sh.s.sum[0][qi][8 * part + j];
-        c1 = c1 * 256 + sh.s.sum[0][qi][8 * part + 4 + j];
-        z0 = z0 * 256 + sh.s.sum[1][qi][8 * (1 - part) + j];
-        z1 = z1 * 256 + sh.s.sum[1][qi][8 * (1 - part) + 4 + j];
-    }
-    if (!part) {                                  // re: cos re - sin im; im: cos im + sin re
-        z0 = -z0;
-        z1 = -z1;
-    }
-    double x;
-    if (q == 3) {
-        const double cs = fma((double)c1, 4294967296.0, (double)c0);
-        const double zs = fma((double)z1, 4294967296.0, (double)z0);
-        x = fma(0.86602540378443864676, zs, 0.5 * cs);
-    } else {
-        x = fma((double)(c1 + z1), 4294967296.0, (double)(c0 + z0));
-    }
-    in_global(reinterpret_cast<T*>(d.x))[2 * ql + part] = (T)ldexp(x, e - 62);
 }
 
 
@@ -497,7 +687,8 @@ extern "C" int qsft_eval_points_blocks(const qsft_eval_points_desc* h) {
 
 // Integer sums for q whose cosines and sines are one constant times small
 // integers, up to the S that int32 digit sums hold (2^23 digits of at most 2^7).
-// They win at every size measured, from S = 10 or 1000 queries up (above).
+// They win at every size measured, from S = 10 or 1000 queries up (above). What
+// the coefficients allow is found by the kernel.
 extern "C" int qsft_eval_points_int(const qsft_eval_points_desc* h) {
     return h && h->q >= 2 && h->q <= 4 && h->S < (1 << 23);
 }

@@ -1,5 +1,8 @@
 """Explicit query points with q in {2, 3, 4}: the exact integer form against sums in 80-bit floats, and
 against the w-table form where a coefficient is not finite."""
+from decimal import Decimal, localcontext
+from fractions import Fraction
+
 import numpy as np
 import pytest
 import torch
@@ -84,3 +87,89 @@ def test_points_mixed_launch():
     K.eval_points(items, L.QSFT_F64)
     for it, ref in zip(items, refs):
         assert np.abs(it["x"].cpu().numpy() - ref).max() <= 1e-13 * np.abs(ref).max() * 10
+
+
+def _exact(q, pts, locq, a):
+    """(re, im, sizes of the parts that meet) of every query in rational numbers, sqrt(3) to 100 digits."""
+    with localcontext() as ctx:
+        ctx.prec = 100
+        half = Fraction(Decimal(3).sqrt()) / 2
+    cos = {2: [1, -1], 3: [2, -1, -1], 4: [1, 0, -1, 0]}[q]
+    sin = {2: [0, 0], 3: [0, 1, -1], 4: [0, 1, 0, -1]}[q]
+    unit = Fraction(1, 2 ** 1074)                                 # of which every component is a whole number
+    ct, st = (Fraction(1, 2), half) if q == 3 else (1, 1)
+    E = (pts.astype(np.int64) @ locq.astype(np.int64)) % q
+    re, im = ([int(Fraction(float(v)) / unit) for v in part] for part in (a.real, a.imag))
+    out = []
+    for row in E.tolist():
+        cr, ci = (ct * unit * sum(cos[e] * v for e, v in zip(row, part)) for part in (re, im))
+        sr, si = (st * unit * sum(sin[e] * v for e, v in zip(row, part)) for part in (re, im))
+        out.append((cr - si, ci + sr, abs(cr) + abs(si), abs(ci) + abs(sr)))
+    return out
+
+
+def _strengths(kind, S, precision, rng):
+    """Components of one size, one part far below the other, or spread over many decades."""
+    re, im = rng.normal(size=S), rng.normal(size=S)
+    if kind == "small im":
+        im = im * 1e-25
+    if kind == "small re":
+        re = re * 1e-18
+    if kind == "decades":
+        re, im = re * 10.0 ** rng.uniform(-9, 9, S), im * 10.0 ** rng.uniform(-9, 9, S)
+    if kind == "many decades":
+        re, im = re * 10.0 ** rng.uniform(-24, 24, S), im * 10.0 ** rng.uniform(-24, 24, S)
+    if kind == "cancelling":                                      # large terms that cancel in pairs, small ones left
+        re[: S // 2 * 2: 2], im[: S // 2 * 2: 2] = 1e9 * re[: S // 2 * 2: 2], 1e9 * im[: S // 2 * 2: 2]
+        re[1::2], im[1::2] = -re[: S // 2 * 2: 2], -im[: S // 2 * 2: 2]
+        re[-1], im[-1] = 1e-7, 3e-8
+    if kind == "whole":
+        re, im = np.rint(re * 8), np.zeros(S)
+    if kind == "subnormal":
+        least = 5e-324 if precision == "fp64" else 2.0 ** -149
+        re, im = np.rint(re * 9) * least, np.rint(im * 9) * least
+    return re + 1j * im
+
+
+@pytest.mark.parametrize("q", [2, 3, 4])
+@pytest.mark.parametrize("n,S,N", [(50, 1, 3), (64, 64, 70), (65, 66, 33), (140, 131, 65), (250, 40, 17)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("kind", ["plain", "small im", "small re", "decades", "cancelling", "whole", "subnormal",
+                                  "many decades"])
+def test_points_every_component_in_full(q, n, S, N, precision, kind):
+    """Each component is the exact sum, rounded once: within half a unit of its own last place, whatever the sizes
+    of the others. q = 3: and 2^-90 of the two sums that meet in it."""
+    print(f"points in full q={q} n={n} S={S} N={N} {precision} {kind}", flush=True)
+    rng = np.random.default_rng(q * 100 + S)
+    locq, pts = rng.integers(0, q, size=(n, S)), rng.integers(0, q, size=(N, n))
+    if kind == "cancelling":
+        locq[:, 1::2] = locq[:, : S // 2 * 2: 2]
+    dev, n_pad = dv.current_device(), dv.n_pad_of(n)
+    at = dv.strengths_tensor(_strengths(kind, S, precision, rng), precision, dev)
+    a = at.cpu().numpy().astype(np.complex128)
+    x = dv.evaluate_points(q, n, dv.digits_tensor(pts, n_pad, dev), dv.digits_tensor(locq.T, n_pad, dev), at,
+                           precision).cpu().numpy().astype(np.complex128)
+    half_ulp = Fraction(1, 2 ** 53) if precision == "fp64" else Fraction(1, 2 ** 24)
+    tiny = Fraction(1, 2 ** 1075) if precision == "fp64" else Fraction(1, 2 ** 150)   # half the smallest number
+    for got, (re, im, pr, pi) in zip(x, _exact(q, pts, locq, a)):
+        for g, ref, parts in ((got.real, re, pr), (got.imag, im, pi)):
+            bound = max(half_ulp * abs(ref) * (1 + Fraction(1, 10 ** 6)), tiny if q == 3 else 0)
+            assert abs(Fraction(float(g)) - ref) <= bound + (parts / 2 ** 90 if q == 3 else 0), (g, float(ref))
+
+
+@pytest.mark.parametrize("q", [2, 3, 4])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_points_of_too_wide_a_range_by_the_table(q, precision):
+    """Components that four limbs do not span (one part of q = 2 is enough) come out as the table form gives them."""
+    rng = np.random.default_rng(q)
+    n, S, N = 70, 150, 130
+    dev, n_pad = dv.current_device(), dv.n_pad_of(n)
+    a = rng.normal(size=S) * 10.0 ** rng.uniform(-18, 18, S) + 1j * rng.normal(size=S)
+    a[:2] = [1e-37 / 3, 2e38]
+    m = dv.digits_tensor(rng.integers(0, q, size=(N, n)), n_pad, dev)
+    k = dv.digits_tensor(rng.integers(0, q, size=(S, n)), n_pad, dev)
+    at = dv.strengths_tensor(a, precision, dev)
+    got = dv.evaluate_points(q, n, m, k, at, precision)
+    ref = torch.empty_like(got)
+    K.EvalPoints([dict(q=q, n=n, S=S, m=m, K=k, a=at, x=ref)], dv.PRECISIONS[precision][0], table=True).launch()
+    np.testing.assert_array_equal(got.cpu().numpy(), ref.cpu().numpy())
