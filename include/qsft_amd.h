@@ -153,6 +153,7 @@ typedef struct qsft_fold_desc {
     double* as;             /* [C][S] complex strengths in sorted order                     */
     uint64_t* key;          /* [C][S] bin << 32 | s, sorted                                 */
     uint32_t* J;            /* [C][S] bins                                                  */
+    uint32_t* bad;          /* [1 + S] strengths that are not finite: their number, then s  */
     int32_t* start;         /* [C][tiles + 1] first sorted position of each tile            */
 } qsft_fold_desc;
 

@@ -88,7 +88,7 @@ class FoldDesc(ctypes.Structure):
                 ("pass_ti", i32 * 4), ("pass_ta", i32 * 4), ("pass_blocks", i32 * 4), ("pass_lds", i32 * 4),
                 ("tiles", i32), ("tile_bins", i32), ("rpw", i32), ("fwd", i32),
                 ("Mt", vp), ("D", vp), ("K", vp), ("a", vp), ("x", vp),
-                ("E", vp), ("as_", vp), ("key", vp), ("J", vp), ("start", vp)]
+                ("E", vp), ("as_", vp), ("key", vp), ("J", vp), ("bad", vp), ("start", vp)]
 
 
 class Request(ctypes.Structure):

@@ -84,6 +84,7 @@ __global__ __launch_bounds__(kPhaseThreads) void k_fold_phase(const SRC src) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int g = lane >> 4, r16 = lane & 15;
     const int s0 = sg * 64 + wave * 16;
+    if (local == 0 && threadIdx.x == 0) in_global(d.bad)[0] = 0;   // (counted by k_fold_rank)
     if (s0 >= S) return;
     const int ptiles = (P + 15) / 16;
     const int dtiles = (d.shared_d ? 1 : C) * ptiles;
@@ -125,6 +126,10 @@ __global__ __launch_bounds__(kPhaseThreads) void k_fold_phase(const SRC src) {
             if (r16 < 4 && s0 + 4 * g + r16 < S) in_global(d.J)[(size_t)c * S + s0 + 4 * g + r16] = (uint32_t)mine;
         }
     }
+}
+
+__device__ __forceinline__ bool finite2(double2 a) {
+    return __builtin_isfinite(a.x) && __builtin_isfinite(a.y);
 }
 
 // Items of one group: its S supports, then (from the next multiple of 64) the
@@ -184,6 +189,14 @@ __global__ __launch_bounds__(kRankThreads) void k_fold_rank(const SRC src) {
             a = make_double2(f.x, f.y);
         } else {
             a = reinterpret_cast<const double2*>(d.a)[item];
+        }
+        if (!finite2(a)) {
+            if (d.fwd) {
+                a = make_double2(__builtin_nan(""), __builtin_nan(""));
+            } else {
+                if (c == 0) in_global(d.bad)[1 + atomicAdd(in_global(d.bad), 1u)] = (uint32_t)item;
+                a = make_double2(0.0, 0.0);
+            }
         }
         reinterpret_cast<double2*>(d.as)[(size_t)c * S + rank] = a;
     }
@@ -315,6 +328,41 @@ __device__ __forceinline__ const QSFT_GLOBAL uint8_t* phase_row(const qsft_fold_
     return gptr(d.E) + ((size_t)(d.shared_d ? 0 : c) * d.P + p) * fold_sp(d.S);
 }
 
+// Strengths that are not finite stay out of the transforms, whose butterflies
+// would meet infinities of both signs and, for q = 4, never the product with a
+// zero cosine or sine: k_fold_rank lists them and takes zero, and here their
+// terms a w^{<m, k>} are added to the finished samples of row p of group c, the
+// elements at(e) for e < E, as the sum over every support has them: an infinity
+// of the right sign or a NaN. (Sub-transforms are sums over all samples of a
+// row, which then are NaN: fwd descriptors take NaN for such a strength.)
+template <typename T, typename G>
+__device__ __forceinline__ void add_not_finite(const qsft_fold_desc& d, uint32_t count, int c, int p,
+                                               cplx_t<T>* __restrict__ x, int E, G at) {
+    const QSFT_GLOBAL uint8_t* ph = phase_row(d, c, p);
+    __syncthreads();                                               // the row's samples are written
+    for (int e = threadIdx.x; e < E; e += blockDim.x) {
+        const int64_t l = at(e);
+        cplx_t<T> v = x[l];
+        for (uint32_t i = 0; i < count; ++i) {
+            const uint32_t s = gptr(d.bad)[1 + i];
+            uint32_t r = ph[s], j = gptr(d.J)[(size_t)c * d.S + s], m = (uint32_t)l;
+            for (int t = 0; t < d.b; ++t, j /= d.q, m /= d.q) r += (j % d.q) * (m % d.q);
+            double sn, cs, ax, ay;
+            sincospi(2.0 * (double)(r % d.q) / (double)d.q, &sn, &cs);
+            if (d.a_prec == QSFT_F32) {
+                ax = reinterpret_cast<const float2*>(d.a)[s].x;
+                ay = reinterpret_cast<const float2*>(d.a)[s].y;
+            } else {
+                ax = reinterpret_cast<const double2*>(d.a)[s].x;
+                ay = reinterpret_cast<const double2*>(d.a)[s].y;
+            }
+            v.x += (T)(ax * cs - ay * sn);
+            v.y += (T)(ax * sn + ay * cs);
+        }
+        x[l] = v;
+    }
+}
+
 // One pass over the axes [d0, d1) of every row (dft.hip's tile scheme). The
 // first pass (FIRST: the innermost axes, so a tile is a contiguous run of
 // bins) folds its terms into the tile; later passes read x. Between passes x
@@ -393,6 +441,8 @@ __global__ __launch_bounds__(TH) void k_fold_pass(const SRC src, int pass, int l
         else tile_store(cur, E, [&](int e, C2 v) { x[goff(e)] = v; });
     } else if (pass == d.n_pass - 1) {
         tile_store(cur, E, [&](int e, C2 v) { x[goff(e)] = C2{v.y, v.x}; });
+        if (const uint32_t bad = d.S > 0 ? cptr(d.bad)[0] : 0)
+            add_not_finite<T>(d, bad, row / d.P, row % d.P, x, E, goff);
     } else {
         tile_store(cur, E, [&](int e, C2 v) { x[goff(e)] = v; });
     }
@@ -560,6 +610,13 @@ __global__ __launch_bounds__(fold4_threads<B>()) __attribute__((
             for (int j = 0; j < 16; ++j) store_c2(x + (xo + tid + j * kTpr), C2{v[j].y, v[j].x});   // (window B - 2)
         }
     }
+    if constexpr (!FWD) {
+        if (const uint32_t bad = d.S > 0 ? cptr(d.bad)[0] : 0) {
+            for (int p = p0; p < p1; ++p)
+                add_not_finite<T>(d, bad, c, p, in_global(reinterpret_cast<C2*>(d.x)) + ((int64_t)c * P + p) * Q, Q,
+                                  [](int e) { return (int64_t)e; });
+        }
+    }
 }
 
 }  // namespace qsft
@@ -590,12 +647,13 @@ bool fold_shape_ok(int q, int n, int b, int C, int P, int S, int n_pad) {
 
 }  // namespace
 
-// Phases (groups x P x 16-padded S bytes), sorted strengths and keys, bins (C x S), tile
-// starts (a first-pass tile holds at least q bins).
+// Phases (groups x P x 16-padded S bytes), sorted strengths and keys, bins (C x S), the
+// strengths that are not finite (a count and at most S), tile starts (a first-pass tile
+// holds at least q bins).
 extern "C" size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, int shared_d) {
     if (!fold_shape_ok(q, 1, b, C, P, S, 64)) return 0;
     return al256((size_t)(shared_d ? 1 : C) * P * fold_sp(S)) + al256((size_t)C * S * 16) +
-           al256((size_t)C * S * 8) + al256((size_t)C * S * 4) + al256((size_t)C * (ipow(q, b) / std::min(q, 32) + 2) * 4);
+           al256((size_t)C * S * 8) + al256((size_t)C * S * 4) + al256(((size_t)S + 1) * 4) + al256((size_t)C * (ipow(q, b) / std::min(q, 32) + 2) * 4);
 }
 
 extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int P, int S, int n_pad, int shared_d,
@@ -624,6 +682,8 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
     w += al256((size_t)C * S * 8);
     d.J = reinterpret_cast<uint32_t*>(w);
     w += al256((size_t)C * S * 4);
+    d.bad = reinterpret_cast<uint32_t*>(w);
+    w += al256(((size_t)S + 1) * 4);
     d.start = reinterpret_cast<int32_t*>(w);
     const int Q = ipow(q, b);
     if (fold_rows4(q, b, precision)) {

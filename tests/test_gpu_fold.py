@@ -143,3 +143,32 @@ def test_fold_gives_the_same_bits_alone_and_beside_larger_rows():
         alone = _item(q, 20, b, *x, "fp32")
         K.EvalFold([alone], L.QSFT_F32, transform=True).launch()
         assert torch.equal(torch.view_as_real(alone["x"]), torch.view_as_real(it["x"])), (q, b)
+
+
+BAD = [complex(np.inf, 0), complex(0, -np.inf), complex(-np.inf, 2), complex(np.inf, np.inf), complex(np.nan, 1),
+       complex(2, np.nan)]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("q,n,b,S", [(2, 9, 5, 30), (2, 20, 14, 70), (3, 7, 4, 65), (4, 9, 3, 30), (4, 20, 4, 100),
+                                     (4, 20, 5, 300), (4, 9, 6, 40), (4, 9, 7, 40), (5, 9, 3, 30), (20, 5, 2, 33),
+                                     (20, 6, 4, 20), (7, 9, 2, 30), (50, 4, 2, 20)])
+def test_fold_of_strengths_that_are_not_finite(q, n, b, S, precision):
+    """One such strength, or several, makes every sample what the sum over all supports makes it: an infinity of
+    the same sign or a NaN. Sub-transforms, sums over such samples, are NaN throughout."""
+    print(f"fold not finite q={q} n={n} b={b} S={S} {precision}", flush=True)
+    code = L.QSFT_F32 if precision == "fp32" else L.QSFT_F64
+    for bad in [[v] for v in BAD] + [[BAD[0], BAD[1]], [BAD[0], -BAD[0], BAD[2]], BAD]:
+        Ms, Ds, loc, a = _inputs(q, n, b, S, 2, 3, seed=S)
+        a[np.random.default_rng(b).permutation(S)[:len(bad)]] = bad
+        it = _item(q, n, b, Ms, Ds, loc, a, precision)
+        it["a"] = dv.strengths_tensor(a, precision, dv.current_device())
+        K.EvalFold([it], code).launch()
+        ref = dict(it, x=torch.empty_like(it["x"]))
+        K.EvalCosets([ref], code).launch()
+        np.testing.assert_array_equal(torch.view_as_real(it["x"]).cpu().numpy(),
+                                      torch.view_as_real(ref["x"]).cpu().numpy())
+        ev = K.EvalFold([it], code, transform=True)
+        ev.launch()
+        K.Dft(ev.rest, code).launch()
+        assert torch.isnan(torch.view_as_real(it["x"])).all()
