@@ -209,21 +209,24 @@ __global__ __launch_bounds__(kRankThreads) void k_fold_rank(const SRC src) {
 // (the terms of one bin), so no two waves touch a bin and none waits for
 // another. A block at a time: each lane forms one term, a segmented scan over
 // the run (as many steps as the longest run in the block needs) leaves a run's
-// sum in its last lane, which adds it. Equal shares keep a row's time even
-// where one bin holds most of the terms (supports of low weight). The blocks
-// are the same for every tile and workgroup size, so the order of a sum
-// depends on the sorted positions only.
+// sum in its last lane, which stores it, or hands it on to the next block in
+// FP64 registers where the run goes on there: a bin is rounded once, however
+// many terms it has. Equal shares keep a row's time even where terms crowd in a
+// few bins, down to one wave's for a single bin. The blocks are the same for
+// every tile and workgroup size, so the order of a sum depends on the sorted
+// positions only.
 //
 // What a lane needs of its position, the same for every row of the group:
 struct Term {
     uint32_t j, s;       // bin and support
     gd2 a;               // strength
-    int flags;           // kTermLive | kTermEmit | kTermWhole | lanes back to the run's first live lane
+    int flags;           // kTermLive | kTermEmit | kTermOpen | kTermOn | lanes back to the run's first live lane
 };
 constexpr int kTermDepth = 63;       // mask of the distance
 constexpr int kTermLive = 64;        // a term of this wave
-constexpr int kTermEmit = 128;       // last lane of the run in the block
-constexpr int kTermWhole = 256;      // ... and the run lies inside the block: its sum is the bin's
+constexpr int kTermEmit = 128;       // last term of the run
+constexpr int kTermOpen = 256;       // lane 63 of a run that goes on in the next block
+constexpr int kTermOn = 512;         // a run that began in an earlier block
 
 struct TermShare {
     int lo, hi, first, last;
@@ -263,7 +266,9 @@ struct TermShare {
             if (lane >= from && lane < to) {
                 const uint64_t before = bm & (~0ull >> (63 - lane));
                 t.flags = kTermLive | (lane - max(before ? 63 - (int)__builtin_clzll(before) : 0, from));
-                if (lane + 1 == to || t.j != kn) t.flags |= kTermEmit | (before && t.j != kn ? kTermWhole : 0);
+                if (t.j != kn) t.flags |= kTermEmit;
+                else if (lane == 63) t.flags |= kTermOpen;
+                if (!before) t.flags |= kTermOn;
             }
         }
         return past == 0;
@@ -275,10 +280,19 @@ __device__ __forceinline__ double lane_below(double v) {
     return dpp_f64<0x138>(v);                                      // wave_shr:1
 }
 
+// FP64 value of lane 63 in all lanes.
+__device__ __forceinline__ double lane63(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, 63);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), 63);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
 // Sums of one block's runs: term(t, sx, sy) forms a live lane's term,
-// put(t, sx, sy) takes the sum of a run in its last lane.
+// put(t, sx, sy) takes the sum of a run in its last lane. cx, cy: the sum so
+// far of the run that the block before left open.
 template <typename TM, typename F>
-__device__ __forceinline__ void term_add(const Term& t, TM term, F put) {
+__device__ __forceinline__ void term_add(const Term& t, double& cx, double& cy, TM term, F put) {
     if (!__ballot(t.flags & kTermLive)) return;
     double sx = 0.0, sy = 0.0;
     if (t.flags & kTermLive) term(t, sx, sy);
@@ -297,7 +311,15 @@ __device__ __forceinline__ void term_add(const Term& t, TM term, F put) {
             }
         }
     }
+    if (t.flags & kTermOn) {
+        sx += cx;
+        sy += cy;
+    }
     if (t.flags & kTermEmit) put(t, sx, sy);
+    if (__ballot(t.flags & kTermOpen)) {
+        cx = lane63(sx);
+        cy = lane63(sy);
+    }
 }
 
 template <typename TM, typename F>
@@ -306,21 +328,11 @@ __device__ __forceinline__ void fold_terms(const qsft_fold_desc& d, int c, int l
     TermShare sh(lo, hi, wave, waves);
     Term t;
     bool more = true;
+    double cx = 0.0, cy = 0.0;
     for (int i0 = sh.first; more; i0 += 64) {
         more = sh.load(d, c, i0, t);
-        term_add(t, term, put);
+        term_add(t, cx, cy, term, put);
     }
-}
-
-// A run's sum into its bin (swapped parts): stored where the run is the whole
-// bin, else added to the bin's earlier blocks.
-template <typename T>
-__device__ __forceinline__ void bin_put(cplx_t<T>& u, const Term& t, double sx, double sy) {
-    if (!(t.flags & kTermWhole)) {
-        sx += (double)u.y;
-        sy += (double)u.x;
-    }
-    u = cplx_t<T>{(T)sy, (T)sx};
 }
 
 // Phases of row p of group c.
@@ -425,7 +437,7 @@ __global__ __launch_bounds__(TH) void k_fold_pass(const SRC src, int pass, int l
                        sx = t.a.x * w.x - t.a.y * w.y;
                        sy = t.a.x * w.y + t.a.y * w.x;
                    },
-                   [&](const Term& t, double sx, double sy) { bin_put<T>(lds[t.j - (uint32_t)base], t, sx, sy); });
+                   [&](const Term& t, double sx, double sy) { lds[t.j - (uint32_t)base] = C2{(T)sy, (T)sx}; });   // swapped
     } else {
         tile_load(lds, E, [&](int e) { return x[goff(e)]; });
     }
@@ -540,12 +552,15 @@ __global__ __launch_bounds__(fold4_threads<B>()) __attribute__((
                     sy = -sy;
                 }
             };
-            auto put = [&](const Term& t, double sx, double sy) { bin_put<T>(lds_all[r][dft4_pad((int)t.j)], t, sx, sy); };
+            auto put = [&](const Term& t, double sx, double sy) {
+                lds_all[r][dft4_pad((int)t.j)] = C2{(T)sy, (T)sx};    // swapped parts
+            };
+            double cx = 0.0, cy = 0.0;
 #pragma unroll
             for (int i = 0; i < kTermBlocks; ++i) {
                 Term t = kept[i];
                 __asm__ volatile("" : "+v"(t.flags));              // or every step's run masks are kept across rows
-                term_add(t, term, put);
+                term_add(t, cx, cy, term, put);
             }
             if (more) {
                 TermShare rest = share;
@@ -553,7 +568,7 @@ __global__ __launch_bounds__(fold4_threads<B>()) __attribute__((
                 bool go = true;
                 for (int i0 = share.first + 64 * kTermBlocks; go; i0 += 64) {
                     go = rest.load(d, c, i0, t);
-                    term_add(t, term, put);
+                    term_add(t, cx, cy, term, put);
                 }
             }
         }

@@ -172,3 +172,27 @@ def test_fold_of_strengths_that_are_not_finite(q, n, b, S, precision):
         ev.launch()
         K.Dft(ev.rest, code).launch()
         assert torch.isnan(torch.view_as_real(it["x"])).all()
+
+
+@pytest.mark.parametrize("q,b", [(2, 6), (2, 13), (4, 3), (4, 4), (4, 5), (4, 6), (4, 7)])
+@pytest.mark.parametrize("S", [64, 65, 300, 1500, 5000])
+def test_fold_rounds_a_crowded_bin_once(q, b, S):
+    """Every support in one bin, FP32: a sample is the bin's sum turned by a power of w, exact for q = 2 and 4, so
+    each part of it is within half a unit of its last place of the sum of its terms (taken in FP64 here: 2^-53 of
+    the sizes of at most S terms each time one is added)."""
+    print(f"fold one bin q={q} b={b} S={S}", flush=True)
+    n, C, P = b + 5, 2, 3
+    Ms, Ds, loc, a = _inputs(q, n, b, S, C, P, S)
+    loc[:b] = loc[:b, :1]                                          # M picks the first b digits: one bin
+    for M in Ms:
+        M[:] = 0
+        M[:b] = np.eye(b, dtype=int)
+    a = a.astype(np.complex64).astype(np.complex128)
+    x = _run(q, n, b, Ms, Ds, loc, a, "fp32")
+    w = np.array([1, 1j, -1, -1j])[::4 // q]
+    lq = (np.arange(q ** b)[:, None] // q ** np.arange(b - 1, -1, -1)) % q
+    turn = w[(lq @ loc[:b, 0]) % q]
+    for c in range(C):
+        ref = (w[(Ds[c] @ loc) % q] @ a)[:, None] * turn[None, :]
+        for got, want in ((x[c].real, ref.real), (x[c].imag, ref.imag)):
+            assert (np.abs(got - want) <= 2.0 ** -24 * (1 + 1e-6) * np.abs(want) + S * 2.0 ** -53 * np.abs(a).sum()).all()
