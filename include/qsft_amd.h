@@ -228,6 +228,8 @@ typedef struct qsft_dft_desc {
     int32_t pass_ti[QSFT_DFT_MAX_PASSES];   /* contiguous inner elements per tile (divides I) */
     int32_t pass_blocks[QSFT_DFT_MAX_PASSES];
     int32_t pass_ta[QSFT_DFT_MAX_PASSES];   /* whole [M, I] blocks per tile (pass_ti = I only) */
+    int32_t order;          /* axes of a pass: 0 innermost first (qsft_dft_plan), 1 outermost  *
+                             * first (qsft_fold_rest)                                         */
 } qsft_dft_desc;
 
 /* Fills the pass fields: the schedule qsft_dft_autotune measured fastest for

@@ -49,7 +49,7 @@ class DftDesc(ctypes.Structure):
                 ("in_", vp), ("out", vp), ("n_pass", i32),
                 ("pass_d0", i32 * QSFT_DFT_MAX_PASSES), ("pass_d1", i32 * QSFT_DFT_MAX_PASSES),
                 ("pass_ti", i32 * QSFT_DFT_MAX_PASSES), ("pass_blocks", i32 * QSFT_DFT_MAX_PASSES),
-                ("pass_ta", i32 * QSFT_DFT_MAX_PASSES)]
+                ("pass_ta", i32 * QSFT_DFT_MAX_PASSES), ("order", i32)]
 
 
 class AssembleDesc(ctypes.Structure):

@@ -96,7 +96,7 @@ __global__ __launch_bounds__(TH) void k_dft_pass(const qsft_dft_desc* __restrict
     }
     __syncthreads();
 
-    C2* cur = tile_axes<T, QR>(lds, lds + E, E, q, mb, ti, tw);
+    C2* cur = tile_axes<T, QR>(lds, lds + E, E, q, mb, ti, tw, d.order != 0);
 
     const bool last = (pass == d.n_pass - 1);
     C2* __restrict__ out = reinterpret_cast<C2*>(d.out) + (int64_t)row * Q;
@@ -311,6 +311,7 @@ int apply_schedule(qsft_dft_desc* h, const Sched& sc) {
         h->pass_blocks[p] = (int)blocks;
     }
     h->n_pass = sc.np;
+    h->order = 0;
     for (int i = sc.np; i < QSFT_DFT_MAX_PASSES; ++i)
         h->pass_d0[i] = h->pass_d1[i] = h->pass_ti[i] = h->pass_ta[i] = h->pass_blocks[i] = 0;
     return QSFT_OK;

@@ -207,16 +207,16 @@ __device__ __forceinline__ void tile_store(const C2* lds, int E, F put) {
 }
 
 // The axis transforms of a tile of E elements, [.., q^mb, ti] with its mb axes
-// innermost first (axis t has stride q^(mb-1-t) ti in the tile), by the whole
-// workgroup, which has synchronised after filling `cur`. The generic radix is
-// out of place (`alt`, E more elements). Returns the buffer that holds the
-// result; the workgroup is synchronised.
+// innermost first, or outermost first (axis t has stride q^(mb-1-t) ti in the
+// tile), by the whole workgroup, which has synchronised after filling `cur`.
+// The generic radix is out of place (`alt`, E more elements). Returns the
+// buffer that holds the result; the workgroup is synchronised.
 template <typename T, int QR>
 __device__ __forceinline__ cplx_t<T>* tile_axes(cplx_t<T>* cur, cplx_t<T>* alt, int E, int q, int mb, int ti,
-                                                const cplx_t<T>* tw) {
+                                                const cplx_t<T>* tw, bool outermost_first = false) {
     const int pencils = E / q;
-    int G = ti;
-    for (int t = mb - 1; t >= 0; --t) {
+    for (int t = 0; t < mb; ++t) {
+        const int G = ti * ipow(q, outermost_first ? mb - 1 - t : t);
         const FastDiv fd((uint32_t)G);
         for (int pc = threadIdx.x; pc < pencils; pc += blockDim.x) {
             const int X = (int)fd.div((uint32_t)pc);
@@ -233,7 +233,6 @@ __device__ __forceinline__ cplx_t<T>* tile_axes(cplx_t<T>* cur, cplx_t<T>* alt, 
             cur = alt;
             alt = tmp;
         }
-        G *= q;
     }
     return cur;
 }

@@ -444,11 +444,13 @@ __global__ __launch_bounds__(TH) void k_fold_pass(const SRC src, int pass, int l
     __syncthreads();
     C2* cur = tile_axes<T, QR>(lds, lds + E, E, q, mb, ti, tw);
     if (d.fwd && pass == d.n_pass - 1) {
-        // the tile now holds samples: back along the same axes, scaled by q^-b as
-        // k_dft_pass scales it if these are all (else its last pass does that)
+        // the tile now holds samples: back along the same axes, the outermost first
+        // as over all passes (the order of the axes, and with it the bits, do not
+        // follow from how they are grouped), scaled by q^-b as k_dft_pass scales
+        // it if these are all (else its last pass does that)
         for (int e = threadIdx.x; e < E; e += blockDim.x) cur[e] = C2{cur[e].y, cur[e].x};
         __syncthreads();
-        cur = tile_axes<T, QR>(cur, cur == lds ? lds + E : lds, E, q, mb, ti, tw);
+        cur = tile_axes<T, QR>(cur, cur == lds ? lds + E : lds, E, q, mb, ti, tw, true);
         if (FIRST) tile_store(cur, E, [&](int e, C2 v) { x[goff(e)] = dft_scaled<T>(v, Q); });
         else tile_store(cur, E, [&](int e, C2 v) { x[goff(e)] = v; });
     } else if (pass == d.n_pass - 1) {
@@ -742,7 +744,8 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
 }
 
 // The forward passes a fwd descriptor's launches leave: those over the axes of
-// every pass but the last, in place on x (n_pass 0: none).
+// every pass but the last, in place on x and from the outermost group inwards
+// (n_pass 0: none).
 extern "C" int qsft_fold_rest(const qsft_fold_desc* h, qsft_dft_desc* out) {
     if (!h || !out || !h->fwd || h->n_pass < 1) {
         qsft_set_error("qsft_fold_rest: a descriptor bound with transform is needed");
@@ -757,12 +760,14 @@ extern "C" int qsft_fold_rest(const qsft_fold_desc* h, qsft_dft_desc* out) {
     r.in = h->x;
     r.out = h->x;
     r.n_pass = h->n_pass - 1;
+    r.order = 1;
     for (int p = 0; p < r.n_pass; ++p) {
-        r.pass_d0[p] = h->pass_d0[p];
-        r.pass_d1[p] = h->pass_d1[p];
-        r.pass_ti[p] = h->pass_ti[p];
-        r.pass_ta[p] = h->pass_ta[p];
-        r.pass_blocks[p] = h->pass_blocks[p];
+        const int f = r.n_pass - 1 - p;
+        r.pass_d0[p] = h->pass_d0[f];
+        r.pass_d1[p] = h->pass_d1[f];
+        r.pass_ti[p] = h->pass_ti[f];
+        r.pass_ta[p] = h->pass_ta[f];
+        r.pass_blocks[p] = h->pass_blocks[f];
     }
     *out = r;
     return QSFT_OK;

@@ -6,6 +6,8 @@ inverse transform has at most b q-point stages, so FP64 is within 1e-12 and
 FP32, with b log2(q) <= 16 rounded additions of partial sums no larger than
 sum |a_s|, within 2e-6 of the largest sample.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -196,3 +198,65 @@ def test_fold_rounds_a_crowded_bin_once(q, b, S):
         ref = (w[(Ds[c] @ loc) % q] @ a)[:, None] * turn[None, :]
         for got, want in ((x[c].real, ref.real), (x[c].imag, ref.imag)):
             assert (np.abs(got - want) <= 2.0 ** -24 * (1 + 1e-6) * np.abs(want) + S * 2.0 ** -53 * np.abs(a).sum()).all()
+
+
+def _scheduled(it, precision, transform, s):
+    """EvalFold of one instance (and the passes left to Dft) on the schedule of the DftDesc s."""
+    code, dev = (L.QSFT_F32 if precision == "fp32" else L.QSFT_F64), dv.current_device()
+    q, b, C, P, S = (it[k] for k in ("q", "b", "C", "P", "S"))
+    nbytes = L.lib.qsft_fold_workspace_bytes(q, b, C, P, S, 0)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    d = L.FoldDesc()
+    L.check(L.lib.qsft_fold_bind(ctypes.byref(d), q, it["n"], b, C, P, S, it["Mt"].shape[-1], 0, code, L.QSFT_F64,
+                                 int(transform), C * P, *(it[k].data_ptr() for k in ("Mt", "D", "K", "a", "x")),
+                                 ws.data_ptr(), nbytes))
+    assert d.rpw == 0                                              # a shape of the tile kernel
+    d.n_pass = s.n_pass
+    for p in range(s.n_pass):
+        d.pass_d0[p], d.pass_d1[p], d.pass_ti[p], d.pass_ta[p] = s.pass_d0[p], s.pass_d1[p], s.pass_ti[p], s.pass_ta[p]
+        d.pass_blocks[p] = s.pass_blocks[p]
+        d.pass_lds[p] = L.lib.qsft_dft_lds_bytes(ctypes.byref(s), p, code)
+        assert 0 < d.pass_lds[p] <= 65536
+    d.tile_bins = q ** (b - s.pass_d0[0]) * s.pass_ta[0]
+    d.tiles = q ** b // d.tile_bins
+    pb, rb = ctypes.c_int(), ctypes.c_int()
+    assert L.lib.qsft_fold_blocks(ctypes.byref(d), ctypes.byref(pb), ctypes.byref(rb)) == 0
+    blocks = [[pb.value], [rb.value]] + [[d.pass_blocks[p]] for p in range(d.n_pass)]
+    buf, dptr, pres, tots = K.pack([d], blocks, dev)
+    st = K.stream_handle()
+    L.check(L.lib.qsft_fold_prep(dptr, pres[0], pres[1], 1, tots[0], tots[1], st))
+    for p in range(d.n_pass):
+        L.check(L.lib.qsft_fold_rows(dptr, pres[2 + p], 1, tots[2 + p], p, code | (q << 8), d.pass_lds[p], st))
+    if transform and d.n_pass > 1:
+        r = L.DftDesc()
+        L.check(L.lib.qsft_fold_rest(ctypes.byref(d), ctypes.byref(r)))
+        K.Dft([dict(q=q, b=b, rows=r.rows, inp=it["x"], out=it["x"], desc=r)], code).launch()
+    torch.cuda.synchronize()                                       # buf and ws are released
+
+
+@pytest.mark.parametrize("transform", [False, True])
+@pytest.mark.parametrize("q,b,precision", [(20, 4, "fp32"), (20, 3, "fp32"), (20, 3, "fp64"), (2, 16, "fp32"),
+                                           (3, 10, "fp64"), (4, 8, "fp32"), (5, 6, "fp64"), (7, 5, "fp32"),
+                                           (11, 3, "fp64")])
+def test_fold_gives_the_same_bits_on_every_schedule(q, b, precision, transform):
+    """Samples and sub-transforms do not depend on how the axes are grouped into passes."""
+    print(f"fold schedules q={q} b={b} {precision} transform={transform}", flush=True)
+    code = L.QSFT_F32 if precision == "fp32" else L.QSFT_F64
+    x = _inputs(q, 20, b, 150, 1, 3, seed=q + b)
+    first, groups = None, set()
+    for cand in range(400):
+        s = L.DftDesc(q=q, b=b, rows=3, in_stride=1, in_row_stride=q ** b)
+        if L.lib.qsft_dft_plan_candidate(ctypes.byref(s), code, cand) != L.QSFT_OK:
+            break
+        split = tuple(s.pass_d0[p] for p in range(s.n_pass))
+        if split in groups or s.n_pass > 1 and len(groups) >= 8:
+            continue
+        if L.lib.qsft_dft_lds_bytes(ctypes.byref(s), 0, code) > 65536:
+            continue
+        groups.add(split)
+        it = _item(q, 20, b, *x, precision)
+        _scheduled(it, precision, transform, s)
+        bits = torch.view_as_real(it["x"])
+        first = bits if first is None else first
+        assert torch.equal(bits, first), split
+    assert len(groups) >= 2
