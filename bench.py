@@ -323,7 +323,6 @@ def k2_stages(E, torch, quiet):
     specs = [E.random_spec(20, 16, 2000, 3, 3, 2, 20.0, rng=rng) for _ in range(16)]
     from qsft_amd import kernels as K
     from qsft_amd import _lib as L
-    K.dft_autotune(20, 3, L.QSFT_F32, specs[0].C * specs[0].P)
     bt = E.Batch(specs, precision="fp32")
     bt.launch(seed_offset=1)
     bt.results()

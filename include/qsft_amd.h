@@ -164,6 +164,8 @@ size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, int shared_d
 int qsft_fold_bind(qsft_fold_desc* host_desc, int q, int n, int b, int C, int P, int S, int n_pad, int shared_d,
                    int precision, int a_precision, int transform, int launch_rows, const int8_t* Mt, const int8_t* D,
                    const int8_t* K, const void* a, void* x, void* ws, size_t ws_bytes);
+/* 1: a row is one pass, whatever was autotuned for its shape. */
+int qsft_fold_whole_rows(int q, int b, int precision);
 int qsft_fold_blocks(const qsft_fold_desc* host_desc, int* phase_blocks, int* rank_blocks);
 /* Instances of any shape share a prep launch. */
 int qsft_fold_prep(const qsft_fold_desc* dev_descs, const int32_t* dev_pre_phase, const int32_t* dev_pre_rank,
@@ -238,22 +240,22 @@ typedef struct qsft_dft_desc {
  * and inner-run lengths). Every schedule applies the same axis transforms in
  * the same order (innermost axis first), so results do not depend on it. */
 int qsft_dft_plan(qsft_dft_desc* host_desc, int precision);
-/* The same, but one pass over whole rows where a row of several passes fits 144 KiB of LDS. */
+/* The same, but where nothing was measured one pass over whole rows if they fit 144 KiB of LDS. */
 int qsft_dft_plan_rows(qsft_dft_desc* host_desc, int precision);
-/* The planner's candidate `index` (0 = the model's best, in the order the
- * autotuner tries them); QSFT_ERR_ARG past the last. */
+/* The planner's candidate `index`, in the order the autotuner tries them (whole
+ * rows if they fit 144 KiB of LDS, then the model's ranking); QSFT_ERR_ARG past the last. */
 int qsft_dft_plan_candidate(qsft_dft_desc* host_desc, int precision, int index);
-/* Autotuner: times the model's best-ranked schedules (at most max_candidates)
+/* Autotuner: times the best-ranked schedules (at most max_candidates)
  * on `rows` rows held in `buf` (rows * q^b elements + 4096 bytes, device
  * memory, overwritten) on `stream`, synchronously, and records the fastest
- * for qsft_dft_plan; *best_ms = its time for the rows. Call once per shape
+ * for qsft_dft_plan and qsft_dft_plan_rows; *best_ms = its time for the rows. Call once per shape
  * before the launches that should use it (not under graph capture). */
 int qsft_dft_autotune(int q, int b, int precision, int rows, void* buf, size_t buf_bytes, int max_candidates,
                       void* stream, float* best_ms);
-/* The schedule qsft_dft_plan returns for (q, b, precision): pass count, axis
+/* The schedule qsft_dft_plan_rows returns for (q, b, precision): pass count, axis
  * groups [d0, d1), TI and TA per pass (arrays of 4); *tuned = 1 if measured. */
 int qsft_dft_schedule(int q, int b, int precision, int* n_pass, int* d0, int* d1, int* ti, int* ta, int* tuned);
-/* Dynamic LDS bytes one instance's pass needs (tile + twiddles; <= 64 KiB for a qsft_dft_plan schedule). */
+/* Dynamic LDS bytes one instance's pass needs (tile + twiddles; > 64 KiB for whole rows only). */
 int qsft_dft_lds_bytes(const qsft_dft_desc* host_desc, int pass, int precision);
 /* lds_bytes: dynamic LDS of the launch, at least qsft_dft_lds_bytes() of every
  * instance's pass; smaller tiles leave more workgroups resident per CU. */

@@ -118,6 +118,7 @@ SIGNATURES = {
     "qsft_eval_mfma": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),
     "qsft_fold_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 6),
     "qsft_fold_bind": (ctypes.c_int, [ctypes.POINTER(FoldDesc)] + [ctypes.c_int] * 12 + [vp] * 6 + [ctypes.c_size_t]),
+    "qsft_fold_whole_rows": (ctypes.c_int, [ctypes.c_int] * 3),
     "qsft_fold_rest": (ctypes.c_int, [ctypes.POINTER(FoldDesc), ctypes.POINTER(DftDesc)]),
     "qsft_fold_blocks": (ctypes.c_int, [ctypes.POINTER(FoldDesc), ctypes.POINTER(ctypes.c_int),
                                         ctypes.POINTER(ctypes.c_int)]),

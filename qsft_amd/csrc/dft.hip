@@ -22,9 +22,10 @@
 // direct sum over a twiddle table (out of place through a second tile).
 //
 // Schedules (passes, axis groups, TI, TA, LDS budget) are enumerated by the
-// host planner and ranked by a bandwidth/occupancy model; qsft_dft_autotune
-// times the best-ranked candidates on the device for one (q, b, precision)
-// and records the fastest, which qsft_dft_plan then returns.
+// host planner and ranked by a bandwidth/occupancy model, one pass over whole
+// rows of up to 144 KiB before all others; qsft_dft_autotune times the
+// best-ranked candidates on the device for one (q, b, precision) and records
+// the fastest, which every plan of that shape then returns.
 //
 // HBM traffic per pass is one read and one write of the rows: 16 B per
 // complex FP32 sample (8 in + 8 out), 32 B in FP64.
@@ -283,12 +284,38 @@ std::vector<Sched> candidates(int q, int b, int prec) {
     return out;
 }
 
-bool schedule_for(int q, int b, int prec, Sched* sc, bool* tuned) {
+// One pass over whole rows, if a row fits the LDS that a workgroup may take.
+bool whole_rows(int q, int b, int prec, Sched* sc) {
+    const long long elem = prec == QSFT_F32 ? 8 : 16, Q = ipow_ll(q, b);
+    if ((radix_compiled(q) ? Q * elem : (2 * Q + q) * elem) > kRowLdsBytes) return false;
+    *sc = Sched{};
+    sc->np = 1;
+    sc->d1[0] = b;
+    sc->ti[0] = sc->ta[0] = 1;
+    return true;
+}
+
+// The schedules that are tried and counted by index: whole rows first where
+// they fit, which the model, made for tiles of at most 64 KiB, does not rank,
+// then the model's order.
+std::vector<Sched> ranked(int q, int b, int prec) {
+    std::vector<Sched> c = candidates(q, b, prec);
+    Sched w;
+    if (whole_rows(q, b, prec, &w)) {
+        c.erase(std::remove_if(c.begin(), c.end(), [&](const Sched& s) { return s.np == 1; }), c.end());
+        c.insert(c.begin(), w);
+    }
+    return c;
+}
+
+// rows: whole rows where they fit and nothing was measured
+bool schedule_for(int q, int b, int prec, bool rows, Sched* sc, bool* tuned) {
     const int key = sched_key(q, b, prec);
     std::lock_guard<std::mutex> g(g_sched_lock);
     auto it = g_tuned.find(key);
     if (it != g_tuned.end()) { *sc = it->second; *tuned = true; return true; }
     *tuned = false;
+    if (rows && whole_rows(q, b, prec, sc)) return true;
     auto im = g_model.find(key);
     if (im != g_model.end()) { *sc = im->second; return true; }
     const std::vector<Sched> c = candidates(q, b, prec);
@@ -319,9 +346,7 @@ int apply_schedule(qsft_dft_desc* h, const Sched& sc) {
 
 }  // namespace
 
-// The schedule of a (q, b, precision): the autotuned one when
-// qsft_dft_autotune has measured it in this process, else the model's best.
-extern "C" int qsft_dft_plan(qsft_dft_desc* h, int precision) {
+static int plan_dft(qsft_dft_desc* h, int precision, bool rows) {
     if (!h || h->q < 2 || h->q > QSFT_MAX_Q || h->b < 1 || h->b > QSFT_MAX_B || h->rows < 0 ||
         h->in_stride < 1 || (precision != QSFT_F32 && precision != QSFT_F64)) {
         qsft_set_error("qsft_dft_plan: bad descriptor");
@@ -329,37 +354,33 @@ extern "C" int qsft_dft_plan(qsft_dft_desc* h, int precision) {
     }
     Sched sc;
     bool tuned = false;
-    if (!schedule_for(h->q, h->b, precision, &sc, &tuned)) {
+    if (!schedule_for(h->q, h->b, precision, rows, &sc, &tuned)) {
         qsft_set_error("qsft_dft_plan: no schedule fits the LDS (q too large)");
         return QSFT_ERR_ARG;
     }
     return apply_schedule(h, sc);
 }
 
-// One pass over whole rows where the planned schedule takes several and a row
-// fits the LDS of a CU. The planner's own schedules stay within 64 KiB.
-extern "C" int qsft_dft_plan_rows(qsft_dft_desc* h, int precision) {
-    const int rc = qsft_dft_plan(h, precision);
-    if (rc != QSFT_OK || h->n_pass == 1) return rc;
-    const long long elem = precision == QSFT_F32 ? 8 : 16, Q = ipow_ll(h->q, h->b);
-    const long long bytes = radix_compiled(h->q) ? Q * elem : (2 * Q + h->q) * elem;
-    if (bytes > kRowLdsBytes) return rc;
-    Sched sc;
-    sc.np = 1;
-    sc.d1[0] = h->b;
-    sc.ti[0] = sc.ta[0] = 1;
-    return apply_schedule(h, sc);
-}
+// The schedule of a (q, b, precision): the autotuned one when
+// qsft_dft_autotune has measured it in this process, else the model's best,
+// which stays within 64 KiB of LDS.
+extern "C" int qsft_dft_plan(qsft_dft_desc* h, int precision) { return plan_dft(h, precision, false); }
 
-// The planner's candidate number `index` (0 = the model's best; the order
-// qsft_dft_autotune tries them in); QSFT_ERR_ARG past the last one.
+// The same, but where nothing was measured one pass over whole rows if they fit
+// the LDS of a CU: q = 20, b = 3 in FP64, 29 us in the model's two passes and
+// 17 as whole rows.
+extern "C" int qsft_dft_plan_rows(qsft_dft_desc* h, int precision) { return plan_dft(h, precision, true); }
+
+// The planner's candidate number `index` (the order qsft_dft_autotune tries
+// them in: whole rows if they fit, then the model's best and on);
+// QSFT_ERR_ARG past the last one.
 extern "C" int qsft_dft_plan_candidate(qsft_dft_desc* h, int precision, int index) {
     if (!h || h->q < 2 || h->q > QSFT_MAX_Q || h->b < 1 || h->b > QSFT_MAX_B || h->rows < 0 ||
         h->in_stride < 1 || (precision != QSFT_F32 && precision != QSFT_F64) || index < 0) {
         qsft_set_error("qsft_dft_plan_candidate: bad arguments");
         return QSFT_ERR_ARG;
     }
-    const std::vector<Sched> c = candidates(h->q, h->b, precision);
+    const std::vector<Sched> c = ranked(h->q, h->b, precision);
     if (index >= (int)c.size()) {
         qsft_set_error("qsft_dft_plan_candidate: no such candidate");
         return QSFT_ERR_ARG;
@@ -428,10 +449,10 @@ extern "C" int qsft_dft_pass(const qsft_dft_desc* d, const int32_t* pre, int n_i
     return qsft_hip_status(e, "qsft_dft_pass");
 }
 
-// Times the model's best-ranked schedules (at most `max_candidates`) on
+// Times the best-ranked schedules (at most `max_candidates`) on
 // `rows` rows of q^b samples held in `buf` (transformed in place, contents
 // irrelevant; the last 4 KiB hold the descriptor and block prefixes), one
-// warm-up and three timed runs each, and records the fastest for qsft_dft_plan.
+// warm-up and three timed runs each, and records the fastest for later plans.
 extern "C" int qsft_dft_autotune(int q, int b, int precision, int rows, void* buf, size_t buf_bytes,
                                  int max_candidates, void* stream, float* best_ms) {
     if (q < 2 || q > QSFT_MAX_Q || b < 1 || b > QSFT_MAX_B || rows < 1 || !buf || max_candidates < 1 ||
@@ -446,7 +467,7 @@ extern "C" int qsft_dft_autotune(int q, int b, int precision, int rows, void* bu
         qsft_set_error("qsft_dft_autotune: buffer smaller than rows * q^b elements + 4096 bytes");
         return QSFT_ERR_ARG;
     }
-    const std::vector<Sched> cand = candidates(q, b, precision);
+    const std::vector<Sched> cand = ranked(q, b, precision);
     if (cand.empty()) { qsft_set_error("qsft_dft_autotune: no schedule fits"); return QSFT_ERR_ARG; }
     hipStream_t st = (hipStream_t)stream;
     char* dev_desc = static_cast<char*>(buf) + data;
@@ -504,7 +525,7 @@ extern "C" int qsft_dft_autotune(int q, int b, int precision, int rows, void* bu
     return QSFT_OK;
 }
 
-// The schedule qsft_dft_plan uses for (q, b, precision): passes, axis groups,
+// The schedule qsft_dft_plan_rows uses for (q, b, precision): passes, axis groups,
 // TI and TA per pass; *tuned = 1 when it was measured by qsft_dft_autotune.
 extern "C" int qsft_dft_schedule(int q, int b, int precision, int* n_pass, int* d0, int* d1, int* ti, int* ta,
                                  int* tuned) {
@@ -515,7 +536,7 @@ extern "C" int qsft_dft_schedule(int q, int b, int precision, int* n_pass, int* 
     }
     Sched sc;
     bool t = false;
-    if (!schedule_for(q, b, precision, &sc, &t)) { qsft_set_error("qsft_dft_schedule: no schedule fits"); return QSFT_ERR_ARG; }
+    if (!schedule_for(q, b, precision, true, &sc, &t)) { qsft_set_error("qsft_dft_schedule: no schedule fits"); return QSFT_ERR_ARG; }
     *n_pass = sc.np;
     for (int p = 0; p < QSFT_DFT_MAX_PASSES; ++p) {
         d0[p] = sc.d0[p]; d1[p] = sc.d1[p]; ti[p] = sc.ti[p]; ta[p] = sc.ta[p];

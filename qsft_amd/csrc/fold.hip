@@ -673,6 +673,12 @@ extern "C" size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, i
            al256((size_t)C * S * 8) + al256((size_t)C * S * 4) + al256(((size_t)S + 1) * 4) + al256((size_t)C * (ipow(q, b) / std::min(q, 32) + 2) * 4);
 }
 
+extern "C" int qsft_fold_whole_rows(int q, int b, int precision) {
+    if (!fold_shape_ok(q, 1, b, 1, 1, 0, 64) || (precision != QSFT_F32 && precision != QSFT_F64)) return 0;
+    const long long elem = precision == QSFT_F32 ? 8 : 16, Q = ipow(q, b);
+    return fold_rows4(q, b, precision) || (radix_compiled(q) ? Q * elem : (2 * Q + q) * elem) <= kRowLdsBytes;
+}
+
 extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int P, int S, int n_pad, int shared_d,
                               int precision, int a_precision, int transform, int launch_rows, const int8_t* Mt,
                               const int8_t* D, const int8_t* K, const void* a, void* x, void* ws, size_t ws_bytes) {
@@ -717,10 +723,15 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
         d.tiles = 1;
         d.tile_bins = Q;
     } else {
-        // whole rows where they fit the LDS, else the sub-DFT planner's schedule, innermost first
+        // whole rows where they fit the LDS, else the sub-DFT planner's schedule,
+        // measured or modelled, innermost first. A measured forward transform says
+        // nothing about whole rows here: one pass writes a row once, where two
+        // write it, read it and write it again, and two more follow for a
+        // sub-transform.
         qsft_dft_desc s{};
         s.q = q; s.b = b; s.rows = C * P; s.in_stride = 1; s.in_row_stride = Q;
-        const int rc = qsft_dft_plan_rows(&s, precision);
+        const int rc = qsft_fold_whole_rows(q, b, precision) ? qsft_dft_plan_candidate(&s, precision, 0)
+                                                              : qsft_dft_plan(&s, precision);
         if (rc != QSFT_OK) return rc;
         d.n_pass = s.n_pass;
         for (int p = 0; p < s.n_pass; ++p) {

@@ -377,7 +377,7 @@ class Dft:
 
     def __init__(self, items, precision, rows4=True, candidate=None):
         """candidate: use the planner's schedule number `candidate` for the
-        pass kernels instead of the tuned / model-best one."""
+        pass kernels instead of the tuned, whole-row or (rows4 off) model-best one."""
         groups = defaultdict(list)
         fast = defaultdict(list)
         for it in items:
@@ -456,7 +456,7 @@ def dft_autotune(q, b, precision, rows, max_candidates=6, device=None):
 
 
 def dft_schedule(q, b, precision):
-    """(passes [(d0, d1, ti, ta)], tuned) the planner uses for (q, b, precision)."""
+    """(passes [(d0, d1, ti, ta)], tuned) that Dft uses for (q, b, precision)."""
     n = ctypes.c_int()
     arrs = [(ctypes.c_int * 4)() for _ in range(4)]
     tuned = ctypes.c_int()

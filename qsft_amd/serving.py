@@ -299,11 +299,12 @@ class Server:
     def tune(self, specs, max_candidates=6):
         """Autotune the sub-DFT schedule of every (q, b) among `specs` not
         tuned yet (FP32, C * P rows of the first request of each shape), before
-        serving them: tuning times kernels synchronously."""
+        serving them: tuning times kernels synchronously. Shapes whose rows the
+        evaluation transforms whole have no schedule to choose."""
         from . import kernels as K
         seen = {}
         for sp in specs:
-            if not (sp.q == 4 and sp.b in (4, 6)):                # those use the whole-row kernel
+            if not lib.qsft_fold_whole_rows(sp.q, sp.b, L.QSFT_F32):
                 seen.setdefault((sp.q, sp.b), sp.C * sp.P)
         for (q, b), rows in seen.items():
             K.dft_autotune(q, b, L.QSFT_F32, rows, max_candidates=max_candidates, device=self.device)

@@ -116,3 +116,29 @@ def test_batch_runtime_sizes_on_the_host():
                                     sigma=0.0, amax=1.0, seed=0))              # noiseless detection needs R = 1
     assert not L.lib.qsft_batch_create(ctypes.cast(bad, ctypes.c_void_p), 1, 15, 3, ctypes.byref(sz))
     assert b"bad request shape" in L.lib.qsft_last_error()
+
+
+@pytest.mark.parametrize("q,b,prec,whole", [(20, 3, L.QSFT_F64, 1), (4, 7, L.QSFT_F32, 1), (5, 6, L.QSFT_F32, 1),
+                                            (7, 4, L.QSFT_F32, 1), (3, 5, L.QSFT_F64, 1), (20, 4, L.QSFT_F32, 0),
+                                            (7, 5, L.QSFT_F32, 0), (2, 15, L.QSFT_F32, 0)])
+def test_the_reported_schedule_is_the_one_that_runs(q, b, prec, whole):
+    """Nothing measured: the schedule of qsft_dft_plan_rows, the autotuner's first candidate where a row fits 144 KiB
+    of LDS."""
+    d, c = (L.DftDesc(q=q, b=b, rows=3, in_stride=1, in_row_stride=q ** b) for _ in range(2))
+    L.check(L.lib.qsft_dft_plan_rows(ctypes.byref(d), prec))
+    L.check(L.lib.qsft_dft_plan_candidate(ctypes.byref(c), prec, 0))
+    n, tuned = ctypes.c_int(), ctypes.c_int()
+    arrs = [(ctypes.c_int * 4)() for _ in range(4)]
+    L.check(L.lib.qsft_dft_schedule(q, b, prec, ctypes.byref(n), *arrs, ctypes.byref(tuned)))
+    assert not tuned.value and n.value == d.n_pass == c.n_pass and (n.value == 1) == bool(whole)
+    for a, x, y in zip(arrs, (d.pass_d0, d.pass_d1, d.pass_ti, d.pass_ta), (c.pass_d0, c.pass_d1, c.pass_ti, c.pass_ta)):
+        assert list(a) == list(x) == list(y)
+    assert L.lib.qsft_fold_whole_rows(q, b, prec) == whole
+    assert L.lib.qsft_dft_lds_bytes(ctypes.byref(d), 0, prec) <= (147456 if whole else 65536)
+    # one whole-row candidate, all others within 64 KiB
+    i = 1
+    while L.lib.qsft_dft_plan_candidate(ctypes.byref(c), prec, i) == L.QSFT_OK:
+        assert c.n_pass > (1 if whole else 0)
+        assert all(0 < L.lib.qsft_dft_lds_bytes(ctypes.byref(c), p, prec) <= 65536 for p in range(c.n_pass))
+        i += 1
+    assert i > 1

@@ -388,3 +388,32 @@ def test_assemble_philox_layout_independent(R, p1, Q):
     K.assemble([dict(args, U=Ur, bin_major=False)])
     K.assemble([dict(args, U=Ub, bin_major=True)])
     assert torch.equal(Ub.transpose(1, 2), Ur)
+
+
+@pytest.mark.parametrize("q,b,precision", [(20, 3, "fp64"), (4, 7, "fp32"), (3, 9, "fp64"), (7, 4, "fp64"),
+                                           (2, 15, "fp32")])
+def test_dft_runs_the_schedule_that_was_measured(q, b, precision):
+    """Whole rows of up to 144 KiB are tried with the others, and what was measured fastest is what later plans return
+    and the schedule query reports."""
+    print(f"dft tuned q={q} b={b} {precision}", flush=True)
+    code = dv.PRECISIONS[precision][0]
+    for cands in (1, 6):
+        K._tuned.pop((q, b, code), None)
+        K.dft_autotune(q, b, code, 4, max_candidates=cands)
+        sched, tuned = K.dft_schedule(q, b, code)
+        assert tuned
+        tried = []
+        for cand in range(cands):
+            d = L.DftDesc(q=q, b=b, rows=4, in_stride=1, in_row_stride=q ** b)
+            if L.lib.qsft_dft_plan_candidate(ctypes.byref(d), code, cand) == L.QSFT_OK:
+                tried.append([(d.pass_d0[p], d.pass_d1[p], d.pass_ti[p], d.pass_ta[p]) for p in range(d.n_pass)])
+        assert sched in tried
+        for plan in (L.lib.qsft_dft_plan, L.lib.qsft_dft_plan_rows):
+            d = L.DftDesc(q=q, b=b, rows=4, in_stride=1, in_row_stride=q ** b)
+            L.check(plan(ctypes.byref(d), code))
+            assert [(d.pass_d0[p], d.pass_d1[p], d.pass_ti[p], d.pass_ta[p]) for p in range(d.n_pass)] == sched
+    x = np.random.default_rng(b).normal(size=(4, q ** b)) + 0j
+    xt = torch.from_numpy(x).to(dv.PRECISIONS[precision][1]).to(dv.current_device())
+    y = torch.empty_like(xt)
+    K.Dft([dict(q=q, b=b, rows=4, inp=xt, out=y)], code, rows4=False, candidate=1).launch()
+    assert torch.equal(torch.view_as_real(dv.subtransform(xt, q, b, precision=precision)), torch.view_as_real(y))

@@ -8,7 +8,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
+    from qsft_amd import _lib as L
     from qsft_amd import engine as E
+    from qsft_amd import kernels as K
     from qsft_amd import serving as SV
 
 
@@ -224,3 +226,13 @@ def test_k3_256_uneven_instances_in_one_batch():
         planted += sp.S
     print(f"noiseless K3 copies: {found} of {planted} keys", flush=True)
     assert found >= 0.95 * planted
+
+
+def test_tune_leaves_shapes_with_whole_rows_alone():
+    """The evaluation transforms whole rows of up to 144 KiB itself: there is nothing to measure for them."""
+    print("tune whole rows", flush=True)
+    rng = np.random.default_rng(8)
+    specs = [E.random_spec(5, 12, 20, 5, 1, 1, 20.0, rng=rng), E.random_spec(4, 12, 20, 5, 1, 1, 20.0, rng=rng),
+             E.random_spec(3, 12, 20, 10, 1, 1, 20.0, rng=rng)]
+    SV.Server(hbm_budget=1 << 40).tune(specs)
+    assert [K.dft_schedule(sp.q, sp.b, L.QSFT_F32)[1] for sp in specs] == [False, False, True]
