@@ -730,9 +730,15 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
         // sub-transform.
         qsft_dft_desc s{};
         s.q = q; s.b = b; s.rows = C * P; s.in_stride = 1; s.in_row_stride = Q;
-        const int rc = qsft_fold_whole_rows(q, b, precision) ? qsft_dft_plan_candidate(&s, precision, 0)
-                                                              : qsft_dft_plan(&s, precision);
-        if (rc != QSFT_OK) return rc;
+        if (qsft_fold_whole_rows(q, b, precision)) {
+            s.n_pass = 1;
+            s.pass_d1[0] = b;
+            s.pass_ti[0] = s.pass_ta[0] = 1;
+            s.pass_blocks[0] = C * P;
+        } else {
+            const int rc = qsft_dft_plan(&s, precision);
+            if (rc != QSFT_OK) return rc;
+        }
         d.n_pass = s.n_pass;
         for (int p = 0; p < s.n_pass; ++p) {
             d.pass_d0[p] = s.pass_d0[p];
