@@ -406,14 +406,16 @@ typedef struct qsft_peel_desc {
 
 /* counter layout (uint32 words); per iteration i at 8 i + :
  *   0 singletons, 1 multitons, 2 distinct balls, 3 active flag,
- *   4 bins scanned in pass i */
+ *   4 bins scanned in pass i
+ * LOG, ITERS, PEELED and LIVE are those of the passes that have ended; words
+ * without a name are the kernels' own. */
 #define QSFT_CTR_ITER_STRIDE 8
 #define QSFT_CTR_LOG 128        /* records appended                                    */
-#define QSFT_CTR_LIVE 129       /* hash slots claimed (keys); LOG and LIVE are one aligned 64-bit word */
+#define QSFT_CTR_OUT 129        /* outputs written                                     */
 #define QSFT_CTR_ERROR 130      /* QSFT_DEVERR_* bits                                  */
 #define QSFT_CTR_ITERS 131      /* iterations that ran                                 */
 #define QSFT_CTR_PEELED 132     /* balls peeled (saturating)                           */
-#define QSFT_CTR_OUT 133        /* outputs written                                     */
+#define QSFT_CTR_LIVE 133       /* hash slots claimed (keys)                           */
 #define QSFT_CTR_WORDS 136
 
 size_t qsft_peel_workspace_bytes(int q, int n, int b, int C, int P, int max_iter, int out_cap);

@@ -26,7 +26,7 @@ QSFT_DFT_MAX_PASSES = 4
 QSFT_PEEL_SHARED_D, QSFT_PEEL_UNIT_D, QSFT_PEEL_UNIT_D_NEG, QSFT_PEEL_SPARSE_U = 1, 2, 4, 8
 QSFT_PEEL_ONE_BIN_WAVES = 16
 QSFT_CTR_ITER_STRIDE = 8
-QSFT_CTR_LOG, QSFT_CTR_OUT, QSFT_CTR_ERROR, QSFT_CTR_ITERS, QSFT_CTR_PEELED, QSFT_CTR_LIVE = 128, 133, 130, 131, 132, 129
+QSFT_CTR_LOG, QSFT_CTR_OUT, QSFT_CTR_ERROR, QSFT_CTR_ITERS, QSFT_CTR_PEELED, QSFT_CTR_LIVE = 128, 129, 130, 131, 132, 133
 QSFT_FIN_FLUSH = 1
 QSFT_CTR_WORDS = 136
 

@@ -61,6 +61,11 @@ constexpr int kSlotThreads = 256;
 constexpr int kSplitFirst = 2;
 constexpr int kSplitLater = 4;
 constexpr uint32_t kNil = 0xFFFFFFFFu;
+// Records appended and, in the next word, hash slots claimed so far: one aligned
+// 64-bit word, so that one atomic takes both. loop_control copies them to
+// QSFT_CTR_LOG and QSFT_CTR_LIVE after each pass.
+constexpr int kCtrTaken = 134;
+static_assert(kCtrTaken % 2 == 0 && kCtrTaken > QSFT_CTR_LIVE && kCtrTaken + 2 <= QSFT_CTR_WORDS, "two words of their own");
 constexpr int kHeldMulti = 1 << 30;   // mark bit: multiton when last scanned, no ball queued on it since
 
 // The per-bin kernels' partition. A batch's block prefix counts blocks of
@@ -902,8 +907,8 @@ __device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int
     uint32_t rbase = 0, lbase = 0;
     if (lane == 0) {
         if (nb_mask) atomicAdd(&ctr[it * QSFT_CTR_ITER_STRIDE + 2], (uint32_t)__popcll(nb_mask));
-        if (ok_mask) rbase = atomicAdd(&ctr[QSFT_CTR_LOG], (uint32_t)__popcll(ok_mask));
-        if (cl_mask) lbase = atomicAdd(&ctr[QSFT_CTR_LIVE], (uint32_t)__popcll(cl_mask));
+        if (ok_mask) rbase = atomicAdd(&ctr[kCtrTaken], (uint32_t)__popcll(ok_mask));
+        if (cl_mask) lbase = atomicAdd(&ctr[kCtrTaken + 1], (uint32_t)__popcll(cl_mask));
     }
     rbase = __shfl(rbase, 0);
     lbase = __shfl(lbase, 0);
@@ -988,13 +993,12 @@ __device__ __forceinline__ void write_records(const qsft_peel_desc& d, int it, c
     }
 }
 
-// records << 0 | claimed slots << 32 added to the adjacent LOG and LIVE words
-// in one atomic (neither word overflows into the other: both count at most the
-// records); the counts before.
+// records << 0 | claimed slots << 32 added to the words at kCtrTaken in one
+// atomic (neither overflows into the other: both count at most the records);
+// the counts before.
 __device__ __forceinline__ uint64_t take_records(uint32_t* ctr, uint32_t records, uint32_t slots) {
-    static_assert(QSFT_CTR_LOG % 2 == 0 && QSFT_CTR_LIVE == QSFT_CTR_LOG + 1, "one 64-bit word");
     if (records == 0 && slots == 0) return 0;
-    return atomicAdd((unsigned long long*)&ctr[QSFT_CTR_LOG], (unsigned long long)records | ((unsigned long long)slots << 32));
+    return atomicAdd((unsigned long long*)&ctr[kCtrTaken], (unsigned long long)records | ((unsigned long long)slots << 32));
 }
 
 // The pass counters of a block: singletons and multitons (adjacent words, one
@@ -1722,7 +1726,7 @@ __device__ __forceinline__ void apply_singleton(const qsft_peel_desc& d, int t, 
 // pass, whose kernel A subtracts it from the column it owns.
 
 // Loop control after pass `it` (one thread; its detection counters are final):
-// the iteration and peel counts, and whether pass it + 1 runs: only if this
+// the iteration, peel, record and slot counts, and whether pass it + 1 runs: only if this
 // pass ran and found a singleton and a multiton, below the peel cap.
 template <bool PERSIST>
 __device__ __forceinline__ void loop_control(const qsft_peel_desc& d, int it, uint32_t active) {
@@ -1735,6 +1739,8 @@ __device__ __forceinline__ void loop_control(const qsft_peel_desc& d, int it, ui
     const uint32_t nm = rd(it * QSFT_CTR_ITER_STRIDE + 1);
     const uint32_t nb = rd(it * QSFT_CTR_ITER_STRIDE + 2);
     uint32_t peeled = rd(QSFT_CTR_PEELED);
+    ctr[QSFT_CTR_LOG] = rd(kCtrTaken);
+    ctr[QSFT_CTR_LIVE] = rd(kCtrTaken + 1);
     if (active) {
         ctr[QSFT_CTR_ITERS] = (uint32_t)(it + 1);
         peeled = (peeled + nb < peeled) ? 0xFFFFFFFFu : peeled + nb;

@@ -142,3 +142,10 @@ def test_the_reported_schedule_is_the_one_that_runs(q, b, prec, whole):
         assert all(0 < L.lib.qsft_dft_lds_bytes(ctypes.byref(c), p, prec) <= 65536 for p in range(c.n_pass))
         i += 1
     assert i > 1
+
+
+def test_counter_words_are_where_this_abi_version_has_them():
+    text = open(os.path.join(ROOT, "include", "qsft_amd.h")).read()
+    words = {k: int(v) for k, v in re.findall(r"#define QSFT_CTR_(\w+) (\d+)", text)}
+    assert words == dict(ITER_STRIDE=8, LOG=128, OUT=129, ERROR=130, ITERS=131, PEELED=132, LIVE=133, WORDS=136)
+    assert all(getattr(L, "QSFT_CTR_" + k) == v for k, v in words.items())

@@ -7,6 +7,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
+    from qsft_amd import _lib as L
     from qsft_amd import engine as E
     from qsft_amd import kernels as K
 
@@ -428,3 +429,20 @@ def test_output_table_is_ranked_by_first_detection(S, count):
         truth = {tuple(c): a for c, a in zip(sp.locq.T, sp.strengths)}
         assert {tuple(r) for r in k} == set(truth)
         assert max(abs(x - truth[tuple(r)]) for r, x in zip(k, v)) < 1e-4
+
+
+@pytest.mark.parametrize("q,n,S,b,R,method,snr", [(4, 50, 1000, 6, 2, "nso", 10.0), (3, 90, 60, 4, 2, "nso", 20.0),
+                                                  (4, 10, 100, 4, 1, "identity", None)])
+@pytest.mark.parametrize("count", [1, 9])
+def test_counters_of_a_finished_loop(q, n, S, b, R, method, snr, count):
+    """One record per singleton, one slot per key, one output per slot."""
+    print(f"counters q={q} n={n} S={S} b={b} count={count}", flush=True)
+    rng = np.random.default_rng(S)
+    bt = E.Batch([E.random_spec(q, n, S, b, 3, R, snr, rng=rng, method=method) for _ in range(count)])
+    bt.launch(seed_offset=1)
+    for i, (k, _, _, info) in enumerate(bt.results(with_info=True)):
+        d, ws = bt.peel.descs[i], bt.peel.ws[i]
+        at = d.ctr - ws.data_ptr()
+        ctr = ws[at:at + 4 * L.QSFT_CTR_WORDS].view(torch.int32).cpu().numpy()
+        assert ctr[L.QSFT_CTR_OUT] == ctr[L.QSFT_CTR_LIVE] == len(k) > 0
+        assert ctr[L.QSFT_CTR_LOG] == info["records"] == sum(s for s, _, _ in info["trace"]) >= len(k)
