@@ -138,8 +138,8 @@ typedef struct qsft_fold_desc {
     int32_t pass_ta[QSFT_DFT_MAX_PASSES], pass_blocks[QSFT_DFT_MAX_PASSES], pass_lds[QSFT_DFT_MAX_PASSES];
     int32_t tiles;          /* tiles of the first pass per row, tile_bins consecutive bins each */
     int32_t tile_bins;
-    int32_t rpw;            /* whole-row kernel (q = 4, b = 4..6, FP32 also 7): row sets of *
-                             * one group per workgroup; 0: the tile kernel                  */
+    int32_t rpw;            /* whole-row kernel (q = 4, b = 4..6, FP32 also 7; few terms):  *
+                             * row sets of one group per workgroup; 0: the tile kernel      */
     int32_t fwd;            /* 1: the last pass transforms its samples back along its axes  *
                              * (all of them where n_pass = 1: x receives sub-transforms);   *
                              * qsft_fold_rest gives the passes that remain                  */

@@ -650,6 +650,18 @@ size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 // rows that k_fold4_rows takes: q = 4, b = 4..6, and in FP32 b = 7 (139 KiB of LDS)
 bool fold_rows4(int q, int b, int precision) { return q == 4 && b >= 4 && b <= (precision == QSFT_F32 ? 7 : 6); }
 
+// Whether the whole-row kernel takes an instance of such rows. Its workgroups of
+// b = 4 and 5 fold their four rows one after the other with one wave and with
+// four, which pays only while the terms are few: the tile kernel (a workgroup
+// a row) takes more. The line depends on the instance alone, so that a request
+// has the same bits in every batch. Rows of 64 instances of C = 3, P = 62,
+// FP32, as sub-transforms, whole-row / tile kernel: b = 4, S = 200 49 / 68 us,
+// S = 400 99 / 75, S = 5000 1820 / 307; b = 5, S = 1000 91 / 124, S = 2000
+// 189 / 167, S = 5000 531 / 304; one such instance, S = 5000: 331 / 30 and 90 / 28.
+bool fold_rows4_takes(int q, int b, int S, int precision) {
+    return fold_rows4(q, b, precision) && S <= (b == 4 ? 256 : b == 5 ? 1600 : 0x7FFFFFFF);
+}
+
 bool fold_shape_ok(int q, int n, int b, int C, int P, int S, int n_pad) {
     if (q < 2 || q > QSFT_MAX_Q || b < 1 || b > QSFT_MAX_B || n < 1 || n > n_pad || n_pad % 64 || n_pad > QSFT_MAX_N ||
         C < 1 || P < 1 || S < 0)
@@ -709,7 +721,7 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
     w += al256(((size_t)S + 1) * 4);
     d.start = reinterpret_cast<int32_t*>(w);
     const int Q = ipow(q, b);
-    if (fold_rows4(q, b, precision)) {
+    if (fold_rows4_takes(q, b, S, precision)) {
         // rows of a group per workgroup: one where the launch has fewer rows than
         // the chip holds (256 CUs x 4 workgroups), up to four where it has many
         d.rpw = launch_rows >= 8192 ? 4 : launch_rows >= 4096 ? 2 : 1;
@@ -908,9 +920,10 @@ extern "C" int qsft_fold_one(int q, int n, int b, int C, int P, int S, int n_pad
         return QSFT_ERR_ARG;
     }
     hipStream_t st = (hipStream_t)stream;
+    const int rows4 = src.d.rpw ? b : 0;
     rc = launch_prep(src, pb, rb, st);
     for (int p = 0; rc == QSFT_OK && p < src.d.n_pass; ++p)
-        rc = precision == QSFT_F32 ? launch_rows<float>(q, b, src.d.fwd, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st)
-                                   : launch_rows<double>(q, b, src.d.fwd, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st);
+        rc = precision == QSFT_F32 ? launch_rows<float>(q, rows4, src.d.fwd, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st)
+                                   : launch_rows<double>(q, rows4, src.d.fwd, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st);
     return rc;
 }

@@ -149,3 +149,18 @@ def test_counter_words_are_where_this_abi_version_has_them():
     words = {k: int(v) for k, v in re.findall(r"#define QSFT_CTR_(\w+) (\d+)", text)}
     assert words == dict(ITER_STRIDE=8, LOG=128, OUT=129, ERROR=130, ITERS=131, PEELED=132, LIVE=133, WORDS=136)
     assert all(getattr(L, "QSFT_CTR_" + k) == v for k, v in words.items())
+
+
+@pytest.mark.parametrize("b,S,rows4", [(4, 0, 1), (4, 256, 1), (4, 257, 0), (4, 100000, 0), (5, 1600, 1), (5, 1601, 0),
+                                       (6, 100000, 1), (3, 10, 0)])
+def test_fold_plan_of_many_terms_leaves_the_one_wave_row_kernel(b, S, rows4):
+    for prec in (L.QSFT_F32, L.QSFT_F64):
+        for transform in (0, 1):
+            for launch_rows in (10, 100000):
+                d, nbytes = L.FoldDesc(), L.lib.qsft_fold_workspace_bytes(4, b, 2, 5, S, 0)
+                at = 1 << 20                                       # (never read here)
+                L.check(L.lib.qsft_fold_bind(ctypes.byref(d), 4, 30, b, 2, 5, S, 64, 0, prec, L.QSFT_F64, transform,
+                                             launch_rows, at, at, at, at, at, at, nbytes))
+                assert (d.rpw > 0) == bool(rows4) and d.n_pass == 1
+                if not rows4:
+                    assert (d.tiles, d.tile_bins, d.pass_blocks[0], d.pass_ta[0]) == (1, 4 ** b, 10, 1)

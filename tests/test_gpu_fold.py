@@ -260,3 +260,27 @@ def test_fold_gives_the_same_bits_on_every_schedule(q, b, precision, transform):
         first = bits if first is None else first
         assert torch.equal(bits, first), split
     assert len(groups) >= 2
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 2e-6)])
+@pytest.mark.parametrize("b,S", [(4, 256), (4, 257), (4, 3000), (5, 1600), (5, 1601), (5, 4097)])
+def test_fold_on_both_sides_of_the_line_between_its_row_kernels(b, S, precision, tol):
+    """q = 4: samples and sub-transforms where the whole-row kernel ends and the tile kernel begins, the two beside
+    each other in one launch, each with the bits it has alone (bounds as above)."""
+    print(f"fold line b={b} S={S} {precision}", flush=True)
+    code = L.QSFT_F32 if precision == "fp32" else L.QSFT_F64
+    x = _inputs(4, 21, b, S, 2, 7, seed=S)
+    few = _inputs(4, 21, b, 50, 2, 7, seed=S)
+    ref = _direct(4, b, *x)
+    for transform in (False, True):
+        items = [_item(4, 21, b, *v, precision) for v in (few, x, few)]
+        K.EvalFold(items, code, transform=transform).launch()
+        bound, want = tol * np.max(np.abs(ref)), ref
+        if transform:
+            want = np.fft.fftn(ref.reshape(2, 7, *[4] * b), axes=range(2, 2 + b)).reshape(2, 7, -1) / 4 ** b
+            bound *= 12 / 4 ** (b / 2)
+        assert np.max(np.abs(items[1]["x"].cpu().numpy() - want)) <= bound
+        for it, v in zip(items, (few, x, few)):
+            alone = _item(4, 21, b, *v, precision)
+            K.EvalFold([alone], code, transform=transform).launch()
+            assert torch.equal(torch.view_as_real(alone["x"]), torch.view_as_real(it["x"]))
