@@ -133,21 +133,53 @@ __device__ __forceinline__ void pencil(cplx_t<T>* v, int st, const cplx_t<T>* tw
     }
 }
 
-// Generic q (not compiled for a fixed radix): out-of-place through a second
-// LDS buffer.
-template <typename T>
-__device__ __forceinline__ void pencil_generic_out(const cplx_t<T>* src, cplx_t<T>* dst, int st, int q,
-                                                   const cplx_t<T>* tw) {
-    for (int k = 0; k < q; ++k) {
-        cplx_t<T> acc = src[0];
-        for (int r = 1; r < q; ++r) {
-            const cplx_t<T> w = tw[(r * k) % q];
-            const cplx_t<T> x = src[r * st];
-            acc.x += x.x * w.x - x.y * w.y;
-            acc.y += x.x * w.y + x.y * w.x;
+// Generic q (not compiled for a fixed radix): one axis (stride G) of a tile of
+// E elements, out of place through a second LDS buffer, N outputs of q terms
+// per thread: a pencil per thread left a workgroup three quarters idle behind
+// q^2 terms one after the other (33 rows of q = 64, b = 2, the samples of S =
+// 10: 690 us a call in FP32, now 42; 710 in FP64, now 62). Bound by its LDS
+// reads, a term and a root of unity for every product: four outputs share their
+// terms where the axis has enough of them (FP64, q = 64: 70 us with one).
+template <typename T, int N>
+__device__ __forceinline__ void axis_generic_by(const cplx_t<T>* src, cplx_t<T>* dst, int E, int q, int G,
+                                                const cplx_t<T>* tw) {
+    const int nk = (q + N - 1) / N;                                // a thread's outputs are nk apart
+    const FastDiv fg((uint32_t)G), fk((uint32_t)nk);
+    const int items = E / q * nk;
+    for (int i = threadIdx.x; i < items; i += blockDim.x) {
+        const int a = (int)fg.div((uint32_t)i), X = (int)fk.div((uint32_t)a), k = a - X * nk;
+        const int p0 = X * q * G + (i - a * G);
+        const cplx_t<T>* v = src + p0;
+        cplx_t<T> acc[N];
+        int rk[N], kn[N];                                          // r k mod q
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            kn[n] = k + n * nk < q ? k + n * nk : 0;               // (past the last output: not stored)
+            rk[n] = 0;
+            acc[n] = v[0];
         }
-        dst[k * st] = acc;
+#pragma unroll(N > 1 ? 2 : 4)
+        for (int r = 1; r < q; ++r) {
+            const cplx_t<T> x = v[r * G];
+#pragma unroll
+            for (int n = 0; n < N; ++n) {
+                rk[n] += kn[n];
+                if (rk[n] >= q) rk[n] -= q;
+                const cplx_t<T> w = tw[rk[n]];
+                acc[n].x += x.x * w.x - x.y * w.y;
+                acc[n].y += x.x * w.y + x.y * w.x;
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+            if (k + n * nk < q) dst[p0 + (k + n * nk) * G] = acc[n];
     }
+}
+template <typename T>
+__device__ __forceinline__ void axis_generic(const cplx_t<T>* src, cplx_t<T>* dst, int E, int q, int G,
+                                             const cplx_t<T>* tw) {
+    if (q >= 16) axis_generic_by<T, 4>(src, dst, E, q, G, tw);
+    else axis_generic_by<T, 1>(src, dst, E, q, G, tw);
 }
 
 __host__ __device__ __forceinline__ bool radix_compiled(int q) {
@@ -217,22 +249,19 @@ __device__ __forceinline__ cplx_t<T>* tile_axes(cplx_t<T>* cur, cplx_t<T>* alt, 
     const int pencils = E / q;
     for (int t = 0; t < mb; ++t) {
         const int G = ti * ipow(q, outermost_first ? mb - 1 - t : t);
-        const FastDiv fd((uint32_t)G);
-        for (int pc = threadIdx.x; pc < pencils; pc += blockDim.x) {
-            const int X = (int)fd.div((uint32_t)pc);
-            const int p0 = X * q * G + (pc - X * G);
-            if constexpr (QR > 0) {
-                pencil<T, QR>(cur + p0, G, tw);
-            } else {
-                pencil_generic_out<T>(cur + p0, alt + p0, G, q, tw);
+        if constexpr (QR > 0) {
+            const FastDiv fd((uint32_t)G);
+            for (int pc = threadIdx.x; pc < pencils; pc += blockDim.x) {
+                const int X = (int)fd.div((uint32_t)pc);
+                pencil<T, QR>(cur + X * q * G + (pc - X * G), G, tw);
             }
-        }
-        __syncthreads();
-        if constexpr (QR == 0) {
+        } else {
+            axis_generic<T>(cur, alt, E, q, G, tw);
             cplx_t<T>* tmp = cur;
             cur = alt;
             alt = tmp;
         }
+        __syncthreads();
     }
     return cur;
 }

@@ -417,3 +417,19 @@ def test_dft_runs_the_schedule_that_was_measured(q, b, precision):
     y = torch.empty_like(xt)
     K.Dft([dict(q=q, b=b, rows=4, inp=xt, out=y)], code, rows4=False, candidate=1).launch()
     assert torch.equal(torch.view_as_real(dv.subtransform(xt, q, b, precision=precision)), torch.view_as_real(y))
+
+
+@pytest.mark.parametrize("q,b", [(6, 3), (15, 2), (16, 1), (16, 2), (17, 2), (18, 2), (19, 2), (33, 2), (62, 1), (63, 2),
+                                 (64, 2)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_dft_generic_radix(q, b, precision):
+    """One and (q >= 16) four outputs of an axis per thread, with axes that four do not divide. A sum of q products
+    in FP32 is off by at most about 2 q 2^-24 of the sizes summed, in FP64 2 q 2^-53."""
+    print(f"dft generic q={q} b={b} {precision}", flush=True)
+    rng = np.random.default_rng(q)
+    x = rng.normal(size=(5, q ** b)) + 1j * rng.normal(size=(5, q ** b))
+    xt = torch.from_numpy(x).to(dv.PRECISIONS[precision][1]).to(dv.current_device())
+    got = dv.subtransform(xt, q, b, precision=precision).cpu().numpy()
+    ref = np.stack([O.gwht(r, q, b) for r in x])
+    eps = 2.0 ** -53 if precision == "fp64" else 2.0 ** -24
+    assert np.max(np.abs(got - ref)) <= 4 * q * b * eps * np.max(np.abs(x))
