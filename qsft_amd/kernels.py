@@ -221,7 +221,7 @@ class EvalFold:
     """
 
     def __init__(self, items, precision, transform=False):
-        self.ws = []
+        self.ws, self.copies = [], []
         launch_rows = sum(it["C"] * it["P"] for it in items)
         descs, phase, rank = [], [], []
         for it in items:
@@ -233,9 +233,10 @@ class EvalFold:
             ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=it["x"].device)
             self.ws.append(ws)
             d = L.FoldDesc()
-            # 16-byte loads: a view that starts elsewhere is copied
-            t = {k: it[k] if it[k].data_ptr() % 16 == 0 else it[k].clone() for k in ("Mt", "D", "K", "a")}
+            # 16-byte loads: a view that starts elsewhere is copied, by each launch, which reads what it holds then
+            t = {k: it[k] if it[k].data_ptr() % 16 == 0 else torch.empty_like(it[k]) for k in ("Mt", "D", "K", "a")}
             self.ws.append(t)
+            self.copies += [(t[k], it[k]) for k in t if t[k] is not it[k]]
             if lib.qsft_fold_bind(ctypes.byref(d), q, n, b, C, P, S, it["Mt"].shape[-1], shared, precision,
                                   L.QSFT_F32 if it["a"].dtype == torch.complex64 else L.QSFT_F64, int(transform),
                                   launch_rows, _ptr(t["Mt"]), _ptr(t["D"]), _ptr(t["K"]), _ptr(t["a"]), _ptr(it["x"]), _ptr(ws),
@@ -281,6 +282,8 @@ class EvalFold:
     def launch_split(self, between):
         """The prep launches (phases, bins, ranks), then `between()`, then the row passes."""
         st = stream_handle()
+        for to, view in self.copies:
+            to.copy_(view)
         pp, pr, tp, tr = self.prep
         L.check(lib.qsft_fold_prep(_vp(self.dptr), _vp(pp), _vp(pr), self.n, tp, tr, st), "qsft_fold_prep")
         between()

@@ -284,3 +284,31 @@ def test_fold_on_both_sides_of_the_line_between_its_row_kernels(b, S, precision,
             alone = _item(4, 21, b, *v, precision)
             K.EvalFold([alone], code, transform=transform).launch()
             assert torch.equal(torch.view_as_real(alone["x"]), torch.view_as_real(it["x"]))
+
+
+def _unaligned(t):
+    """The same values in a view that starts one element into its storage."""
+    v = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    return v.copy_(t)
+
+
+@pytest.mark.parametrize("q,b", [(4, 4), (3, 3)])
+def test_fold_reads_views_that_start_anywhere_at_every_launch(q, b):
+    """Mt, D, K and complex64 a that are not 16-byte aligned, changed between the launches of one EvalFold."""
+    print(f"fold unaligned views q={q} b={b}", flush=True)
+    first, second = (_item(q, 13, b, *_inputs(q, 13, b, 37, 2, 5, seed=s), "fp32") for s in (1, 2))
+    want = []
+    for it in (first, second):
+        it["a"] = it["a"].to(torch.complex64)
+        K.EvalFold([it], L.QSFT_F32).launch()
+        want.append(it["x"].clone())
+        x = dv.evaluate_cosets(q, 13, b, *(_unaligned(it[k]) for k in ("Mt", "D", "K", "a")), "fp32")
+        assert torch.equal(torch.view_as_real(x), torch.view_as_real(want[-1]))
+    views = dict(first, **{k: _unaligned(first[k]) for k in ("Mt", "D", "K", "a")})
+    assert all(views[k].data_ptr() % 16 for k in ("Mt", "D", "K", "a"))
+    ev = K.EvalFold([views], L.QSFT_F32)
+    for it, x in zip((first, second, first), (want[0], want[1], want[0])):
+        for k in ("Mt", "D", "K", "a"):
+            views[k].copy_(it[k])
+        ev.launch()
+        assert torch.equal(torch.view_as_real(views["x"]), torch.view_as_real(x))
