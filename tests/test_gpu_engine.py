@@ -446,3 +446,23 @@ def test_counters_of_a_finished_loop(q, n, S, b, R, method, snr, count):
         ctr = ws[at:at + 4 * L.QSFT_CTR_WORDS].view(torch.int32).cpu().numpy()
         assert ctr[L.QSFT_CTR_OUT] == ctr[L.QSFT_CTR_LIVE] == len(k) > 0
         assert ctr[L.QSFT_CTR_LOG] == info["records"] == sum(s for s, _, _ in info["trace"]) >= len(k)
+
+
+@pytest.mark.parametrize("mode,precision", [("direct", "fp64"), ("direct", "fp32"), ("mfma", "fp32")])
+def test_every_evaluator_recovers_the_same_spectrum(mode, precision):
+    """The other evaluators through the whole engine: the support and the coefficients of the folded samples to the
+    precision of the samples (1e-14 and 2e-6 of the largest sample, at most the sum of 200 strengths in [1, 10], either
+    way)."""
+    print(f"engine {mode} {precision}", flush=True)
+    rng = np.random.default_rng(21)
+    specs = [E.random_spec(4, 30, 200, 5, 3, 1, None, rng=rng, method="identity"),
+             E.random_spec(20, 12, 60, 2, 3, 1, None, rng=rng, method="identity"),
+             E.random_spec(3, 16, 80, 4, 2, 1, None, rng=rng, method="identity")]
+    out = []
+    for m in (mode, "fold"):
+        bt = E.Batch(specs, precision=precision, eval_mode=m)
+        bt.launch(seed_offset=1)
+        out.append([(k, v) for k, v, _, _ in bt.results()])
+    for a, b in zip(*out):
+        assert len(a[0]) > 0
+        _same(a, b, rtol=2000 * 2 * (1e-14 if precision == "fp64" else 2e-6))

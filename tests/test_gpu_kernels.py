@@ -433,3 +433,38 @@ def test_dft_generic_radix(q, b, precision):
     ref = np.stack([O.gwht(r, q, b) for r in x])
     eps = 2.0 ** -53 if precision == "fp64" else 2.0 ** -24
     assert np.max(np.abs(got - ref)) <= 4 * q * b * eps * np.max(np.abs(x))
+
+
+@pytest.mark.parametrize("q,b,bb,precision", [(4, 8, 7, "fp32"), (20, 4, 3, "fp64"), (2, 15, 14, "fp32"), (3, 9, 8, "fp64"),
+                                              (7, 5, 4, "fp64")])
+def test_dft_strided_whole_rows(q, b, bb, precision):
+    """all_bs: whole rows of 64 to 144 KiB of LDS from every q-th sample, with the bits of contiguous rows."""
+    print(f"dft strided whole rows q={q} b={b} {precision}", flush=True)
+    g = torch.Generator().manual_seed(q)
+    x = torch.view_as_complex(torch.randn((3, q ** b, 2), dtype=torch.float64, generator=g))
+    x = x.to(dv.PRECISIONS[precision][1]).to(dv.current_device())
+    got = dv.subtransform(x, q, bb, in_stride=q ** (b - bb), precision=precision)
+    assert torch.equal(torch.view_as_real(got),
+                       torch.view_as_real(dv.subtransform(x[:, ::q ** (b - bb)].contiguous(), q, bb, precision=precision)))
+    ref = np.stack([O.gwht(r[::q ** (b - bb)], q, bb) for r in x.cpu().numpy().astype(np.complex128)])
+    assert rel_err(got.cpu().numpy(), ref) < (1e-13 if precision == "fp64" else 3e-6)
+
+
+@pytest.mark.parametrize("q,n,b,S,C,R", CASES)
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_eval_direct_sums_match_oracle(q, n, b, S, C, R, precision):
+    """The sums over every support at every query (eval_cosets), with the oracle's bounds of the folded samples."""
+    print(f"direct sums q={q} n={n} b={b} S={S} C={C} R={R} {precision}", flush=True)
+    Ms, D, locq, a = _setup(q, n, b, S, C, R, seed=q * 1000 + n)
+    dev, n_pad = dv.current_device(), dv.n_pad_of(n)
+    code, dt = dv.PRECISIONS[precision]
+    x = torch.empty((C, D.shape[0], q ** b), dtype=dt, device=dev)
+    K.eval_cosets([dict(q=q, n=n, b=b, C=C, P=D.shape[0], S=S, Mt=dv.Mt_tensor(Ms, b, n_pad, dev),
+                        D=dv.D_tensor([D] * C, n_pad, dev), K=dv.digits_tensor(locq.T, n_pad, dev),
+                        a=dv.strengths_tensor(a, precision, dev), x=x)], code)
+    x = x.cpu().numpy()
+    tol = max(1e-12, 4e-16 * 2 * np.pi * n * (q - 1) ** 2 / q) if precision == "fp64" else 2e-6
+    for c in range(C):
+        for p in [0, D.shape[0] // 2, D.shape[0] - 1]:
+            ref = O.eval_synthetic(O.coset_digits(Ms[c], D[p:p + 1], q, b)[0], locq, a, q)
+            assert rel_err(x[c, p], ref) < tol, (c, p)
