@@ -155,9 +155,14 @@ typedef struct qsft_fold_desc {
     uint32_t* J;            /* [C][S] bins                                                  */
     uint32_t* bad;          /* [1 + S] strengths that are not finite: their number, then s  */
     int32_t* start;         /* [C][tiles + 1] first sorted position of each tile            */
+    uint32_t* chunk;        /* QSFT_FOLD_CHUNKS and many supports: [C][S] bins sorted within *
+                             * chunks, [C][S] ranks there; else null                        */
 } qsft_fold_desc;
 
 size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, int shared_d);
+/* Added to `transform` by a caller that runs qsft_fold_chunks: instances of many
+ * supports (more than 8192) are then ranked in two steps, with the same results. */
+#define QSFT_FOLD_CHUNKS 2
 /* Fills a host descriptor (schedule: whole rows where they fit the LDS, else the
  * sub-DFT planner's passes). precision: of x; transform: sub-transforms instead of
  * samples, the passes of qsft_fold_rest included; launch_rows: rows (C * P) of all instances of the launch; ws 256-byte aligned. */
@@ -170,6 +175,10 @@ int qsft_fold_blocks(const qsft_fold_desc* host_desc, int* phase_blocks, int* ra
 /* Instances of any shape share a prep launch. */
 int qsft_fold_prep(const qsft_fold_desc* dev_descs, const int32_t* dev_pre_phase, const int32_t* dev_pre_rank,
                    int n_inst, int phase_blocks, int rank_blocks, void* stream);
+/* Between the phases of a prep launch (rank_blocks 0) and its ranks (phase_blocks
+ * 0), if any instance has chunks. */
+int qsft_fold_chunks(const qsft_fold_desc* dev_descs, const int32_t* dev_pre_rank, int n_inst, int rank_blocks,
+                     void* stream);
 /* Row pass `pass` (dev_pre counts pass_blocks). word: low nibble QSFT_F32 / QSFT_F64, bits 8..15 = q, bits
  * 16..23 = b of a whole-row launch (descriptors with rpw > 0, all of one b; 0: the tile kernel, any b);
  * bit 24: the descriptors' fwd (whole-row launches). All instances of a launch share q.

@@ -28,6 +28,7 @@ QSFT_PEEL_ONE_BIN_WAVES = 16
 QSFT_CTR_ITER_STRIDE = 8
 QSFT_CTR_LOG, QSFT_CTR_OUT, QSFT_CTR_ERROR, QSFT_CTR_ITERS, QSFT_CTR_PEELED, QSFT_CTR_LIVE = 128, 129, 130, 131, 132, 133
 QSFT_FIN_FLUSH = 1
+QSFT_FOLD_CHUNKS = 2
 QSFT_CTR_WORDS = 136
 
 i32, i64, u64, f64, vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_uint64, ctypes.c_double, ctypes.c_void_p
@@ -88,7 +89,7 @@ class FoldDesc(ctypes.Structure):
                 ("pass_ti", i32 * 4), ("pass_ta", i32 * 4), ("pass_blocks", i32 * 4), ("pass_lds", i32 * 4),
                 ("tiles", i32), ("tile_bins", i32), ("rpw", i32), ("fwd", i32),
                 ("Mt", vp), ("D", vp), ("K", vp), ("a", vp), ("x", vp),
-                ("E", vp), ("as_", vp), ("key", vp), ("J", vp), ("bad", vp), ("start", vp)]
+                ("E", vp), ("as_", vp), ("key", vp), ("J", vp), ("bad", vp), ("start", vp), ("chunk", vp)]
 
 
 class Request(ctypes.Structure):
@@ -123,6 +124,7 @@ SIGNATURES = {
     "qsft_fold_blocks": (ctypes.c_int, [ctypes.POINTER(FoldDesc), ctypes.POINTER(ctypes.c_int),
                                         ctypes.POINTER(ctypes.c_int)]),
     "qsft_fold_prep": (ctypes.c_int, [vp, vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]),
+    "qsft_fold_chunks": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int, vp]),
     "qsft_fold_rows": (ctypes.c_int, [vp, vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                       vp]),
     "qsft_fold_one": (ctypes.c_int, [ctypes.c_int] * 10 + [vp] * 6 + [ctypes.c_size_t, vp]),

@@ -136,6 +136,7 @@ struct Batch {
     bool bound = false, launched = false;
     size_t fold_desc = 0, fold_pre_phase = 0, fold_pre_rank = 0;
     int fold_phase = 0, fold_rank = 0;
+    bool fold_chunks = false;              // a request of so many supports that they are ranked in two steps
     std::vector<FoldLaunch> fold;
     std::vector<DftLaunch> dft;
     size_t asm_desc = 0, asm_pre = 0;
@@ -223,14 +224,16 @@ int build_plan(Batch& B, bool write) {
         for (int i = 0; i < nreq; ++i) all_rows += (long long)B.req[i].C * B.lay[i].P;
         const int launch_rows = (int)(all_rows < 0x7FFFFFFF ? all_rows : 0x7FFFFFFF);
         B.rest.assign(nreq, qsft_dft_desc{});
+        B.fold_chunks = false;
         for (int i = 0; i < nreq; ++i) {
             const qsft_request& r = B.req[i];
             const ReqLayout& l = B.lay[i];
             const int rc = qsft_fold_bind(&descs[i], r.q, r.n, r.b, r.C, l.P, r.S, l.n_pad, 1, QSFT_F32, QSFT_F64,
-                                          1, launch_rows, (const int8_t*)in_ptr(i, l.mt), (const int8_t*)in_ptr(i, l.d),
+                                          1 | QSFT_FOLD_CHUNKS, launch_rows, (const int8_t*)in_ptr(i, l.mt), (const int8_t*)in_ptr(i, l.d),
                                           (const int8_t*)work_ptr(i, l.k), in_ptr(i, l.a), work_ptr(i, l.x),
                                           work_ptr(i, l.fw), l.fw_bytes);
             if (rc != QSFT_OK) return rc;
+            B.fold_chunks |= descs[i].chunk != nullptr;
             const int rr = qsft_fold_rest(&descs[i], &B.rest[i]);
             if (rr != QSFT_OK) return rr;
             if (qsft_fold_blocks(&descs[i], &phase[i], &rank[i]) != 0) {
@@ -601,8 +604,14 @@ int enqueue(Batch* B, int upload, const void* input_host, uint64_t seed_offset, 
         if (e != hipSuccess) return qsft_hip_status(e, "qsft_batch_launch(stage)");
     }
     const qsft_fold_desc* fd = (const qsft_fold_desc*)(P + B->fold_desc);
-    rc = qsft_fold_prep(fd, (const int32_t*)(P + B->fold_pre_phase), (const int32_t*)(P + B->fold_pre_rank),
-                        (int)B->req.size(), B->fold_phase, B->fold_rank, st);
+    const int32_t* fpp = (const int32_t*)(P + B->fold_pre_phase);
+    const int32_t* fpr = (const int32_t*)(P + B->fold_pre_rank);
+    const int nreq = (int)B->req.size();
+    rc = qsft_fold_prep(fd, fpp, fpr, nreq, B->fold_phase, B->fold_chunks ? 0 : B->fold_rank, st);
+    if (rc == QSFT_OK && B->fold_chunks) {
+        rc = qsft_fold_chunks(fd, fpr, nreq, B->fold_rank, st);
+        if (rc == QSFT_OK) rc = qsft_fold_prep(fd, fpp, fpr, nreq, 0, B->fold_rank, st);
+    }
     if (rc != QSFT_OK) return rc;
     for (const FoldLaunch& L : B->fold) {
         rc = qsft_fold_rows(fd, (const int32_t*)(P + L.pre), (int)B->req.size(), L.blocks, L.pass, L.word, L.lds, st);

@@ -143,6 +143,7 @@ __device__ __forceinline__ void pencil(cplx_t<T>* v, int st, const cplx_t<T>* tw
 template <typename T, int N>
 __device__ __forceinline__ void axis_generic_by(const cplx_t<T>* src, cplx_t<T>* dst, int E, int q, int G,
                                                 const cplx_t<T>* tw) {
+    constexpr int kUnroll = N > 1 ? 2 : 4;
     const int nk = (q + N - 1) / N;                                // a thread's outputs are nk apart
     const FastDiv fg((uint32_t)G), fk((uint32_t)nk);
     const int items = E / q * nk;
@@ -158,7 +159,7 @@ __device__ __forceinline__ void axis_generic_by(const cplx_t<T>* src, cplx_t<T>*
             rk[n] = 0;
             acc[n] = v[0];
         }
-#pragma unroll(N > 1 ? 2 : 4)
+#pragma unroll kUnroll
         for (int r = 1; r < q; ++r) {
             const cplx_t<T> x = v[r * G];
 #pragma unroll

@@ -20,7 +20,8 @@
 //     counted against LDS tiles of the bins: the terms of a bin are adjacent
 //     and always summed in ascending s, so the sums have the same bits on
 //     every run. Also the first sorted position of every tile of the row
-//     kernel.
+//     kernel. Many supports are ranked in two steps: within chunks of 2048
+//     (k_fold_chunk), then by a binary search in every other chunk.
 //   * k_fold_pass / k_fold4_rows: a workgroup clears a tile of bins of one row
 //     in LDS, adds the tile's terms and runs the
 //     inverse transform over the tile's axes; k_fold4_rows (q = 4, b = 4
@@ -48,8 +49,17 @@ constexpr int kPhaseThreads = 256;   // four waves, 16 supports each
 constexpr int kPhaseTiles = 4;       // 16-row tiles of [D; M] per workgroup
 constexpr int kRankThreads = 1024;
 constexpr int kRankTileKeys = 2048;
+// Supports up to which every one is compared with every other, S^2 comparisons a
+// group; beyond, S / 2048 searches of twelve steps each. A call of few samples,
+// C = 3, one step / two: S = 8000 111 us / -, 10000 129 / 107, 30000 600 / 295,
+// 100000 4720 / 1004, 300000 36400 / 4320.
+constexpr int kRankDirect = 8192;
 
 __host__ __device__ __forceinline__ int fold_sp(int S) { return (S + 15) / 16 * 16; }
+// chunks of kRankTileKeys supports that are ranked by themselves first; 0: one step
+__host__ __device__ __forceinline__ int fold_chunks(int S) {
+    return S > kRankDirect ? (S + kRankTileKeys - 1) / kRankTileKeys : 0;
+}
 // tile boundaries ranked with the supports: none where a row is one tile
 __host__ __device__ __forceinline__ int fold_bounds(int tiles) { return tiles > 1 ? tiles + 1 : 0; }
 
@@ -132,6 +142,82 @@ __device__ __forceinline__ bool finite2(double2 a) {
     return __builtin_isfinite(a.x) && __builtin_isfinite(a.y);
 }
 
+// The keys of one LDS tile (the supports from t0, tn of them, then padding that
+// counts nowhere) below bin j, or of bin j and a support before `upto`: this
+// wave's sixteenth of them.
+__device__ __forceinline__ uint32_t rank_in_tile(const uint32_t* keys, int t0, int tn, uint32_t j, int upto, int wave) {
+    constexpr int kWaves = kRankThreads / 64;
+    const int share = ((tn + kWaves - 1) / kWaves + 3) & ~3;
+    const int z = min(tn, (wave + 1) * share);
+    uint32_t rank = 0;
+#pragma unroll 4
+    for (int t = wave * share; t < z; t += 4) {
+        const uint4 k = *reinterpret_cast<const uint4*>(keys + t);
+        const int at = t0 + t;
+        rank += k.x < j + (at < upto ? 1u : 0u) ? 1u : 0u;
+        rank += k.y < j + (at + 1 < upto ? 1u : 0u) ? 1u : 0u;
+        rank += k.z < j + (at + 2 < upto ? 1u : 0u) ? 1u : 0u;
+        rank += k.w < j + (at + 3 < upto ? 1u : 0u) ? 1u : 0u;
+    }
+    return rank;
+}
+
+// First step of many supports, 64 of one chunk per workgroup: their ranks in the
+// chunk, and the chunk's bins in that order.
+template <typename SRC>
+__global__ __launch_bounds__(kRankThreads) void k_fold_chunk(const SRC src) {
+    constexpr int kWaves = kRankThreads / 64;
+    __shared__ __align__(16) uint32_t keys[kRankTileKeys];
+    __shared__ uint32_t part[kWaves][64];
+    int local;
+    const qsft_fold_desc& d = src.at(blockIdx.x, local);
+    if (!d.chunk) return;
+    const int S = d.S, S64 = (S + 63) / 64 * 64;
+    const int per_c = (S64 + fold_bounds(d.tiles) + 63) / 64;
+    const int c = local / per_c, first = (local - c * per_c) * 64;
+    if (first >= S) return;                                        // tile boundaries
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, item = first + lane;
+    const uint32_t* __restrict__ J = in_global(d.J) + (size_t)c * S;
+    const int t0 = first / kRankTileKeys * kRankTileKeys, tn = min(kRankTileKeys, S - t0);
+    for (int t = threadIdx.x; t < kRankTileKeys; t += kRankThreads) keys[t] = t < tn ? J[t0 + t] : 0xFFFFFFFFu;
+    __syncthreads();
+    const uint32_t j = item < S ? keys[item - t0] : 0;
+    part[wave][lane] = rank_in_tile(keys, t0, tn, j, item, wave);
+    __syncthreads();
+    if (wave != 0 || item >= S) return;
+    uint32_t rank = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) rank += part[w][lane];
+    uint32_t* __restrict__ out = in_global(d.chunk) + (size_t)c * S;
+    out[t0 + rank] = j;
+    out[(size_t)d.C * S + item] = rank;
+}
+
+// Keys below j among the chunks (in order) of one group, those of bin j too in
+// the chunks before `own`, whose own count is left out: this wave's share of the
+// chunks, four searches at once.
+__device__ __forceinline__ uint32_t rank_in_chunks(const uint32_t* __restrict__ sorted, int S, int chunks, uint32_t j,
+                                                   int own, int wave) {
+    constexpr int kWaves = kRankThreads / 64, kAtOnce = 4;
+    uint32_t rank = 0;
+    for (int c0 = wave * kAtOnce; c0 < chunks; c0 += kWaves * kAtOnce) {
+        int pos[kAtOnce];
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) pos[i] = 0;
+        for (int step = kRankTileKeys; step > 0; step >>= 1) {
+#pragma unroll
+            for (int i = 0; i < kAtOnce; ++i) {
+                const int ch = c0 + i, t0 = ch * kRankTileKeys;
+                const int tn = ch < chunks && ch != own ? min(kRankTileKeys, S - t0) : 0;
+                if (pos[i] + step <= tn && sorted[t0 + pos[i] + step - 1] < j + (ch < own ? 1u : 0u)) pos[i] += step;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i) rank += (uint32_t)pos[i];
+    }
+    return rank;
+}
+
 // Items of one group: its S supports, then (from the next multiple of 64) the
 // tiles + 1 tile boundaries. An item's rank among the supports by (bin, s) is
 // its sorted position, where its key and strength are written; a boundary's is
@@ -158,21 +244,18 @@ __global__ __launch_bounds__(kRankThreads) void k_fold_rank(const SRC src) {
     if (bound) j = (uint32_t)(item - S64) * (uint32_t)d.tile_bins;
     const int upto = item < S64 ? item : 0;                        // equal bins count before this index
     uint32_t rank = 0;
-    for (int t0 = 0; t0 < S; t0 += kRankTileKeys) {
-        const int tn = min(kRankTileKeys, S - t0);
-        const int share = ((tn + kWaves - 1) / kWaves + 3) & ~3;
-        __syncthreads();                                           // the previous tile is consumed
-        for (int t = threadIdx.x; t < kRankTileKeys; t += kRankThreads) keys[t] = t < tn ? J[t0 + t] : 0xFFFFFFFFu;
-        __syncthreads();
-        const int z = min(tn, (wave + 1) * share);
-#pragma unroll 4
-        for (int t = wave * share; t < z; t += 4) {                // padded keys count nowhere
-            const uint4 k = *reinterpret_cast<const uint4*>(keys + t);
-            const int at = t0 + t;
-            rank += k.x < j + (at < upto ? 1u : 0u) ? 1u : 0u;
-            rank += k.y < j + (at + 1 < upto ? 1u : 0u) ? 1u : 0u;
-            rank += k.z < j + (at + 2 < upto ? 1u : 0u) ? 1u : 0u;
-            rank += k.w < j + (at + 3 < upto ? 1u : 0u) ? 1u : 0u;
+    if (d.chunk) {                                                 // (block-uniform)
+        const uint32_t* __restrict__ sorted = in_global(d.chunk) + (size_t)c * S;
+        const int own = support ? item / kRankTileKeys : -1;
+        rank = rank_in_chunks(sorted, S, fold_chunks(S), j, own, wave);
+        if (wave == 0 && support) rank += sorted[(size_t)d.C * S + item];
+    } else {
+        for (int t0 = 0; t0 < S; t0 += kRankTileKeys) {
+            const int tn = min(kRankTileKeys, S - t0);
+            __syncthreads();                                       // the previous tile is consumed
+            for (int t = threadIdx.x; t < kRankTileKeys; t += kRankThreads) keys[t] = t < tn ? J[t0 + t] : 0xFFFFFFFFu;
+            __syncthreads();
+            rank += rank_in_tile(keys, t0, tn, j, upto, wave);
         }
     }
     part[wave][lane] = rank;
@@ -678,11 +761,12 @@ bool fold_shape_ok(int q, int n, int b, int C, int P, int S, int n_pad) {
 
 // Phases (groups x P x 16-padded S bytes), sorted strengths and keys, bins (C x S), the
 // strengths that are not finite (a count and at most S), tile starts (a first-pass tile
-// holds at least q bins).
+// holds at least q bins), sorted bins of chunks and ranks in them (C x S each).
 extern "C" size_t qsft_fold_workspace_bytes(int q, int b, int C, int P, int S, int shared_d) {
     if (!fold_shape_ok(q, 1, b, C, P, S, 64)) return 0;
     return al256((size_t)(shared_d ? 1 : C) * P * fold_sp(S)) + al256((size_t)C * S * 16) +
-           al256((size_t)C * S * 8) + al256((size_t)C * S * 4) + al256(((size_t)S + 1) * 4) + al256((size_t)C * (ipow(q, b) / std::min(q, 32) + 2) * 4);
+           al256((size_t)C * S * 8) + al256((size_t)C * S * 4) + al256(((size_t)S + 1) * 4) +
+           al256((size_t)C * (ipow(q, b) / std::min(q, 32) + 2) * 4) + (fold_chunks(S) ? al256((size_t)C * S * 8) : 0);
 }
 
 extern "C" int qsft_fold_whole_rows(int q, int b, int precision) {
@@ -720,6 +804,8 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
     d.bad = reinterpret_cast<uint32_t*>(w);
     w += al256(((size_t)S + 1) * 4);
     d.start = reinterpret_cast<int32_t*>(w);
+    w += al256((size_t)C * (ipow(q, b) / std::min(q, 32) + 2) * 4);
+    if ((transform & QSFT_FOLD_CHUNKS) && fold_chunks(S)) d.chunk = reinterpret_cast<uint32_t*>(w);
     const int Q = ipow(q, b);
     if (fold_rows4_takes(q, b, S, precision)) {
         // rows of a group per workgroup: one where the launch has fewer rows than
@@ -767,7 +853,7 @@ extern "C" int qsft_fold_bind(qsft_fold_desc* h, int q, int n, int b, int C, int
         d.tile_bins = ipow(q, b - s.pass_d0[0]) * s.pass_ta[0];   // whole innermost axes: contiguous bins
         d.tiles = Q / d.tile_bins;
     }
-    d.fwd = transform != 0;
+    d.fwd = (transform & ~QSFT_FOLD_CHUNKS) != 0;
     *h = d;
     return QSFT_OK;
 }
@@ -820,6 +906,12 @@ namespace {
 
 using FoldBatch = DescBatch<qsft_fold_desc>;
 using FoldOne = DescOne<qsft_fold_desc>;
+
+template <typename SRC>
+int launch_chunks(const SRC& src, int rank_blocks, hipStream_t st) {
+    if (rank_blocks > 0) hipLaunchKernelGGL(k_fold_chunk<SRC>, dim3(rank_blocks), dim3(kRankThreads), 0, st, src);
+    return qsft_hip_status(hipGetLastError(), "qsft_fold(chunks)");
+}
 
 template <typename SRC>
 int launch_prep(const SRC& src, int phase_blocks, int rank_blocks, hipStream_t st) {
@@ -882,6 +974,15 @@ int launch_rows(int q, int b, bool fwd, const SRC& src, int blocks, int pass, in
 
 }  // namespace
 
+extern "C" int qsft_fold_chunks(const qsft_fold_desc* d, const int32_t* pre_rank, int n_inst, int rank_blocks,
+                                void* stream) {
+    if (!d || !pre_rank || n_inst < 1 || rank_blocks < 0) {
+        qsft_set_error("qsft_fold_chunks: bad arguments");
+        return QSFT_ERR_ARG;
+    }
+    return launch_chunks(FoldBatch{d, pre_rank, n_inst}, rank_blocks, (hipStream_t)stream);
+}
+
 extern "C" int qsft_fold_prep(const qsft_fold_desc* d, const int32_t* pre_phase, const int32_t* pre_rank, int n_inst,
                               int phase_blocks, int rank_blocks, void* stream) {
     if (!d || !pre_phase || !pre_rank || n_inst < 1 || phase_blocks < 0 || rank_blocks < 0) {
@@ -911,8 +1012,8 @@ extern "C" int qsft_fold_one(int q, int n, int b, int C, int P, int S, int n_pad
                              int a_precision, const int8_t* Mt, const int8_t* D, const int8_t* K, const void* a,
                              void* x, void* ws, size_t ws_bytes, void* stream) {
     FoldOne src;
-    int rc = qsft_fold_bind(&src.d, q, n, b, C, P, S, n_pad, shared_d, precision, a_precision, 0, C * P, Mt, D, K, a,
-                            x, ws, ws_bytes);
+    int rc = qsft_fold_bind(&src.d, q, n, b, C, P, S, n_pad, shared_d, precision, a_precision, QSFT_FOLD_CHUNKS, C * P,
+                            Mt, D, K, a, x, ws, ws_bytes);
     if (rc != QSFT_OK) return rc;
     int pb = 0, rb = 0;
     if (qsft_fold_blocks(&src.d, &pb, &rb) != 0) {
@@ -921,7 +1022,9 @@ extern "C" int qsft_fold_one(int q, int n, int b, int C, int P, int S, int n_pad
     }
     hipStream_t st = (hipStream_t)stream;
     const int rows4 = src.d.rpw ? b : 0;
-    rc = launch_prep(src, pb, rb, st);
+    rc = launch_prep(src, pb, 0, st);
+    if (rc == QSFT_OK && src.d.chunk) rc = launch_chunks(src, rb, st);
+    if (rc == QSFT_OK) rc = launch_prep(src, 0, rb, st);
     for (int p = 0; rc == QSFT_OK && p < src.d.n_pass; ++p)
         rc = precision == QSFT_F32 ? launch_rows<float>(q, rows4, src.d.fwd, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st)
                                    : launch_rows<double>(q, rows4, src.d.fwd, src, src.d.pass_blocks[p], p, src.d.pass_lds[p], st);

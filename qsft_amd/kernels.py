@@ -238,7 +238,8 @@ class EvalFold:
             self.ws.append(t)
             self.copies += [(t[k], it[k]) for k in t if t[k] is not it[k]]
             if lib.qsft_fold_bind(ctypes.byref(d), q, n, b, C, P, S, it["Mt"].shape[-1], shared, precision,
-                                  L.QSFT_F32 if it["a"].dtype == torch.complex64 else L.QSFT_F64, int(transform),
+                                  L.QSFT_F32 if it["a"].dtype == torch.complex64 else L.QSFT_F64,
+                                  int(transform) | L.QSFT_FOLD_CHUNKS,
                                   launch_rows, _ptr(t["Mt"]), _ptr(t["D"]), _ptr(t["K"]), _ptr(t["a"]), _ptr(it["x"]), _ptr(ws),
                                   nbytes) != L.QSFT_OK:
                 raise ValueError(f"bad eval shape {[it[k] for k in ('q', 'n', 'b', 'C', 'P', 'S')]}")
@@ -273,6 +274,7 @@ class EvalFold:
             at += len(ix)
         self.buf, self.dptr, pres, tots = pack(sd, lists, items[0]["x"].device)
         self.n = len(sd)
+        self.chunks = any(d.chunk for d in descs)
         self.prep = (pres[0], pres[1], tots[0], tots[1])
         self.rows = [(pres[2 + k], tots[2 + k], p, word, lds) for k, (p, word, _, lds) in enumerate(plan)]
 
@@ -285,7 +287,11 @@ class EvalFold:
         for to, view in self.copies:
             to.copy_(view)
         pp, pr, tp, tr = self.prep
-        L.check(lib.qsft_fold_prep(_vp(self.dptr), _vp(pp), _vp(pr), self.n, tp, tr, st), "qsft_fold_prep")
+        L.check(lib.qsft_fold_prep(_vp(self.dptr), _vp(pp), _vp(pr), self.n, tp, 0 if self.chunks else tr, st),
+                "qsft_fold_prep")
+        if self.chunks:
+            L.check(lib.qsft_fold_chunks(_vp(self.dptr), _vp(pr), self.n, tr, st), "qsft_fold_chunks")
+            L.check(lib.qsft_fold_prep(_vp(self.dptr), _vp(pp), _vp(pr), self.n, 0, tr, st), "qsft_fold_prep")
         between()
         for pre, tot, p, word, lds in self.rows:
             L.check(lib.qsft_fold_rows(_vp(self.dptr), _vp(pre), self.n, tot, p, word, lds, st), "qsft_fold_rows")

@@ -312,3 +312,46 @@ def test_fold_reads_views_that_start_anywhere_at_every_launch(q, b):
             views[k].copy_(it[k])
         ev.launch()
         assert torch.equal(torch.view_as_real(views["x"]), torch.view_as_real(x))
+
+
+@pytest.mark.parametrize("q,b,S", [(2, 3, 8193), (2, 1, 12289), (3, 7, 8200), (4, 4, 10240), (4, 6, 16385), (20, 4, 8250),
+                                   (2, 16, 9000), (7, 5, 8193), (4, 7, 67000)])
+def test_fold_ranks_many_supports_in_two_steps(q, b, S):
+    """More than 8192 supports are ranked within chunks of 2048 and by a search in the others: the bits of the one-step
+    ranking, alone and in a launch with few supports, for bins of many supports of all chunks and for several tiles."""
+    print(f"fold two-step ranks q={q} b={b} S={S}", flush=True)
+    x = _inputs(q, 17, b, S, 2, 3, seed=S)
+    few = _inputs(q, 17, b, 70, 2, 3, seed=1)
+    it, small = _item(q, 17, b, *x, "fp64"), _item(q, 17, b, *few, "fp64")
+    ev = K.EvalFold([small, it], L.QSFT_F64)
+    assert ev.chunks
+    ev.launch()
+    got, got_small = it["x"].clone(), small["x"].clone()
+    if S * q ** b < 10 ** 7:
+        ref = _direct(q, b, *x)
+        assert np.max(np.abs(got.cpu().numpy() - ref)) <= 1e-12 * np.max(np.abs(ref))
+    nbytes = L.lib.qsft_fold_workspace_bytes(q, b, 2, 3, S, 0)
+    for one_step in (True, False):
+        it["x"].fill_(0)
+        if one_step:
+            d = L.FoldDesc()
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=it["x"].device)
+            L.check(L.lib.qsft_fold_bind(ctypes.byref(d), q, 17, b, 2, 3, S, it["Mt"].shape[-1], 0, L.QSFT_F64, L.QSFT_F64,
+                                         0, 6, *(it[k].data_ptr() for k in ("Mt", "D", "K", "a", "x")), ws.data_ptr(),
+                                         nbytes))
+            assert not d.chunk
+            pb, rb = ctypes.c_int(), ctypes.c_int()
+            assert L.lib.qsft_fold_blocks(ctypes.byref(d), ctypes.byref(pb), ctypes.byref(rb)) == 0
+            buf, dptr, pres, tots = K.pack([d], [[pb.value], [rb.value]] + [[d.pass_blocks[p]] for p in range(d.n_pass)],
+                                           it["x"].device)
+            st = K.stream_handle()
+            L.check(L.lib.qsft_fold_prep(dptr, pres[0], pres[1], 1, tots[0], tots[1], st))
+            for p in range(d.n_pass):
+                L.check(L.lib.qsft_fold_rows(dptr, pres[2 + p], 1, tots[2 + p], p,
+                                             L.QSFT_F64 | (q << 8) | ((b << 16) if d.rpw else 0), d.pass_lds[p], st))
+            torch.cuda.synchronize()
+        else:
+            K.eval_fold(q, 17, b, *(it[k] for k in ("Mt", "D", "K", "a", "x")))
+        assert torch.equal(torch.view_as_real(it["x"]), torch.view_as_real(got))
+    K.EvalFold([small], L.QSFT_F64).launch()
+    assert torch.equal(torch.view_as_real(small["x"]), torch.view_as_real(got_small))

@@ -236,3 +236,19 @@ def test_tune_leaves_shapes_with_whole_rows_alone():
              E.random_spec(3, 12, 20, 10, 1, 1, 20.0, rng=rng)]
     SV.Server(hbm_budget=1 << 40).tune(specs)
     assert [K.dft_schedule(sp.q, sp.b, L.QSFT_F32)[1] for sp in specs] == [False, False, True]
+
+
+def test_a_request_of_many_supports_equals_the_engine():
+    """More than 8192 supports (ranked in two steps) beside few, in the native runtime and in the engine: the same rows."""
+    print("runtime vs engine, many supports", flush=True)
+    rng = np.random.default_rng(13)
+    specs = [E.random_spec(4, 40, 8300, 7, 2, 1, None, rng=rng, method="identity"),
+             E.random_spec(4, 12, 100, 4, 3, 1, None, rng=rng, method="identity")]
+    sb = SV.ServedBatch(specs, torch.device("cuda", torch.cuda.current_device()))
+    sb.launch(seed_offset=0)
+    sb.wait()
+    ref = E.Batch(specs, precision="fp32")
+    ref.launch(seed_offset=0)
+    for g, (k, v, order, _) in zip(sb.results(), ref.results()):
+        assert len(k) > 0 and _rows(g.k, g.values)[0] == _rows(k, v)[0]
+        assert np.array_equal(_bits(g.values), _bits(v)) and np.array_equal(np.asarray(g.order), order)
