@@ -861,74 +861,9 @@ __device__ __forceinline__ uint64_t scan_marks(const qsft_peel_desc& d, int it, 
 }
 
 // Hash registration of a wave's ns buffered singletons, one lane each, so the
-// atomics of up to 64 registrations are in flight together. Every lane of the
-// wave takes part (ballots).
-template <int CAP>
-__device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int it, int ns,
-                                                    const SingletonBuf<CAP>& sb, int lane) {
-    uint32_t* __restrict__ ctr = in_global(d.ctr);
-    const int CQ = d.C * d.Q;
-    int slot = -1;
-    bool claimed = false;                                      // this lane's k took a new slot
-    bool newball = false;
-    int t = 0;
-    uint64_t tm = 0;
-    double2 rho = make_double2(0.0, 0.0);
-    if (lane < ns) {
-        t = sb.t[lane];
-        rho = sb.rho[lane];
-        const uint64_t hv = sb.h[lane];
-        const uint64_t tg = hv | 1ull;
-        const uint32_t mask = (1u << d.hcap_log2) - 1u;
-        uint32_t pos = (uint32_t)(hv >> 32) & mask;
-        for (uint32_t probe = 0; probe <= mask; ++probe) {
-            const unsigned long long old = atomicCAS((unsigned long long*)&in_global(d.tag)[pos], 0ull, (unsigned long long)tg);
-            if (old == 0ull || old == tg) {
-                slot = (int)pos;
-                claimed = old == 0ull;
-                break;
-            }
-            pos = (pos + 1) & mask;
-        }
-        if (slot < 0) {
-            atomicOr(&ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_TABLE_FULL);
-        } else {
-            in_global(d.slot_bin)[t] = slot;
-            in_global(d.sstamp)[t] = it + 1;                                 // kernel B peels only registered bins
-            tm = ((uint64_t)(it + 1) << 32) | (uint32_t)t;
-            atomicMin((unsigned long long*)&in_global(d.owner)[slot], (unsigned long long)tm);
-            const unsigned long long prev = atomicMax((unsigned long long*)&in_global(d.last)[slot], (unsigned long long)tm);
-            newball = (prev >> 32) != (unsigned long long)(it + 1);
-        }
-    }
-    const uint64_t nb_mask = __ballot(newball);
-    const uint64_t ok_mask = __ballot(slot >= 0);
-    const uint64_t cl_mask = __ballot(claimed);
-    uint32_t rbase = 0, lbase = 0;
-    if (lane == 0) {
-        if (nb_mask) atomicAdd(&ctr[it * QSFT_CTR_ITER_STRIDE + 2], (uint32_t)__popcll(nb_mask));
-        if (ok_mask) rbase = atomicAdd(&ctr[kCtrTaken], (uint32_t)__popcll(ok_mask));
-        if (cl_mask) lbase = atomicAdd(&ctr[kCtrTaken + 1], (uint32_t)__popcll(cl_mask));
-    }
-    rbase = __shfl(rbase, 0);
-    lbase = __shfl(lbase, 0);
-    if (claimed) in_global(d.live)[lbase + (uint32_t)__popcll(cl_mask & ((1ull << lane) - 1ull))] = (uint32_t)slot;
-    if (slot >= 0) {
-        const uint32_t rix = rbase + (uint32_t)__popcll(ok_mask & ((1ull << lane) - 1ull));
-        if ((uint64_t)rix >= (uint64_t)d.max_iter * (uint64_t)CQ) {   // cannot happen: one record per bin per pass
-            atomicOr(&ctr[QSFT_CTR_ERROR], (uint32_t)QSFT_DEVERR_BAD_SHAPE);
-        } else {
-            in_global(d.rec_time)[rix] = tm;
-            in_global(d.rec_rho)[2 * (size_t)rix] = rho.x;
-            in_global(d.rec_rho)[2 * (size_t)rix + 1] = rho.y;
-            in_global(d.rec_next)[rix] = atomicExch(&in_global(d.head)[slot], rix);
-            atomicAdd(&in_global(d.count)[slot], 1u);
-        }
-    }
-}
-
-// The same in two parts, for waves that end together (finish_block): first the
+// atomics of up to 64 registrations are in flight together, in two parts: the
 // slots; then, with the first record and list position of the wave, the records.
+// Every lane of the wave takes part (ballots).
 struct Claim {
     int slot, t;
     bool claimed;                                              // this lane's k took a new slot
@@ -999,6 +934,21 @@ __device__ __forceinline__ void write_records(const qsft_peel_desc& d, int it, c
 __device__ __forceinline__ uint64_t take_records(uint32_t* ctr, uint32_t records, uint32_t slots) {
     if (records == 0 && slots == 0) return 0;
     return atomicAdd((unsigned long long*)&ctr[kCtrTaken], (unsigned long long)records | ((unsigned long long)slots << 32));
+}
+
+// Both parts for one wave by itself.
+template <int CAP>
+__device__ __forceinline__ void register_singletons(const qsft_peel_desc& d, int it, int ns,
+                                                    const SingletonBuf<CAP>& sb, int lane) {
+    uint32_t* __restrict__ ctr = in_global(d.ctr);
+    const Claim c = claim_slots(d, it, ns, sb, lane);
+    uint64_t base = 0;
+    if (lane == 0) {
+        if (c.nb_mask) atomicAdd(&ctr[it * QSFT_CTR_ITER_STRIDE + 2], (uint32_t)__popcll(c.nb_mask));
+        base = take_records(ctr, (uint32_t)__popcll(c.ok_mask), (uint32_t)__popcll(c.cl_mask));
+    }
+    base = __shfl((unsigned long long)base, 0);
+    write_records(d, it, c, (uint32_t)base, (uint32_t)(base >> 32), lane);
 }
 
 // The pass counters of a block: singletons and multitons (adjacent words, one
