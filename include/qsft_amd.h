@@ -125,7 +125,7 @@ int qsft_eval_mfma(const qsft_eval_mfma_desc* dev_descs, const int32_t* dev_pre_
  * a_s w^{<d_p, k_s>} summed into their bins. qsft_fold_prep forms the phases
  * <d_p, k_s> and the bins by an int8 MFMA contraction (exact int32, mod q) and
  * sorts the supports of each group by bin; qsft_fold_rows folds the terms of each
- * row into LDS (FP64 sums in ascending s: the same bits on every run) and
+ * row into LDS (FP64 sums in one order: the same bits on every run) and
  * transforms them, n_pass launches. Replaces the same reference code as
  * qsft_eval_cosets. */
 typedef struct qsft_fold_desc {
@@ -524,8 +524,9 @@ typedef struct qsft_request {
     int32_t _pad0;
     double cutoff;              /* zeroton threshold per row (reference: 1e-9 + 1.5 noise_sd^2 / q^b) */
     double sigma;               /* transform-domain noise sd per bin (noise_sd / sqrt(q^b)); 0: none */
-    double amax;                /* max |a_s| (> 0), or 0: computed from the strengths when the   *
-                                 * request is packed (qsft_batch_pack_input)                    */
+    double amax;                /* 0: strengths that are all zero or not finite are refused when *
+                                 * the request is packed (qsft_batch_pack_input), which then    *
+                                 * stores max |a_s| here; > 0: taken unchecked. No other use    */
     uint64_t seed;              /* Philox key of the request's noise                            */
 } qsft_request;
 

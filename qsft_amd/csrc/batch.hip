@@ -477,8 +477,8 @@ extern "C" int qsft_batch_pack_input(void* h, int i, const int8_t* M, const int8
     // through references would be reloaded on every store
     const int n = r.n, b = r.b, C = r.C, P = l.P, S = r.S, np = l.n_pad;
     if (!(r.amax > 0.0)) {
-        // amax 0: max |a_s| from the strengths, as sqrt(max(re^2 + im^2)) with
-        // every product and sum rounded (no fused multiply-add)
+        // amax 0: the strengths are checked, by max |a_s| = sqrt(max(re^2 + im^2))
+        // with every product and sum rounded (no fused multiply-add)
         double m2 = 0.0;
         bool nan = false;
         for (int s = 0; s < S; ++s) {

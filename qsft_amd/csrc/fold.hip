@@ -18,8 +18,8 @@
 //     b products with M_c^T.
 //   * k_fold_rank: per group the supports sorted by (bin, s), each at its rank,
 //     counted against LDS tiles of the bins: the terms of a bin are adjacent
-//     and always summed in ascending s, so the sums have the same bits on
-//     every run. Also the first sorted position of every tile of the row
+//     and always summed in one order (a scan over blocks of 64 sorted
+//     positions), so the sums have the same bits on every run. Also the first sorted position of every tile of the row
 //     kernel. Many supports are ranked in two steps: within chunks of 2048
 //     (k_fold_chunk), then by a binary search in every other chunk.
 //   * k_fold_pass / k_fold4_rows: a workgroup clears a tile of bins of one row
@@ -32,11 +32,15 @@
 // swapped on the way in and out, so it shares the forward radix kernels: the
 // fold stores swapped terms and the last pass swaps back.
 //
-// Bound: HBM. A row is written once (8 or 16 bytes a sample) where it fits one
-// tile; nothing else of that order is read. Measured against the sums over
-// every support that these kernels replaced: one q = 4, n = 50, S = 1000,
-// b = 6, 306-row signal in FP64 463 -> 23 us a call, 64 of them in FP32 in one
-// launch 0.91 -> 0.29 ms; q = 20, S = 2000, b = 3, FP32 570 -> 32 us.
+// HBM is all that it cannot do without: a row is written once (8 or 16 bytes a
+// sample) where it fits one tile; nothing else of that order is read. One
+// instance is bound by three dependent launches, many by the VALU (see
+// k_fold4_rows). Measured against the sums over every support that these
+// kernels replaced: one q = 4, n = 50, S = 1000, b = 6, 306-row signal in FP64
+// 463 -> 23 us a call, 64 of them in FP32 in one launch 0.91 -> 0.26 ms; q = 20,
+// S = 2000, b = 3, FP32 570 -> 27 us. FP32 against FP64, of the samples' size:
+// 6e-8 to 1.3e-7 for every S (the direct sums 5e-8 at S = 10, 1e-7 at 300, 3e-7
+// at 5000; generic radices up to 2e-7).
 #include <algorithm>
 
 #include "dft_tile.h"
@@ -561,9 +565,9 @@ __global__ __launch_bounds__(TH) void k_fold_pass(const SRC src, int pass, int l
 // then the others upwards, so that the stores are 128-byte segments), and x
 // receives that.
 // 64 instances of q = 4, S = 1000, b = 6, P = 102 in FP32: 0.227 ms for the
-// samples and 0.268 ms for k_dft4_rows as two launches, 0.214 ms in one (3.0
-// TB/s of writes: bound by the chain of exchanges at four waves per SIMD, all
-// that 34 KiB of LDS a row allow).
+// samples and 0.268 ms for k_dft4_rows as two launches, 0.23 ms in one (2.8
+// TB/s of writes). Bound by its VALU, 70 % busy, between the chain of exchanges
+// (LDS 43 %) at four waves per SIMD, all that 34 KiB of LDS a row allow.
 typedef float gf2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void store_c2(QSFT_GLOBAL float2* p, float2 v) {
     *reinterpret_cast<QSFT_GLOBAL gf2*>(p) = gf2{v.x, v.y};
@@ -730,7 +734,7 @@ namespace {
 
 size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// rows that k_fold4_rows takes: q = 4, b = 4..6, and in FP32 b = 7 (139 KiB of LDS)
+// rows that k_fold4_rows takes: q = 4, b = 4..6, and in FP32 b = 7 (144 KiB of LDS)
 bool fold_rows4(int q, int b, int precision) { return q == 4 && b >= 4 && b <= (precision == QSFT_F32 ? 7 : 6); }
 
 // Whether the whole-row kernel takes an instance of such rows. Its workgroups of

@@ -87,7 +87,7 @@ def request_struct(sp, max_iter=15):
     else:
         raise ValueError(f"detection method {sp.method!r}")
     Q = sp.q ** sp.b
-    # amax 0: the runtime takes max |a_s| from the strengths while it packs them
+    # amax 0: the runtime refuses strengths that are all zero or not finite while it packs them
     return L.Request(sp.q, sp.n, sp.b, sp.C, sp.R, sp.strengths.size, method, 0, float(sp.threshold()),
                      float(sp.noise_sd) / Q ** 0.5 if sp.noise_sd > 0 else 0.0, 0.0,
                      int(sp.seed) & 0xFFFFFFFFFFFFFFFF)
